@@ -957,6 +957,9 @@ static size_t bwd_slot_floats(int S, int large) {
                                     : (size_t)8 * kb::kb_slot_ld(S, large);
 }
 
+// rows of level d that the backward solves (level 0: one per class)
+static int level_rows(const kb_plan* p, int d) { return d == 0 ? p->n_cls0 : p->level_ptr[d + 1] - p->level_ptr[d]; }
+
 static int ensure_backward_work(kb_plan* p, int use_col) {
   const int S = p->S, C = p->C;
   // resident workgroups of the backward row kernel: its per-level grid
@@ -976,6 +979,12 @@ static int ensure_backward_work(kb_plan* p, int use_col) {
   const char* lv = getenv("KB_BWD_LARGE");
   const int large = (lv && lv[0] == '0') ? 0 : (lv && lv[0] == '2') ? 2 : 1;
   int nb_max = std::max(1, n_cu * kb::bwd_blocks_per_cu(S, use_col, variant, large));
+  // short rows: at most four workgroups per CU (each adds a bucket slot to read
+  // back), and never more than the widest level has rows
+  nb_max = std::min(nb_max, 4 * n_cu);
+  int widest = 1;
+  for (int d = 0; d < p->n_levels; ++d) widest = std::max(widest, level_rows(p, d));
+  nb_max = std::min(nb_max, widest);
   // KB_BWD_GRID=n caps the persistent grid at n workgroups (tests: every
   // workgroup then walks many rows of a level)
   const char* gv = getenv("KB_BWD_GRID");
@@ -1159,7 +1168,7 @@ static int backward_level(kb_plan* p, kb::BwdParams& B, int d, int first, int n,
   // level 0 (rows without splits) runs by class: one adjoint solve per class of identical rows
   B.class_mode = d == 0 ? 1 : 0;
   if (d == 0) kb::launch_bwd_level0_prep(B, p->level_ptr[1], p->n_cls0, st);
-  B.variant = p->b_variant == 1 ? ((S > 1024 || n < 2 * grid) ? 2 : 0) : p->b_variant;
+  B.variant = p->b_variant == 1 && S > 1024 ? 2 : p->b_variant;
   kb::launch_bwd_wave(B, first, n, std::min(n, grid), poff, st);
   if (p->prof) KB_HIP(hipEventRecord(p->ev_bwd[2 * d + 1], st));
   return 0;
@@ -1206,8 +1215,6 @@ static int backward_finish(kb_plan* p, const kb_backward_io* io, int n_partials,
   KB_HIP(hipGetLastError());
   return 0;
 }
-
-static int level_rows(const kb_plan* p, int d) { return d == 0 ? p->n_cls0 : p->level_ptr[d + 1] - p->level_ptr[d]; }
 
 extern "C" int kb_backward(kb_plan* p, const kb_backward_io* io, void* stream) {
   hipStream_t st = (hipStream_t)stream;

@@ -1162,6 +1162,9 @@ void launch_bwd_wave(const BwdParams& P, int first, int W, int nb, int poff, hip
   KB_BWD_CASE(64, 2)
   KB_BWD_CASE(128, 2)
   KB_BWD_CASE(256, 2)
+  if (P.variant != 0) {
+    KB_BWD_CASE(512, 2)
+  }
   KB_BWD_CASE(256, 4)
   KB_BWD_CASE(512, 4)
   KB_BWD_CASE(1024, 4)
@@ -1186,6 +1189,9 @@ int bwd_blocks_per_cu(int S, int use_col, int variant, int large) {
   KB_BWD_OCC(64, 2)
   KB_BWD_OCC(128, 2)
   KB_BWD_OCC(256, 2)
+  if (variant != 0) {
+    KB_BWD_OCC(512, 2)
+  }
   KB_BWD_OCC(256, 4)
   KB_BWD_OCC(512, 4)
   KB_BWD_OCC(1024, 4)
@@ -1245,8 +1251,12 @@ __global__ void bwd_reduce_stage1(const float* contrib, int C, int S, size_t slo
   const int a = j / S;
   const size_t off = (size_t)a * ld + (j - a * S);
   const int r0 = chunk * RED_CHUNK, r1 = min(C, r0 + RED_CHUNK);
+  float x[RED_CHUNK];
+#pragma unroll
+  for (int u = 0; u < RED_CHUNK; ++u) x[u] = r0 + u < r1 ? contrib[(size_t)(r0 + u) * slot_stride + off] : 0.0f;
   double acc = 0.0;
-  for (int r = r0; r < r1; ++r) acc += (double)contrib[(size_t)r * slot_stride + off];
+#pragma unroll
+  for (int u = 0; u < RED_CHUNK; ++u) acc += (double)x[u];
   partial[(size_t)chunk * 8 * S + j] = acc;
 }
 
@@ -1259,7 +1269,15 @@ __global__ void bwd_reduce_stage2(const double* partial, int n_chunks, int S, co
   const int a = j / S, s = j - a * S;
   const size_t src = (size_t)a * S + pre[s];
   double acc = 0.0;
-  for (int c = 0; c < n_chunks; ++c) acc += partial[(size_t)c * 8 * S + src];
+  int c = 0;
+  for (; c + 8 <= n_chunks; c += 8) {  // eight loads in flight, added in chunk order
+    double x[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) x[u] = partial[(size_t)(c + u) * 8 * S + src];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc += x[u];
+  }
+  for (; c < n_chunks; ++c) acc += partial[(size_t)c * 8 * S + src];
   out[j] = acc;
 }
 

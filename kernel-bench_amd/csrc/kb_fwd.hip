@@ -629,12 +629,18 @@ void launch_fwd_wave(const FwdParams& P, int first, int W, hipStream_t st) {
   if (P.wide == 1) {  // fewer, wider threads per row (tuning knob)
     KB_FWD_CASE(256, 8, fwd_row_kernel)
   }
-  if (P.wide == 2 || (P.wide == 0 && W < P.narrow_below)) {  // more, narrower threads per row
+  // 1024 x 2: on every level by the knob; by default on rows of 1025..2048
+  // states where few rows share a CU (narrow_below, forward_setup).  Shorter
+  // rows never take it: half or more of its wavefronts would carry padding.
+  if (P.wide == 2 || (P.wide == 0 && S > 1024 && W < P.narrow_below)) {
     KB_FWD_CASE(1024, 2, fwd_row_kernel)
   }
   KB_FWD_CASE(64, 2, fwd_row_kernel)
   KB_FWD_CASE(128, 2, fwd_row_kernel)
   KB_FWD_CASE(256, 2, fwd_row_kernel)
+  if (P.wide == 0 && W < P.narrow_below) {
+    KB_FWD_CASE(512, 2, fwd_row_kernel)
+  }
   KB_FWD_CASE(256, 4, fwd_row_kernel)
   KB_FWD_CASE(512, 4, fwd_row_kernel)
   KB_FWD_CASE(1024, 4, fwd_row_kernel)
