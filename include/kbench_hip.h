@@ -229,7 +229,7 @@ typedef struct kb_e_adjoint_io {
   const double* q_extra;     /* [S] added to q, or null */
   double* w_out;             /* [S] the E adjoint, or null */
   double* g_out;             /* [5,S] cotangents of (pS, pD, pL, max_coupling, col) per state */
-  double* work;              /* [KB_E_ADJOINT_WORK_VECTORS, S] scratch */
+  double* work;              /* [KB_E_ADJOINT_WORK_VECTORS, S] scratch (this library's kernels leave it alone) */
   int32_t* status;           /* [2] device: iterations, failure flag */
 } kb_e_adjoint_io;
 

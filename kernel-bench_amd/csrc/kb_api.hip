@@ -66,7 +66,7 @@ int alloc(T** dst, size_t n) {
 
 struct kb_plan {
   int S = 0, C = 0, n_fam = 0, n_waves = 0;
-  int n_jump = 0, n_tlevels = 0, n_blevels = 0;
+  int n_jump = 0, n_blevels = 0;
   std::vector<int> wave_start, wave_size, wave_split;
   // dependency levels: rows grouped by clade-DAG depth (0 = no splits); a row
   // only reads its own children, so level order is a valid schedule
@@ -103,7 +103,6 @@ struct kb_plan {
   // device tables
   int* d_parent = nullptr; int* d_c1 = nullptr; int* d_c2 = nullptr; int* d_jump = nullptr;
   int* d_blevel_ptr = nullptr; int* d_blevel_node = nullptr;
-  int* d_tlevel_ptr = nullptr; int* d_tlevel_node = nullptr;
   int* d_sub_start = nullptr; int* d_sub_end = nullptr;
   int* d_item = nullptr; int* d_leaf = nullptr; int* d_roots = nullptr;
   int* d_split_ptr = nullptr; int* d_split_l = nullptr; int* d_split_r = nullptr; float* d_split_lsp = nullptr;
@@ -121,8 +120,6 @@ struct kb_plan {
   int* d_pflag = nullptr; int* d_endpos = nullptr; int* d_tin = nullptr; int* d_euler = nullptr;
   int* d_post = nullptr;
   int* d_om_tab = nullptr;  // owner-major position tables of the large backward kernel (2048 < S <= 8192)
-  int* d_euler_col = nullptr; int* d_tin_col = nullptr;  // the Euler tour in column terms
-  kb::TreeScanDev tscan() const { return kb::TreeScanDev{S, d_pre, d_endpos, d_euler_col, d_tin_col}; }
   double* E64 = nullptr; int* n_e_iter = nullptr; double* loss_terms = nullptr; double* loss64 = nullptr;
   int* d_root_index = nullptr;
   int64_t n_splits = 0;
@@ -132,7 +129,7 @@ struct kb_plan {
   float* b_rhsc = nullptr;
   unsigned char* b_m_mask = nullptr;
   unsigned char* b_cls_active = nullptr;
-  float* b_contrib = nullptr; double* b_partial = nullptr; double* b_acc = nullptr; double* b_work = nullptr;
+  float* b_contrib = nullptr; double* b_partial = nullptr; double* b_acc = nullptr;
   float* b_om_const = nullptr;  // owner-major constants of the large backward kernel
   int* b_status = nullptr;
   int* h_status = nullptr;  // pinned host copy of b_status (kb_backward_stats)
@@ -257,12 +254,6 @@ int kb_plan_create(const kb_layout* L, kb_plan** out) {
     }
   int maxd = 0;
   for (int s = 0; s < S; ++s) maxd = std::max(maxd, depth[s]);
-  std::vector<int> tptr(maxd + 2, 0), tnode;
-  for (int d = 0; d <= maxd; ++d) {
-    for (int s = 0; s < S; ++s)
-      if (depth[s] == d) tnode.push_back(s);
-    tptr[d + 1] = (int)tnode.size();
-  }
   std::vector<int> bptr(1, 0), bnode;
   for (int d = maxd; d >= 0; --d) {
     bool any = false;
@@ -334,7 +325,6 @@ int kb_plan_create(const kb_layout* L, kb_plan** out) {
     }
   }
   p->n_jump = n_jump;
-  p->n_tlevels = maxd + 1;
   p->n_blevels = (int)bptr.size() - 1;
 
   // ---- rows, splits, waves (int64 values range-checked before narrowing)
@@ -538,8 +528,6 @@ int kb_plan_create(const kb_layout* L, kb_plan** out) {
   rc |= upload(&p->d_jump, jump);
   rc |= upload(&p->d_blevel_ptr, bptr);
   rc |= upload(&p->d_blevel_node, bnode);
-  rc |= upload(&p->d_tlevel_ptr, tptr);
-  rc |= upload(&p->d_tlevel_node, tnode);
   rc |= upload(&p->d_sub_start, ss);
   rc |= upload(&p->d_sub_end, se);
   rc |= upload(&p->d_item, item);
@@ -743,13 +731,6 @@ int kb_plan_create(const kb_layout* L, kb_plan** out) {
       rc |= upload(&p->d_om_tab, om);
     }
   }
-  {
-    std::vector<int> ecol(euler.size()), tcol(S);
-    for (size_t q = 0; q < euler.size(); ++q) ecol[q] = (pcol[euler[q] >> 1] << 1) | (euler[q] & 1);
-    for (int s = 0; s < S; ++s) tcol[s] = tin[pre[s]];
-    rc |= upload(&p->d_euler_col, ecol);
-    rc |= upload(&p->d_tin_col, tcol);
-  }
   rc |= alloc(&p->c_Ebar, S);
   rc |= alloc(&p->c_E, S);
   rc |= alloc(&p->c_mt, S);
@@ -770,7 +751,7 @@ int kb_plan_create(const kb_layout* L, kb_plan** out) {
   rc |= alloc(&p->loss_terms, std::max(1, L->n_fam));
   rc |= alloc(&p->loss64, 1);
   for (void* ptr : {(void*)p->d_parent, (void*)p->d_c1, (void*)p->d_c2, (void*)p->d_jump, (void*)p->d_blevel_ptr,
-                    (void*)p->d_blevel_node, (void*)p->d_tlevel_ptr, (void*)p->d_tlevel_node, (void*)p->d_sub_start,
+                    (void*)p->d_blevel_node, (void*)p->d_sub_start,
                     (void*)p->d_sub_end, (void*)p->d_item, (void*)p->d_leaf, (void*)p->d_roots, (void*)p->d_split_ptr,
                     (void*)p->d_split_l, (void*)p->d_split_r, (void*)p->d_split_lsp, (void*)p->d_split_parent,
                     (void*)p->d_child_ptr, (void*)p->d_child_in, (void*)p->d_bslot, (void*)p->d_unnorm, (void*)p->c_DL, (void*)p->c_SL1,
@@ -782,7 +763,7 @@ int kb_plan_create(const kb_layout* L, kb_plan** out) {
                     (void*)p->d_dup_rows, (void*)p->d_cls_ptr, (void*)p->d_cls_rows, (void*)p->d_ck_ptr, (void*)p->d_cls_ck_ptr, (void*)p->d_rep_of, (void*)p->d_m_side_ptr, (void*)p->d_m_side, (void*)p->d_m_root,
                     (void*)p->d_dts,
                     (void*)p->d_c1pos, (void*)p->d_c2pos, (void*)p->d_ppos, (void*)p->d_pflag, (void*)p->d_endpos,
-                    (void*)p->d_tin, (void*)p->d_euler, (void*)p->d_post, (void*)p->d_om_tab, (void*)p->d_euler_col, (void*)p->d_tin_col, (void*)p->c_Ebar, (void*)p->c_E, (void*)p->c_mt,
+                    (void*)p->d_tin, (void*)p->d_euler, (void*)p->d_post, (void*)p->d_om_tab, (void*)p->c_Ebar, (void*)p->c_E, (void*)p->c_mt,
                     (void*)p->c_col})
     p->owned.push_back(ptr);
   if (rc) {
@@ -820,12 +801,8 @@ static int forward_setup(kb_plan* p, const kb_forward_io* io, hipStream_t st, kb
 
   kb::EStepParams E{};
   E.tr = p->tree();
-  E.ts = p->tscan();
   E.pd = p->predev();
   E.S = S;
-  E.n_tlevels = p->n_tlevels;
-  E.tlevel_ptr = p->d_tlevel_ptr;
-  E.tlevel_node = p->d_tlevel_node;
   E.theta = io->theta;
   E.statewise = io->statewise;
   E.col_weights = io->col_weights;
@@ -1031,7 +1008,6 @@ static int ensure_backward_work(kb_plan* p, int use_col) {
   rc |= alloc(&p->b_contrib, (size_t)2 * std::max(1, p->b_n_partials) * p->b_slot);
   rc |= alloc(&p->b_partial, (size_t)kb::reduce_chunks(2 * std::max(1, p->b_n_partials)) * 8 * S);
   rc |= alloc(&p->b_acc, (size_t)8 * S);
-  rc |= alloc(&p->b_work, (size_t)kb::epilogue_work_vectors() * S);
   rc |= alloc(&p->b_status, 2);
   rc |= alloc(&p->b_DL, S);
   rc |= alloc(&p->b_SL1, S);
@@ -1045,7 +1021,7 @@ static int ensure_backward_work(kb_plan* p, int use_col) {
   for (void* ptr : {(void*)p->b_Ebar, (void*)p->b_E, (void*)p->b_mt, (void*)p->b_col,
                     (void*)p->b_staging, (void*)p->b_split_on, (void*)p->b_mask, (void*)p->b_contrib,
                     (void*)p->b_rhs0, (void*)p->b_rhsc, (void*)p->b_cls_active, (void*)p->b_ck_any, (void*)p->b_m_mask,
-                    (void*)p->b_partial, (void*)p->b_acc, (void*)p->b_work, (void*)p->b_status, (void*)p->b_DL,
+                    (void*)p->b_partial, (void*)p->b_acc, (void*)p->b_status, (void*)p->b_DL,
                     (void*)p->b_SL1, (void*)p->b_SL2, (void*)p->b_pS, (void*)p->b_pD})
     p->owned.push_back(ptr);
   return rc ? KB_ERR_HIP : 0;
@@ -1185,12 +1161,8 @@ static int backward_finish(kb_plan* p, const kb_backward_io* io, int n_partials,
 
   kb::EpiParams X{};
   X.tr = p->tree();
-  X.ts = p->tscan();
   X.pd = p->predev();
   X.S = S;
-  X.n_tlevels = p->n_tlevels;
-  X.tlevel_ptr = p->d_tlevel_ptr;
-  X.tlevel_node = p->d_tlevel_node;
   X.E = io->E;
   X.log_pS = io->log_pS;
   X.log_pD = io->log_pD;
@@ -1209,7 +1181,6 @@ static int backward_finish(kb_plan* p, const kb_backward_io* io, int n_partials,
   X.breakdown = io->bicgstab_breakdown_tol;
   X.grad_theta = io->grad_theta;
   X.grad_col = io->grad_col;
-  X.work = p->b_work;
   X.status = p->b_status;
   kb::launch_epilogue(X, st);
   KB_HIP(hipGetLastError());
@@ -1295,16 +1266,10 @@ int kb_e_adjoint(kb_plan* p, const kb_e_adjoint_io* io, void* stream) {
   if (io->bicgstab_max_iter < 1) return set_error(KB_ERR_ARG, "max_iter must be at least 1");
   if (!(io->bicgstab_tol > 0.0)) return set_error(KB_ERR_ARG, "tol must be positive");
   if (!(io->bicgstab_breakdown_tol > 0.0)) return set_error(KB_ERR_ARG, "breakdown_tol must be positive");
-  if (kb::epilogue_work_vectors() > KB_E_ADJOINT_WORK_VECTORS)
-    return set_error(KB_ERR_HIP, "the epilogue needs %d work vectors", kb::epilogue_work_vectors());
   kb::EpiParams X{};
   X.tr = p->tree();
-  X.ts = p->tscan();
   X.pd = p->predev();
   X.S = p->S;
-  X.n_tlevels = p->n_tlevels;
-  X.tlevel_ptr = p->d_tlevel_ptr;
-  X.tlevel_node = p->d_tlevel_node;
   X.E = io->E;
   X.log_pS = io->log_pS;
   X.log_pD = io->log_pD;
@@ -1319,7 +1284,6 @@ int kb_e_adjoint(kb_plan* p, const kb_e_adjoint_io* io, void* stream) {
   X.max_iter = io->bicgstab_max_iter;
   X.tol = io->bicgstab_tol;
   X.breakdown = io->bicgstab_breakdown_tol;
-  X.work = io->work;
   X.status = io->status;
   X.q_extra = io->q_extra;
   X.no_norm = io->with_norm ? 0 : 1;

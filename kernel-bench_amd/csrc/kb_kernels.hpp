@@ -16,12 +16,8 @@ int set_error(int code, const char* fmt, ...);
 // ----------------------------------------------------------------------------
 struct EStepParams {
   TreeDev tr;
-  TreeScanDev ts;
-  PreDev pd;                  // preorder tables (register-resident kernel)
+  PreDev pd;                  // preorder tables
   int S;
-  int n_tlevels;              // depth levels, root first
-  const int* tlevel_ptr;      // [n_tlevels + 1]
-  const int* tlevel_node;     // [S]
   const int* pre;             // [S] column -> preorder position (layout of the c_* / lin_* constants)
   const float* theta;         // [S,3] (statewise) or [3]
   int statewise;
@@ -196,12 +192,8 @@ __host__ __device__ inline int kb_slot_ld(int S, int large) {
 
 struct EpiParams {
   TreeDev tr;
-  TreeScanDev ts;
-  PreDev pd;                  // preorder tables (register-resident kernel)
+  PreDev pd;                  // preorder tables
   int S;
-  int n_tlevels;
-  const int* tlevel_ptr;
-  const int* tlevel_node;
   const float* E; const float* log_pS; const float* log_pD; const float* log_pL; const float* mt;
   const float* col;
   int statewise;
@@ -216,7 +208,6 @@ struct EpiParams {
   double breakdown;
   float* grad_theta;
   float* grad_col;
-  double* work;               // [N_WORK, S]
   int* status;                // [0] iterations, [1] failure flag
   const double* q_extra;      // [S] added to q_E, or null
   int no_norm;                // 1: q_E without the loss normaliser's term
@@ -243,6 +234,5 @@ void launch_bwd_reduce(const float* contrib, int C, int S, size_t slot_stride, i
                        double* out, hipStream_t st);
 int reduce_chunks(int C);
 void launch_epilogue(const EpiParams& P, hipStream_t st);
-int epilogue_work_vectors();
 
 }  // namespace kb
