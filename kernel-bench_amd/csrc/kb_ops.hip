@@ -272,197 +272,404 @@ struct WsArgs {
   const T* leaf_logp;
 };
 
-// n_sweeps self-loop sweeps of one row; between sweeps the row stays in LDS
-// (Pr), so the result equals n_sweeps one-sweep launches bit for bit.  The
-// thread's tree entries (children, Euler events, entry events) and the row's
-// constants are read once, before the first sweep.
-template <typename T, int CPT>
-__global__ __launch_bounds__(NT) void wave_step_kernel(OpsTree t, WsArgs<T> a) {
-  extern __shared__ unsigned char smraw[];
-  T* Pr = reinterpret_cast<T*>(smraw);  // input row, later the final-Pibar work row
-  T* X = Pr + t.S;                      // linear row, then path sums, then the new row
-  T* EV = X + t.S;                      // 2S Euler scan
-  __shared__ T red[NW];
+// One sweep of rows [ws, ws + W) (float64: n_sweeps of them), one workgroup
+// per row in flight.  Threads own preorder positions: the path sums are an
+// inclusive preorder scan minus an exclusive postorder scan, both in registers
+// (two barriers), and the row passes through LDS once each way between column
+// and preorder order.
+//
+// A sweep is evaluated in linear space relative to the row's largest entry,
+// 2^-M y' = a x + emc (rowsum - ps) + k1 x[c1] + k2 x[c2] + (leaf + dts) 2^-M,
+// so an entry takes one exponential per input and one logarithm instead of
+// seven and two.  Rows (or constants) whose finite values span more than R
+// binary orders, and non-finite ones, are evaluated term by term in log space,
+// where nothing underflows: both forms in one kernel, chosen per row.
+//
+// A workgroup walks its rows with the position tables and the linear constants
+// in registers (formed again when the item changes) and the next row's loads
+// in flight.  Measured: see launch_wave_step.
+// hardware exponential and logarithm for float (arguments that keep clear of
+// denormals, or whose denormal results vanish next to the sums they enter)
+__device__ __forceinline__ float fexp2(float x) { return kb::exp2_hw(x); }
+__device__ __forceinline__ double fexp2(double x) { return exp2(x); }
+__device__ __forceinline__ float flog2(float x) { return kb::log2_hw(x); }
+__device__ __forceinline__ double flog2(double x) { return log2(x); }
+
+// z = mantissa * 2^exponent, mantissa in [1/2, 1)
+__device__ __forceinline__ float mantissa(float z) { return __builtin_amdgcn_frexp_mantf(z); }
+__device__ __forceinline__ double mantissa(double z) { return __builtin_amdgcn_frexp_mant(z); }
+__device__ __forceinline__ int exponent(float z) { return __builtin_amdgcn_frexp_expf(z); }
+__device__ __forceinline__ int exponent(double z) { return __builtin_amdgcn_frexp_exp(z); }
+__device__ __forceinline__ float xceil(float x) { return ceilf(x); }
+__device__ __forceinline__ double xceil(double x) { return ceil(x); }
+
+// float rows of two positions per thread: six wavefronts per SIMD (at most 80
+// VGPRs; eight spill, and the spills cost more than the wavefronts give)
+template <typename T>
+constexpr int step_min_waves(int cpt) { return std::is_same_v<T, float> && cpt == 2 ? 6 : 1; }
+
+// see wave_step_kernel: four rows of constants in LDS
+template <typename T>
+__host__ __device__ constexpr bool step_consts_in_lds(int maxs) { return 4 * maxs * (int)sizeof(T) <= 64 * 1024; }
+
+template <typename T, int BT, int CPT, bool WEIGHTED>
+__global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(OpsTree t, WsArgs<T> a) {
+  constexpr int MAXS = BT * CPT, BW = BT / 64, ZERO = MAXS, SEG = 64 * CPT, LD = MAXS + 64;
+  constexpr int NONE = 0xffff;
+  constexpr bool CHAINS = !std::is_same_v<T, float>;  // (float chains: wave_step_lin_kernel)
+  constexpr T R = std::is_same_v<T, float> ? T(60) : T(400);
+  extern __shared__ __align__(16) unsigned char smraw[];
+  T* X = reinterpret_cast<T*>(smraw);  // the row's values at preorder positions; [ZERO] stays 0
+  T* Q = X + LD;                       // the split term, then the postorder scan
+  // the linear constants of the own positions: in LDS where they fit in 64 KB,
+  // which leaves registers for more rows per CU
+  constexpr bool KC = step_consts_in_lds<T>(MAXS);
+  T* Kc = Q + LD;
+  __shared__ T wP[BW], wQ[BW], wA[BW], wB[BW];
   const int S = t.S;
-  const int w = blockIdx.x;
-  const long long grow = a.ws + w;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const T NI = ninf<T>();
-  const long long item = a.item[grow];
-  const size_t cb = (size_t)(item * a.cstride);
-  const T* in = a.Pi_in + (size_t)(a.pi_ws + w) * S;
-#pragma unroll
-  for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
-    if (s < S) Pr[s] = in[s];
-  }
-  const long long lstate = a.use_leaf ? a.leaf_state[grow] : -1;
-  int c1v[CPT], c2v[CPT], tinv[CPT], evv[2 * CPT];
-  T kmt[CPT], kDL[CPT], kEb[CPT], kE[CPT], kS1[CPT], kS2[CPT], klf[CPT], kd[CPT], kcol[CPT];
-#pragma unroll
-  for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
-    c1v[k] = c2v[k] = -1;
-    tinv[k] = 0;
-    kmt[k] = kDL[k] = kEb[k] = kE[k] = kS1[k] = kS2[k] = kcol[k] = T(0);
-    klf[k] = kd[k] = NI;
-    if (s < S) {
-      const size_t ci = cb + s;
-      c1v[k] = t.c1[s];
-      c2v[k] = t.c2[s];
-      tinv[k] = t.tin[s];
-      kmt[k] = a.mt[ci];
-      kDL[k] = a.DL[ci];
-      kEb[k] = a.Ebar[ci];
-      kE[k] = a.E[ci];
-      kS1[k] = a.SL1[ci];
-      kS2[k] = a.SL2[ci];
-      if (lstate == s) klf[k] = a.leaf_logp[(size_t)item * S + s];
-      if (a.dts) kd[k] = a.dts[(size_t)w * S + s];
-      if (a.use_col) kcol[k] = a.col[s];
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < 2 * CPT; ++j) {
-    const int q = threadIdx.x + j * NT;
-    evv[j] = q < 2 * S ? t.ev[q] : 0;
-  }
-  // ancestors-or-self path sums of x (LDS, column order) into ps (may alias x):
-  // +x at the entry event and -x at the exit event of each column, scanned,
-  // read back at the entry event
-  auto path_sums_own = [&](const T* x, T* ps) {
-#pragma unroll
-    for (int j = 0; j < 2 * CPT; ++j) {
-      const int q = threadIdx.x + j * NT;
-      if (q < 2 * S) {
-        const int e = evv[j];
-        const T v = x[e >> 1];
-        EV[q] = (e & 1) ? -v : v;
-      }
-    }
-    __syncthreads();
-    block_scan(EV, 2 * S, red);
+  // Tables of the own positions i = tid*CPT + k, two 16-bit entries a word:
+  // child2's position and the position at postorder slot i (ZERO: none);
+  // tin(i) - i and the preorder position of column tid + k*BT (NONE: past the
+  // row).  Child1 of i is i + 1.
+  unsigned cq[CPT], np[CPT];
+  auto load_tables = [&]() {
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
-      const int s = threadIdx.x + k * NT;
-      if (s < S) ps[s] = EV[tinv[k]];
+      const int i = kb::own_pos_c<BT, CPT>(k);
+      const int c2 = i < S ? t.pc2[i] : -1, q = i < S ? t.ppost[i] : ZERO;
+      cq[k] = (unsigned)(c2 >= 0 ? c2 : ZERO) | ((unsigned)q << 16);
+      const int sc = tid + k * BT;
+      np[k] = (unsigned)(i < S ? t.pnex[i] : 0) | ((unsigned)(sc < S ? t.ppos[sc] : NONE) << 16);
     }
-    __syncthreads();
   };
-  __syncthreads();
-  T wv[CPT], res[CPT];
-  T ldiff = 0;
-  for (int sweep = 0; sweep < a.n_sweeps; ++sweep) {
-    // row max / sum of (col +) Pi, then Pibar(Pi) = log2(rowsum - pathsum) + M + mt
-    T lm = NI;
+  load_tables();
+  auto own = [&](int k) { return kb::own_pos_c<BT, CPT>(k); };
+  if (tid < 64) {
+    X[MAXS + tid] = T(0);
+    Q[MAXS + tid] = T(0);
+  }
+  T cw[WEIGHTED ? CPT : 1], cwq[WEIGHTED ? CPT : 1];
+  bool out_of_range = false;
+  auto ranged = [&](T x) { out_of_range = out_of_range || !((x >= -R && x <= R) || x == NI); };
+  if constexpr (WEIGHTED) {
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
-      const int s = threadIdx.x + k * NT;
-      wv[k] = NI;
-      if (s < S) {
-        wv[k] = a.use_col ? kcol[k] + Pr[s] : Pr[s];
-        lm = tmax(lm, wv[k]);
+      cw[k] = cwq[k] = T(0);
+      if (own(k) < S) {
+        const T c = a.col[t.pcol[own(k)]];
+        ranged(c);
+        cw[k] = xexp2(c);
+        cwq[k] = xexp2(a.col[t.pcol[cq[k] >> 16]]);
       }
     }
-    const T M = block_max(lm, red);
-    const T Ms = msafe(M);
-    T ls = 0;
+  }
+  const bool col_out = out_of_range;
+  T kr[4][KC ? 1 : CPT];
+  auto load_consts = [&](size_t cb) {  // -> a constant is out of range
+    out_of_range = col_out;
+    T ca[CPT], ce[CPT], ck1[CPT], ck2[CPT];
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
-      const int s = threadIdx.x + k * NT;
-      if (s < S) {
-        const T x = xexp2(wv[k] - Ms);
-        X[s] = x;
-        ls += x;
-      }
-    }
-    const T rowsum = block_sum(ls, red);
-    path_sums_own(X, X);
-    ldiff = 0;
-#pragma unroll
-    for (int k = 0; k < CPT; ++k) {
-      const int s = threadIdx.x + k * NT;
-      res[k] = NI;
-      if (s < S) {
-        const T denom = rowsum - X[s];
-        const T pibar_w = denom > T(0) ? xlog2(denom) + M + kmt[k] : NI;
-        const T pi_w = Pr[s];
-        const T ps1 = c1v[k] >= 0 ? Pr[c1v[k]] : NI;
-        const T ps2 = c2v[k] >= 0 ? Pr[c2v[k]] : NI;
-        const T t0 = kDL[k] + pi_w;
-        const T t1 = pi_w + kEb[k];
-        const T t2 = pibar_w + kE[k];
-        const T t3 = kS1[k] + ps1;
-        const T t4 = kS2[k] + ps2;
-        const T t5 = klf[k];
-        T m = tmax(tmax(tmax(t0, t1), tmax(t2, t3)), tmax(t4, t5));
-        const T d = kd[k];
-        if (a.dts) m = tmax(m, d);
-        const T ms = msafe(m);
-        T sum = xexp2(t0 - ms) + xexp2(t1 - ms) + xexp2(t2 - ms) + xexp2(t3 - ms) + xexp2(t4 - ms) + xexp2(t5 - ms);
-        if (a.dts) sum += xexp2(d - ms);
-        res[k] = xlog2(sum) + m;
-        if (res[k] != NI && pi_w != NI) {
-          const T df = res[k] - pi_w;
-          ldiff = tmax(ldiff, df < T(0) ? -df : df);
+      ca[k] = ce[k] = ck1[k] = ck2[k] = T(0);
+      if (own(k) < S) {
+        const size_t ci = cb + t.pcol[own(k)];
+        const T dl = a.DL[ci], eb = a.Ebar[ci], em = a.E[ci] + a.mt[ci];
+        ca[k] = xexp2(dl) + xexp2(eb);
+        ce[k] = xexp2(em);
+        ranged(dl);
+        ranged(eb);
+        ranged(em);
+        if (t.pc1[own(k)] >= 0) {
+          const T s1 = a.SL1[ci];
+          ck1[k] = xexp2(s1);
+          ranged(s1);
+        }
+        if ((cq[k] & 0xffff) != ZERO) {
+          const T s2 = a.SL2[ci];
+          ck2[k] = xexp2(s2);
+          ranged(s2);
         }
       }
     }
-    __syncthreads();  // every read of X / Pr above is done
-    if (sweep + 1 < a.n_sweeps) {
+    if constexpr (KC) {
+      own_store<CPT>(Kc, ca);
+      own_store<CPT>(Kc + MAXS, ce);
+      own_store<CPT>(Kc + 2 * MAXS, ck1);
+      own_store<CPT>(Kc + 3 * MAXS, ck2);
+    } else {
 #pragma unroll
       for (int k = 0; k < CPT; ++k) {
-        const int s = threadIdx.x + k * NT;
-        if (s < S) Pr[s] = res[k];
+        kr[0][k] = ca[k];
+        kr[1][k] = ce[k];
+        kr[2][k] = ck1[k];
+        kr[3][k] = ck2[k];
+      }
+    }
+    return __syncthreads_or(out_of_range) != 0;
+  };
+  auto konst = [&](int j, T (&v)[CPT]) {
+    if constexpr (KC) {
+      own_load<CPT>(Kc + j * MAXS, v);
+    } else {
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) v[k] = kr[j][k];
+    }
+  };
+  // Publishes v (own positions; with WGT its sums are column-weighted) and
+  // returns the ancestors-or-self sums and the total; with WGT or an unweighted
+  // sweep (KIDS) also the children's values.
+  auto path_sums = [&](auto wgt_, auto kids_, const T (&v)[CPT], T (&ps)[CPT], T& total, T (&x2)[CPT], T& x1last) {
+    constexpr bool WGT = decltype(wgt_)::value && WEIGHTED, KIDS = decltype(kids_)::value;
+    T sp[CPT], ta = T(0);
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) {
+      ta += WGT ? cw[WGT ? k : 0] * v[k] : v[k];
+      sp[k] = ta;
+    }
+    const T wa = wscan(ta);
+    own_store<CPT>(X, v);
+    if (lane == 63) wP[wv] = wa;
+    __syncthreads();
+    const T tp = kb::lds_wave_values<BW>(wP, lane, T(0));
+    T yq[CPT];
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) {
+      yq[k] = X[cq[k] >> 16];
+      if constexpr (KIDS) x2[k] = X[cq[k] & 0xffff];
+    }
+    if constexpr (KIDS) x1last = X[tid * CPT + CPT];
+    const T ip = wscan_first<BW>(tp);
+    total = lane_of(ip, BW - 1);
+    const T offp = lane_of(ip - tp, wv) + (wa - ta);
+    T sq[CPT], tb = T(0);
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) {
+      sq[k] = tb;
+      tb += WGT ? cwq[WGT ? k : 0] * yq[k] : yq[k];
+    }
+    const T wb = wscan(tb);
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) sq[k] += wb - tb;
+    own_store<CPT>(Q, sq);
+    if (lane == 63) wQ[wv] = wb;
+    __syncthreads();
+    const T tq = kb::lds_wave_values<BW>(wQ, lane, T(0));
+    const T eq = wscan_first<BW>(tq) - tq;
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) {
+      const int n = np[k] & 0xffff;
+      ps[k] = (sp[k] + offp) - (Q[n] + (BW > 1 ? shfl_of(eq, n / SEG) : T(0)));
+    }
+  };
+  // the largest value over the workgroup (two barriers)
+  auto wg_max = [&](T x) {
+    x = wmax63(x);
+    __syncthreads();
+    if (lane == 63) wA[wv] = x;
+    __syncthreads();
+    return wmax_first<BW>(wA, lane);
+  };
+  long long citem = -1;
+  bool cbad = false;
+  for (int w = blockIdx.x; w < a.W; w += gridDim.x) {
+    // (opaque in every row: the LDS addresses formed from the packed tables
+    // would otherwise be kept in registers through the loop)
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) asm("" : "+v"(cq[k]), "+v"(np[k]));
+    const long long grow = a.ws + w;
+    const long long item = a.item[grow];
+    const size_t cb = (size_t)(item * a.cstride);
+    if (citem < 0 || (a.cstride != 0 && item != citem)) cbad = load_consts(cb);
+    citem = item;
+    const T* in = a.Pi_in + (size_t)(a.pi_ws + w) * S;
+    const T* dt = a.dts ? a.dts + (size_t)w * S : nullptr;
+    T vin[CPT], vdt[CPT];  // columns tid + j*BT
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) {
+      const int sc = tid + j * BT;
+      vin[j] = sc < S ? kb::ldg(in, sc) : NI;
+      vdt[j] = dt && sc < S ? kb::ldg(dt, sc) : NI;
+    }
+    const long long lstate = a.use_leaf ? a.leaf_state[grow] : -1;
+    const bool has_leaf = lstate >= 0 && lstate < S;
+    const int lpos = has_leaf ? t.ppos[lstate] : -1;
+    const T lval = has_leaf ? a.leaf_logp[(size_t)item * S + lstate] : NI;
+    T* out = a.Pi_out + (size_t)grow * S;
+    // largest and (negated) smallest finite input; one that is NaN or +inf
+    // makes the range infinite
+    T hi = lval, lo = lval == NI ? NI : -lval;
+    auto span = [&](T x) {
+      hi = tmax(hi, x);
+      lo = tmax(lo, x == NI ? NI : x == x ? -x : -NI);
+    };
+    auto publish_span = [&]() {
+      hi = wmax63(hi);
+      lo = wmax63(lo);
+      if (lane == 63) {
+        wA[wv] = hi;
+        wB[wv] = lo;
       }
       __syncthreads();
-    }
-  }
-  T* out = a.Pi_out + (size_t)grow * S;
+      hi = wmax_first<BW>(wA, lane);
+      lo = wmax_first<BW>(wB, lane);
+    };
 #pragma unroll
-  for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
-    if (s < S) out[s] = res[k];
-  }
-  if (a.resid) {
-    const T md = block_max(ldiff, red);
-    if (threadIdx.x == 0) a.resid[grow] = (float)md;
-  }
-  if (!a.store_final) return;
-  __syncthreads();
-  T lm2 = NI;
-#pragma unroll
-  for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
-    wv[k] = NI;
-    if (s < S) {
-      wv[k] = a.use_col ? kcol[k] + res[k] : res[k];
-      lm2 = tmax(lm2, wv[k]);
+    for (int j = 0; j < CPT; ++j) {
+      span(vin[j]);
+      span(vdt[j]);
+      const unsigned i = np[j] >> 16;
+      if (i != NONE) {
+        X[i] = vin[j];
+        Q[i] = vdt[j];
+      }
     }
-  }
-  const T M2 = block_max(lm2, red);
-  const T Ms2 = msafe(M2);
-  T ls2 = 0;
+    publish_span();
+    T pr[CPT], dd[CPT], res[CPT];
+    own_load<CPT>(X, pr);
+    own_load<CPT>(Q, dd);
 #pragma unroll
-  for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
-    if (s < S) {
-      const T x = xexp2(wv[k] - Ms2);
-      Pr[s] = x;
-      ls2 += x;
-    }
-  }
-  const T rowsum2 = block_sum(ls2, red);
-  path_sums_own(Pr, Pr);
-  T* pb = a.Pibar + (size_t)grow * S;
+    for (int k = 0; k < CPT; ++k)
+      if (own(k) >= S) pr[k] = dd[k] = NI;
+    for (int sweep = 0;; ++sweep) {
+      // (hi and lo of a row without finite entries are -inf)
+      if (!cbad && (hi == NI || hi + lo <= R)) {
+        // an integer reference: Pi - Ms and the exponent of the result are exact,
+        // and the result is rounded once
+        const T Ms = xceil(msafe(hi));
+        T x[CPT], x2[CPT], ps[CPT], tot, x1last;
 #pragma unroll
-  for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
-    if (s < S) {
-      const T denom = rowsum2 - Pr[s];
-      pb[s] = denom > T(0) ? xlog2(denom) + M2 + kmt[k] : NI;
+        for (int k = 0; k < CPT; ++k) x[k] = fexp2(pr[k] - Ms);  // 0 at padding positions
+        path_sums(std::true_type{}, std::true_type{}, x, ps, tot, x2, x1last);
+        T ca[CPT], ce[CPT], ck1[CPT], ck2[CPT];
+        konst(0, ca);
+        konst(1, ce);
+        konst(2, ck1);
+        konst(3, ck2);
+#pragma unroll
+        for (int k = 0; k < CPT; ++k) {
+          T z = ca[k] * x[k];
+          z += ck1[k] * (k + 1 < CPT ? x[k + 1 < CPT ? k + 1 : k] : x1last);
+          z += ck2[k] * x2[k];
+          z += ce[k] * tmax(tot - ps[k], T(0));
+          z += fexp2(dd[k] - Ms);
+          if (own(k) == lpos) z += fexp2(lval - Ms);
+          // (0 at padding positions)
+          res[k] = z > T(0) ? flog2(mantissa(z)) + (Ms + (T)exponent(z)) : NI;
+        }
+      } else {
+        // term by term in log space: values 2^(col + Pi - M) in Q, Pi in X, the
+        // path sums by following the parents; the results go straight to the
+        // output row and are read back
+        T lm = NI;
+#pragma unroll
+        for (int k = 0; k < CPT; ++k)
+          if (own(k) < S) lm = tmax(lm, a.use_col ? a.col[t.pcol[own(k)]] + pr[k] : pr[k]);
+        const T M = wg_max(lm);
+        const T Mw = msafe(M);
+        T ls = T(0);
+#pragma unroll
+        for (int k = 0; k < CPT; ++k)
+          if (own(k) < S) {
+            const T xw = xexp2((a.use_col ? a.col[t.pcol[own(k)]] + pr[k] : pr[k]) - Mw);
+            X[own(k)] = pr[k];
+            Q[own(k)] = xw;
+            ls += xw;
+          }
+        const T wa = lane_of(wscan(ls), 63);
+        if (lane == 63) wP[wv] = wa;
+        __syncthreads();
+        T tot = wP[0];
+#pragma unroll 1
+        for (int i = 1; i < BW; ++i) tot += wP[i];
+#pragma unroll 1
+        for (int i = tid * CPT; i < min(S, tid * CPT + CPT); ++i) {
+          const int sc = t.pcol[i];
+          const size_t ci = cb + sc;
+          T ps = T(0);
+          for (int n = sc; n >= 0; n = t.par[n]) ps += Q[t.ppos[n]];
+          const T denom = tot - ps, p = X[i];
+          const int c1 = t.pc1[i], c2 = t.pc2[i];
+          const T pibar = denom > T(0) ? xlog2(denom) + M + a.mt[ci] : NI;
+          const T t0 = a.DL[ci] + p;
+          const T t1 = p + a.Ebar[ci];
+          const T t2 = pibar + a.E[ci];
+          const T t3 = a.SL1[ci] + (c1 >= 0 ? X[c1] : NI);
+          const T t4 = a.SL2[ci] + (c2 >= 0 ? X[c2] : NI);
+          const T t5 = i == lpos ? lval : NI;
+          const T d = a.dts ? a.dts[(size_t)w * S + sc] : NI;
+          const T m = tmax(tmax(tmax(tmax(t0, t1), tmax(t2, t3)), tmax(t4, t5)), d);
+          const T ms = msafe(m);
+          const T sum = xexp2(t0 - ms) + xexp2(t1 - ms) + xexp2(t2 - ms) + xexp2(t3 - ms) + xexp2(t4 - ms) +
+                        xexp2(t5 - ms) + xexp2(d - ms);
+          out[sc] = xlog2(sum) + m;
+        }
+#pragma unroll
+        for (int k = 0; k < CPT; ++k) res[k] = own(k) < S ? out[t.pcol[own(k)]] : NI;
+        __syncthreads();  // X and Q are written again below
+        // tables and constants are read again, so that this branch, which few
+        // rows take, does not hold the others' registers
+        load_tables();
+        citem = -1;
+      }
+      if (a.resid && sweep + 1 >= a.n_sweeps) {
+        T ldiff = T(0);
+#pragma unroll
+        for (int k = 0; k < CPT; ++k)
+          if (res[k] != NI && pr[k] != NI) {
+            const T df = res[k] - pr[k];
+            ldiff = tmax(ldiff, df < T(0) ? -df : df);
+          }
+        ldiff = wg_max(ldiff);
+        if (tid == 0) a.resid[grow] = (float)ldiff;
+      }
+      if (!CHAINS || sweep + 1 >= a.n_sweeps) break;
+      hi = lval;
+      lo = lval == NI ? NI : -lval;
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) {
+        pr[k] = res[k];
+        span(pr[k]);
+        span(dd[k]);
+      }
+      publish_span();
     }
+    if (a.store_final) {
+      T lm = NI, x[CPT], x2[CPT], ps[CPT], tot, x1last;
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) {
+        x[k] = WEIGHTED && own(k) < S ? a.col[t.pcol[own(k)]] + res[k] : res[k];
+        lm = tmax(lm, x[k]);
+      }
+      const T M = wg_max(lm);  // (its barriers: every earlier read of X and Q is done)
+      const T Mw = msafe(M);
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) x[k] = own(k) < S ? fexp2(x[k] - Mw) : T(0);
+      path_sums(std::false_type{}, std::false_type{}, x, ps, tot, x2, x1last);
+      __syncthreads();  // Q is written again
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) {
+        const T denom = tot - ps[k];
+        x[k] = own(k) < S && denom > T(0) ? flog2(denom) + M + a.mt[cb + t.pcol[own(k)]] : NI;
+      }
+      own_store<CPT>(Q, x);
+      if (tid == 0) a.rowmax[grow] = M;
+    }
+    own_store<CPT>(X, res);
+    __syncthreads();
+    T* pbo = a.store_final ? a.Pibar + (size_t)grow * S : nullptr;
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) {
+      const unsigned i = np[j] >> 16;
+      if (i != NONE) {
+        const int sc = tid + j * BT;
+        kb::stg(out, sc, X[i]);
+        if (pbo) kb::stg(pbo, sc, Q[i]);
+      }
+    }
+    __syncthreads();  // X and Q are free for the next row
   }
-  if (threadIdx.x == 0) a.rowmax[grow] = M2;
 }
 
 // Sweep chains (n_sweeps > 1) of float32 rows in linear space, as the
@@ -2071,13 +2278,22 @@ int estep_vjp_launch(const kb_tree* tr, const kb_estep_vjp_io* io, double* work,
 }  // namespace
 
 namespace {
-// Chains of float sweeps run the linear-space preorder-ownership kernel (three
-// LDS rows of NT * CPT + 64 floats; its set-up -- tables, linear constants, the
-// row permuted through LDS -- pays off over several sweeps); single sweeps and
-// float64 rows the log-space Euler-tour one.  A chain agrees with the same
-// sweeps launched one at a time to float32 rounding.
+// Chains of float sweeps run the linear-space preorder-ownership kernel, which
+// keeps the row in linear space between sweeps (three LDS rows of NT * CPT + 64
+// floats); single sweeps and float64 rows wave_step_kernel.  A chain agrees
+// with the same sweeps launched one at a time to float32 rounding.
+template <typename T, int BT, int CPT>
+int launch_step(const kbo::OpsTree& t, const kbo::WsArgs<T>& a, int W, hipStream_t st) {
+  constexpr int MAXS = BT * CPT;
+  const size_t lds = (2 * (MAXS + 64) + (kbo::step_consts_in_lds<T>(MAXS) ? 4 * MAXS : 0)) * sizeof(T);
+  auto k = a.use_col ? kbo::wave_step_kernel<T, BT, CPT, true> : kbo::wave_step_kernel<T, BT, CPT, false>;
+  if (int rc = set_lds(k, lds)) return rc;
+  hipLaunchKernelGGL(k, dim3(std::min(W, resident_blocks(k, BT, lds))), dim3(BT), lds, st, t, a);
+  return 0;
+}
+
 template <typename T, int CPT>
-int launch_wave_step(const kbo::OpsTree& t, const kbo::WsArgs<T>& a, int W, size_t lds, hipStream_t st) {
+int launch_wave_step(const kbo::OpsTree& t, const kbo::WsArgs<T>& a, int W, hipStream_t st) {
   if constexpr (std::is_same_v<T, float>) {
     if (a.n_sweeps > 1) {
       const size_t lds_lin = (size_t)3 * (kbo::NT * CPT + 64) * sizeof(float);
@@ -2087,10 +2303,26 @@ int launch_wave_step(const kbo::OpsTree& t, const kbo::WsArgs<T>& a, int W, size
       return 0;
     }
   }
-  auto k = kbo::wave_step_kernel<T, CPT>;
-  if (int rc = set_lds(k, lds)) return rc;
-  hipLaunchKernelGGL(k, dim3(W), dim3(kbo::NT), lds, st, t, a);
-  return 0;
+  // The smallest shape that holds the row.  Times of the 15 sweeps and the split
+  // term of a wave through the wrappers, against one 1024-thread workgroup per
+  // row with an Euler-tour scan and log-space sums: 2047 states, 2140 rows 1044 ->
+  // 514 us (512 x 4; 1024 x 2 579 us); 1023 states, 1908 rows 658 -> 279 us (512
+  // x 2; 256 x 4 314 us); 127 states, 2104 rows 567 -> 246 us (the calls' host
+  // time); 4095 states, 721 rows 644 -> 517 us; 7999 states, 652 rows 2338 ->
+  // 1711 us.  float64: 2047 states 3440 -> 1170 us (512 x 4; 1024 x 2 spills,
+  // 1470 us), 1023 states 1342 -> 590 us (256 x 4; 512 x 2 700 us), 511 states
+  // 1024 -> 335 us.  A sweep of 2140 x 2047 floats moves 53 MB (10 us at 5.3
+  // TB/s) in about 32 us: barriers and the LDS round trips of a row, with two to
+  // three rows per CU.
+  const int S = t.S;
+  constexpr bool F32 = std::is_same_v<T, float>;
+  if (S <= 128) return launch_step<T, 64, 2>(t, a, W, st);
+  if (S <= 256) return launch_step<T, 128, 2>(t, a, W, st);
+  if (S <= 512) return launch_step<T, 256, 2>(t, a, W, st);
+  if (S <= 1024) return launch_step<T, F32 ? 512 : 256, F32 ? 2 : 4>(t, a, W, st);
+  if (S <= 2048) return launch_step<T, 512, 4>(t, a, W, st);
+  if (S <= 4096) return launch_step<T, 1024, 4>(t, a, W, st);
+  return launch_step<T, 1024, 8>(t, a, W, st);
 }
 
 // float32 rows of the per-call wave backward run the preorder-ownership kernel
@@ -2149,7 +2381,7 @@ int kb_wave_step(const kb_tree* tr, const kb_wave_step_io* io, void* stream) {
                      io->pi_residual, (const T*)io->dts, (const T*)io->max_coupling, (const T*)io->DL,
                      (const T*)io->Ebar, (const T*)io->E, (const T*)io->SL1, (const T*)io->SL2,
                      (const T*)io->col_log_probs, io->item_idx, io->leaf_state, (const T*)io->leaf_logp};
-    if (int rc = launch_wave_step<T, CPT>(t, a, io->W, lds, st_of(stream))) return rc;
+    if (int rc = launch_wave_step<T, CPT>(t, a, io->W, st_of(stream))) return rc;
   });
   KBO_HIP(hipGetLastError());
   return 0;

@@ -162,6 +162,68 @@ __device__ __forceinline__ T complement_of(const OpsTree& t, const T* pre, int s
   return (p > 0 ? pre[p - 1] : T(0)) + (total - pre[e - 1]);
 }
 
+// ---- preorder ownership, any T ------------------------------------------------
+// Thread t owns positions t*CPT + k (kb_rowops.hpp); float and double forms of
+// the wavefront scans and own-position LDS accesses under one name.
+
+__device__ __forceinline__ float wscan(float x) { return kb::wave_scan_incl(x); }
+__device__ __forceinline__ double wscan(double x) { return kb::wave_scan_incl_f64(x); }
+template <int N> __device__ __forceinline__ float wscan_first(float x) { return kb::wave_scan_first<N>(x); }
+template <int N> __device__ __forceinline__ double wscan_first(double x) { return kb::wave_scan_first_f64<N>(x); }
+__device__ __forceinline__ float lane_of(float x, int l) { return kb::lane_value(x, l); }
+__device__ __forceinline__ double lane_of(double x, int l) { return kb::lane_value_f64(x, l); }
+__device__ __forceinline__ float shfl_of(float x, int l) { return __shfl(x, l, 64); }
+__device__ __forceinline__ double shfl_of(double x, int l) { return kb::shfl_f64(x, l); }
+
+template <int CTRL, int ROW_MASK = 0xf>
+__device__ __forceinline__ float dpp_ninf(float x) {  // lanes without a source read -inf
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(-__builtin_inff()), __float_as_int(x), CTRL,
+                                                    ROW_MASK, 0xf, false));
+}
+template <int CTRL, int ROW_MASK = 0xf>
+__device__ __forceinline__ double dpp_ninf(double x) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+  const unsigned long long n = (unsigned long long)__double_as_longlong(-__builtin_inf());
+  const int lo = __builtin_amdgcn_update_dpp((int)(unsigned)n, (int)(unsigned)b, CTRL, ROW_MASK, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp((int)(unsigned)(n >> 32), (int)(unsigned)(b >> 32), CTRL, ROW_MASK, 0xf, false);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+// Maximum over the wavefront, in lane 63 (the scan's data movement).
+template <typename T>
+__device__ __forceinline__ T wmax63(T x) {
+  x = tmax(x, dpp_ninf<0x111>(x));
+  x = tmax(x, dpp_ninf<0x112>(x));
+  x = tmax(x, dpp_ninf<0x114>(x));
+  x = tmax(x, dpp_ninf<0x118>(x));
+  x = tmax(x, dpp_ninf<0x142, 0xa>(x));
+  x = tmax(x, dpp_ninf<0x143, 0xc>(x));
+  return x;
+}
+
+// Maximum of the N (a power of two, at most 16) per-wavefront values w[0..N-1].
+template <int N, typename T>
+__device__ __forceinline__ T wmax_first(const T* w, int lane) {
+  T x = w[lane & (N - 1)];
+  if constexpr (N > 1) x = tmax(x, dpp_ninf<0x111>(x));
+  if constexpr (N > 2) x = tmax(x, dpp_ninf<0x112>(x));
+  if constexpr (N > 4) x = tmax(x, dpp_ninf<0x114>(x));
+  if constexpr (N > 8) x = tmax(x, dpp_ninf<0x118>(x));
+  return lane_of(x, N - 1);
+}
+
+template <int CPT> __device__ __forceinline__ void own_store(float* lds, const float (&v)[CPT]) { kb::lds_store_own<CPT>(lds, v); }
+template <int CPT> __device__ __forceinline__ void own_store(double* lds, const double (&v)[CPT]) { kb::lds_store_own_f64<CPT>(lds, v); }
+template <int CPT> __device__ __forceinline__ void own_load(const float* lds, float (&v)[CPT]) { kb::lds_load_own<CPT>(lds, v); }
+template <int CPT> __device__ __forceinline__ void own_load(const double* lds, double (&v)[CPT]) {
+  const double* p = lds + threadIdx.x * CPT;
+#pragma unroll
+  for (int k = 0; k < CPT; k += 2) {
+    const double2 q = *reinterpret_cast<const double2*>(p + k);
+    v[k] = q.x;
+    v[k + 1] = q.y;
+  }
+}
+
 // float64 path sums / subtree sums over depth levels (in place).
 __device__ void level_path_sums(const OpsTree& t, double* x) {
   for (int d = 1; d < t.n_levels; ++d) {
@@ -341,6 +403,25 @@ inline int set_lds(F* kernel, size_t bytes) {
   KBO_HIP(hipFuncSetAttribute(key.first, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
   raised[key] = bytes;
   return 0;
+}
+
+// Workgroups of `nt` threads and `lds` bytes of dynamic LDS that the current
+// device holds at once: the grid of the kernels that walk their rows.  Asked
+// of the runtime once per kernel and device.
+template <typename F>
+inline int resident_blocks(F* kernel, int nt, size_t lds) {
+  static std::mutex mu;
+  static std::map<std::pair<const void*, int>, int> known;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 1;
+  const auto key = std::make_pair(reinterpret_cast<const void*>(kernel), dev);
+  std::lock_guard<std::mutex> lock(mu);
+  auto it = known.find(key);
+  if (it != known.end()) return it->second;
+  int n_cu = 1, occ = 0;
+  if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n_cu = 1;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, nt, lds) != hipSuccess) occ = 1;
+  return known[key] = n_cu * std::max(1, occ);
 }
 
 }  // namespace kbo_host

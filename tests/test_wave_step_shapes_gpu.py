@@ -1,0 +1,125 @@
+"""``compute_wave_step`` at the edges of its launch shapes and of its two row forms, against the oracle.
+
+A row (with its constants) whose finite values span at most 60 binary orders (float32; 400 in
+float64) is swept in linear space, any other term by term in log space.  Rows of both kinds,
+rows with -inf entries, a single finite entry or none, and two items whose constants alternate
+over the rows share one launch.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+import kbench_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+W = 6
+
+
+def _case(leaves, dt, weighted, wide_consts, leaf):
+    from kbench import synth
+
+    rng = np.random.default_rng(leaves + 7 * weighted)
+    tree = synth.yule_tree(leaves, rng)
+    h = synth.state_helpers_from_tree(tree)
+    S = tree.S
+    rnd = lambda a: np.asarray(a).astype(dt).astype(np.float64)
+    low = np.where(np.asarray(h["node_child1"]) < S, -8.0, 0.0)
+    span = 90.0 if dt == np.float32 else 500.0
+    Pi = -30.0 + rng.uniform(-12.0, 0.0, (W, S)) + low
+    Pi[1, rng.random(S) < 0.5] = -np.inf
+    Pi[2] = -20.0 + rng.uniform(-span, 0.0, S) + low
+    Pi[2, 0] = -20.0
+    Pi[3] = -np.inf
+    Pi[4] = -np.inf
+    Pi[4, S // 2] = -5.0
+    dts = Pi - rng.uniform(1.0, 9.0, (W, S))
+    dts[3] = -40.0 + low
+    dts[5] = -np.inf
+    c = {k: rng.uniform(-4.0, -0.5, (2, S)) for k in ("DL", "Ebar", "E", "SL1", "SL2", "leaf")}
+    c["mt"] = rng.uniform(-12.0, -9.0, (2, S))
+    if wide_consts:
+        c["DL"][1, S // 3] = -span
+    col = np.log2(rng.dirichlet(np.full(S, 50.0))) if weighted else np.full(S, -np.log2(S))
+    c, Pi, dts, col = {k: rnd(v) for k, v in c.items()}, rnd(Pi), rnd(dts), rnd(col)
+    items = np.arange(W) % 2
+    leaf_state = rng.integers(0, S, W) if leaf else None
+    consts = O.WaveConsts(mt=c["mt"], DL=c["DL"], Ebar=c["Ebar"], E=c["E"], SL1=c["SL1"], SL2=c["SL2"],
+                          leaf_logp=c["leaf"], col=col, use_col_weights=weighted)
+    return tree, h, S, Pi, dts, c, col, items, leaf_state, consts
+
+
+def _device_sweep(case, dt, weighted, *, sweeps=1, store=True):
+    from kbench.core.kernels import wave_step
+
+    tree, h, S, Pi, dts, c, col, items, leaf_state, _ = case
+    t = lambda a, d=dt: torch.as_tensor(np.ascontiguousarray(a), dtype=d, device="cuda")
+    ints = lambda a: torch.as_tensor(np.asarray(a), dtype=torch.int64, device="cuda")
+    bufs = [t(Pi), torch.full((W, S), 7.0, dtype=dt, device="cuda")]
+    pibar, rmax = (torch.full(s, 7.0, dtype=dt, device="cuda") for s in ((W, S), (W,)))
+    resid = torch.full((W,), 7.0, device="cuda") if sweeps == 1 else None
+    consts = [t(c[k]) for k in ("mt", "DL", "Ebar", "E", "SL1", "SL2")]
+    dev = dict(leaf_state_idx=ints(leaf_state if leaf_state is not None else np.zeros(W)), leaf_logp=t(c["leaf"]),
+               item_idx=ints(items))
+    topo = [ints(h[k]) for k in ("node_child1", "node_child2", "node_parent")]
+    d = None if leaf_state is not None else t(dts)
+    colt = t(col)
+    for k in range(sweeps):
+        wave_step.compute_wave_step(
+            bufs[k % 2], bufs[(k + 1) % 2], pibar, 0, W, S, *consts, colt, *topo, int(h["max_ancestor_depth"]), d,
+            **dev, pibar_row_max=rmax, store_final_pibar=store and k == sweeps - 1,
+            has_leaf_term=leaf_state is not None, use_col_weights=weighted, pi_residual_out=resid)
+    torch.cuda.synchronize()
+    return bufs[sweeps % 2].cpu().numpy(), pibar.cpu().numpy(), rmax.cpu().numpy(), resid
+
+
+# 4097 double rows need more LDS than the entry point allows (refused before any launch)
+@pytest.mark.parametrize("leaves,kind", [(n, k) for n in (1, 2, 64, 65, 128, 129, 256, 257, 512, 513, 1024, 1025, 2049)
+                                         for k in ("float32", "float64") if not (k == "float64" and n > 2048)])
+def test_one_sweep_matches_oracle(leaves, kind):
+    dt, tdt = (np.float32, torch.float32) if kind == "float32" else (np.float64, torch.float64)
+    for weighted, wide_consts, leaf in ((False, False, False), (True, False, True), (False, True, True)):
+        if leaves == 1 and weighted:
+            continue  # one column: its weight is the whole distribution
+        case = _case(leaves, dt, weighted, wide_consts, leaf)
+        tree, h, S, Pi, dts, c, col, items, leaf_state, consts = case
+        print(f"[sweep] S={S} {kind} weighted={weighted} wide_consts={wide_consts} leaf={leaf}", flush=True)
+        out, pibar, rmax, resid = _device_sweep(case, tdt, weighted)
+        otree = O.Tree.from_helpers(h)
+        with np.errstate(all="ignore"):
+            ref = O.wave_sweep(Pi, items, consts, otree, leaf_state=leaf_state, dts_r=None if leaf else dts)
+            wcol = col if weighted else 0.0
+            # each row's transfer term and its noise: a prefix-sum difference carries roundings of the
+            # row's total (eps each, of which sqrt(S) survive), whatever the share of the others is
+            eps = np.finfo(dt).eps
+            noise = eps * (8.0 + 2.0 * np.sqrt(S))
+            total = lambda x: np.exp2(x + wcol).sum(axis=1, keepdims=True)
+            unit = np.exp2((c["E"] + c["mt"])[items]) * total(Pi)
+            # a log2 value carries a few roundings of its own size and of its inputs'
+            size = 4.0 * eps * np.nanmax(np.abs(np.where(np.isfinite(Pi), Pi, 0.0)), axis=1, keepdims=True) + 16.0 * eps
+            y, y_ref = np.exp2(out.astype(np.float64)), np.exp2(ref)
+            assert (np.abs(y - y_ref) <= size * y_ref + noise * unit).all(), "Pi"
+            # Pibar and row_max belong to the rows written
+            o64 = out.astype(np.float64)
+            pb_ref, max_ref = O._pibar_from_pi(o64, col, c["mt"][items], otree, weighted)
+            scale = np.exp2(c["mt"][items]) * total(o64)
+            size = size + 4.0 * eps * np.abs(c["mt"][items])
+            pb = np.exp2(pibar.astype(np.float64))
+            assert (np.abs(pb - np.exp2(pb_ref)) <= size * np.exp2(pb_ref) + noise * scale).all(), "Pibar"
+            assert np.allclose(rmax, max_ref, rtol=2.0 * eps, atol=0.0, equal_nan=True), "row_max"
+            f = np.isfinite(out) & np.isfinite(Pi)
+            want = np.abs(np.where(f, o64, 0.0) - np.where(f, Pi, 0.0)).max(axis=1)
+        assert np.allclose(resid.cpu().numpy(), want, rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("leaves", [40, 400])
+def test_float64_chain_is_bitwise_its_single_sweeps(leaves, monkeypatch):
+    from kbench.core.kernels import wave_step
+
+    case = _case(leaves, np.float64, True, False, False)
+    one = _device_sweep(case, torch.float64, True, sweeps=3)
+    monkeypatch.setattr(wave_step, "FUSE_SWEEPS", True)
+    chain = _device_sweep(case, torch.float64, True, sweeps=3)
+    for a, b in zip(one[:3], chain[:3]):
+        assert np.array_equal(a, b, equal_nan=True)
