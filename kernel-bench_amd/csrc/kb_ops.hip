@@ -37,132 +37,289 @@ struct EsArgs {
   int* n_iter;
 };
 
-// One E-step of row values E (LDS, float64 log2) -> new values in En[k],
-// plus E_s1, E_s2, Ebar in registers.  X is LDS scratch (S doubles).
-template <typename T, int CPT>
-__device__ void estep_eval(const OpsTree& t, const EsArgs<T>& a, size_t base, const double* Ev, double* X,
-                           double* red, double (&En)[CPT], double (&Es1)[CPT], double (&Es2)[CPT],
-                           double (&Eb)[CPT]) {
-  const int S = t.S;
-  const double NI = -__builtin_inf();
-  double wE[CPT];
-  double lm = NI;
-#pragma unroll
-  for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
-    wE[k] = NI;
-    if (s < S) {
-      wE[k] = Ev[s] + (a.use_col ? (double)a.col[s] : 0.0);
-      lm = fmax(lm, wE[k]);
-    }
-  }
-  const double M = block_max(lm, red);
-  const double Ms = M == NI ? 0.0 : M;
-  double ls = 0.0;
-#pragma unroll
-  for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
-    if (s < S) {
-      const double x = exp2(wE[k] - Ms);
-      X[s] = x;
-      ls += x;
-    }
-  }
-  const double rowsum = block_sum(ls, red);  // its barrier publishes X
-  level_path_sums(t, X);
-#pragma unroll
-  for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
-    if (s < S) {
-      const size_t i = base + s;
-      const int c1 = t.c1[s], c2 = t.c2[s];
-      Es1[k] = c1 >= 0 ? Ev[c1] : NI;
-      Es2[k] = c2 >= 0 ? Ev[c2] : NI;
-      const double denom = rowsum - X[s];
-      Eb[k] = denom > 0.0 ? log2(denom) + M + (double)a.mt[i] : NI;
-      const double E = Ev[s];
-      const double t0 = (double)a.pS[i] + Es1[k] + Es2[k];
-      const double t1 = (double)a.pD[i] + 2.0 * E;
-      const double t2 = E + Eb[k];
-      const double t3 = (double)a.pL[i];
-      const double m = fmax(fmax(t0, t1), fmax(t2, t3));
-      const double ms = m == NI ? 0.0 : m;
-      En[k] = log2(exp2(t0 - ms) + exp2(t1 - ms) + exp2(t2 - ms) + exp2(t3 - ms)) + m;
-    }
-  }
-  __syncthreads();  // X and Ev reads done before the caller rewrites them
+// Largest value over a BT-thread workgroup; ends with a barrier (red: BT / 64).
+template <int BT, typename V>
+__device__ __forceinline__ V wg_max_of(V x, V* red) {
+  x = wave_max(x);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+  __syncthreads();
+  V m = red[0];
+  for (int i = 1; i < BT / 64; ++i) m = tmax(m, red[i]);
+  __syncthreads();
+  return m;
+}
+template <int BT, typename V>
+__device__ __forceinline__ V wg_sum_of(V x, V* red) {
+  x = wave_sum(x);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+  __syncthreads();
+  V m = red[0];
+  for (int i = 1; i < BT / 64; ++i) m += red[i];
+  __syncthreads();
+  return m;
 }
 
-template <typename T, int CPT>
-__global__ __launch_bounds__(NT) void estep_kernel(OpsTree t, EsArgs<T> a) {
-  extern __shared__ double sm[];
-  double* Ev = sm;
-  double* X = sm + t.S;
-  __shared__ double red[NW];
-  const int S = t.S;
-  const size_t base = (size_t)blockIdx.x * S;
-#pragma unroll
-  for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
-    if (s < S) Ev[s] = (double)a.E[base + s];
-  }
+// One row of estep_kernel term by term in log space (column order, Ev and X:
+// LDS rows), for values that linear float64 might not hold: the path sums by
+// following the parents.
+template <typename T, int BT, int CPT>
+__device__ void estep_row_log(const OpsTree& t, const EsArgs<T>& a, size_t base, double* Ev, double* X, double* red) {
+  const int S = t.S, tid = threadIdx.x;
+  const double NI = -__builtin_inf();
+  for (int s = tid; s < S; s += BT) Ev[s] = (double)a.E[base + s];
   __syncthreads();
-  double En[CPT], Es1[CPT], Es2[CPT], Eb[CPT];
-  if (a.mode == 0) {
-    estep_eval<T, CPT>(t, a, base, Ev, X, red, En, Es1, Es2, Eb);
-    double ld = 0.0;
-#pragma unroll
-    for (int k = 0; k < CPT; ++k) {
-      const int s = threadIdx.x + k * NT;
-      if (s < S) {
-        const T en = (T)En[k];
-        a.E_out[base + s] = en;
-        a.Es1[base + s] = (T)Es1[k];
-        a.Es2[base + s] = (T)Es2[k];
-        a.Ebar[base + s] = (T)Eb[k];
-        const T d = en - a.E[base + s];
-        ld = fmax(ld, (double)(d < T(0) ? -d : d));
-      }
+  double M = NI;
+  // X[s] = the others' sum of 2^(E + col - M); M the row's maximum
+  auto others = [&]() {
+    double lm = NI, ls = 0.0, den[CPT];
+    for (int s = tid; s < S; s += BT) lm = fmax(lm, Ev[s] + (a.use_col ? (double)a.col[s] : 0.0));
+    M = wg_max_of<BT>(lm, red);
+    const double Ms = M == NI ? 0.0 : M;
+    for (int s = tid; s < S; s += BT) {
+      X[s] = exp2(Ev[s] + (a.use_col ? (double)a.col[s] : 0.0) - Ms);
+      ls += X[s];
     }
-    const double md = block_max(ld, red);
-    if (a.max_diff && threadIdx.x == 0) a.max_diff[blockIdx.x] = (T)md;
-    return;
-  }
-  // fixed point: iterate while max |E_new - E| >= tol
-  int it = 0;
-  for (;;) {
-    estep_eval<T, CPT>(t, a, base, Ev, X, red, En, Es1, Es2, Eb);
-    double ld = 0.0;
+    const double tot = wg_sum_of<BT>(ls, red);
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
-      const int s = threadIdx.x + k * NT;
+      den[k] = tot;
+      const int s = tid + k * BT;
       if (s < S) {
-        const double d = En[k] - Ev[s];
-        if (!(fabs(d) < a.tol) && !(En[k] == Ev[s])) ld = fmax(ld, d != d ? __builtin_inf() : fabs(d));
+        double ps = 0.0;
+        for (int n = s; n >= 0; n = t.par[n]) ps += X[n];
+        den[k] = tot - ps;
       }
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < CPT; ++k) {
-      const int s = threadIdx.x + k * NT;
-      if (s < S) Ev[s] = En[k];
+    for (int k = 0; k < CPT; ++k)
+      if (tid + k * BT < S) X[tid + k * BT] = den[k];
+  };
+  auto ebar_of = [&](int s) { return X[s] > 0.0 ? log2(X[s]) + M + (double)a.mt[base + s] : NI; };
+  auto step_of = [&](int s) {
+    const size_t i = base + s;
+    const double E = Ev[s];
+    const double t0 = (double)a.pS[i] + (t.c1[s] >= 0 ? Ev[t.c1[s]] : NI) + (t.c2[s] >= 0 ? Ev[t.c2[s]] : NI);
+    const double t1 = (double)a.pD[i] + 2.0 * E;
+    const double t2 = E + ebar_of(s);
+    const double t3 = (double)a.pL[i];
+    const double m = fmax(fmax(t0, t1), fmax(t2, t3));
+    const double ms = m == NI ? 0.0 : m;
+    return log2(exp2(t0 - ms) + exp2(t1 - ms) + exp2(t2 - ms) + exp2(t3 - ms)) + m;
+  };
+  auto child = [&](int c) { return c >= 0 ? Ev[c] : NI; };
+  if (a.mode == 0) {
+    others();
+    double ld = 0.0;
+#pragma unroll 1
+    for (int s = tid; s < S; s += BT) {
+      const T en = (T)step_of(s);
+      a.E_out[base + s] = en;
+      a.Es1[base + s] = (T)child(t.c1[s]);
+      a.Es2[base + s] = (T)child(t.c2[s]);
+      a.Ebar[base + s] = (T)ebar_of(s);
+      const T d = en - a.E[base + s];
+      ld = fmax(ld, (double)(d < T(0) ? -d : d));
     }
-    ++it;
-    const double md = block_max(ld, red);  // barrier also publishes Ev
-    if (md < a.tol || it >= a.max_iter) break;
+    const double md = wg_max_of<BT>(ld, red);
+    if (a.max_diff && tid == 0) a.max_diff[blockIdx.x] = (T)md;
+    return;
   }
-  estep_eval<T, CPT>(t, a, base, Ev, X, red, En, Es1, Es2, Eb);
+  for (int it = 1;; ++it) {
+    others();
+    double ld = 0.0;
+#pragma unroll 1
+    for (int s = tid; s < S; s += BT) {
+      const double en = step_of(s), d = en - Ev[s];
+      if (!(fabs(d) < a.tol) && !(en == Ev[s])) ld = fmax(ld, d != d ? __builtin_inf() : fabs(d));
+      X[s] = en;
+    }
+    const double md = wg_max_of<BT>(ld, red);
+    for (int s = tid; s < S; s += BT) Ev[s] = X[s];
+    __syncthreads();
+    if (md < a.tol || it >= a.max_iter) {
+      if (a.n_iter && tid == 0) a.n_iter[blockIdx.x] = it;
+      break;
+    }
+  }
+  others();
+#pragma unroll 1
+  for (int s = tid; s < S; s += BT) {
+    a.E_out[base + s] = (T)Ev[s];
+    a.Es1[base + s] = (T)child(t.c1[s]);
+    a.Es2[base + s] = (T)child(t.c2[s]);
+    a.Ebar[base + s] = (T)ebar_of(s);
+  }
+}
+
+// One E step (mode 0) or the E fixed point (mode 1) of an item row, in linear
+// float64 at preorder positions as kb_estep.hip's estep_pre_kernel: e = 2^E,
+//   e' = 2^pS e[c1] e[c2] + 2^pD e^2 + e 2^mt (rowsum - ps) + 2^pL,
+// path sums from an inclusive preorder and an exclusive postorder register
+// scan, two barriers per step, and no exponential or logarithm inside the
+// iteration.  Rows with a parameter or start outside [-400, 400] (log2), which
+// products of float64 might not hold, are evaluated in log space.
+// Bound by one row's latency (two barriers and two scans a step).  100 rows of
+// 1023 states: 16 iterations and one step 290 -> 39 us (against a 1024-thread
+// workgroup summing by tree levels, with eight transcendentals an entry and
+// iteration), one VJP 23 -> 12 us.
+template <typename T, int BT, int CPT, bool WEIGHTED>
+__global__ __launch_bounds__(BT) void estep_kernel(OpsTree t, EsArgs<T> a) {
+  constexpr int MAXS = BT * CPT, BW = BT / 64, ZERO = MAXS, SEG = 64 * CPT;
+  extern __shared__ __align__(16) unsigned char smraw[];
+  double* X = reinterpret_cast<double*>(smraw);  // e at preorder positions
+  double* Q = X + MAXS + 64;                     // wavefront-local exclusive postorder scan
+  __shared__ double wP[BW], wQ[BW], red[BW];
+  __shared__ int wok[BW];
+  const int S = t.S;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const size_t base = (size_t)blockIdx.x * S;
+  const double NI = -__builtin_inf();
+  int colk[CPT], c2p[CPT], nex[CPT], qp[CPT];
+  bool h1[CPT], ranged = true;
+  double e[CPT], kS[CPT], kD[CPT], kL[CPT], kM[CPT], w[WEIGHTED ? CPT : 1], wq[WEIGHTED ? CPT : 1];
+  auto in_range = [&](double x) { ranged = ranged && x >= -400.0 && x <= 400.0; };
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
-    if (s < S) {
-      a.E_out[base + s] = (T)Ev[s];
-      a.Es1[base + s] = (T)Es1[k];
-      a.Es2[base + s] = (T)Es2[k];
-      a.Ebar[base + s] = (T)Eb[k];
+    const int i = tid * CPT + k;
+    colk[k] = -1;
+    c2p[k] = qp[k] = ZERO;
+    nex[k] = 0;
+    h1[k] = false;
+    e[k] = kS[k] = kD[k] = kL[k] = kM[k] = 0.0;
+    if constexpr (WEIGHTED) w[k] = wq[k] = 0.0;
+    if (i < S) {
+      const int s = colk[k] = t.pcol[i];
+      const int c2 = t.pc2[i];
+      c2p[k] = c2 >= 0 ? c2 : ZERO;
+      h1[k] = t.pc1[i] >= 0;  // child1 of i is i + 1
+      nex[k] = t.pnex[i];
+      qp[k] = t.ppost[i];
+      const double E = a.E[base + s], ps = a.pS[base + s], pd = a.pD[base + s], pl = a.pL[base + s], mt = a.mt[base + s];
+      in_range(E);
+      in_range(ps);
+      in_range(pd);
+      in_range(pl);
+      in_range(mt);
+      e[k] = exp2(E);
+      // (a missing child is the probability 0)
+      kS[k] = h1[k] && c2 >= 0 ? exp2(ps) : 0.0;
+      kD[k] = exp2(pd);
+      kL[k] = exp2(pl);
+      kM[k] = exp2(mt);
+      if constexpr (WEIGHTED) {
+        const double c = a.col[s];
+        in_range(c);
+        w[k] = exp2(c);
+        wq[k] = exp2((double)a.col[t.pcol[qp[k]]]);
+      }
     }
   }
-  if (a.n_iter && threadIdx.x == 0) a.n_iter[blockIdx.x] = it;
+  if (tid < 64) X[MAXS + tid] = Q[MAXS + tid] = 0.0;
+  if (!__syncthreads_and(ranged)) {
+    estep_row_log<T, BT, CPT>(t, a, base, X, Q, red);
+    return;
+  }
+  const double hi = exp2(a.tol), lo = exp2(-a.tol);
+  bool ok = true;  // the last update moved the own positions by less than tol
+  double e1[CPT], e2[CPT], ps[CPT], tot = 0.0;
+  int it = 0;
+  for (;;) {
+    double sp[CPT], ta = 0.0;
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) {
+      ta += WEIGHTED ? w[WEIGHTED ? k : 0] * e[k] : e[k];
+      sp[k] = ta;
+    }
+    const double wa = wscan(ta);
+    own_store<CPT>(X, e);
+    const bool wave_ok = __ballot(!ok) == 0;
+    if (lane == 63) {
+      wP[wv] = wa;
+      wok[wv] = wave_ok ? 1 : 0;
+    }
+    __syncthreads();
+    const int fl = kb::lds_wave_values<BW>(wok, lane, 1);
+    const bool stop = it > 0 && (a.mode == 0 || __ballot(fl == 0) == 0 || it >= a.max_iter);
+    const double tp = kb::lds_wave_values<BW>(wP, lane, 0.0);
+    double yq[CPT];
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) {
+      yq[k] = X[qp[k]];
+      if constexpr (WEIGHTED) yq[k] *= wq[k];
+      e2[k] = X[c2p[k]];
+    }
+    const double e1last = X[tid * CPT + CPT];
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) e1[k] = k + 1 < CPT ? e[k + 1 < CPT ? k + 1 : k] : e1last;
+    const double ip = wscan_first<BW>(tp);
+    tot = lane_of(ip, BW - 1);
+    const double offp = lane_of(ip - tp, wv) + (wa - ta);
+    double sq[CPT], tb = 0.0;
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) {
+      sq[k] = tb;
+      tb += yq[k];
+    }
+    const double wb = wscan(tb);
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) sq[k] += wb - tb;
+    own_store<CPT>(Q, sq);
+    if (lane == 63) wQ[wv] = wb;
+    __syncthreads();
+    const double tq = kb::lds_wave_values<BW>(wQ, lane, 0.0);
+    const double eq = wscan_first<BW>(tq) - tq;
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) ps[k] = (sp[k] + offp) - (Q[nex[k]] + (BW > 1 ? shfl_of(eq, nex[k] / SEG) : 0.0));
+    // (mode 0 stops after one step; its outputs are those of the point before it)
+    if (stop) break;
+    if (a.mode == 0) {
+      double ld = 0.0;
+#pragma unroll
+      for (int k = 0; k < CPT; ++k)
+        if (colk[k] >= 0) {
+          const size_t o = base + colk[k];
+          const double na = tot - ps[k];
+          const double en = kS[k] * e1[k] * e2[k] + kD[k] * e[k] * e[k] + (na > 0.0 ? e[k] * kM[k] * na : 0.0) + kL[k];
+          const T En = (T)log2(en), Eo = a.E[o];
+          a.E_out[o] = En;
+          a.Ebar[o] = (T)(na > 0.0 ? log2(na) + (double)a.mt[o] : NI);
+          const int c1 = t.c1[colk[k]], c2 = t.c2[colk[k]];
+          a.Es1[o] = c1 >= 0 ? a.E[base + c1] : (T)NI;
+          a.Es2[o] = c2 >= 0 ? a.E[base + c2] : (T)NI;
+          const T d = En - Eo;
+          ld = fmax(ld, (double)(d < T(0) ? -d : d));
+        }
+      if (a.max_diff) {
+        const double md = wg_max_of<BT>(ld, red);
+        if (tid == 0) a.max_diff[blockIdx.x] = (T)md;
+      }
+      return;
+    }
+    ok = true;
+#pragma unroll
+    for (int k = 0; k < CPT; ++k)
+      if (colk[k] >= 0) {
+        const double na = tot - ps[k];
+        const double eb = na > 0.0 ? kM[k] * na : 0.0;
+        const double en = kS[k] * e1[k] * e2[k] + kD[k] * e[k] * e[k] + e[k] * eb + kL[k];
+        // |log2(en / e)| < tol without a logarithm (e > 0)
+        if (!(en < e[k] * hi && en > e[k] * lo) && en != e[k]) ok = false;
+        e[k] = en;
+      }
+    ++it;
+  }
+#pragma unroll
+  for (int k = 0; k < CPT; ++k)
+    if (colk[k] >= 0) {
+      const size_t o = base + colk[k];
+      const double na = tot - ps[k];
+      a.E_out[o] = (T)log2(e[k]);
+      a.Es1[o] = (T)(h1[k] ? log2(e1[k]) : NI);
+      a.Es2[o] = (T)(c2p[k] != ZERO ? log2(e2[k]) : NI);
+      a.Ebar[o] = (T)(na > 0.0 ? log2(na) + (double)a.mt[o] : NI);
+    }
+  if (a.n_iter && tid == 0) a.n_iter[blockIdx.x] = it;
 }
 
 template <typename T>
@@ -173,49 +330,83 @@ struct EvArgs {
   double* work;  // [G, S] per-row contribution to grad_col
 };
 
-template <typename T, int CPT>
-__global__ __launch_bounds__(NT) void estep_vjp_kernel(OpsTree t, EvArgs<T> a) {
-  extern __shared__ double sm[];
-  double* X = sm;       // r, then path sums, then u / subtree sums
-  double* PC = sm + t.S;  // q0 + g_s1 / q0 + g_s2 of each column's parent
-  __shared__ double red[NW];
+// VJP of one E step of an item row, float64 at preorder positions: the path
+// sums as in estep_kernel, the subtree sums of u from one preorder scan, and
+// each parent hands its children their terms through LDS.
+template <typename T, int BT, int CPT>
+__global__ __launch_bounds__(BT) void estep_vjp_kernel(OpsTree t, EvArgs<T> a) {
+  constexpr int MAXS = BT * CPT, BW = BT / 64, ZERO = MAXS, SEG = 64 * CPT;
+  extern __shared__ __align__(16) unsigned char smraw[];
+  double* X = reinterpret_cast<double*>(smraw);  // r, then what each position gets from its parent
+  double* Q = X + MAXS + 64;                     // postorder scan, then the preorder scan of u
+  __shared__ double wP[BW], wQ[BW], red[BW];
   const int S = t.S;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const size_t base = (size_t)blockIdx.x * S;
   const double NI = -__builtin_inf();
-  double r[CPT], wbar[CPT], ge[CPT];
-  double lm = NI;
+  int colk[CPT], c2p[CPT], nex[CPT], qp[CPT], endm1[CPT];
+  bool h1[CPT];
+  double r[CPT], lm = NI;
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
+    const int i = tid * CPT + k;
+    colk[k] = -1;
+    c2p[k] = qp[k] = endm1[k] = ZERO;
+    nex[k] = 0;
+    h1[k] = false;
     r[k] = NI;
-    if (s < S) {
+    if (i < S) {
+      const int s = colk[k] = t.pcol[i];
+      const int c2 = t.pc2[i];
+      c2p[k] = c2 >= 0 ? c2 : ZERO;
+      h1[k] = t.pc1[i] >= 0;
+      nex[k] = t.pnex[i];
+      qp[k] = t.ppost[i];
+      endm1[k] = t.pend[s] - 1;
       r[k] = (double)a.E[base + s] + (a.use_col ? (double)a.col[s] : 0.0);
       lm = fmax(lm, r[k]);
-      PC[s] = 0.0;
     }
   }
-  const double M = block_max(lm, red);
+  if (tid < 64) X[MAXS + tid] = Q[MAXS + tid] = 0.0;
+  const double M = wg_max_of<BT>(lm, red);
   const double Ms = M == NI ? 0.0 : M;
-  double ls = 0.0;
+  // path sums of r
+  double sp[CPT], ta = 0.0;
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
-    if (s < S) {
-      r[k] = exp2(r[k] - Ms);
-      X[s] = r[k];
-      ls += r[k];
-    }
+    r[k] = colk[k] >= 0 ? exp2(r[k] - Ms) : 0.0;
+    ta += r[k];
+    sp[k] = ta;
   }
-  const double rowsum = block_sum(ls, red);
-  level_path_sums(t, X);
-  double lu = 0.0;
+  const double wa = wscan(ta);
+  own_store<CPT>(X, r);
+  if (lane == 63) wP[wv] = wa;
+  __syncthreads();
+  const double tp = kb::lds_wave_values<BW>(wP, lane, 0.0);
+  const double ip = wscan_first<BW>(tp);
+  const double rowsum = lane_of(ip, BW - 1);
+  const double offp = lane_of(ip - tp, wv) + (wa - ta);
+  double sq[CPT], tb = 0.0;
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
-    wbar[k] = 0.0;
-    ge[k] = 0.0;
-    if (s < S) {
-      const size_t i = base + s;
+    sq[k] = tb;
+    tb += X[qp[k]];
+  }
+  const double wb = wscan(tb);
+#pragma unroll
+  for (int k = 0; k < CPT; ++k) sq[k] += wb - tb;
+  own_store<CPT>(Q, sq);
+  if (lane == 63) wQ[wv] = wb;
+  __syncthreads();
+  const double tq = kb::lds_wave_values<BW>(wQ, lane, 0.0);
+  const double eq = wscan_first<BW>(tq) - tq;
+  double ge[CPT], u[CPT], tu = 0.0;
+#pragma unroll
+  for (int k = 0; k < CPT; ++k) {
+    ge[k] = u[k] = 0.0;
+    const double off = BW > 1 ? shfl_of(eq, nex[k] / SEG) : 0.0;
+    if (colk[k] >= 0) {
+      const size_t i = base + colk[k];
       const double En = a.En[i], E = a.E[i];
       const double gN = a.gN[i];
       const double t0 = (double)a.pS[i] + (double)a.Es1[i] + (double)a.Es2[i];
@@ -224,36 +415,40 @@ __global__ __launch_bounds__(NT) void estep_vjp_kernel(OpsTree t, EvArgs<T> a) {
       const double t3 = (double)a.pL[i];
       const double q0 = gN * exp2(t0 - En), q1 = gN * exp2(t1 - En);
       const double q2 = gN * exp2(t2 - En), q3 = gN * exp2(t3 - En);
-      wbar[k] = q2 + (double)a.gB[i];
+      const double wbar = q2 + (double)a.gB[i];
       a.gpS[i] = (T)q0;
       a.gpD[i] = (T)q1;
       a.gpL[i] = (T)q3;
-      a.gmt[i] = (T)wbar[k];
+      a.gmt[i] = (T)wbar;
       ge[k] = 2.0 * q1 + q2;
-      const int c1 = t.c1[s], c2 = t.c2[s];
-      if (c1 >= 0) PC[c1] = q0 + (double)a.g1[i];
-      if (c2 >= 0) PC[c2] = q0 + (double)a.g2[i];
-      const double denom = rowsum - X[s];
-      const double u = denom > 0.0 ? wbar[k] / denom : 0.0;
-      lu += u;
-      wbar[k] = u;  // reuse: u
+      if (h1[k]) X[tid * CPT + k + 1] = q0 + (double)a.g1[i];
+      if (c2p[k] != ZERO) X[c2p[k]] = q0 + (double)a.g2[i];
+      const double denom = rowsum - ((sp[k] + offp) - (Q[nex[k]] + off));
+      u[k] = denom > 0.0 ? wbar / denom : 0.0;
     }
+    tu += u[k];
+    sp[k] = tu;
   }
-  const double total_u = block_sum(lu, red);  // barrier: X reads and PC writes done
+  const double wu = wscan(tu);
 #pragma unroll
-  for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
-    if (s < S) X[s] = wbar[k];
-  }
+  for (int k = 0; k < CPT; ++k) sp[k] += wu - tu;  // wavefront-local inclusive scan of u
+  __syncthreads();  // Q was read
+  own_store<CPT>(Q, sp);
+  if (lane == 63) wP[wv] = wu;
   __syncthreads();
-  level_subtree_sums(t, X);
+  const double tv = kb::lds_wave_values<BW>(wP, lane, 0.0);
+  const double iv = wscan_first<BW>(tv);
+  const double ev = iv - tv;
+  const double total = lane_of(iv, BW - 1), offv = lane_of(ev, wv);
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
-    if (s < S) {
-      const double pv = r[k] * (total_u - X[s]);
-      a.gE[base + s] = (T)(ge[k] + PC[s] + pv);
-      a.work[base + s] = pv;
+    const double oe = BW > 1 ? shfl_of(ev, min(endm1[k], MAXS - 1) / SEG) : 0.0;
+    if (colk[k] >= 0) {
+      const int i = tid * CPT + k;
+      const double before = (sp[k] + offv) - u[k];
+      const double pv = r[k] * (before + (total - (Q[endm1[k]] + oe)));
+      a.gE[base + colk[k]] = (T)(ge[k] + (i > 0 ? X[i] : 0.0) + pv);
+      a.work[base + colk[k]] = pv;
     }
   }
 }
@@ -2223,6 +2418,43 @@ int kb_ops_max_states(int dtype) {
   return (int)std::min<size_t>(8192, s);
 }
 
+}  // extern "C"
+
+// The smallest shape that holds the tree (see estep_kernel).
+#define KBO_ESTEP_SHAPE(S, ...)                                                      \
+  do {                                                                               \
+    if ((S) <= 128) { constexpr int BT = 64, CPT = 2; __VA_ARGS__; }                 \
+    else if ((S) <= 256) { constexpr int BT = 128, CPT = 2; __VA_ARGS__; }           \
+    else if ((S) <= 512) { constexpr int BT = 256, CPT = 2; __VA_ARGS__; }           \
+    else if ((S) <= 1024) { constexpr int BT = 512, CPT = 2; __VA_ARGS__; }          \
+    else if ((S) <= 2048) { constexpr int BT = 512, CPT = 4; __VA_ARGS__; }          \
+    else if ((S) <= 4096) { constexpr int BT = 1024, CPT = 4; __VA_ARGS__; }         \
+    else { constexpr int BT = 1024, CPT = 8; __VA_ARGS__; }                          \
+  } while (0)
+
+template <typename T>
+static int launch_estep_rows(const kbo::OpsTree& t, const kbo::EsArgs<T>& a, hipStream_t st) {
+  KBO_ESTEP_SHAPE(t.S, {
+    const size_t lds = (size_t)2 * (BT * CPT + 64) * sizeof(double);
+    auto k = a.use_col ? kbo::estep_kernel<T, BT, CPT, true> : kbo::estep_kernel<T, BT, CPT, false>;
+    if (int rc = set_lds(k, lds)) return rc;
+    hipLaunchKernelGGL(k, dim3(a.G), dim3(BT), lds, st, t, a);
+  });
+  return 0;
+}
+template <typename T>
+static int launch_estep_vjp_rows(const kbo::OpsTree& t, const kbo::EvArgs<T>& a, hipStream_t st) {
+  KBO_ESTEP_SHAPE(t.S, {
+    const size_t lds = (size_t)2 * (BT * CPT + 64) * sizeof(double);
+    auto k = kbo::estep_vjp_kernel<T, BT, CPT>;
+    if (int rc = set_lds(k, lds)) return rc;
+    hipLaunchKernelGGL(k, dim3(a.G), dim3(BT), lds, st, t, a);
+  });
+  return 0;
+}
+
+extern "C" {
+
 int kb_estep(const kb_tree* tr, const kb_estep_io* io, void* stream) {
   if (!tr || !io) return kb::set_error(KB_ERR_ARG, "null argument");
   if (int rc = dtype_ok(io->dtype)) return rc;
@@ -2231,17 +2463,13 @@ int kb_estep(const kb_tree* tr, const kb_estep_io* io, void* stream) {
     return kb::set_error(KB_ERR_ARG, "max_iter must be >= 1 and tol > 0");
   if (io->G == 0) return 0;
   const int S = tr->S;
-  const size_t lds = (size_t)2 * S * sizeof(double);
-  if (int rc = check_lds(lds, S, KB_F64)) return rc;
   const kbo::OpsTree t = tr->dev();
   KBO_DISPATCH(io->dtype, S, {
     kbo::EsArgs<T> a{io->G, S, io->mode, io->use_col_weights, io->max_iter, io->tol,
                      (const T*)io->E, (const T*)io->log_pS, (const T*)io->log_pD, (const T*)io->log_pL,
                      (const T*)io->max_coupling, (const T*)io->col_log_probs,
                      (T*)io->E_out, (T*)io->E_s1, (T*)io->E_s2, (T*)io->Ebar, (T*)io->max_diff, io->n_iter};
-    auto k = kbo::estep_kernel<T, CPT>;
-    if (int rc = set_lds(k, lds)) return rc;
-    hipLaunchKernelGGL(k, dim3(io->G), dim3(kbo::NT), lds, st_of(stream), t, a);
+    if (int rc = launch_estep_rows<T>(t, a, st_of(stream))) return rc;
   });
   KBO_HIP(hipGetLastError());
   return 0;
@@ -2254,8 +2482,6 @@ namespace {
 // The E-step VJP launches with `work` ([G, S] float64) as the grad_col staging rows.
 int estep_vjp_launch(const kb_tree* tr, const kb_estep_vjp_io* io, double* work, void* stream) {
   const int S = tr->S;
-  const size_t lds = (size_t)2 * S * sizeof(double);
-  if (int rc = check_lds(lds, S, KB_F64)) return rc;
   const kbo::OpsTree t = tr->dev();
   KBO_DISPATCH(io->dtype, S, {
     kbo::EvArgs<T> a{io->G, S, io->use_col_weights,
@@ -2264,9 +2490,7 @@ int estep_vjp_launch(const kb_tree* tr, const kb_estep_vjp_io* io, double* work,
                      (const T*)io->g_E_new, (const T*)io->g_E_s1, (const T*)io->g_E_s2, (const T*)io->g_Ebar,
                      (T*)io->grad_E, (T*)io->grad_log_pS, (T*)io->grad_log_pD, (T*)io->grad_log_pL,
                      (T*)io->grad_max_coupling, work};
-    auto k = kbo::estep_vjp_kernel<T, CPT>;
-    if (int rc = set_lds(k, lds)) return rc;
-    hipLaunchKernelGGL(k, dim3(io->G), dim3(kbo::NT), lds, st_of(stream), t, a);
+    if (int rc = launch_estep_vjp_rows<T>(t, a, st_of(stream))) return rc;
     // grad_col += sum over item rows of the per-row contributions (fixed row order)
     hipLaunchKernelGGL((kbo::rows_sum_stage2<T>), dim3((S + 255) / 256), dim3(256), 0, st_of(stream), S, io->G,
                        (const double*)work, (T*)io->grad_col_log_probs);

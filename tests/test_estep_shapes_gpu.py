@@ -1,0 +1,73 @@
+"""The per-call E step, its fixed point and its VJP at the edges of their launch shapes, against the oracle.
+
+Item rows whose parameters all lie in [-400, 400] (log2) run in linear float64, any other row in
+log space: one row of each launch has a probability of 0 and one a rate of 2^-600.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+import kbench_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("leaves", [2, 64, 65, 128, 129, 256, 257, 512, 513, 1024, 1025, 2049])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_e_step_rows_match_oracle(leaves, weighted):
+    from kbench import synth
+    from kbench.core.kernels.e_step import e_fixed_point_triton, e_step_triton_autograd
+
+    rng = np.random.default_rng(leaves)
+    tree = synth.yule_tree(leaves, rng)
+    h = synth.state_helpers_from_tree(tree)
+    S, G = tree.S, 4
+    logits = rng.uniform(-3.0, -1.0, (G, S, 3))
+    r = O.log2_softmax(np.concatenate([np.zeros((G, S, 1)), logits], axis=-1))
+    pS, pD, pL, pT = (r[..., k].copy() for k in range(4))
+    pL[2, : leaves // 2] = -np.inf      # leaves that cannot go extinct by loss
+    pD[3, S - 1] = -600.0
+    col = np.log2(rng.dirichlet(np.full(S, 20.0))) if weighted else np.full(S, -np.log2(S))
+    otree = O.Tree.from_helpers(h)
+    norm = O.col_valid_log_normalizer(col, otree) if weighted else np.asarray(h["unnorm_row_max"])
+    mt = pT + norm
+    E0 = np.full((G, S), -1.0)
+    t = lambda a: torch.as_tensor(np.ascontiguousarray(a), dtype=torch.float64, device="cuda")
+    topo = [torch.as_tensor(np.asarray(h[k])).cuda() for k in ("node_parent", "node_child1", "node_child2")]
+    topo.append(int(h["max_ancestor_depth"]))
+    print(f"[e step] S={S} weighted={weighted}", flush=True)
+    params = [t(x) for x in (pS, pD, pL, mt)]
+    got = e_fixed_point_triton(t(E0), *params, t(col), *topo, max_iter=500, tol=1e-10, use_col_weights=weighted)
+    with np.errstate(all="ignore"):
+        want = [np.empty((G, S)) for _ in range(4)]
+        for g in range(G):  # rows stop on their own
+            row = lambda a: a[g:g + 1]
+            for o, x in zip(want, O.e_fixed_point(row(E0), row(pS), row(pD), row(pL), row(mt), col, otree, weighted,
+                                                  500, 1e-10)):
+                o[g] = x[0]
+    # an iterate at the stopping line may take one more step: 1e-10; the others' sum is a difference
+    # of prefix sums of S values (float64)
+    for name, a, b in zip(("E", "E_s1", "E_s2", "Ebar"), got, want):
+        a = a.cpu().numpy()
+        assert np.array_equal(np.isfinite(a), np.isfinite(b)), name
+        f = np.isfinite(b)
+        assert np.abs(a[f] - b[f]).max(initial=0.0) <= 1e-9, name
+    # one step and its VJP at that point
+    E = want[0]
+    cot = [rng.normal(size=(G, S)) for _ in range(4)]
+    for c, o in zip(cot, O.e_step(E, pS, pD, pL, mt, col, otree, weighted)):
+        c[~np.isfinite(o)] = 0.0  # (an output of -inf has no cotangent)
+    leaves_ = [x.requires_grad_(True) for x in (t(E), *(p.clone() for p in params), t(col))]
+    out = e_step_triton_autograd(*leaves_, *topo, use_col_weights=weighted)
+    with np.errstate(all="ignore"):
+        ref = O.e_step(E, pS, pD, pL, mt, col, otree, weighted)
+        ref_g = O.e_step_vjp(E, pS, pD, pL, mt, col, otree, weighted, *cot)
+    for a, b in zip(out, ref):
+        a = a.detach().cpu().numpy()
+        assert np.array_equal(np.isfinite(a), np.isfinite(b))
+        f = np.isfinite(b)
+        assert np.abs(a[f] - b[f]).max(initial=0.0) <= 1e-10
+    grads = torch.autograd.grad(out, leaves_, grad_outputs=[t(c) for c in cot])
+    for name, a, b in zip(("E", "pS", "pD", "pL", "mt", "col"), grads, ref_g):
+        assert np.abs(a.cpu().numpy() - b).max() <= 1e-10 * max(1.0, np.abs(b).max()), name
