@@ -1440,35 +1440,39 @@ __global__ __launch_bounds__(NT) void wave_bwd_kernel(OpsTree t, WbArgs<T> a) {
   }
 }
 
-// float32 rows at preorder ownership (thread t owns positions t*CPT + k, as
-// the whole-pass backward row kernel): the root-path sums of p' from an
-// inclusive preorder and an exclusive postorder scan, one barrier per Neumann
-// term (wavefront-local scans published, the readers add the wavefront
-// offsets), and the [W, S] outputs written back in column order through LDS.
-// Same mathematics as wave_bwd_kernel.
-template <int CPT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kb::pre_waves_per_eu(CPT)))) void wave_bwd_pre_kernel(OpsTree t, WbArgs<float> a) {
-  constexpr int MAXS = NT * CPT;
+// Rows at preorder ownership (thread t owns positions t*CPT + k, as the
+// whole-pass backward row kernel): the root-path sums of p' from an inclusive
+// preorder and an exclusive postorder scan, one barrier per Neumann term
+// (wavefront-local scans published, the readers add the wavefront offsets),
+// and the [W, S] outputs written back in column order through LDS.  Same
+// mathematics as wave_bwd_kernel.  Shapes and figures: launch_wave_bwd.
+template <typename T>
+constexpr int wave_bwd_waves(int cpt) { return cpt > 2 ? 1 : std::is_same_v<T, float> ? 8 : 4; }
+
+template <typename T, int BT, int CPT>
+__global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(wave_bwd_waves<T>(CPT)))) void wave_bwd_pre_kernel(OpsTree t, WbArgs<T> a) {
+  constexpr int BW = BT / 64;
+  constexpr int MAXS = BT * CPT;
   constexpr int LD = MAXS + 64;  // [MAXS] is the padding slot, kept at 0
   constexpr int ZERO = MAXS;
   constexpr int SEG = 64 * CPT;  // postorder slots per wavefront
   extern __shared__ __align__(16) unsigned char smraw[];
-  float* L0 = reinterpret_cast<float*>(smraw);
-  float* L1 = L0 + LD;
-  float* L2 = L1 + LD;
-  float* L3 = L2 + LD;
-  __shared__ float wA[NW], wB[NW];
+  T* L0 = reinterpret_cast<T*>(smraw);
+  T* L1 = L0 + LD;
+  T* L2 = L1 + LD;
+  T* L3 = L2 + LD;
+  __shared__ T wA[BW], wB[BW];
   const int S = a.S;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int w = blockIdx.x;
   const long long grow = a.ws + w;
   const size_t ob = (size_t)w * S;
-  const float NI = -__builtin_inff();
+  const T NI = ninf<T>();
   const bool act = a.active ? a.active[w] != 0 : true;
   if (!act) {
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
-      const int s = tid + k * NT;
+      const int s = tid + k * BT;
       if (s < S) {
         a.v[ob + s] = 0;
         a.aw0[ob + s] = 0;
@@ -1480,18 +1484,18 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kb::pre_wave
         a.col_rows[ob + s] = 0;
       }
     }
-    if (a.relres && tid == 0) a.relres[w] = 0.0f;
+    if (a.relres && tid == 0) a.relres[w] = T(0.0);
     return;
   }
   const long long item = a.item ? a.item[grow] : 0;
   const size_t cb = a.clayout == 1 ? ob : (a.clayout == 2 ? (size_t)item * S : 0);
-  const float* pirow = a.Pi + (size_t)grow * S;
-  const float* pbrow = a.Pibar + (size_t)grow * S;
-  const float rms = msafe(a.rowmax[grow]);
+  const T* pirow = a.Pi + (size_t)grow * S;
+  const T* pbrow = a.Pibar + (size_t)grow * S;
+  const T rms = msafe(a.rowmax[grow]);
   // Pi and Pibar to their preorder positions (coalesced column reads)
 #pragma unroll
   for (int j = 0; j < CPT; ++j) {
-    const int sc = tid + j * NT;
+    const int sc = tid + j * BT;
     if (sc < S) {
       const int p = t.ppos[sc];
       L0[p] = pirow[sc];
@@ -1499,17 +1503,17 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kb::pre_wave
     }
   }
   if (tid < 64) {
-    L0[MAXS + tid] = 0.0f;
-    L1[MAXS + tid] = 0.0f;
-    L2[MAXS + tid] = 0.0f;
-    L3[MAXS + tid] = 0.0f;
+    L0[MAXS + tid] = T(0.0);
+    L1[MAXS + tid] = T(0.0);
+    L2[MAXS + tid] = T(0.0);
+    L3[MAXS + tid] = T(0.0);
   }
   // own positions: column, children, parent, subtree end - 1, postorder slot, tin - i
   int colk[CPT], c1p[CPT], c2p[CPT], ppar[CPT], endm1[CPT], wend[CPT], qp[CPT], nex[CPT];
   bool okp[CPT];
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    const int i = kb::own_pos_c<NT, CPT>(k);
+    const int i = kb::own_pos_c<BT, CPT>(k);
     okp[k] = i < S;
     colk[k] = okp[k] ? t.pcol[i] : 0;
     c1p[k] = okp[k] ? t.pc1[i] : -1;
@@ -1522,74 +1526,74 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kb::pre_wave
     nex[k] = okp[k] ? t.pnex[i] : 0;
   }
   __syncthreads();
-  float piv[CPT], pbv[CPT];
-  kb::lds_load_own<CPT>(L0, piv);
-  kb::lds_load_own<CPT>(L1, pbv);
+  T piv[CPT], pbv[CPT];
+  own_load<CPT>(L0, piv);
+  own_load<CPT>(L1, pbv);
   // p' = 2^(col + Pi - rowmax) and its root-path sums ps(i) = Pre(i) - PostEx(tin(i) - i)
-  float pp[CPT], sp[CPT], ta = 0.0f;
+  T pp[CPT], sp[CPT], ta = T(0.0);
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    pp[k] = okp[k] ? xexp2((a.use_col ? a.col[colk[k]] + piv[k] : piv[k]) - rms) : 0.0f;
+    pp[k] = okp[k] ? xexp2((a.use_col ? a.col[colk[k]] + piv[k] : piv[k]) - rms) : T(0.0);
     ta += pp[k];
     sp[k] = ta;
   }
-  const float wa = kb::wave_scan_incl(ta);
-  kb::lds_store_own<CPT>(L2, pp);
+  const T wa = wscan(ta);
+  own_store<CPT>(L2, pp);
   if (lane == 63) wA[wv] = wa;
   __syncthreads();
-  float ps[CPT], ch1[CPT], ch2[CPT], row_sum;
+  T ps[CPT], ch1[CPT], ch2[CPT], row_sum;
   {
-    const float tp = kb::lds_wave_values<NW>(wA, lane, 0.0f);
-    float yq[CPT];
+    const T tp = kb::lds_wave_values<BW>(wA, lane, T(0));
+    T yq[CPT];
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       yq[k] = L2[qp[k]];
       ch1[k] = c1p[k] >= 0 ? L0[c1p[k]] : NI;
       ch2[k] = c2p[k] >= 0 ? L0[c2p[k]] : NI;
     }
-    const float ip = kb::wave_scan_first<NW>(tp);
-    row_sum = kb::lane_value(ip, NW - 1);
-    const float offp = kb::lane_value(ip - tp, wv) + (wa - ta);
-    float sq[CPT], tb = 0.0f;
+    const T ip = wscan_first<BW>(tp);
+    row_sum = lane_of(ip, BW - 1);
+    const T offp = lane_of(ip - tp, wv) + (wa - ta);
+    T sq[CPT], tb = T(0.0);
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       sq[k] = tb;
       tb += yq[k];
     }
-    const float wb = kb::wave_scan_incl(tb);
+    const T wb = wscan(tb);
 #pragma unroll
     for (int k = 0; k < CPT; ++k) sq[k] += wb - tb;
-    kb::lds_store_own<CPT>(L3, sq);
+    own_store<CPT>(L3, sq);
     if (lane == 63) wB[wv] = wb;
     __syncthreads();
-    const float tq = kb::lds_wave_values<NW>(wB, lane, 0.0f);
-    const float eq = kb::wave_scan_first<NW>(tq) - tq;
+    const T tq = kb::lds_wave_values<BW>(wB, lane, T(0.0));
+    const T eq = wscan_first<BW>(tq) - tq;
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       const int n = nex[k];
-      ps[k] = (sp[k] + offp) - (L3[n] + __shfl(eq, n / SEG, 64));
+      ps[k] = (sp[k] + offp) - (L3[n] + shfl_of(eq, n / SEG));
     }
   }
   // J^T coefficients; the child-edge weights (q3 into child1, q4 into child2)
   // scattered by the parent's owner into L1; the rhs and initial rows staged
   // into L2 / L0 (free since the scans above), all under one barrier
   const long long lstate = a.use_leaf ? a.leaf_state[grow] : -1;
-  float diag[CPT], pcoef[CPT], q[6][CPT];
+  T diag[CPT], pcoef[CPT], q[6][CPT];
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    diag[k] = pcoef[k] = 0.0f;
+    diag[k] = pcoef[k] = T(0.0);
 #pragma unroll
-    for (int j = 0; j < 6; ++j) q[j][k] = 0.0f;
+    for (int j = 0; j < 6; ++j) q[j][k] = T(0.0);
     if (okp[k]) {
       const int s = colk[k];
       const size_t ci = cb + s;
-      const float pi = piv[k];
-      const float t0 = a.DL[ci] + pi;
-      const float t1 = pi + a.Ebar[ci];
-      const float t2 = pbv[k] + a.E[ci];
-      const float t3 = a.SL1[ci] + ch1[k];
-      const float t4 = a.SL2[ci] + ch2[k];
-      float t5 = NI;
+      const T pi = piv[k];
+      const T t0 = a.DL[ci] + pi;
+      const T t1 = pi + a.Ebar[ci];
+      const T t2 = pbv[k] + a.E[ci];
+      const T t3 = a.SL1[ci] + ch1[k];
+      const T t4 = a.SL2[ci] + ch2[k];
+      T t5 = NI;
       if (a.use_leaf) {
         if (lstate == s) {
           if (a.leaf_mode == 3) t5 = a.leaf_logp[0];
@@ -1600,26 +1604,26 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kb::pre_wave
       } else if (a.leaf_term) {
         t5 = a.leaf_term[ob + s];
       }
-      const float m = tmax(tmax(tmax(t0, t1), tmax(t2, t3)), tmax(t4, t5));
-      const float ms = msafe(m);
-      const float e0 = xexp2(t0 - ms), e1 = xexp2(t1 - ms), e2 = xexp2(t2 - ms);
-      const float e3 = xexp2(t3 - ms), e4 = xexp2(t4 - ms), e5 = xexp2(t5 - ms);
-      const float sum = e0 + e1 + e2 + e3 + e4 + e5;
-      const float isum = sum > 0.0f ? 1.0f / sum : 0.0f;
-      float wl = 1.0f;
+      const T m = tmax(tmax(tmax(t0, t1), tmax(t2, t3)), tmax(t4, t5));
+      const T ms = msafe(m);
+      const T e0 = xexp2(t0 - ms), e1 = xexp2(t1 - ms), e2 = xexp2(t2 - ms);
+      const T e3 = xexp2(t3 - ms), e4 = xexp2(t4 - ms), e5 = xexp2(t5 - ms);
+      const T sum = e0 + e1 + e2 + e3 + e4 + e5;
+      const T isum = sum > T(0.0) ? T(1.0) / sum : T(0.0);
+      T wl = T(1.0);
       if (a.dts) {
-        const float dl = xlog2(sum) + m;
-        const float dr = a.dts[ob + s];
-        const float pm = tmax(dl, dr);
-        const float pms = msafe(pm);
-        const float pnew = xlog2(xexp2(dl - pms) + xexp2(dr - pms)) + pm;
-        wl = dl != NI ? xexp2(dl - pnew) : 0.0f;
+        const T dl = xlog2(sum) + m;
+        const T dr = a.dts[ob + s];
+        const T pm = tmax(dl, dr);
+        const T pms = msafe(pm);
+        const T pnew = xlog2(xexp2(dl - pms) + xexp2(dr - pms)) + pm;
+        wl = dl != NI ? xexp2(dl - pnew) : T(0.0);
       }
-      const float denom = row_sum - ps[k];
-      const float idn = denom > 0.0f ? 1.0f / denom : 0.0f;
+      const T denom = row_sum - ps[k];
+      const T idn = denom > T(0.0) ? T(1.0) / denom : T(0.0);
       diag[k] = wl * (e0 + e1) * isum;
       pcoef[k] = wl * e2 * isum * idn;
-      const float c = wl * isum;
+      const T c = wl * isum;
       q[0][k] = c * e0;
       q[1][k] = c * e1;
       q[2][k] = c * e2;
@@ -1632,7 +1636,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kb::pre_wave
   }
 #pragma unroll
   for (int j = 0; j < CPT; ++j) {
-    const int sc = tid + j * NT;
+    const int sc = tid + j * BT;
     if (sc < S) {
       const int p = t.ppos[sc];
       L2[p] = a.rhs[ob + sc];
@@ -1640,51 +1644,63 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kb::pre_wave
     }
   }
   __syncthreads();
-  float edge[CPT], rh[CPT], v[CPT], term[CPT];
-  kb::lds_load_own<CPT>(L1, edge);
-  kb::lds_load_own<CPT>(L2, rh);
-  if (a.v0) kb::lds_load_own<CPT>(L0, v);
+  T edge[CPT], rh[CPT], v[CPT], term[CPT];
+  own_load<CPT>(L1, edge);
+  own_load<CPT>(L2, rh);
+  if (a.v0) own_load<CPT>(L0, v);
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    edge[k] = ppar[k] != ZERO ? edge[k] : 0.0f;
-    if (!okp[k]) rh[k] = 0.0f;
+    edge[k] = ppar[k] != ZERO ? edge[k] : T(0.0);
+    if (!okp[k]) rh[k] = T(0.0);
     // Neumann: term_0 = rhs; fixed point from initial_v: the term is v itself
-    v[k] = a.v0 ? (okp[k] ? v[k] : 0.0f) : rh[k];
+    v[k] = a.v0 ? (okp[k] ? v[k] : T(0.0)) : rh[k];
     term[k] = v[k];
   }
   // Neumann series v = sum_{n <= N} (J^T)^n rhs, or N steps of v <- rhs + J^T v.
   // Buffers alternate by parity: (Tb, Lb) = (L0, L2) for even terms, (L1, L3)
   // for odd ones; every thread read its own L0..L2 entries above, and the
   // other threads' entries are read only after each term's barrier.
-  auto neumann_term = [&](float* Tb, float* Lb, float* wt) {
-    float sc[CPT];
+  // the scan of u at the own positions, wavefront-local, published in Lb / wt
+  auto publish_scan = [&](const T (&u)[CPT], T (&sc)[CPT], T* Lb, T* wt) {
 #pragma unroll
-    for (int k = 0; k < CPT; ++k) sc[k] = term[k] * pcoef[k] + (k > 0 ? sc[k - 1] : 0.0f);
-    const float tsum = sc[CPT - 1];
-    const float ws = kb::wave_scan_incl(tsum);
+    for (int k = 0; k < CPT; ++k) sc[k] = u[k] + (k > 0 ? sc[k > 0 ? k - 1 : 0] : T(0));
+    const T tsum = sc[CPT - 1];
+    const T ws = wscan(tsum);
     if (lane == 63) wt[wv] = ws;
 #pragma unroll
     for (int k = 0; k < CPT; ++k) sc[k] += ws - tsum;
-    kb::lds_store_own<CPT>(Lb, sc);
-    kb::lds_store_own<CPT>(Tb, term);
-    __syncthreads();
-    float le[CPT], tpar[CPT];
+    own_store<CPT>(Lb, sc);
+  };
+  // after a barrier: the sum of u outside each own position's subtree
+  auto outside = [&](const T (&sc)[CPT], const T* Lb, const T* wt, T (&x)[CPT]) {
+    T le[CPT];
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) le[k] = Lb[endm1[k]];
+    const T wtot = kb::lds_wave_values<BW>(wt, lane, T(0));
+    const T wincl = wscan_first<BW>(wtot);
+    const T wexcl = wincl - wtot;
+    const T A = lane_of(wincl, BW - 1);
+    const T woff = lane_of(wexcl, wv);
+    const T p0 = prev_lane(sc[CPT - 1]) + woff;
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
-      le[k] = Lb[endm1[k]];
-      tpar[k] = Tb[ppar[k]];
+      const T pm1 = k == 0 ? p0 : sc[k > 0 ? k - 1 : 0] + woff;
+      x[k] = pm1 + (A - (le[k] + (BW > 1 ? shfl_of(wexcl, wend[k]) : T(0))));
     }
-    const float wtot = lane < NW ? wt[lane] : 0.0f;
-    const float wincl = kb::wave_scan_first<NW>(wtot);
-    const float wexcl = wincl - wtot;
-    const float A = kb::lane_value(wincl, NW - 1);
-    const float woff = kb::lane_value(wexcl, wv);
-    const float p0 = kb::wave_prev_lane(sc[CPT - 1]) + woff;
+  };
+  auto neumann_term = [&](T* Tb, T* Lb, T* wt) {
+    T u[CPT], sc[CPT], tpar[CPT], x[CPT];
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) u[k] = term[k] * pcoef[k];
+    publish_scan(u, sc, Lb, wt);
+    own_store<CPT>(Tb, term);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) tpar[k] = Tb[ppar[k]];
+    outside(sc, Lb, wt, x);
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
-      const float pm1 = k == 0 ? p0 : sc[k - 1] + woff;
-      const float nt = term[k] * diag[k] + pp[k] * (pm1 + (A - (le[k] + __shfl(wexcl, wend[k], 64)))) +
-                       tpar[k] * edge[k];
+      const T nt = term[k] * diag[k] + pp[k] * x[k] + tpar[k] * edge[k];
       if (a.v0) {
         v[k] = rh[k] + nt;
         term[k] = v[k];
@@ -1703,29 +1719,29 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kb::pre_wave
     if (n < a.n_terms) neumann_term(L0, L2, wA);
   }
   // column gradient p' (A - subtree(v pcoef)), in the next parity's buffers
-  float colg[CPT];
+  T colg[CPT];
   {
     const int n = a.n_terms;
-    float* Pb = (n & 1) ? L3 : L2;
-    float* wt = (n & 1) ? wB : wA;
-    float u[CPT], sc[CPT], pm1[CPT], rest[CPT];
+    T* Pb = (n & 1) ? L3 : L2;
+    T* wt = (n & 1) ? wB : wA;
+    T u[CPT], sc[CPT], x[CPT];
 #pragma unroll
     for (int k = 0; k < CPT; ++k) u[k] = v[k] * pcoef[k];
-    kb::local_scan_publish<NT, CPT>(sc, u, Pb, wt);
+    publish_scan(u, sc, Pb, wt);
     __syncthreads();
-    kb::subtree_terms<NT, CPT>(sc, Pb, wt, endm1, wend, pm1, rest);
+    outside(sc, Pb, wt, x);
 #pragma unroll
-    for (int k = 0; k < CPT; ++k) colg[k] = okp[k] ? pp[k] * (pm1[k] + rest[k]) : 0.0f;
+    for (int k = 0; k < CPT; ++k) colg[k] = okp[k] ? pp[k] * x[k] : T(0);
   }
   // outputs in column order, four rows at a time through L0..L3
-  float* const outs[8] = {a.v, a.aw0, a.aw1, a.aw2, a.aw3, a.aw4, a.aw345, a.col_rows};
+  T* const outs[8] = {a.v, a.aw0, a.aw1, a.aw2, a.aw3, a.aw4, a.aw345, a.col_rows};
 #pragma unroll
   for (int half = 0; half < 2; ++half) {
     __syncthreads();  // the previous readers of L0..L3 are done
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int o = 4 * half + r;
-      float x[CPT];
+      T x[CPT];
 #pragma unroll
       for (int k = 0; k < CPT; ++k) {
         if (o == 0) x[k] = v[k];
@@ -1733,32 +1749,33 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kb::pre_wave
         else if (o == 6) x[k] = v[k] * (q[3][k] + q[4][k] + q[5][k]);
         else x[k] = v[k] * q[o - 1][k];
       }
-      kb::lds_store_own<CPT>(L0 + r * LD, x);
+      own_store<CPT>(L0 + r * LD, x);
     }
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      float* dst = outs[4 * half + r] + ob;
+      T* dst = outs[4 * half + r] + ob;
 #pragma unroll
       for (int j = 0; j < CPT; ++j) {
-        const int sc = tid + j * NT;
+        const int sc = tid + j * BT;
         if (sc < S) dst[sc] = L0[r * LD + t.ppos[sc]];
       }
     }
   }
   if (a.relres) {
-    float ln = 0.0f, lv = 0.0f;
+    T ln = T(0), lv = T(0);
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
-      ln += term[k] * term[k];
-      lv += v[k] * v[k];
+      const float tf = (float)term[k], vf = (float)v[k];
+      ln += (T)(tf * tf);
+      lv += (T)(vf * vf);
     }
-    const float n2 = block_sum(ln, wA);
-    const float v2 = block_sum(lv, wB);
+    const T n2 = wg_sum_of<BT>(ln, wA);
+    const T v2 = wg_sum_of<BT>(lv, wB);
     if (tid == 0) {
       const float tiny = 1.17549435e-38f;
-      const float den = fmaxf(sqrtf(v2), tiny);
-      a.relres[w] = a.n_terms > 0 ? sqrtf(n2) / den : 0.0f;
+      const float den = fmaxf(sqrtf((float)v2), tiny);
+      a.relres[w] = a.n_terms > 0 ? sqrtf((float)n2) / den : 0.0f;
     }
   }
 }
@@ -2549,17 +2566,30 @@ int launch_wave_step(const kbo::OpsTree& t, const kbo::WsArgs<T>& a, int W, hipS
   return launch_step<T, 1024, 8>(t, a, W, st);
 }
 
-// float32 rows of the per-call wave backward run the preorder-ownership kernel
-template <typename T, int CPT>
+template <typename T, int BT, int CPT>
+int launch_bwd(const kbo::OpsTree& t, const kbo::WbArgs<T>& a, int W, hipStream_t st) {
+  const size_t lds = (size_t)4 * (BT * CPT + 64) * sizeof(T);
+  auto k = kbo::wave_bwd_pre_kernel<T, BT, CPT>;
+  if (int rc = set_lds(k, lds)) return rc;
+  hipLaunchKernelGGL(k, dim3(W), dim3(BT), lds, st, t, a);
+  return 0;
+}
+
+// The preorder-ownership kernel on the smallest shape that holds the row; its
+// four padded LDS rows do not hold doubles past 4096 states, where the
+// column-order kernel (four rows of S) goes on.
+template <typename T>
 int launch_wave_bwd(const kbo::OpsTree& t, const kbo::WbArgs<T>& a, int W, size_t lds, hipStream_t st) {
-  if constexpr (std::is_same_v<T, float>) {
-    const size_t lds_pre = (size_t)4 * (kbo::NT * CPT + 64) * sizeof(float);
-    auto k = kbo::wave_bwd_pre_kernel<CPT>;
-    if (int rc = set_lds(k, lds_pre)) return rc;
-    hipLaunchKernelGGL(k, dim3(W), dim3(kbo::NT), lds_pre, st, t, a);
-    return 0;
-  }
-  auto k = kbo::wave_bwd_kernel<T, CPT>;
+  constexpr bool F32 = std::is_same_v<T, float>;
+  const int S = t.S;
+  if (S <= 128) return launch_bwd<T, 64, 2>(t, a, W, st);
+  if (S <= 256) return launch_bwd<T, 128, 2>(t, a, W, st);
+  if (S <= 512) return launch_bwd<T, 256, 2>(t, a, W, st);
+  if (S <= 1024) return launch_bwd<T, 512, 2>(t, a, W, st);
+  if (S <= 2048) return launch_bwd<T, 1024, 2>(t, a, W, st);
+  if (S <= 4096) return launch_bwd<T, 1024, 4>(t, a, W, st);
+  if constexpr (F32) return launch_bwd<T, 1024, 8>(t, a, W, st);
+  auto k = kbo::wave_bwd_kernel<T, 8>;
   if (int rc = set_lds(k, lds)) return rc;
   hipLaunchKernelGGL(k, dim3(W), dim3(kbo::NT), lds, st, t, a);
   return 0;
@@ -2693,7 +2723,7 @@ int kb_wave_backward(const kb_tree* tr, const kb_wave_bwd_io* io, void* stream) 
                      (const T*)io->col_log_probs, io->item_idx, io->leaf_state, (const T*)io->leaf_logp,
                      (const T*)io->leaf_term, (T*)io->v, (T*)io->aw0, (T*)io->aw1, (T*)io->aw2, (T*)io->aw345,
                      (T*)io->aw3, (T*)io->aw4, (T*)io->col_rows, io->relres};
-    if (int rc = launch_wave_bwd<T, CPT>(t, a, io->W, lds, st_of(stream))) return rc;
+    if (int rc = launch_wave_bwd<T>(t, a, io->W, lds, st_of(stream))) return rc;
   });
   KBO_HIP(hipGetLastError());
   return 0;

@@ -175,6 +175,9 @@ __device__ __forceinline__ double lane_of(double x, int l) { return kb::lane_val
 __device__ __forceinline__ float shfl_of(float x, int l) { return __shfl(x, l, 64); }
 __device__ __forceinline__ double shfl_of(double x, int l) { return kb::shfl_f64(x, l); }
 
+__device__ __forceinline__ float prev_lane(float x) { return kb::wave_prev_lane(x); }
+__device__ __forceinline__ double prev_lane(double x) { return kb::wave_prev_lane_f64(x); }
+
 template <int CTRL, int ROW_MASK = 0xf>
 __device__ __forceinline__ float dpp_ninf(float x) {  // lanes without a source read -inf
   return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(-__builtin_inff()), __float_as_int(x), CTRL,
