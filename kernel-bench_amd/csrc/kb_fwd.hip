@@ -283,10 +283,13 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
   constexpr bool OMT = CPT == 8;
   int c2p[CPT], nex[CPT], qp[CPT], pre_s[CPT];
   bool h1[CPT];
-  // Below 1024 threads the tables and row constants are read with one vector
-  // load per row (they start their allocations); the 1024 x 2 shape keeps one
-  // load per position, which measured faster there.
-  constexpr bool VEC = NT < 1024;
+  // The tables and row constants are read with one vector load per row (they
+  // start their allocations): with one load per position a wavefront's read is
+  // spread over CPT times its bytes (with the row constants of the leaf, split
+  // and output phases: whole solves of 8191 states 12.1 -> 10.9 ms, of 3001
+  // weighted states 2.75 -> 2.64 ms).  The 1024 x 2 shape keeps one load per
+  // position, which measured faster there.
+  constexpr bool VEC = CPT > 2 || NT < 1024;
   if constexpr (VEC) {
     int a[CPT], tn[CPT];
     gld_own<CPT>(T.c1pos, S, a, -1);
@@ -364,6 +367,24 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
     const int lend = T.endpos[lpos];
     leaf_obs = P.pS[lpos];
     const float leaf_col = WEIGHTED ? P.col[lpos] : 0.0f;
+    // a row constant at the own positions (rows of four or more positions per
+    // thread: one vector load; the others' loads per position measured faster
+    // in this phase)
+    auto kc_own = [&](const float* c, float (&x)[CPT]) {
+      if constexpr (CPT > 2 && NT == 1024) {
+        gld_own<CPT>(c, S, x, 0.0f);
+      } else {
+#pragma unroll
+        for (int k = 0; k < CPT; ++k) x[k] = own_pos_c<NT, CPT>(k) < S ? c[own_pos_c<NT, CPT>(k)] : 0.0f;
+      }
+    };
+    float kmt[CPT], kDL[CPT], kEb[CPT], kE[CPT], kS1[CPT], kS2[CPT];
+    kc_own(P.mt, kmt);
+    kc_own(P.DL, kDL);
+    kc_own(P.Ebar, kEb);
+    kc_own(P.E, kE);
+    kc_own(P.SL1, kS1);
+    kc_own(P.SL2, kS2);
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       const int i = own_pos_c<NT, CPT>(k);
@@ -371,17 +392,16 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
       if (i < S) {
         const bool hit = i == lpos;
         const bool desc = i >= lpos && i < lend;
-        const int ci = i;
         const float pi_w = hit ? leaf_obs : KB_NEG_INF;
-        const float pibar_w = desc ? KB_NEG_INF : P.mt[ci] + leaf_col + leaf_obs;
+        const float pibar_w = desc ? KB_NEG_INF : kmt[k] + leaf_col + leaf_obs;
         const float pi_s1 = (h1[k] && i + 1 == lpos) ? leaf_obs : KB_NEG_INF;
         const float pi_s2 = c2p[k] == lpos ? leaf_obs : KB_NEG_INF;  // padding ZERO never equals lpos
-        const float t0 = P.DL[ci] + pi_w;
-        const float t1 = pi_w + P.Ebar[ci];
-        const float t2 = pibar_w + P.E[ci];
-        const float t3 = P.SL1[ci] + pi_s1;
-        const float t4 = P.SL2[ci] + pi_s2;
-        const float t5 = hit ? P.pS[ci] : KB_NEG_INF;
+        const float t0 = kDL[k] + pi_w;
+        const float t1 = pi_w + kEb[k];
+        const float t2 = pibar_w + kE[k];
+        const float t3 = kS1[k] + pi_s1;
+        const float t4 = kS2[k] + pi_s2;
+        const float t5 = hit ? leaf_obs : KB_NEG_INF;
         const float m = fmaxf(fmaxf(fmaxf(t0, t1), fmaxf(t2, t3)), fmaxf(t4, t5));
         const float ms = fsafe(m);
         const float sum = exp2_hw(t0 - ms) + exp2_hw(t1 - ms) + exp2_hw(t2 - ms) + exp2_hw(t3 - ms) +
@@ -399,6 +419,10 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
       acc[k] = 0.0f;
     }
     const int b = P.split_ptr[row], e = P.split_ptr[row + 1];
+    if constexpr (!EARLY && NT == 1024) {
+      gld_own<CPT>(P.pD, S, kd, 0.0f);
+      gld_own<CPT>(P.pS, S, ks, 0.0f);
+    }
     for (int si = b; si < e; ++si) {
       const size_t l = (size_t)P.split_l[si] * S, r = (size_t)P.split_r[si] * S;
       const float lsp = P.split_lsp[si];
@@ -427,7 +451,7 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
         const int i = own_pos_c<NT, CPT>(k);
         if (i < S) {
           const bool h2 = c2p[k] != ZERO;
-          const float d = EARLY ? kd[k] : P.pD[i], sp = EARLY ? ks[k] : P.pS[i];
+          const float d = EARLY || NT == 1024 ? kd[k] : P.pD[i], sp = EARLY || NT == 1024 ? ks[k] : P.pS[i];
           const float t0 = lsp + d + pl[k] + pr[k];
           const float t1 = lsp + pl[k] + br[k];
           const float t2 = lsp + pr[k] + bl[k];
@@ -565,17 +589,23 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
   const float M = Ms + (float)kexp;
   float piv[CPT], pbv[CPT];
   float lmax = KB_NEG_INF;
+  float omt[CPT], ocol[CPT];
+  if constexpr (CPT > 2 && NT == 1024) {
+    gld_own<CPT>(P.mt, S, omt, 0.0f);
+    if constexpr (WEIGHTED) gld_own<CPT>(P.col, S, ocol, 0.0f);
+  }
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
     const int i = own_pos_c<NT, CPT>(k);
     piv[k] = KB_NEG_INF;
     pbv[k] = KB_NEG_INF;
     if (i < S) {
+      const float mt = CPT > 2 && NT == 1024 ? omt[k] : P.mt[i];
       const float x = y[k] * f;
       piv[k] = x > 0.0f ? log2f(x) + M : KB_NEG_INF;
       const float na = rowsum - ps[k] * f;
-      pbv[k] = na > 0.0f ? log2f(na) + M + P.mt[i] : KB_NEG_INF;
-      lmax = fmaxf(lmax, WEIGHTED ? P.col[i] + piv[k] : piv[k]);
+      pbv[k] = na > 0.0f ? log2f(na) + M + mt : KB_NEG_INF;
+      lmax = fmaxf(lmax, WEIGHTED ? (CPT > 2 && NT == 1024 ? ocol[k] : P.col[i]) + piv[k] : piv[k]);
     }
   }
   // Lb[2], Lb[3] are unused since the staging
