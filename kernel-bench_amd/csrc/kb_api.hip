@@ -726,7 +726,6 @@ int kb_plan_create(const kb_layout* L, kb_plan** out) {
         const int pa = ok && ppos[i] >= 0 ? ppos[i] : zero;
         const int e1 = ok ? endpos[i] - 1 : zero;
         om[kb::OMT_PK * (size_t)ld + o] = pa | (e1 << 16) | ((ok && ppos[i] >= 0 && pflag[i]) ? (1 << 30) : 0);
-        om[kb::OMT_PN * (size_t)ld + o] = ok ? (post[i] | ((tin[i] - i) << 16)) : zero;
       }
       rc |= upload(&p->d_om_tab, om);
     }
@@ -889,10 +888,9 @@ static int forward_setup(kb_plan* p, const kb_forward_io* io, hipStream_t st, kb
   F.row_kind = p->d_row_kind;
   F.dup_ptr = p->d_dup_ptr;
   F.dup_rows = p->d_dup_rows;
-  F.om_tab = p->d_om_tab;
   {
-    // rows of 4097..8192 states: the contiguous-ownership kernel on the
-    // owner-major tables (KB_FWD_LARGE=0: the Euler-tour kernel)
+    // rows of 4097..8192 states: the contiguous-ownership kernel
+    // (KB_FWD_LARGE=0: the Euler-tour kernel)
     const char* lv = getenv("KB_FWD_LARGE");
     F.large = (lv && lv[0] == '0') ? 0 : 1;
   }

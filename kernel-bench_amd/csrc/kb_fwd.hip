@@ -20,8 +20,7 @@
 // k2 = 2^SL2 prepared once per solve.  NA(x)[s] = rowsum - pathsum(s) as in
 // the reference; the path sums come from an Euler-tour prefix scan.
 // Two layouts of the sweep loop:
-//  * fwd_row_kernel (rows of up to 8192 positions; 8 per thread with the
-//    owner-major tables): two barriers per sweep.  Thread t owns preorder
+//  * fwd_row_kernel (rows of up to 8192 positions): two barriers per sweep.  Thread t owns preorder
 //    positions t*CPT+k and postorder slots t*CPT+k.  The path sum is
 //    ps(i) = Pre(i) - PostEx(tin(i) - i),  Pre the inclusive preorder prefix
 //    sum and PostEx the exclusive postorder prefix sum (the nodes left before
@@ -31,8 +30,8 @@
 //    of its postorder slots and scans them (phase B), published under the
 //    second barrier; phase C forms the path sums, the wavefront offsets being
 //    applied by the readers.
-//  * fwd_row_kernel_euler (rows past 4096 positions without the owner-major
-//    tables): wavefront-segment ownership and an Euler-tour scan, three
+//  * fwd_row_kernel_euler (rows past 4096 positions, by a tuning knob only):
+//    wavefront-segment ownership and an Euler-tour scan, three
 //    barriers per sweep, half the LDS.
 #include "kb_device.hpp"
 #include "kb_kernels.hpp"
@@ -257,6 +256,14 @@ __global__ __launch_bounds__(NT, (NT == 1024 && CPT == 2) ? 8 : 1) void fwd_row_
 // would spill).
 #define FWD_MIN_WAVES(NT, CPT, W) (((NT) == 512 && (CPT) == 4 && !(W)) ? 6 : 1)
 
+// the LDS word at a byte offset, and the value of lane (byte / 4)
+__device__ __forceinline__ float lds_at(const float* p, unsigned byte) {
+  return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + byte);
+}
+__device__ __forceinline__ float lane_gather(float x, unsigned byte) {
+  return __int_as_float(__builtin_amdgcn_ds_bpermute((int)byte, __float_as_int(x)));
+}
+
 template <int NT, int CPT, bool WEIGHTED>
 __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_kernel(FwdParams P, int first) {
   constexpr int MAXS = NT * CPT;
@@ -277,10 +284,12 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
   // Tables of the own positions i = tid*CPT + k and of the own postorder slots.
   // In preorder (child1 first) child1 of i is i + 1: from registers, except
   // for the last own position, whose child1 is read from X.  With 8 positions
-  // per thread (and the owner-major tables given) the sweeps read child2, the
-  // postorder slot and tin(i) - i from those tables in every sweep instead of
-  // holding them in registers.
-  constexpr bool OMT = CPT == 8;
+  // per thread the sweeps hold child2, the postorder slot and tin(i) - i as
+  // 16-bit LDS byte offsets (pk, pc2): 12 registers of the 128 instead of 24,
+  // which is what lets a row stay in registers (rows of 8191 states read the
+  // three tables from L2 in every sweep before: whole solves 10.96 -> 10.85 ms).
+  constexpr bool PACK = CPT == 8;
+  static_assert(!PACK || MAXS * 4 <= 0xffff, "LDS byte offsets in 16 bits");
   int c2p[CPT], nex[CPT], qp[CPT], pre_s[CPT];
   bool h1[CPT];
   // The tables and row constants are read with one vector load per row (they
@@ -320,6 +329,22 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
     }
   }
   const int c1last = h1[CPT - 1] ? own_pos_c<NT, CPT>(CPT - 1) + 1 : ZERO;
+  unsigned pk[CPT], pc2[CPT / 2 + 1];
+  auto opaque = [&](int epoch) {  // unpacked where they are used, not held unpacked
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) asm("; %1" : "+v"(pk[k]) : "s"(epoch));
+#pragma unroll
+    for (int k = 0; k < CPT / 2; ++k) asm("; %1" : "+v"(pc2[k]) : "s"(epoch));
+  };
+  if constexpr (PACK) {
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) pk[k] = (unsigned)qp[k] * 4u | ((unsigned)nex[k] * 4u) << 16;
+#pragma unroll
+    for (int k = 0; k < CPT; k += 2) pc2[k / 2] = (unsigned)c2p[k] * 4u | ((unsigned)c2p[k + 1] * 4u) << 16;
+    opaque(-2);
+  }
+  // child2 of own position k (ZERO: none)
+  auto c2_of = [&](int k) { return PACK ? (int)(((k & 1) ? pc2[k / 2] >> 16 : pc2[k / 2] & 0xffffu) >> 2) : c2p[k]; };
 
   // Per-position row constants.  Shapes of two positions per thread have
   // registers to spare and run the levels with few rows per CU, where a row's
@@ -395,7 +420,7 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
         const float pi_w = hit ? leaf_obs : KB_NEG_INF;
         const float pibar_w = desc ? KB_NEG_INF : kmt[k] + leaf_col + leaf_obs;
         const float pi_s1 = (h1[k] && i + 1 == lpos) ? leaf_obs : KB_NEG_INF;
-        const float pi_s2 = c2p[k] == lpos ? leaf_obs : KB_NEG_INF;  // padding ZERO never equals lpos
+        const float pi_s2 = c2_of(k) == lpos ? leaf_obs : KB_NEG_INF;  // padding ZERO never equals lpos
         const float t0 = kDL[k] + pi_w;
         const float t1 = pi_w + kEb[k];
         const float t2 = pibar_w + kE[k];
@@ -431,7 +456,7 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
       for (int j = 0; j < CPT; ++j) {
         const int sj = tid + j * NT;
         if (sj < S) {
-          const int i = pre_s[j];
+          const int i = PACK ? T.pre[sj] : pre_s[j];
           Lb[0][i] = P.pi[l + sj];
           Lb[1][i] = P.pi[r + sj];
           Lb[2][i] = P.pibar[l + sj];
@@ -450,7 +475,8 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
       for (int k = 0; k < CPT; ++k) {
         const int i = own_pos_c<NT, CPT>(k);
         if (i < S) {
-          const bool h2 = c2p[k] != ZERO;
+          const int c2 = c2_of(k);
+          const bool h2 = c2 != ZERO;
           const float d = EARLY || NT == 1024 ? kd[k] : P.pD[i], sp = EARLY || NT == 1024 ? ks[k] : P.pS[i];
           const float t0 = lsp + d + pl[k] + pr[k];
           const float t1 = lsp + pl[k] + br[k];
@@ -463,7 +489,7 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
             l1 = pl_last;
             r1 = pr_last;
           }
-          const float l2 = h2 ? Lb[0][c2p[k]] : KB_NEG_INF, r2 = h2 ? Lb[1][c2p[k]] : KB_NEG_INF;
+          const float l2 = h2 ? Lb[0][c2] : KB_NEG_INF, r2 = h2 ? Lb[1][c2] : KB_NEG_INF;
           const float t3 = lsp + sp + l1 + r2;
           const float t4 = lsp + sp + r1 + l2;
           const float m5 = fmaxf(fmaxf(fmaxf(t0, t1), fmaxf(t2, t3)), t4);
@@ -487,6 +513,7 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
   if (tid < 64) {  // padding slots read by the child gathers (after the staging)
     X[MAXS + tid] = 0.0f;
     Q[MAXS + tid] = 0.0f;
+    if constexpr (PACK && WEIGHTED) Lb[3][MAXS + tid] = 0.0f;
   }
 
   // ---- linear space relative to the row maximum
@@ -504,21 +531,18 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
     y[k] = ok ? exp2f(v[k] - Ms) : 0.0f;
     dl[k] = leaf_row ? (i == lpos ? leaf_lin : 0.0f) : y[k];
     cw[k] = WEIGHTED ? (ok ? P.colw[i] : 0.0f) : 1.0f;
-    cwq[k] = WEIGHTED ? (qp[k] < S ? P.colw[qp[k]] : 0.0f) : 1.0f;
+    if constexpr (!(PACK && WEIGHTED)) cwq[k] = WEIGHTED ? (qp[k] < S ? P.colw[qp[k]] : 0.0f) : 1.0f;
   }
+  // Packed rows keep the column weights in Lb[3] (unused since the staging),
+  // read at the own positions and at the postorder slots.
+  if constexpr (PACK && WEIGHTED) lds_store_own<CPT>(Lb[3], cw);
   int kexp = 0;
   float ps[CPT], rowsum = 0.0f, f = 1.0f;
 
   for (int sweep = 0;; ++sweep) {
-    if constexpr (OMT) {  // (the launcher requires the tables for this shape)
-#pragma unroll
-      for (int k = 0; k < CPT; ++k) {
-        const int c2 = ldg(fresh(P.om_tab + (size_t)OMT_C2 * MAXS + k * NT, sweep), tid);
-        const int pn = ldg(fresh(P.om_tab + (size_t)OMT_PN * MAXS + k * NT, sweep), tid);
-        c2p[k] = c2 >= 0 ? c2 : ZERO;
-        qp[k] = pn & 0xffff;
-        nex[k] = pn >> 16;
-      }
+    if constexpr (PACK) {
+      opaque(sweep);
+      if constexpr (WEIGHTED) lds_load_own<CPT>(Lb[3], cw);
     }
     // phase A: publish y; inclusive preorder scan (wavefront-local) in registers
     float sp[CPT], ta = 0.0f;
@@ -537,8 +561,14 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
     float yq[CPT], x2[CPT];
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
-      yq[k] = X[qp[k]];
-      x2[k] = X[c2p[k]];
+      if constexpr (PACK) {
+        yq[k] = lds_at(X, pk[k] & 0xffffu);
+        x2[k] = lds_at(X, (k & 1) ? pc2[k / 2] >> 16 : pc2[k / 2] & 0xffffu);
+        if constexpr (WEIGHTED) cwq[k] = lds_at(Lb[3], pk[k] & 0xffffu);
+      } else {
+        yq[k] = X[qp[k]];
+        x2[k] = X[c2p[k]];
+      }
     }
     const float x1last = X[c1last];
     const float ip = wave_scan_first<NW>(tp);
@@ -567,8 +597,13 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
     const float eq = iq - tq;
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
-      const int n = nex[k];
-      ps[k] = (sp[k] + offp) - (Q[n] + __shfl(eq, n / SEG, 64));
+      if constexpr (PACK) {
+        const unsigned n4 = pk[k] >> 16;  // the lane is n4 / (4 SEG); bpermute takes it times four, rounding down
+        ps[k] = (sp[k] + offp) - (lds_at(Q, n4) + lane_gather(eq, n4 / SEG));
+      } else {
+        const int n = nex[k];
+        ps[k] = (sp[k] + offp) - (Q[n] + __shfl(eq, n / SEG, 64));
+      }
     }
     if (sweep == P.n_sweeps) break;
     // y' = f (a y + k1 y[c1] + k2 y[c2] + emc (tsum - ps)) + dl 2^-kexp: f is a
@@ -674,7 +709,7 @@ void launch_fwd_wave(const FwdParams& P, int first, int W, hipStream_t st) {
   KB_FWD_CASE(256, 4, fwd_row_kernel)
   KB_FWD_CASE(512, 4, fwd_row_kernel)
   KB_FWD_CASE(1024, 4, fwd_row_kernel)
-  if (P.om_tab && P.large) {
+  if (P.large) {
     KB_FWD_CASE(1024, 8, fwd_row_kernel)
   }
   KB_FWD_CASE(1024, 8, fwd_row_kernel_euler)

@@ -68,8 +68,7 @@ struct FwdParams {
   const int* row_kind;        // 1: leaf row, 0: split row
   const int* dup_ptr;         // [slots + 1] rows identical to the row of each slot ...
   const int* dup_rows;        // ... which receive the same outputs
-  const int* om_tab;          // owner-major position tables (OmTab) for rows of 4097..8192 states, or null
-  int large;                  // 1: rows of 4097..8192 states run fwd_row_kernel on om_tab (else the Euler kernel)
+  int large;                  // 1: rows of 4097..8192 states run fwd_row_kernel (else the Euler kernel)
   // outputs
   float* pi; float* pibar; float* rowmax;
   float* dts_out;             // [C, S] preorder split term of every computed split row
@@ -101,10 +100,9 @@ struct BwdConstArgs {
 // wavefront's reads of one slot k are contiguous.
 enum OmConst { OMC_DL, OMC_EBAR, OMC_E, OMC_SL1, OMC_SL2, OMC_PD, OMC_PS, OMC_MT, OMC_COL, KB_OM_CONSTS };
 // position tables: child-1 / child-2 positions (-1: leaf); parent position
-// (ZERO = 1024*CPT for the root) | (subtree end - 1) << 16 | child-1 flag << 30;
-// postorder slot's position | (tin(i) - i) << 16.  Positions >= S: -1, -1,
-// ZERO | ZERO << 16, ZERO.
-enum OmTab { OMT_C1, OMT_C2, OMT_PK, OMT_PN, KB_OM_TABS };
+// (ZERO = 1024*CPT for the root) | (subtree end - 1) << 16 | child-1 flag << 30.
+// Positions >= S: -1, -1, ZERO | ZERO << 16.
+enum OmTab { OMT_C1, OMT_C2, OMT_PK, KB_OM_TABS };
 
 // The backward's record of a schedule slot (KB_BREC ints): the row's first
 // two child sides (-1: none; bit 30 of the second: more sides follow), the
