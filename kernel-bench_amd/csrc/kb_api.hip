@@ -93,7 +93,7 @@ struct kb_plan {
   int* d_m_side_ptr = nullptr;         // level-0 members (cls_rows order): staging sides
   int* d_m_side = nullptr;
   int* d_m_root = nullptr;
-  float* d_dts = nullptr;              // [C, S] split terms stored by the forward (preorder rows)
+  float* d_dts = nullptr;              // [C, kb_stage_ld(S)] split terms stored by the forward (preorder rows)
   int64_t fwd_token = 0;               // counter of forwards on this plan
   const float* fwd_pi = nullptr;       // outputs of the forward with token fwd_token
   const float* fwd_pibar = nullptr;
@@ -698,7 +698,7 @@ int kb_plan_create(const kb_layout* L, kb_plan** out) {
     rc |= upload(&p->d_m_side, ms);
     rc |= upload(&p->d_m_root, mroot);
   }
-  rc |= alloc(&p->d_dts, (size_t)std::max(1, C) * S);
+  rc |= alloc(&p->d_dts, (size_t)std::max(1, C) * kb::kb_stage_ld(S));
   rc |= upload(&p->d_pre, pre);
   rc |= upload(&p->d_pcol, pcol);
   rc |= upload(&p->d_c1pos, c1pos);
@@ -716,10 +716,10 @@ int kb_plan_create(const kb_layout* L, kb_plan** out) {
     rc |= upload(&p->d_post, post);
     if (S > 1024 && S <= 8192) {
       // owner-major position tables of bwd_row_large_kernel (kb::OmTab)
-      const int ld = kb::kb_large_ld(S), nt = kb::kb_large_nt(S), cpt = ld / nt, zero = ld;
+      const int ld = kb::kb_large_ld(S), cpt = ld / kb::kb_large_nt(S), zero = ld;
       std::vector<int> om((size_t)kb::KB_OM_TABS * ld);
       for (int i = 0; i < ld; ++i) {
-        const size_t o = (size_t)(i % cpt) * nt + i / cpt;
+        const size_t o = kb::kb_om_index(i, cpt);
         const bool ok = i < S;
         om[kb::OMT_C1 * (size_t)ld + o] = ok ? c1pos[i] : -1;
         om[kb::OMT_C2 * (size_t)ld + o] = ok ? c2pos[i] : -1;
@@ -995,11 +995,13 @@ static int ensure_backward_work(kb_plan* p, int use_col) {
   }
   const int64_t NS = p->n_splits;
   int rc = 0;
-  rc |= alloc(&p->b_staging, (size_t)std::max<int64_t>(1, 2 * NS) * kb::kb_stage_ld(S) + kb::KB_STAGE_TAIL);
+  // (the large-row kernels keep the family roots' v behind the child sides)
+  const int64_t n_stage = 2 * NS + (S > 1024 && S <= 8192 ? p->n_fam : 0);
+  rc |= alloc(&p->b_staging, (size_t)std::max<int64_t>(1, n_stage) * kb::kb_stage_ld(S) + kb::KB_STAGE_TAIL);
   rc |= alloc(&p->b_split_on, (size_t)std::max<int64_t>(1, NS));
   rc |= alloc(&p->b_mask, (size_t)std::max(1, C));
   rc |= alloc(&p->b_rhs0, (size_t)std::max(1, C > 0 ? p->level_ptr[1] : 1) * S);
-  rc |= alloc(&p->b_rhsc, (size_t)std::max(1, p->n_cls0) * S);
+  rc |= alloc(&p->b_rhsc, (size_t)std::max(1, p->n_cls0) * kb::kb_stage_ld(S));
   rc |= alloc(&p->b_m_mask, (size_t)std::max(1, C > 0 ? p->level_ptr[1] : 1));
   rc |= alloc(&p->b_cls_active, (size_t)std::max(1, p->n_cls0));
   rc |= alloc(&p->b_ck_any, (size_t)std::max(1, p->n_chunks0));
@@ -1105,6 +1107,7 @@ static int backward_setup(kb_plan* p, const kb_backward_io* io, hipStream_t st, 
   B.child_in = p->d_child_in;
   B.bslot = p->d_bslot;
   B.staging = p->b_staging;
+  B.n_splits = (int)p->n_splits;
   B.split_on = p->b_split_on;
   B.mask = io->active_mask ? (unsigned char*)io->active_mask : p->b_mask;
   B.contrib = p->b_contrib;
@@ -1148,8 +1151,10 @@ static int backward_level(kb_plan* p, kb::BwdParams& B, int d, int first, int n,
   return 0;
 }
 
-static int backward_finish(kb_plan* p, const kb_backward_io* io, int n_partials, hipStream_t st) {
+static int backward_finish(kb_plan* p, const kb_backward_io* io, const kb::BwdParams& B, int n_partials, hipStream_t st) {
   const int S = p->S;
+  if (p->n_levels > 0)
+    kb::launch_bwd_buckets_large(B, p->level_ptr[1], p->C - p->level_ptr[1], p->n_cls0, p->b_nb_max, st);
   KB_HIP(hipGetLastError());
   kb::launch_bwd_reduce(p->b_contrib, n_partials, S, p->b_slot, kb::kb_slot_ld(S, p->b_large), p->b_partial,
                         p->d_pre, p->b_acc, st);
@@ -1191,7 +1196,7 @@ extern "C" int kb_backward(kb_plan* p, const kb_backward_io* io, void* stream) {
   int rc = backward_setup(p, io, st, B, 0);
   for (int d = p ? p->n_levels - 1 : -1; !rc && d >= 0; --d)
     rc = backward_level(p, B, d, p->level_ptr[d], level_rows(p, d), p->b_nb_max, 0, st);
-  return rc ? rc : backward_finish(p, io, p->b_n_partials, st);
+  return rc ? rc : backward_finish(p, io, B, p->b_n_partials, st);
 }
 
 extern "C" int kb_solve(kb_plan* p, const kb_forward_io* fio, const kb_backward_io* bio, void* stream) {
@@ -1251,7 +1256,7 @@ extern "C" int kb_solve(kb_plan* p, const kb_forward_io* fio, const kb_backward_
   if (rc) return rc;
   KB_HIP(hipStreamWaitEvent(st, p->ev_join, 0));
   for (int d = low - 1; !rc && d >= 0; --d) rc = backward_level(p, B, d, p->level_ptr[d], level_rows(p, d), p->b_nb_max, 0, st);
-  return rc ? rc : backward_finish(p, &b2, p->b_nb_max + eg, st);
+  return rc ? rc : backward_finish(p, &b2, B, p->b_nb_max + eg, st);
 }
 
 extern "C" {

@@ -250,7 +250,7 @@ __global__ __launch_bounds__(NT) void bwd_row_kernel(BwdParams P, int first, int
     const int rmr = q == 0 ? frow : q == 1 ? fl0 : fr0;
     nrm = rmr >= 0 ? P.rowmax[rmr] : 0.0f;
     const bool dts = !leaf && P.dts_in;
-    const size_t db = (size_t)rep * S;
+    const size_t db = (size_t)rep * SG;
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       const int i = own_pos_c<NT, CPT>(k);
@@ -378,7 +378,7 @@ __global__ __launch_bounds__(NT) void bwd_row_kernel(BwdParams P, int first, int
   if (P.class_mode) {
     // the summed adjoint of the class's active members (bwd_gather0 / bwd_classsum0)
     any_active = P.cls_active[rr] != 0;
-    const float* src = P.rhsc + (size_t)rr * S;
+    const float* src = P.rhsc + (size_t)rr * SG;
 #pragma unroll
     for (int k = 0; k < CPT; ++k)
       if (okp[k]) rhs[k] = src[own_pos_c<NT, CPT>(k)];
@@ -488,7 +488,7 @@ __global__ __launch_bounds__(NT) void bwd_row_kernel(BwdParams P, int first, int
   for (int k = 0; k < CPT; ++k) dts[k] = KB_NEG_INF;
   if (!leaf_row && P.dts_in) {
     if (cm) {
-      const float* src = P.dts_in + (size_t)P.rep_of[row] * S;
+      const float* src = P.dts_in + (size_t)P.rep_of[row] * SG;
 #pragma unroll
       for (int k = 0; k < CPT; ++k)
         if (okp[k]) dts[k] = src[own_pos_c<NT, CPT>(k)];
@@ -1014,7 +1014,7 @@ __global__ __launch_bounds__(256) void bwd_classsum0_kernel(BwdParams P) {
       if (i < S) acc += P.rhs0[(size_t)(m0 + j) * S + i];
     }
   }
-  if (i < S) P.rhsc[(size_t)c * S + i] = acc;
+  if (i < S) P.rhsc[(size_t)c * kb_stage_ld(S) + i] = acc;
   if (blockIdx.y == 0 && threadIdx.x == 0) P.cls_active[c] = any ? 1 : 0;
 }
 
@@ -1136,7 +1136,7 @@ __global__ __launch_bounds__(256) void bwd_chunksum0_kernel(BwdParams P) {
     any |= P.ck_any[k];
     if (i < S) acc += P.rhs0[(size_t)k * S + i];
   }
-  if (i < S) P.rhsc[(size_t)c * S + i] = acc;
+  if (i < S) P.rhsc[(size_t)c * kb_stage_ld(S) + i] = acc;
   if (blockIdx.y == 0 && threadIdx.x == 0) P.cls_active[c] = any ? 1 : 0;
 }
 
@@ -1220,8 +1220,8 @@ __global__ __launch_bounds__(256) void bwd_consts_kernel(BwdConstArgs A) {
   A.mt_pre[i] = A.mt[s];
   A.col_pre[i] = A.col[s];
   if (A.om) {
-    const int ld = kb_large_ld(A.S), nt = kb_large_nt(A.S), cpt = ld / nt;
-    float* o = A.om + (i % cpt) * nt + i / cpt;
+    const int ld = kb_large_ld(A.S);
+    float* o = A.om + kb_om_index(i, ld / kb_large_nt(A.S));
     o[OMC_DL * ld] = dl;
     o[OMC_EBAR * ld] = A.Ebar[s];
     o[OMC_E * ld] = A.E[s];

@@ -7,20 +7,25 @@
 // buckets, split adjoints into the children's staging rows.
 //
 // At these sizes a row needs 1024 threads owning 4 or 8 preorder positions
-// each, and 16 wavefronts per workgroup leave 128 VGPRs per thread.  The
-// general kernel keeps per-position tables, six coefficient rows and eight
-// bucket rows in registers across the whole row and spills hundreds of
-// registers there.  This kernel keeps across phases only what the Neumann
-// series needs:
-//  * per-position tables (children, parent, subtree end, postorder slot) are
-//    read from memory in the phase that uses them (L2-resident, 32 KB each);
-//  * per-position constants are read from memory where they are used;
-//  * the J^T coefficients q_0..q_5 are recomputed after the Neumann series
-//    from Pi*, Pibar* and the split term (same code, same values) instead of
-//    being held through it;
-//  * the gradient buckets are added into this workgroup's bucket slot in
-//    memory after every row (each thread updates only its own positions, in
-//    row order, so the sums keep a fixed order).
+// each, and 16 wavefronts per workgroup leave 128 VGPRs per thread: per-position
+// tables, six coefficient rows and eight bucket rows do not fit beside the
+// Neumann series.  So a row is solved and its gradient buckets are summed in
+// two kernels:
+//  * bwd_row_large_kernel solves the rows of one level: adjoint, coefficients,
+//    Neumann series, split adjoints into the children's staging rows.  It keeps
+//    across phases only what the series needs, writes the row's v, and adds the
+//    column-gradient bucket (the one that needs the row's scans) to this
+//    workgroup's slot in memory;
+//  * bwd_buckets_large_kernel runs once, after the last level, over all rows:
+//    it recomputes q_0..q_5 and the split shares (same code, same values) from
+//    v, Pi*, Pibar* and the split term, and holds the seven other bucket rows in
+//    registers over every row of its workgroup.
+// One kernel for both read and wrote the eight bucket rows of its slot (0.5 MB,
+// 0.75 MB for a split row, of 8191 positions) on every row, more than L2 holds
+// for 256 workgroups: @@FIG@@.
+// v takes the staging row of the row's first child side (only this row reads
+// it, and has by then), an extra staging row for a family root, and the class's
+// adjoint row for a class of level-0 rows.
 #include "kb_device.hpp"
 #include "kb_kernels.hpp"
 #include "kb_rowops.hpp"
@@ -68,6 +73,13 @@ __device__ __forceinline__ Coef6 coef_at(const CoefK& K, float piv, float pbv, f
 
 }  // namespace
 
+// Where a solved row's v is kept for bwd_buckets_large_kernel: the staging row
+// of its first child side s0, the extra staging row of a family root, or none.
+__device__ __forceinline__ float* bwd_v_row(const BwdParams& P, int s0, int fam) {
+  if (s0 < 0 && fam < 0) return nullptr;
+  return P.staging + (s0 >= 0 ? (size_t)s0 : (size_t)2 * P.n_splits + fam) * kb_stage_ld(P.S);
+}
+
 template <int N>
 __device__ __forceinline__ void vld(const float* p, float (&x)[N]) {
 #pragma unroll
@@ -88,15 +100,6 @@ __device__ __forceinline__ void vst(float* p, const float (&x)[N]) {
 
 __device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 __device__ __forceinline__ float f4(const float4& v, int j) { return j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w; }
-// *p = b + x (four floats)
-__device__ __forceinline__ void st4_add(float* p, float4 b, const float (&x)[4]) {
-  b.x += x[0];
-  b.y += x[1];
-  b.z += x[2];
-  b.w += x[3];
-  *reinterpret_cast<float4*>(p) = b;
-}
-
 // NT threads (1024, or 512 for rows of at most 2048 states) own CPT positions
 // each; at most 128 VGPRs, so 16 wavefronts per CU are resident (two
 // workgroups of 512).
@@ -131,15 +134,15 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
     R3[MAXS + tid] = 0.0f;
   }
   // this workgroup's slot (KB_LARGE_SLOT_ROWS rows of MAXS floats, preorder
-  // positions): the eight bucket rows, then the current row's split term, Pi*
-  // and Pibar*.  srow(j) is this thread's first own position of row j.
+  // positions): the eight bucket rows, then the current row's Pi*.  srow(j) is
+  // this thread's first own position of row j.
   float* const slot = P.contrib + (size_t)(poff + (int)blockIdx.x) * KB_LARGE_SLOT_ROWS * MAXS;
   int ep = 0;  // epoch of the current phase (see fresh)
   auto srow = [&](int j) {
     return reinterpret_cast<float*>(reinterpret_cast<char*>(fresh(slot + (size_t)j * MAXS, ep)) +
                                     (unsigned)(tid * CPT) * 4u);
   };
-  enum { SL_DTS = 8, SL_PI = 9, SL_PIBAR = 10 };
+  enum { SL_COL = 7, SL_PI = 8 };
   // own position k; with 8 positions per thread recomputed where it is used
   // (the positions and the LDS addresses derived from them would otherwise be
   // held across the row loop)
@@ -148,25 +151,30 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
     if constexpr (CPT > 4) asm("; %1" : "+v"(b) : "s"(ep));
     return b + k;
   };
-  // a global row in column order -> LDS at preorder positions (coalesced reads)
-  auto stage = [&](float* dst, const float* src) {
+  // two global rows in column order -> LDS at preorder positions (coalesced reads)
+  auto stage2 = [&](float* d0, const float* s0, float* d1, const float* s1) {
     int sp[CPT];
-    float x[CPT];
+    float x[CPT], y[CPT];
 #pragma unroll
     for (int j = 0; j < CPT; ++j) {
       const int s = tid + j * NT;
       sp[j] = s < S ? ldg(fresh(T.pre, ep), s) : -1;
-      x[j] = s < S ? ldg(fresh(src, ep), s) : 0.0f;
+      x[j] = s < S ? ldg(fresh(s0, ep), s) : 0.0f;
+      y[j] = s < S ? ldg(fresh(s1, ep), s) : 0.0f;
     }
 #pragma unroll
     for (int j = 0; j < CPT; ++j)
-      if (sp[j] >= 0) dst[sp[j]] = x[j];
+      if (sp[j] >= 0) {
+        d0[sp[j]] = x[j];
+        d1[sp[j]] = y[j];
+      }
   };
   auto field = [](int rec, int f) { return __builtin_amdgcn_readlane(rec, f); };
   // row j of the owner-major tables / constants at own position k (one
   // contiguous read per wavefront)
-  auto omi = [&](int j, int k) { return ldg(fresh(P.om_tab + (size_t)j * MAXS + k * NT, ep), tid); };
-  auto omf = [&](int j, int k) { return ldg(fresh(P.om_const + (size_t)j * MAXS + k * NT, ep), tid); };
+  const int om0 = (tid >> 6) * 64 * CPT + (tid & 63);  // kb_om_index(tid * CPT, CPT)
+  auto omi = [&](int j, int k) { return ldg(fresh(P.om_tab + (size_t)j * MAXS, ep) + k * 64, om0); };
+  auto omf = [&](int j, int k) { return ldg(fresh(P.om_const + (size_t)j * MAXS, ep) + k * 64, om0); };
   auto coef_k = [&](int k) {
     return CoefK{omf(OMC_DL, k), omf(OMC_EBAR, k), omf(OMC_E, k), omf(OMC_SL1, k), omf(OMC_SL2, k), omf(OMC_PS, k)};
   };
@@ -211,19 +219,13 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
     float rhs[CPT], dts[CPT];
 #pragma unroll
     for (int k = 0; k < CPT; ++k) dts[k] = KB_NEG_INF;
-    if (!leaf_row && P.dts_in) {
-      const float* src = P.dts_in + (size_t)(cm ? P.rep_of[row] : f_rep) * S;
-#pragma unroll
-      for (int k = 0; k < CPT; ++k)
-        if (pos(k) < S) dts[k] = ldg(fresh(src, ep), pos(k));
-    }
+    if (!leaf_row && P.dts_in)
+      gld_own<CPT>(fresh(P.dts_in + (size_t)(cm ? P.rep_of[row] : f_rep) * kb_stage_ld(S), ep), S, dts, KB_NEG_INF);
     bool any_active = false;
     float row_amax = 0.0f;  // max |adjoint| of the row
     if (cm) {
       any_active = P.cls_active[rr] != 0;
-      const float* src = P.rhsc + (size_t)rr * S;
-#pragma unroll
-      for (int k = 0; k < CPT; ++k) rhs[k] = pos(k) < S ? ldg(fresh(src, ep), pos(k)) : 0.0f;
+      gld_own<CPT>(fresh(P.rhsc + (size_t)rr * kb_stage_ld(S), ep), S, rhs, 0.0f);
     } else {
       const int s1 = f_s1 < 0 ? -1 : (f_s1 & ((1 << 30) - 1));
       const bool on0 = f_s0 >= 0 && P.split_on[f_s0 >> 1];
@@ -231,12 +233,8 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
       const float* st0 = P.staging + (size_t)(f_s0 >= 0 ? f_s0 : 0) * kb_stage_ld(S);
       const float* st1 = P.staging + (size_t)(s1 >= 0 ? s1 : 0) * kb_stage_ld(S);
       float a0[CPT], a1[CPT];
-#pragma unroll
-      for (int k = 0; k < CPT; ++k) {
-        const bool ok = pos(k) < S;
-        a0[k] = ok && f_s0 >= 0 ? ldg(fresh(st0, ep), pos(k)) : 0.0f;
-        a1[k] = ok && s1 >= 0 ? ldg(fresh(st1, ep), pos(k)) : 0.0f;
-      }
+      gld_own<CPT>(fresh(st0, ep), f_s0 >= 0 ? S : 0, a0, 0.0f);
+      gld_own<CPT>(fresh(st1, ep), s1 >= 0 ? S : 0, a1, 0.0f);
 #pragma unroll
       for (int k = 0; k < CPT; ++k) {
         rhs[k] = 0.0f;
@@ -247,10 +245,10 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
       for (int j = 0; j < n2; ++j) {
         const int side = P.child_in[P.child_ptr[row] + 2 + j];
         if (!P.split_on[side >> 1]) continue;
-        const float* st = P.staging + (size_t)side * kb_stage_ld(S);
+        float a[CPT];
+        gld_own<CPT>(fresh(P.staging + (size_t)side * kb_stage_ld(S), ep), S, a, 0.0f);
 #pragma unroll
-        for (int k = 0; k < CPT; ++k)
-          if (pos(k) < S) rhs[k] += ldg(fresh(st, ep), pos(k));
+        for (int k = 0; k < CPT; ++k) rhs[k] += a[k];
       }
     }
     const bool mask_early = !cm && fam < 0;
@@ -319,15 +317,13 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
     const float rms = fsafe(P.rowmax[row]);
     const int lpos = cm ? (leaf_row ? T.pre[P.leaf_state[row]] : -1) : f_lpos;
     // Pibar* at the own positions (each thread reads its own positions only,
-    // before any thread restages R1); Pi* and Pibar* kept in the slot for the
-    // phases after the Neumann series
+    // before any thread restages R1); Pi* kept in the slot for the split adjoints
     float pbv[CPT];
     lds_load_own<CPT>(R1, pbv);
 #pragma unroll
     for (int k = 0; k < CPT; ++k)
       if (pos(k) >= S) pbv[k] = KB_NEG_INF;
-    vst<CPT>(srow(SL_PI), piv);
-    vst<CPT>(srow(SL_PIBAR), pbv);
+    if (se > sb) vst<CPT>(srow(SL_PI), piv);
     // the reductions above reused scratch, and the split term below restages
     // R0..R3 when it is not stored
     if (fam >= 0 || (!leaf_row && !P.dts_in)) __syncthreads();
@@ -342,10 +338,8 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
       for (int si = sb; si < se; ++si) {
         const size_t l = (size_t)P.split_l[si] * S, r = (size_t)P.split_r[si] * S;
         const float lsp = P.split_lsp[si];
-        stage(R0, P.pi + l);
-        stage(R1, P.pi + r);
-        stage(R2, P.pibar + l);
-        stage(R3, P.pibar + r);
+        stage2(R0, P.pi + l, R1, P.pi + r);
+        stage2(R2, P.pibar + l, R3, P.pibar + r);
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < CPT; ++k) {
@@ -372,7 +366,6 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
 #pragma unroll
       for (int k = 0; k < CPT; ++k) dts[k] = log2f(acc[k]) + dts[k];
     }
-    vst<CPT>(srow(SL_DTS), dts);
 
     // ---- 4. J^T coefficients at Pi* (wave_backward.py:264-416)
     ep = rr * 16 + 4;
@@ -522,75 +515,34 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
     }
 
     ep = rr * 16 + 6;
-    // ---- 6. self-loop column gradient and parameter buckets.  The buffers of
-    // the next term's parity are free: Pi* goes back to its Tb buffer for the
-    // recomputed coefficients' child gathers, the scan of u = v * pcoef to its
-    // Lb buffer.
+    // ---- 6. v for the bucket kernel, and the self-loop's column gradient (the
+    // scan of u = v * pcoef in the Lb buffer of the next term's parity)
+    {
+      float* vr = cm ? P.rhsc + (size_t)rr * kb_stage_ld(S) : bwd_v_row(P, f_s0, fam);
+      if (vr) gst_own<CPT>(vr, S, v);
+    }
+    float gcol[CPT];
     {
       // the buffers the last term did not write (its readers may still be
       // reading its own)
-      float* Pt = (calls & 1) ? R1 : R0;
       float* Pb = (calls & 1) ? R3 : R2;
       float* wt = (calls & 1) ? wB : wA;
-      {
-        float x[CPT];
-        vld<CPT>(srow(SL_PI), x);
-        lds_store_own<CPT>(Pt, x);
+      float x[CPT], sc[CPT];
 #pragma unroll
-        for (int k = 0; k < CPT; ++k) x[k] = v[k] * pcoef[k];
-        float sc[CPT];
-        local_scan_publish<NT, CPT>(sc, x, Pb, wt);
-        __syncthreads();
-        float A, woff, wexcl;
-        scan_offsets(wt, A, woff, wexcl);
-        const float p0 = wave_prev_lane(sc[CPT - 1]) + woff;
-        int pkt[CPT];
-        pk_now(pkt, ep);
-        // the column-gradient term p' (P(i-1) + A - P(end(i)-1)), in pcoef's
-        // registers (pcoef is not needed after this)
+      for (int k = 0; k < CPT; ++k) x[k] = v[k] * pcoef[k];
+      local_scan_publish<NT, CPT>(sc, x, Pb, wt);
+      __syncthreads();
+      float A, woff, wexcl;
+      scan_offsets(wt, A, woff, wexcl);
+      const float p0 = wave_prev_lane(sc[CPT - 1]) + woff;
+      int pkt[CPT];
+      pk_now(pkt, ep);
+      // p' (P(i-1) + A - P(end(i)-1))
 #pragma unroll
-        for (int k = 0; k < CPT; ++k) {
-          const float pm1 = k == 0 ? p0 : sc[k - 1] + woff;
-          const float rest = A - (Pb[endm1_of(pkt[k])] + __shfl(wexcl, wend_of(pkt[k]), 64));
-          pcoef[k] = pos(k) < S ? pp[k] * (pm1 + rest) : 0.0f;
-        }
-      }
-      // a group's bucket loads are all issued before its stores (a load after a
-      // store to the slot would wait for that store)
-#pragma unroll
-      for (int g = 0; g < NG; ++g) {
-        float4 bk[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) bk[j] = ld4(srow(j) + 4 * g);
-        float pb4[4], dt4[4];
-        vld<4>(srow(SL_PIBAR) + 4 * g, pb4);
-        vld<4>(srow(SL_DTS) + 4 * g, dt4);
-        const float4 pt4 = ld4(Pt + tid * CPT + 4 * g);  // own positions of Pi* (vector LDS read)
-        float x[8][4];
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-          const int k = 4 * g + kk;
-          const int i = pos(k);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) x[j][kk] = 0.0f;
-          if (i < S) {
-            const int c1 = omi(OMT_C1, k), c2 = omi(OMT_C2, k);
-            const Coef6 c = coef_at(coef_k(k), f4(pt4, kk), pb4[kk], dt4[kk], c1 >= 0 ? Pt[c1] : KB_NEG_INF,
-                                    c2 >= 0 ? Pt[c2] : KB_NEG_INF, leaf_row, i == lpos);
-            const float aw0 = v[k] * c.q[0], aw1 = v[k] * c.q[1], aw2 = v[k] * c.q[2];
-            const float aw3 = v[k] * c.q[3], aw4 = v[k] * c.q[4], aw5 = v[k] * c.q[5];
-            x[0][kk] = aw0;
-            x[1][kk] = aw3 + aw4 + aw5;
-            x[2][kk] = aw0 + aw2;
-            x[3][kk] = aw1;
-            x[4][kk] = aw4;
-            x[5][kk] = aw3;
-            x[6][kk] = aw2;
-            x[7][kk] = pcoef[k];
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) st4_add(srow(j) + 4 * g, bk[j], x[j]);
+      for (int k = 0; k < CPT; ++k) {
+        const float pm1 = k == 0 ? p0 : sc[k - 1] + woff;
+        const float rest = A - (Pb[endm1_of(pkt[k])] + __shfl(wexcl, wend_of(pkt[k]), 64));
+        gcol[k] = pos(k) < S ? pp[k] * (pm1 + rest) : 0.0f;
       }
     }
 
@@ -603,26 +555,23 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
       const float rmsl = fsafe(rml), rmsr = fsafe(rmr);
       ep = -4 * si - 1;
       __syncthreads();  // previous readers of R0..R3 are done
-      stage(R0, P.pi + l);
-      stage(R1, P.pi + r);
-      stage(R2, P.pibar + l);
-      stage(R3, P.pibar + r);
+      stage2(R0, P.pi + l, R1, P.pi + r);
+      stage2(R2, P.pibar + l, R3, P.pibar + r);
       __syncthreads();
       ep = -4 * si - 2;
       // pass 1 (own positions, four at a time): the five split-term shares
       // vd_j; vd3 / vd4 replace the own positions of the children's Pibar
       // rows (R2 / R3, read only at own positions) for the child positions'
-      // parent reads; buckets 0, 1, 6 take vd0, vd3 + vd4, vd1 + vd2
+      // parent reads
       float av[CPT], bv[CPT], udl[CPT], udr[CPT], ppl[CPT], ppr[CPT];
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
-        const float4 b0 = ld4(srow(0) + 4 * g), b1 = ld4(srow(1) + 4 * g), b6 = ld4(srow(6) + 4 * g);
         float pv4[4];
         vld<4>(srow(SL_PI) + 4 * g, pv4);
         // own positions of the four staged child rows (vector LDS reads)
         const float4 pl4 = ld4(R0 + tid * CPT + 4 * g), pr4 = ld4(R1 + tid * CPT + 4 * g);
         const float4 bl4 = ld4(R2 + tid * CPT + 4 * g), br4 = ld4(R3 + tid * CPT + 4 * g);
-        float y0[4], y1[4], y2[4], d3[4], d4[4];
+        float d3[4], d4[4];
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
           const int k = 4 * g + kk;
@@ -653,22 +602,13 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
           }
           av[k] = vd0 + vd1;
           bv[k] = vd0 + vd2;
-          y0[kk] = vd0;
-          y1[kk] = vd3 + vd4;
-          y2[kk] = vd1 + vd2;
           d3[kk] = vd3;
           d4[kk] = vd4;
         }
         *reinterpret_cast<float4*>(R2 + tid * CPT + 4 * g) = make_float4(d3[0], d3[1], d3[2], d3[3]);
         *reinterpret_cast<float4*>(R3 + tid * CPT + 4 * g) = make_float4(d4[0], d4[1], d4[2], d4[3]);
-        st4_add(srow(0) + 4 * g, b0, y0);
-        st4_add(srow(1) + 4 * g, b1, y1);
-        st4_add(srow(6) + 4 * g, b6, y2);
       }
       __syncthreads();  // the staged children (R0, R1) fully read; vd3 / vd4 published
-      float4 b7[NG];
-#pragma unroll
-      for (int g = 0; g < NG; ++g) b7[g] = ld4(srow(7) + 4 * g);
       float scl[CPT], scr[CPT];
       local_scan_publish<NT, CPT>(scl, udl, R0, wA);
       local_scan_publish<NT, CPT>(scr, udr, R1, wA + NW);
@@ -685,7 +625,7 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
       pk_now(pkt, ep);
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
-        float y3[4];
+        float yl[4], yr[4];
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
           const int k = 4 * g + kk;
@@ -693,9 +633,9 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
           const int e1 = endm1_of(pkt[k]), we = wend_of(pkt[k]);
           const float pml = k == 0 ? p0l : scl[k - 1] + woffl;
           const float pmr = k == 0 ? p0r : scr[k - 1] + woffr;
+          yl[kk] = yr[kk] = 0.0f;
           const float rsl = Al - (R0[e1] + __shfl(wexl, we, 64));
           const float rsr = Ar - (R1[e1] + __shfl(wexr, we, 64));
-          y3[kk] = 0.0f;
           if (i < S) {
             const float tl = ppl[k] * (pml + rsl);
             const float tr = ppr[k] * (pmr + rsr);
@@ -704,16 +644,199 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
             const float sh3 = R2[pa], sh4 = R3[pa];  // padding slot holds 0
             const float shl = first_child ? sh3 : sh4;
             const float shr = first_child ? sh4 : sh3;
-            stg(stl, i, av[k] + shl + tl);
-            stg(str, i, bv[k] + shr + tr);
-            y3[kk] = tl + tr;
+            yl[kk] = av[k] + shl + tl;
+            yr[kk] = bv[k] + shr + tr;
+            gcol[k] += tl + tr;
           }
         }
-        st4_add(srow(7) + 4 * g, b7[g], y3);
+        // (rows are a multiple of four floats long: the tail goes to padding)
+        if (pos(4 * g) < S) {
+          *reinterpret_cast<float4*>(stl + pos(4 * g)) = make_float4(yl[0], yl[1], yl[2], yl[3]);
+          *reinterpret_cast<float4*>(str + pos(4 * g)) = make_float4(yr[0], yr[1], yr[2], yr[3]);
+        }
       }
       if (tid == 0) P.split_on[si] = 1;
     }
+    float old[CPT];
+    vld<CPT>(srow(SL_COL), old);
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) old[k] += gcol[k];
+    vst<CPT>(srow(SL_COL), old);
   }  // rows
+}
+
+// The seven other bucket rows of all solved rows: levels 1 and up (schedule
+// slots first .. first + n_rows) and the n_cls classes of level 0, workgroup b
+// taking items b, b + gridDim.x, ... in order into slot b, whose rows 0..6 it
+// writes once.  128 VGPRs: 7 * CPT sums stay in registers; per row the two or
+// six rows it reads are staged through LDS to preorder positions.  Measured
+// @@FIG2@@.
+template <int NT, int CPT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4)))
+void bwd_buckets_large_kernel(BwdParams P, int first, int n_rows, int n_cls) {
+  constexpr int MAXS = NT * CPT;
+  constexpr int LD = MAXS + 64;
+  static_assert(CPT == 4 || CPT == 8, "4 or 8 positions per thread");
+  __shared__ __align__(16) float L[4 * LD];
+  float* R0 = L;
+  float* R1 = L + LD;
+  float* R2 = L + 2 * LD;
+  float* R3 = L + 3 * LD;
+  const PreDev& T = P.pre;
+  const int S = P.S;
+  const int tid = threadIdx.x;
+  int ep = 0;
+  auto pos = [&](int k) {
+    int b = tid * CPT;
+    if constexpr (CPT > 4) asm("; %1" : "+v"(b) : "s"(ep));
+    return b + k;
+  };
+  auto stage2 = [&](float* d0, const float* s0, float* d1, const float* s1) {
+    int sp[CPT];
+    float x[CPT], y[CPT];
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) {
+      const int s = tid + j * NT;
+      sp[j] = s < S ? ldg(fresh(T.pre, ep), s) : -1;
+      x[j] = s < S ? ldg(fresh(s0, ep), s) : 0.0f;
+      y[j] = s < S ? ldg(fresh(s1, ep), s) : 0.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < CPT; ++j)
+      if (sp[j] >= 0) {
+        d0[sp[j]] = x[j];
+        d1[sp[j]] = y[j];
+      }
+  };
+  auto field = [](int rec, int f) { return __builtin_amdgcn_readlane(rec, f); };
+  const int om0 = (tid >> 6) * 64 * CPT + (tid & 63);  // kb_om_index(tid * CPT, CPT)
+  auto omi = [&](int j, int k) { return ldg(fresh(P.om_tab + (size_t)j * MAXS, ep) + k * 64, om0); };
+  auto omf = [&](int j, int k) { return ldg(fresh(P.om_const + (size_t)j * MAXS, ep) + k * 64, om0); };
+  auto coef_k = [&](int k) {
+    return CoefK{omf(OMC_DL, k), omf(OMC_EBAR, k), omf(OMC_E, k), omf(OMC_SL1, k), omf(OMC_SL2, k), omf(OMC_PS, k)};
+  };
+  enum { B_PD, B_PS, B_E, B_EBAR, B_SL2, B_SL1, B_MT, NB };
+  float acc[NB][CPT];
+#pragma unroll
+  for (int j = 0; j < NB; ++j)
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) acc[j][k] = 0.0f;
+
+  for (int it = blockIdx.x; it < n_rows + n_cls; it += gridDim.x) {
+    const bool cm = it >= n_rows;
+    const int c = it - n_rows;
+    const int rec = cm ? 0 : P.bslot[(size_t)KB_BREC * (first + it) + (tid & (KB_BREC - 1))];
+    const int row = cm ? P.cls_rows[P.cls_ptr[c]] : field(rec, BR_ROW);
+    if (!(cm ? P.cls_active[c] : P.mask[row])) continue;
+    const float* vr = cm ? P.rhsc + (size_t)c * kb_stage_ld(S) : bwd_v_row(P, field(rec, BR_S0), field(rec, BR_FAM));
+    if (!vr) continue;  // neither a root nor anyone's child: v = 0
+    const bool leaf_row = (cm ? P.row_kind[row] : field(rec, BR_LEAF)) != 0;
+    const int lpos = cm ? (leaf_row ? T.pre[P.leaf_state[row]] : -1) : field(rec, BR_LPOS);
+    const int sb = cm ? P.split_ptr[row] : field(rec, BR_SB), se = cm ? P.split_ptr[row + 1] : field(rec, BR_SE);
+    ep = 8 * it + 1;
+    float v[CPT], dts[CPT];
+    gld_own<CPT>(fresh(vr, ep), S, v, 0.0f);
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) dts[k] = KB_NEG_INF;
+    if (!leaf_row) {
+      if (P.dts_in) {
+        gld_own<CPT>(fresh(P.dts_in + (size_t)(cm ? P.rep_of[row] : field(rec, BR_REP)) * kb_stage_ld(S), ep), S, dts,
+                     KB_NEG_INF);
+      } else {
+        // the split term at Pi*, as in bwd_row_large_kernel
+        float sum[CPT];
+#pragma unroll
+        for (int k = 0; k < CPT; ++k) sum[k] = 0.0f;
+        for (int si = sb; si < se; ++si) {
+          const size_t l = (size_t)P.split_l[si] * S, r = (size_t)P.split_r[si] * S;
+          const float lsp = P.split_lsp[si];
+          __syncthreads();
+          stage2(R0, P.pi + l, R1, P.pi + r);
+          stage2(R2, P.pibar + l, R3, P.pibar + r);
+          __syncthreads();
+#pragma unroll
+          for (int k = 0; k < CPT; ++k) {
+            const int i = pos(k);
+            if (i < S) {
+              const int c1 = omi(OMT_C1, k), c2 = omi(OMT_C2, k);
+              const float pl = R0[i], pr = R1[i];
+              const float l1 = c1 >= 0 ? R0[c1] : KB_NEG_INF, r1 = c1 >= 0 ? R1[c1] : KB_NEG_INF;
+              const float l2 = c2 >= 0 ? R0[c2] : KB_NEG_INF, r2 = c2 >= 0 ? R1[c2] : KB_NEG_INF;
+              const float t0 = lsp + omf(OMC_PD, k) + pl + pr;
+              const float t1 = lsp + pl + R3[i];
+              const float t2 = lsp + pr + R2[i];
+              const float sp = omf(OMC_PS, k);
+              const float t3 = lsp + sp + l1 + r2;
+              const float t4 = lsp + sp + r1 + l2;
+              const float m5 = fmaxf(fmaxf(fmaxf(t0, t1), fmaxf(t2, t3)), t4);
+              const float ms = fsafe(m5);
+              const float s5 = exp2f(t0 - ms) + exp2f(t1 - ms) + exp2f(t2 - ms) + exp2f(t3 - ms) + exp2f(t4 - ms);
+              lse_merge(dts[k], sum[k], m5, s5);
+            }
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < CPT; ++k) dts[k] = log2f(sum[k]) + dts[k];
+      }
+    }
+    __syncthreads();  // LDS of the previous row or split is no longer read
+    stage2(R0, P.pi + (size_t)row * S, R1, P.pibar + (size_t)row * S);
+    __syncthreads();
+    ep = 8 * it + 2;
+    float piv[CPT];
+    lds_load_own<CPT>(R0, piv);
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) {
+      const int i = pos(k);
+      if (i < S) {
+        const int c1 = omi(OMT_C1, k), c2 = omi(OMT_C2, k);
+        const Coef6 q = coef_at(coef_k(k), piv[k], R1[i], dts[k], c1 >= 0 ? R0[c1] : KB_NEG_INF,
+                                c2 >= 0 ? R0[c2] : KB_NEG_INF, leaf_row, i == lpos);
+        const float aw0 = v[k] * q.q[0], aw1 = v[k] * q.q[1], aw2 = v[k] * q.q[2];
+        const float aw3 = v[k] * q.q[3], aw4 = v[k] * q.q[4], aw5 = v[k] * q.q[5];
+        acc[B_PD][k] += aw0;
+        acc[B_PS][k] += aw3 + aw4 + aw5;
+        acc[B_E][k] += aw0 + aw2;
+        acc[B_EBAR][k] += aw1;
+        acc[B_SL2][k] += aw4;
+        acc[B_SL1][k] += aw3;
+        acc[B_MT][k] += aw2;
+      }
+    }
+    for (int si = sb; si < se; ++si) {
+      const size_t l = (size_t)P.split_l[si] * S, r = (size_t)P.split_r[si] * S;
+      const float lsp = P.split_lsp[si];
+      ep = -4 * si - 1;
+      __syncthreads();
+      stage2(R0, P.pi + l, R1, P.pi + r);
+      stage2(R2, P.pibar + l, R3, P.pibar + r);
+      __syncthreads();
+      ep = -4 * si - 2;
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) {
+        const int i = pos(k);
+        if (i < S && piv[k] != KB_NEG_INF) {
+          const int c1 = omi(OMT_C1, k), c2 = omi(OMT_C2, k);
+          const float pl = R0[i], pr = R1[i], bl = R2[i], br = R3[i];
+          const float l1 = c1 >= 0 ? R0[c1] : KB_NEG_INF, r1 = c1 >= 0 ? R1[c1] : KB_NEG_INF;
+          const float l2 = c2 >= 0 ? R0[c2] : KB_NEG_INF, r2 = c2 >= 0 ? R1[c2] : KB_NEG_INF;
+          const float d = omf(OMC_PD, k), sp = omf(OMC_PS, k);
+          const float base = lsp - piv[k];
+          const float vd0 = v[k] * exp2_hw(base + (d + pl + pr));
+          const float vd1 = v[k] * exp2_hw(base + (pl + br));
+          const float vd2 = v[k] * exp2_hw(base + (pr + bl));
+          const float vd3 = v[k] * exp2_hw(base + (sp + l1 + r2));
+          const float vd4 = v[k] * exp2_hw(base + (sp + r1 + l2));
+          acc[B_PD][k] += vd0;
+          acc[B_PS][k] += vd3 + vd4;
+          acc[B_MT][k] += vd1 + vd2;
+        }
+      }
+    }
+  }
+  float* const slot = P.contrib + (size_t)blockIdx.x * KB_LARGE_SLOT_ROWS * MAXS + tid * CPT;
+#pragma unroll
+  for (int j = 0; j < NB; ++j) vst<CPT>(slot + (size_t)j * MAXS, acc[j]);
 }
 
 #define KB_BWD_LARGE_CASE(NT_, CPT_)                                                                           \
@@ -740,6 +863,18 @@ bool launch_bwd_large(const BwdParams& P, int first, int W, int nb, int poff, hi
   KB_BWD_LARGE_CASE(1024, 4)
   KB_BWD_LARGE_CASE(1024, 8)
   return false;
+}
+
+void launch_bwd_buckets_large(const BwdParams& P, int first, int n_rows, int n_cls, int nb, hipStream_t st) {
+  const int S = P.S;
+  if (!kb_use_large(S, P.large) || n_rows + n_cls <= 0) return;
+  const dim3 g(std::min(nb, n_rows + n_cls));
+  if (kb_large_nt(S) == 512)
+    hipLaunchKernelGGL((bwd_buckets_large_kernel<512, 4>), g, dim3(512), 0, st, P, first, n_rows, n_cls);
+  else if (S <= 4096)
+    hipLaunchKernelGGL((bwd_buckets_large_kernel<1024, 4>), g, dim3(1024), 0, st, P, first, n_rows, n_cls);
+  else
+    hipLaunchKernelGGL((bwd_buckets_large_kernel<1024, 8>), g, dim3(1024), 0, st, P, first, n_rows, n_cls);
 }
 
 int bwd_large_blocks_per_cu(int S, int use_col) {

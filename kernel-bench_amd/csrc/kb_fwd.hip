@@ -153,7 +153,7 @@ __global__ __launch_bounds__(NT, (NT == 1024 && CPT == 2) ? 8 : 1) void fwd_row_
 #pragma unroll
     for (int k = 0; k < CPT; ++k) v[k] = log2_hw(acc[k]) + m[k];
     if (P.dts_out) {  // the backward reuses the split term at Pi*
-      float* dst = P.dts_out + (size_t)row * S;
+      float* dst = P.dts_out + (size_t)row * kb_stage_ld(S);
 #pragma unroll
       for (int k = 0; k < CPT; ++k)
         if (own_pos<NT, CPT>(k) < S) dst[own_pos<NT, CPT>(k)] = v[k];
@@ -503,12 +503,8 @@ __global__ __launch_bounds__(NT, FWD_MIN_WAVES(NT, CPT, WEIGHTED)) void fwd_row_
     __syncthreads();  // the staging buffers become the sweep buffers
 #pragma unroll
     for (int k = 0; k < CPT; ++k) v[k] = log2_hw(acc[k]) + m[k];
-    if (P.dts_out) {  // the backward reuses the split term at Pi*
-      float* dst = P.dts_out + (size_t)row * S;
-#pragma unroll
-      for (int k = 0; k < CPT; ++k)
-        if (own_pos_c<NT, CPT>(k) < S) dst[own_pos_c<NT, CPT>(k)] = v[k];
-    }
+    if (P.dts_out)  // the backward reuses the split term at Pi*
+      gst_own<CPT>(P.dts_out + (size_t)row * kb_stage_ld(S), S, v);
   }
   if (tid < 64) {  // padding slots read by the child gathers (after the staging)
     X[MAXS + tid] = 0.0f;

@@ -71,7 +71,7 @@ struct FwdParams {
   int large;                  // 1: rows of 4097..8192 states run fwd_row_kernel (else the Euler kernel)
   // outputs
   float* pi; float* pibar; float* rowmax;
-  float* dts_out;             // [C, S] preorder split term of every computed split row
+  float* dts_out;             // [C, kb_stage_ld(S)] preorder split term of every computed split row
 };
 
 // Pi / Pibar / row-max rows src[i] -> dst[i], i < n.
@@ -94,10 +94,14 @@ struct BwdConstArgs {
   float* zero; size_t n_zero;  // n_zero floats set to zero by the same launch (the bucket slots)
 };
 
-// Owner-major layout of bwd_row_large_kernel's per-position tables: with
-// 1024 threads owning CPT positions each (thread t: t*CPT .. t*CPT+CPT-1),
-// row j holds position t*CPT + k at [j*1024*CPT + k*1024 + t], so a
-// wavefront's reads of one slot k are contiguous.
+// Owner-major layout of the large-row backward kernels' per-position tables:
+// with CPT positions per thread (thread t: t*CPT .. t*CPT+CPT-1) a row holds
+// position t*CPT + k at kb_om_index, so a wavefront's reads of one slot k are
+// contiguous and its slots 256 bytes apart (the loads' immediate offsets).
+__host__ __device__ inline int kb_om_index(int i, int cpt) {
+  const int t = i / cpt, k = i % cpt;
+  return (t >> 6) * 64 * cpt + k * 64 + (t & 63);
+}
 enum OmConst { OMC_DL, OMC_EBAR, OMC_E, OMC_SL1, OMC_SL2, OMC_PD, OMC_PS, OMC_MT, OMC_COL, KB_OM_CONSTS };
 // position tables: child-1 / child-2 positions (-1: leaf); parent position
 // (ZERO = 1024*CPT for the root) | (subtree end - 1) << 16 | child-1 flag << 30.
@@ -134,7 +138,8 @@ struct BwdParams {
   const int* split_ptr; const int* split_l; const int* split_r; const float* split_lsp;
   const int* child_ptr; const int* child_in;
   const int* bslot;           // [KB_BREC * C] record of every schedule slot (BrecField)
-  float* staging;             // [2 * n_splits, kb_stage_ld(S)]
+  float* staging;             // [2 * n_splits (+ n_fam for the large-row kernels), kb_stage_ld(S)]
+  int n_splits;
   unsigned char* split_on;    // [n_splits]
   unsigned char* mask;        // [C]
   float* contrib;             // [n_partials, 8, kb_slot_ld(S)] gradient buckets, one slot per workgroup
@@ -146,13 +151,13 @@ struct BwdParams {
   const int* om_tab;          // [KB_OM_TABS, kb_large_ld(S)] owner-major position tables (OmTab)
   const float* om_const;      // [KB_OM_CONSTS, kb_large_ld(S)] owner-major constants (OmConst)
   float* rhs0;                // [rows of level 0, S] preorder adjoint rows, in cls_rows order
-  float* rhsc;                // [classes of level 0, S] summed adjoint of each class
+  float* rhsc;                // [classes of level 0, kb_stage_ld(S)] summed adjoint of each class
   const int* m_side_ptr;      // [members + 1] staging sides of each level-0 member (cls_rows order)
   const int* m_side;
   const int* m_root;          // [members] family of a member that is a root row, else -1
   unsigned char* m_mask;      // [members] active mask in member order
   unsigned char* cls_active;  // [classes of level 0] any member active
-  const float* dts_in;        // [C, S] preorder split terms stored by the forward, or null: recompute
+  const float* dts_in;        // [C, kb_stage_ld(S)] preorder split terms stored by the forward, or null: recompute
   const int* rep_of;          // [C] row -> row whose stored split term it shares
   const int* cls_ptr;         // [n_classes + 1]
   const int* cls_rows;        // member rows, representative first
@@ -165,9 +170,9 @@ struct BwdParams {
 
 constexpr int KB_CHUNK0 = 8;
 // Workgroup slot of bwd_row_large_kernel: KB_LARGE_SLOT_ROWS rows of
-// kb_large_ld(S) floats (8 bucket rows, then the row's split term, Pi* and
-// Pibar*); other row kernels use 8 rows of kb_slot_ld(S).
-constexpr int KB_LARGE_SLOT_ROWS = 11;
+// kb_large_ld(S) floats (8 bucket rows, then the current row's Pi*); other row
+// kernels use 8 rows of kb_slot_ld(S).
+constexpr int KB_LARGE_SLOT_ROWS = 9;
 // large = 1: rows of 2049..8192 states; large = 2: also rows of 1025..2048
 // states (512 threads x 4 positions)
 __host__ __device__ inline bool kb_use_large(int S, int large) {
@@ -223,6 +228,10 @@ int bwd_blocks_per_cu(int S, int use_col, int variant, int large);
 // false if P.large is off or S is outside that range.
 bool launch_bwd_large(const BwdParams& P, int first, int n, int nb, int poff, hipStream_t st);
 int bwd_large_blocks_per_cu(int S, int use_col);
+// After the last level of the low-register kernel (nothing otherwise): bucket
+// rows 0..6 of all its rows, the schedule slots first .. first + n_rows and the
+// n_cls classes of level 0, into the slots 0 .. nb.
+void launch_bwd_buckets_large(const BwdParams& P, int first, int n_rows, int n_cls, int nb, hipStream_t st);
 // Level-0 adjoint rows, masks and class sums.
 void launch_bwd_level0_prep(const BwdParams& P, int n_members, int n_cls, hipStream_t st);
 // Sums the bucket rows of C workgroup slots (slot_stride floats apart, bucket
