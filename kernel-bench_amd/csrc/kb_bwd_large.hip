@@ -22,7 +22,9 @@
 //    registers over every row of its workgroup.
 // One kernel for both read and wrote the eight bucket rows of its slot (0.5 MB,
 // 0.75 MB for a split row, of 8191 positions) on every row, more than L2 holds
-// for 256 workgroups: @@FIG@@.
+// for 256 workgroups.  Measured per whole solve, with the vector row accesses of
+// both: 8191 states 10.85 -> 9.3 ms (row kernels 7.1 -> 4.8 ms, buckets 0.73
+// ms), 3001 weighted states 2.58 -> 2.37 ms.
 // v takes the staging row of the row's first child side (only this row reads
 // it, and has by then), an extra staging row for a family root, and the class's
 // adjoint row for a class of level-0 rows.
@@ -72,6 +74,9 @@ __device__ __forceinline__ Coef6 coef_at(const CoefK& K, float piv, float pbv, f
 }
 
 }  // namespace
+
+// a workgroup-uniform value, in a scalar register
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 // Where a solved row's v is kept for bwd_buckets_large_kernel: the staging row
 // of its first child side s0, the extra staging row of a family root, or none.
@@ -151,20 +156,25 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
     if constexpr (CPT > 4) asm("; %1" : "+v"(b) : "s"(ep));
     return b + k;
   };
+  // Column tid + j*NT of a row: with 4 positions per thread columns past the
+  // row read and store its last one again (no branches); with 8 the loads all
+  // in flight at once would spill, and the guarded form measured faster.
+  constexpr bool CLAMP = CPT == 4;
+  auto column = [&](int j) { return CLAMP ? min(tid + j * NT, S - 1) : tid + j * NT; };
   // two global rows in column order -> LDS at preorder positions (coalesced reads)
   auto stage2 = [&](float* d0, const float* s0, float* d1, const float* s1) {
     int sp[CPT];
     float x[CPT], y[CPT];
 #pragma unroll
     for (int j = 0; j < CPT; ++j) {
-      const int s = tid + j * NT;
-      sp[j] = s < S ? ldg(fresh(T.pre, ep), s) : -1;
-      x[j] = s < S ? ldg(fresh(s0, ep), s) : 0.0f;
-      y[j] = s < S ? ldg(fresh(s1, ep), s) : 0.0f;
+      const int s = column(j);
+      sp[j] = CLAMP || s < S ? ldg(fresh(T.pre, ep), s) : -1;
+      x[j] = CLAMP || s < S ? ldg(fresh(s0, ep), s) : 0.0f;
+      y[j] = CLAMP || s < S ? ldg(fresh(s1, ep), s) : 0.0f;
     }
 #pragma unroll
     for (int j = 0; j < CPT; ++j)
-      if (sp[j] >= 0) {
+      if (CLAMP || sp[j] >= 0) {
         d0[sp[j]] = x[j];
         d1[sp[j]] = y[j];
       }
@@ -196,7 +206,7 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
     const int f_row = field(rec, BR_ROW), f_leaf = field(rec, BR_LEAF), f_sb = field(rec, BR_SB);
     const int f_se = field(rec, BR_SE), f_fam = field(rec, BR_FAM), f_s0 = field(rec, BR_S0);
     const int f_s1 = field(rec, BR_S1), f_lpos = field(rec, BR_LPOS), f_rep = field(rec, BR_REP);
-    const int row = cm ? P.cls_rows[P.cls_ptr[rr]] : f_row;
+    const int row = cm ? uniform(P.cls_rows[P.cls_ptr[rr]]) : f_row;
     const bool leaf_row = (cm ? P.row_kind[row] : f_leaf) != 0;
     const int sb = cm ? P.split_ptr[row] : f_sb, se = cm ? P.split_ptr[row + 1] : f_se;
     const int fam = cm ? -1 : f_fam;
@@ -211,10 +221,10 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
     int spre[CPT];
 #pragma unroll
     for (int j = 0; j < CPT; ++j) {
-      const int s = tid + j * NT;
-      spre[j] = s < S ? ldg(fresh(T.pre, ep), s) : -1;
-      nPi[j] = s < S ? ldg(fresh(P.pi + rb, ep), s) : 0.0f;
-      nPb[j] = s < S ? ldg(fresh(P.pibar + rb, ep), s) : 0.0f;
+      const int s = column(j);
+      spre[j] = CLAMP || s < S ? ldg(fresh(T.pre, ep), s) : -1;
+      nPi[j] = CLAMP || s < S ? ldg(fresh(P.pi + rb, ep), s) : 0.0f;
+      nPb[j] = CLAMP || s < S ? ldg(fresh(P.pibar + rb, ep), s) : 0.0f;
     }
     float rhs[CPT], dts[CPT];
 #pragma unroll
@@ -263,7 +273,7 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
     }
 #pragma unroll
     for (int j = 0; j < CPT; ++j)
-      if (spre[j] >= 0) {
+      if (CLAMP || spre[j] >= 0) {
         R0[spre[j]] = nPi[j];
         R1[spre[j]] = nPb[j];
       }
@@ -336,7 +346,7 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
 #pragma unroll
       for (int k = 0; k < CPT; ++k) acc[k] = 0.0f;
       for (int si = sb; si < se; ++si) {
-        const size_t l = (size_t)P.split_l[si] * S, r = (size_t)P.split_r[si] * S;
+        const size_t l = (size_t)uniform(P.split_l[si]) * S, r = (size_t)uniform(P.split_r[si]) * S;
         const float lsp = P.split_lsp[si];
         stage2(R0, P.pi + l, R1, P.pi + r);
         stage2(R2, P.pibar + l, R3, P.pibar + r);
@@ -548,7 +558,7 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
 
     // ---- 7. split adjoints into the child rows (staging, preorder layout)
     for (int si = sb; si < se; ++si) {
-      const int lrow = P.split_l[si], rrow = P.split_r[si];
+      const int lrow = uniform(P.split_l[si]), rrow = uniform(P.split_r[si]);
       const size_t l = (size_t)lrow * S, r = (size_t)rrow * S;
       const float lsp = P.split_lsp[si];
       const float rml = P.rowmax[lrow], rmr = P.rowmax[rrow];
@@ -668,15 +678,26 @@ void bwd_row_large_kernel(BwdParams P, int first, int n_rows, int poff) {
 // The seven other bucket rows of all solved rows: levels 1 and up (schedule
 // slots first .. first + n_rows) and the n_cls classes of level 0, workgroup b
 // taking items b, b + gridDim.x, ... in order into slot b, whose rows 0..6 it
-// writes once.  128 VGPRs: 7 * CPT sums stay in registers; per row the two or
-// six rows it reads are staged through LDS to preorder positions.  Measured
-// @@FIG2@@.
+// writes once.
+//
+// One row is in flight per CU (four LDS rows), so the row's loads are issued
+// together ahead of its arithmetic: record and mask one row early, then v, the
+// split term, Pi*, Pibar* and the first split's children's Pi; the children's
+// Pibar while the coefficients are computed (with 8 positions per thread the
+// children are loaded in the split loop instead: the loads ahead spilled, 731 us
+// against 1305).  128 VGPRs hold 7 * CPT sums and the position tables packed 16
+// bits each.  Against one load per position, tables from memory and no loads
+// ahead: 11000 rows of 8191 states 953 -> 731 us, 5500 of 3001 186 -> 144 us.
 template <int NT, int CPT>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4)))
 void bwd_buckets_large_kernel(BwdParams P, int first, int n_rows, int n_cls) {
   constexpr int MAXS = NT * CPT;
   constexpr int LD = MAXS + 64;
+  constexpr int ZERO = MAXS;
+  constexpr int NG = CPT / 4;
+  constexpr bool PREF = CPT == 4;
   static_assert(CPT == 4 || CPT == 8, "4 or 8 positions per thread");
+  static_assert(MAXS <= 8192, "positions in 16 bits");
   __shared__ __align__(16) float L[4 * LD];
   float* R0 = L;
   float* R1 = L + LD;
@@ -691,29 +712,51 @@ void bwd_buckets_large_kernel(BwdParams P, int first, int n_rows, int n_cls) {
     if constexpr (CPT > 4) asm("; %1" : "+v"(b) : "s"(ep));
     return b + k;
   };
-  auto stage2 = [&](float* d0, const float* s0, float* d1, const float* s1) {
-    int sp[CPT];
-    float x[CPT], y[CPT];
-#pragma unroll
-    for (int j = 0; j < CPT; ++j) {
-      const int s = tid + j * NT;
-      sp[j] = s < S ? ldg(fresh(T.pre, ep), s) : -1;
-      x[j] = s < S ? ldg(fresh(s0, ep), s) : 0.0f;
-      y[j] = s < S ? ldg(fresh(s1, ep), s) : 0.0f;
-    }
-#pragma unroll
-    for (int j = 0; j < CPT; ++j)
-      if (sp[j] >= 0) {
-        d0[sp[j]] = x[j];
-        d1[sp[j]] = y[j];
-      }
-  };
   auto field = [](int rec, int f) { return __builtin_amdgcn_readlane(rec, f); };
   const int om0 = (tid >> 6) * 64 * CPT + (tid & 63);  // kb_om_index(tid * CPT, CPT)
-  auto omi = [&](int j, int k) { return ldg(fresh(P.om_tab + (size_t)j * MAXS, ep) + k * 64, om0); };
   auto omf = [&](int j, int k) { return ldg(fresh(P.om_const + (size_t)j * MAXS, ep) + k * 64, om0); };
   auto coef_k = [&](int k) {
     return CoefK{omf(OMC_DL, k), omf(OMC_EBAR, k), omf(OMC_E, k), omf(OMC_SL1, k), omf(OMC_SL2, k), omf(OMC_PS, k)};
+  };
+  // preorder position of column tid + j*NT, child2 (ZERO: none) of own position
+  // k, two to a register; bit k of has1: own position k has a child1 (k + 1)
+  unsigned pre2[CPT / 2], c22[CPT / 2], has1 = 0;
+#pragma unroll
+  for (int k = 0; k < CPT; k += 2) {
+    auto pre_of = [&](int s) { return (unsigned)T.pre[min(s, S - 1)]; };
+    auto c2_at = [&](int j) {
+      const int c2 = P.om_tab[(size_t)OMT_C2 * MAXS + j * 64 + om0];
+      return c2 >= 0 ? (unsigned)c2 : (unsigned)ZERO;
+    };
+    pre2[k / 2] = pre_of(tid + k * NT) | pre_of(tid + (k + 1) * NT) << 16;
+    c22[k / 2] = c2_at(k) | c2_at(k + 1) << 16;
+  }
+#pragma unroll
+  for (int k = 0; k < CPT; ++k) has1 |= P.om_tab[(size_t)OMT_C1 * MAXS + k * 64 + om0] >= 0 ? 1u << k : 0u;
+  auto opaque = [&]() {  // unpacked where they are used, not held unpacked
+#pragma unroll
+    for (int k = 0; k < CPT / 2; ++k) {
+      asm("; %1" : "+v"(pre2[k]) : "s"(ep));
+      asm("; %1" : "+v"(c22[k]) : "s"(ep));
+    }
+  };
+  auto half = [](const unsigned (&x)[CPT / 2], int k) { return (int)((k & 1) ? x[k / 2] >> 16 : x[k / 2] & 0xffffu); };
+  auto load_row = [&](const float* src, float (&x)[CPT]) {  // columns tid + j*NT (the last one past the row)
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) x[j] = ldg(fresh(src, ep), min(tid + j * NT, S - 1));
+  };
+  auto put_row = [&](float* dst, const float (&x)[CPT]) {
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) dst[half(pre2, j)] = x[j];
+  };
+  // child1 / child2 of own position k = 4g + kk in the staged row Rw (-inf: none);
+  // q: the row's own positions 4g .. 4g+3
+  auto child1 = [&](const float* Rw, const float4& q, int k) {
+    return (has1 >> k) & 1 ? ((k & 3) < 3 ? f4(q, (k & 3) + 1) : Rw[pos(k) + 1]) : KB_NEG_INF;
+  };
+  auto child2 = [&](const float* Rw, int k) {
+    const int c2 = half(c22, k);
+    return c2 != ZERO ? Rw[c2] : KB_NEG_INF;
   };
   enum { B_PD, B_PS, B_E, B_EBAR, B_SL2, B_SL1, B_MT, NB };
   float acc[NB][CPT];
@@ -722,20 +765,44 @@ void bwd_buckets_large_kernel(BwdParams P, int first, int n_rows, int n_cls) {
 #pragma unroll
     for (int k = 0; k < CPT; ++k) acc[j][k] = 0.0f;
 
-  for (int it = blockIdx.x; it < n_rows + n_cls; it += gridDim.x) {
+  // the sums as single registers: as vectors of four the compiler spills them
+  auto pin = [&]() {
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) asm("" : "+v"(acc[j][k]));
+  };
+  const int n_items = n_rows + n_cls;
+  auto load_rec = [&](int it) {
+    return it < n_rows ? P.bslot[(size_t)KB_BREC * (first + it) + (tid & (KB_BREC - 1))] : 0;
+  };
+  auto load_on = [&](int it, int rec) {
+    return it >= n_items ? 0 : it >= n_rows ? (int)P.cls_active[it - n_rows] : (int)P.mask[field(rec, BR_ROW)];
+  };
+  int nrec = load_rec(blockIdx.x), non = load_on(blockIdx.x, nrec);
+  for (int it = blockIdx.x; it < n_items; it += gridDim.x) {
+    const int rec = nrec, on = __builtin_amdgcn_readfirstlane(non);
+    const int nit = it + (int)gridDim.x;
+    nrec = load_rec(nit);
     const bool cm = it >= n_rows;
     const int c = it - n_rows;
-    const int rec = cm ? 0 : P.bslot[(size_t)KB_BREC * (first + it) + (tid & (KB_BREC - 1))];
-    const int row = cm ? P.cls_rows[P.cls_ptr[c]] : field(rec, BR_ROW);
-    if (!(cm ? P.cls_active[c] : P.mask[row])) continue;
+    // (no row: neither a root nor anyone's child, v = 0)
     const float* vr = cm ? P.rhsc + (size_t)c * kb_stage_ld(S) : bwd_v_row(P, field(rec, BR_S0), field(rec, BR_FAM));
-    if (!vr) continue;  // neither a root nor anyone's child: v = 0
+    if (!on || !vr) {
+      non = load_on(nit, nrec);
+      continue;
+    }
+    const int row = cm ? uniform(P.cls_rows[P.cls_ptr[c]]) : field(rec, BR_ROW);
     const bool leaf_row = (cm ? P.row_kind[row] : field(rec, BR_LEAF)) != 0;
     const int lpos = cm ? (leaf_row ? T.pre[P.leaf_state[row]] : -1) : field(rec, BR_LPOS);
     const int sb = cm ? P.split_ptr[row] : field(rec, BR_SB), se = cm ? P.split_ptr[row + 1] : field(rec, BR_SE);
+    const bool split = se > sb;
+    const size_t l0 = split ? (size_t)(cm ? uniform(P.split_l[sb]) : field(rec, BR_L0)) * S : 0;
+    const size_t r0 = split ? (size_t)(cm ? uniform(P.split_r[sb]) : field(rec, BR_R0)) * S : 0;
+    const float lsp0 = split ? (cm ? P.split_lsp[sb] : __int_as_float(field(rec, BR_LSP0))) : 0.0f;
     ep = 8 * it + 1;
+    opaque();
     float v[CPT], dts[CPT];
-    gld_own<CPT>(fresh(vr, ep), S, v, 0.0f);
 #pragma unroll
     for (int k = 0; k < CPT; ++k) dts[k] = KB_NEG_INF;
     if (!leaf_row) {
@@ -748,30 +815,40 @@ void bwd_buckets_large_kernel(BwdParams P, int first, int n_rows, int n_cls) {
 #pragma unroll
         for (int k = 0; k < CPT; ++k) sum[k] = 0.0f;
         for (int si = sb; si < se; ++si) {
-          const size_t l = (size_t)P.split_l[si] * S, r = (size_t)P.split_r[si] * S;
+          const size_t l = (size_t)uniform(P.split_l[si]) * S, r = (size_t)uniform(P.split_r[si]) * S;
           const float lsp = P.split_lsp[si];
           __syncthreads();
-          stage2(R0, P.pi + l, R1, P.pi + r);
-          stage2(R2, P.pibar + l, R3, P.pibar + r);
+          float x[CPT], y[CPT];
+          load_row(P.pi + l, x);
+          load_row(P.pi + r, y);
+          put_row(R0, x);
+          put_row(R1, y);
+          load_row(P.pibar + l, x);
+          load_row(P.pibar + r, y);
+          put_row(R2, x);
+          put_row(R3, y);
           __syncthreads();
 #pragma unroll
-          for (int k = 0; k < CPT; ++k) {
-            const int i = pos(k);
-            if (i < S) {
-              const int c1 = omi(OMT_C1, k), c2 = omi(OMT_C2, k);
-              const float pl = R0[i], pr = R1[i];
-              const float l1 = c1 >= 0 ? R0[c1] : KB_NEG_INF, r1 = c1 >= 0 ? R1[c1] : KB_NEG_INF;
-              const float l2 = c2 >= 0 ? R0[c2] : KB_NEG_INF, r2 = c2 >= 0 ? R1[c2] : KB_NEG_INF;
-              const float t0 = lsp + omf(OMC_PD, k) + pl + pr;
-              const float t1 = lsp + pl + R3[i];
-              const float t2 = lsp + pr + R2[i];
-              const float sp = omf(OMC_PS, k);
-              const float t3 = lsp + sp + l1 + r2;
-              const float t4 = lsp + sp + r1 + l2;
-              const float m5 = fmaxf(fmaxf(fmaxf(t0, t1), fmaxf(t2, t3)), t4);
-              const float ms = fsafe(m5);
-              const float s5 = exp2f(t0 - ms) + exp2f(t1 - ms) + exp2f(t2 - ms) + exp2f(t3 - ms) + exp2f(t4 - ms);
-              lse_merge(dts[k], sum[k], m5, s5);
+          for (int g = 0; g < NG; ++g) {
+            const float4 pl4 = ld4(R0 + tid * CPT + 4 * g), pr4 = ld4(R1 + tid * CPT + 4 * g);
+            const float4 bl4 = ld4(R2 + tid * CPT + 4 * g), br4 = ld4(R3 + tid * CPT + 4 * g);
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) {
+              const int k = 4 * g + kk;
+              if (pos(k) < S) {
+                const float pl = f4(pl4, kk), pr = f4(pr4, kk);
+                const float l1 = child1(R0, pl4, k), r1 = child1(R1, pr4, k), l2 = child2(R0, k), r2 = child2(R1, k);
+                const float t0 = lsp + omf(OMC_PD, k) + pl + pr;
+                const float t1 = lsp + pl + f4(br4, kk);
+                const float t2 = lsp + pr + f4(bl4, kk);
+                const float sp = omf(OMC_PS, k);
+                const float t3 = lsp + sp + l1 + r2;
+                const float t4 = lsp + sp + r1 + l2;
+                const float m5 = fmaxf(fmaxf(fmaxf(t0, t1), fmaxf(t2, t3)), t4);
+                const float ms = fsafe(m5);
+                const float s5 = exp2f(t0 - ms) + exp2f(t1 - ms) + exp2f(t2 - ms) + exp2f(t3 - ms) + exp2f(t4 - ms);
+                lse_merge(dts[k], sum[k], m5, s5);
+              }
             }
           }
         }
@@ -779,59 +856,109 @@ void bwd_buckets_large_kernel(BwdParams P, int first, int n_rows, int n_cls) {
         for (int k = 0; k < CPT; ++k) dts[k] = log2f(sum[k]) + dts[k];
       }
     }
-    __syncthreads();  // LDS of the previous row or split is no longer read
-    stage2(R0, P.pi + (size_t)row * S, R1, P.pibar + (size_t)row * S);
+    gld_own<CPT>(fresh(vr, ep), S, v, 0.0f);
+    {
+      float a[CPT], b[CPT], x[CPT], y[CPT];
+      load_row(P.pi + (size_t)row * S, a);
+      load_row(P.pibar + (size_t)row * S, b);
+      if (PREF && split) {
+        load_row(P.pi + l0, x);
+        load_row(P.pi + r0, y);
+      }
+      __syncthreads();  // LDS of the previous row or split is no longer read
+      put_row(R0, a);
+      put_row(R1, b);
+      if (PREF && split) {
+        put_row(R2, x);
+        put_row(R3, y);
+      }
+    }
     __syncthreads();
+    non = load_on(nit, nrec);
     ep = 8 * it + 2;
+    opaque();
+    float bx[CPT], by[CPT];  // the first split's children's Pibar, in flight below
+    if (PREF && split) {
+      load_row(P.pibar + l0, bx);
+      load_row(P.pibar + r0, by);
+    }
     float piv[CPT];
     lds_load_own<CPT>(R0, piv);
 #pragma unroll
-    for (int k = 0; k < CPT; ++k) {
-      const int i = pos(k);
-      if (i < S) {
-        const int c1 = omi(OMT_C1, k), c2 = omi(OMT_C2, k);
-        const Coef6 q = coef_at(coef_k(k), piv[k], R1[i], dts[k], c1 >= 0 ? R0[c1] : KB_NEG_INF,
-                                c2 >= 0 ? R0[c2] : KB_NEG_INF, leaf_row, i == lpos);
-        const float aw0 = v[k] * q.q[0], aw1 = v[k] * q.q[1], aw2 = v[k] * q.q[2];
-        const float aw3 = v[k] * q.q[3], aw4 = v[k] * q.q[4], aw5 = v[k] * q.q[5];
-        acc[B_PD][k] += aw0;
-        acc[B_PS][k] += aw3 + aw4 + aw5;
-        acc[B_E][k] += aw0 + aw2;
-        acc[B_EBAR][k] += aw1;
-        acc[B_SL2][k] += aw4;
-        acc[B_SL1][k] += aw3;
-        acc[B_MT][k] += aw2;
-      }
-    }
-    for (int si = sb; si < se; ++si) {
-      const size_t l = (size_t)P.split_l[si] * S, r = (size_t)P.split_r[si] * S;
-      const float lsp = P.split_lsp[si];
-      ep = -4 * si - 1;
-      __syncthreads();
-      stage2(R0, P.pi + l, R1, P.pi + r);
-      stage2(R2, P.pibar + l, R3, P.pibar + r);
-      __syncthreads();
-      ep = -4 * si - 2;
+    for (int g = 0; g < NG; ++g) {
+      const float4 pi4 = make_float4(piv[4 * g], piv[4 * g + 1], piv[4 * g + 2], piv[4 * g + 3]);
+      const float4 pb4 = ld4(R1 + tid * CPT + 4 * g);
 #pragma unroll
-      for (int k = 0; k < CPT; ++k) {
+      for (int kk = 0; kk < 4; ++kk) {
+        const int k = 4 * g + kk;
         const int i = pos(k);
-        if (i < S && piv[k] != KB_NEG_INF) {
-          const int c1 = omi(OMT_C1, k), c2 = omi(OMT_C2, k);
-          const float pl = R0[i], pr = R1[i], bl = R2[i], br = R3[i];
-          const float l1 = c1 >= 0 ? R0[c1] : KB_NEG_INF, r1 = c1 >= 0 ? R1[c1] : KB_NEG_INF;
-          const float l2 = c2 >= 0 ? R0[c2] : KB_NEG_INF, r2 = c2 >= 0 ? R1[c2] : KB_NEG_INF;
-          const float d = omf(OMC_PD, k), sp = omf(OMC_PS, k);
-          const float base = lsp - piv[k];
-          const float vd0 = v[k] * exp2_hw(base + (d + pl + pr));
-          const float vd1 = v[k] * exp2_hw(base + (pl + br));
-          const float vd2 = v[k] * exp2_hw(base + (pr + bl));
-          const float vd3 = v[k] * exp2_hw(base + (sp + l1 + r2));
-          const float vd4 = v[k] * exp2_hw(base + (sp + r1 + l2));
-          acc[B_PD][k] += vd0;
-          acc[B_PS][k] += vd3 + vd4;
-          acc[B_MT][k] += vd1 + vd2;
+        if (i < S) {
+          const Coef6 q = coef_at(coef_k(k), piv[k], f4(pb4, kk), dts[k], child1(R0, pi4, k), child2(R0, k), leaf_row,
+                                  i == lpos);
+          const float aw0 = v[k] * q.q[0], aw1 = v[k] * q.q[1], aw2 = v[k] * q.q[2];
+          const float aw3 = v[k] * q.q[3], aw4 = v[k] * q.q[4], aw5 = v[k] * q.q[5];
+          acc[B_PD][k] += aw0;
+          acc[B_PS][k] += aw3 + aw4 + aw5;
+          acc[B_E][k] += aw0 + aw2;
+          acc[B_EBAR][k] += aw1;
+          acc[B_SL2][k] += aw4;
+          acc[B_SL1][k] += aw3;
+          acc[B_MT][k] += aw2;
         }
       }
+    }
+    pin();
+    for (int si = sb; si < se; ++si) {
+      float lsp = lsp0;
+      __syncthreads();
+      ep = -4 * si - 1;
+      opaque();
+      if (!PREF || si > sb) {
+        const size_t l = (size_t)uniform(P.split_l[si]) * S, r = (size_t)uniform(P.split_r[si]) * S;
+        lsp = P.split_lsp[si];
+        float x[CPT], y[CPT];
+        load_row(P.pi + l, x);
+        load_row(P.pi + r, y);
+        if (PREF) {
+          load_row(P.pibar + l, bx);
+          load_row(P.pibar + r, by);
+        }
+        put_row(R2, x);
+        put_row(R3, y);
+        if (!PREF) {
+          load_row(P.pibar + l, bx);
+          load_row(P.pibar + r, by);
+        }
+      }
+      put_row(R0, bx);
+      put_row(R1, by);
+      __syncthreads();
+      ep = -4 * si - 2;
+      opaque();
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        const float4 pl4 = ld4(R2 + tid * CPT + 4 * g), pr4 = ld4(R3 + tid * CPT + 4 * g);
+        const float4 bl4 = ld4(R0 + tid * CPT + 4 * g), br4 = ld4(R1 + tid * CPT + 4 * g);
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+          const int k = 4 * g + kk;
+          if (pos(k) < S && piv[k] != KB_NEG_INF) {
+            const float pl = f4(pl4, kk), pr = f4(pr4, kk), bl = f4(bl4, kk), br = f4(br4, kk);
+            const float l1 = child1(R2, pl4, k), r1 = child1(R3, pr4, k), l2 = child2(R2, k), r2 = child2(R3, k);
+            const float d = omf(OMC_PD, k), sp = omf(OMC_PS, k);
+            const float base = lsp - piv[k];
+            const float vd0 = v[k] * exp2_hw(base + (d + pl + pr));
+            const float vd1 = v[k] * exp2_hw(base + (pl + br));
+            const float vd2 = v[k] * exp2_hw(base + (pr + bl));
+            const float vd3 = v[k] * exp2_hw(base + (sp + l1 + r2));
+            const float vd4 = v[k] * exp2_hw(base + (sp + r1 + l2));
+            acc[B_PD][k] += vd0;
+            acc[B_PS][k] += vd3 + vd4;
+            acc[B_MT][k] += vd1 + vd2;
+          }
+        }
+      }
+      pin();
     }
   }
   float* const slot = P.contrib + (size_t)blockIdx.x * KB_LARGE_SLOT_ROWS * MAXS + tid * CPT;
