@@ -44,3 +44,27 @@ def test_solve_at_shape_edges_matches_oracle(leaves):
     assert ok and (ma <= 2e-4 or mr <= 1e-5)
     assert np.abs(saved["E"].cpu().numpy() - ref["E"]).max() <= 1e-6
     assert rt <= 1e-4 and rc <= 1e-4
+
+
+@pytest.mark.parametrize("leaves", [65, 513, 1025, 1501, 2049])
+def test_backward_of_an_older_forward_matches_its_solve(leaves):
+    """Outputs of a forward that is no longer the plan's last: its split terms are gone, and every
+    backward kernel recomputes them (the solve's own backward reads the stored ones)."""
+    from kbench import synth
+    from kbench.fused import FusedSolver, problem_to_captured
+    from kbench.runtime import make_static
+
+    cap = problem_to_captured(synth.build_problem(synth.ProblemConfig(
+        leaves, 4, n_nni=3, family_leaves_median=12.0, family_leaves_sigma=0.5, family_leaves_max=40,
+        statewise=False, seed=leaves)))
+    static = make_static(cap, "cuda")
+    solver = FusedSolver(static, static.solver_options)
+    theta = cap["inputs"]["theta"].cuda()
+    cw = torch.from_numpy(np.random.default_rng(7).normal(0.0, 0.5, size=solver.S).astype(np.float32)).cuda()
+    _, saved, gt, gc = solver.solve(theta, cw)
+    solver.run_forward(theta - 0.5, cw)
+    gt2, gc2 = solver.run_backward(theta, cw, saved)
+    print(f"[older forward] S={solver.S}", flush=True)
+    # the split terms differ by float32 rounding only (exp2 / log2 of the two kernels)
+    assert kbtest.norm_rel(gt2.cpu().numpy(), gt.cpu().numpy()) <= 1e-5
+    assert kbtest.norm_rel(gc2.cpu().numpy(), gc.cpu().numpy()) <= 1e-5
