@@ -1796,13 +1796,19 @@ struct DcArgs {
   T *gPl, *gPr, *prow, *psum, *mrow;
 };
 
-template <typename T, int CPT>
-__global__ __launch_bounds__(NT)
-__attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? kb::pre_waves_per_eu(CPT) : 1))) void dts_cross_kernel(DcArgs<T> a) {
-  extern __shared__ unsigned char smraw[];
+// One split per workgroup of the smallest shape that holds a row; memory-bound
+// (six rows read, two to eight written), so what counts is how many splits a CU
+// has in flight: up to 2048 threads of them instead of two 1024-thread
+// workgroups.  The up to six row sums share one exchange (each took two
+// barriers).  Measured against 1024 threads for every row: 2047 states 81 -> 76
+// us a wave, 1023 states (18 mostly narrow waves) 211 -> 166 us.
+template <typename T, int BT, int CPT>
+__global__ __launch_bounds__(BT) void dts_cross_kernel(DcArgs<T> a) {
+  constexpr int BW = BT / 64;
+  extern __shared__ __align__(16) unsigned char smraw[];
   T* Lr = reinterpret_cast<T*>(smraw);
   T* Rr = Lr + a.S;
-  __shared__ T red[NW];
+  __shared__ T red[6][BW];
   const int S = a.S;
   const long long i = blockIdx.x;
   const long long N = a.N;
@@ -1814,7 +1820,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? kb::pre_waves_per_eu(CPT) : 
   if (!act) {
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
-      const int s = threadIdx.x + k * NT;
+      const int s = threadIdx.x + k * BT;
       if (s < S) {
         sideL[s] = 0;
         sideR[s] = 0;
@@ -1877,7 +1883,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? kb::pre_waves_per_eu(CPT) : 
   }
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
+    const int s = threadIdx.x + k * BT;
     vd3[k] = vd4[k] = 0;
     c1v[k] = c2v[k] = -1;
     if (s < S) {
@@ -1950,6 +1956,22 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? kb::pre_waves_per_eu(CPT) : 
       }
     }
   }
+  {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    auto put = [&](int j, T x) {
+      if (lane == 63) red[j][wv] = x;
+    };
+    if (a.psum) {
+      put(0, wscan(sd));
+      put(1, wscan(ss));
+    }
+    if (a.output_ud) {
+      put(2, wscan(sul));
+      put(3, wscan(sur));
+      put(4, a.side_thr > 0.0 ? wscan(bl) : wmax63(bl));
+      put(5, a.side_thr > 0.0 ? wscan(br) : wmax63(br));
+    }
+  }
   __syncthreads();
   // speciation terms land in the children's columns (each column has one parent)
 #pragma unroll
@@ -1966,41 +1988,39 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? kb::pre_waves_per_eu(CPT) : 
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
+    const int s = threadIdx.x + k * BT;
     if (s < S) {
       sideL[s] = Lr[s];
       sideR[s] = Rr[s];
     }
   }
-  if (a.psum) {
-    const T tsd = block_sum(sd, red);
-    const T tss = block_sum(ss, red);
-    if (threadIdx.x == 0) {
-      a.psum[i] = tsd;
-      a.psum[N + i] = tss;
+  if (threadIdx.x == 0) {
+    auto sum = [&](int j) {
+      T x = red[j][0];
+#pragma unroll
+      for (int w = 1; w < BW; ++w) x += red[j][w];
+      return x;
+    };
+    auto top = [&](int j) {
+      T x = red[j][0];
+#pragma unroll
+      for (int w = 1; w < BW; ++w) x = tmax(x, red[j][w]);
+      return x;
+    };
+    if (a.psum) {
+      a.psum[i] = sum(0);
+      a.psum[N + i] = sum(1);
     }
-  }
-  if (a.output_ud) {
-    const T tl = block_sum(sul, red);
-    const T tr = block_sum(sur, red);
-    T ql, qr;
-    if (a.side_thr > 0.0) {
-      ql = block_sum(bl, red);
-      qr = block_sum(br, red);
-    } else {
-      ql = block_max(bl, red);
-      qr = block_max(br, red);
-    }
-    if (threadIdx.x == 0) {
-      a.A[i] = tl;
-      a.A[N + i] = tr;
+    if (a.output_ud) {
+      a.A[i] = sum(2);
+      a.A[N + i] = sum(3);
       if (a.side_active) {
         if (a.side_thr > 0.0) {
-          a.side_active[i] = (double)ql > a.side_thr;
-          a.side_active[N + i] = (double)qr > a.side_thr;
+          a.side_active[i] = (double)sum(4) > a.side_thr;
+          a.side_active[N + i] = (double)sum(5) > a.side_thr;
         } else {
-          a.side_active[i] = ql != T(0);
-          a.side_active[N + i] = qr != T(0);
+          a.side_active[i] = top(4) != T(0);
+          a.side_active[N + i] = top(5) != T(0);
         }
       }
     }
@@ -2020,13 +2040,23 @@ struct PvArgs {
   T* contrib;
 };
 
-template <typename T, int CPT>
-__global__ __launch_bounds__(NT) void pibar_vjp_kernel(OpsTree t, PvArgs<T> a) {
-  extern __shared__ unsigned char smraw[];
-  T* U = reinterpret_cast<T*>(smraw);
-  T* Up = U + t.S;
-  __shared__ T red[NW];
+// One side per workgroup of the smallest shape that holds a row.  The row's ud
+// goes to its preorder positions in LDS, is scanned in registers (thread t owns
+// positions t*CPT + k, one wavefront scan, published with the wavefront totals
+// under one barrier), and each column reads its two prefix values back: two
+// barriers in all, and the Pi row is loaded ahead of them.  Measured against an
+// LDS block scan on 1024 threads: 2047 states 57 -> 34 us a wave, 1023 states
+// (18 waves) 144 -> 105 us.
+template <typename T, int BT, int CPT>
+__global__ __launch_bounds__(BT) void pibar_vjp_kernel(OpsTree t, PvArgs<T> a) {
+  constexpr int BW = BT / 64;
+  constexpr int MAXS = BT * CPT;
+  constexpr int SEG = 64 * CPT;  // positions per wavefront
+  extern __shared__ __align__(16) unsigned char smraw[];
+  T* L = reinterpret_cast<T*>(smraw);
+  __shared__ T wA[BW];
   const int S = a.S;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const long long row = blockIdx.x;
   const long long si = row < a.N ? row : row - a.N;
   T* crow = a.contrib + (size_t)row * S;
@@ -2035,58 +2065,115 @@ __global__ __launch_bounds__(NT) void pibar_vjp_kernel(OpsTree t, PvArgs<T> a) {
   if (!go) {
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
-      const int s = threadIdx.x + k * NT;
+      const int s = tid + k * BT;
       if (s < S) crow[s] = 0;
     }
     return;
   }
   const long long child = row < a.N ? a.sl[si] : a.sr[si];
   T* udr = a.ud + (size_t)row * S;
+  const T* pr = a.Pi + (size_t)child * S;
+  int pos[CPT], end[CPT];
+  T pic[CPT];
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
-    if (s < S) U[s] = udr[s];
+    const int s = tid + k * BT;
+    pos[k] = 0;
+    end[k] = 1;
+    pic[k] = T(0);
+    if (s < S) {
+      pos[k] = t.ppos[s];
+      end[k] = t.pend[s];
+      pic[k] = a.use_col ? a.col[s] + pr[s] : pr[s];
+      L[pos[k]] = udr[s];
+    }
   }
+  for (int i = S + tid; i < MAXS; i += BT) L[i] = T(0);
   __syncthreads();
-  subtree_scan(t, U, Up, red);
+  T sc[CPT], run = T(0);
+  own_load<CPT>(L, sc);
+#pragma unroll
+  for (int k = 0; k < CPT; ++k) {
+    run += sc[k];
+    sc[k] = run;
+  }
+  const T ws = wscan(run);
+#pragma unroll
+  for (int k = 0; k < CPT; ++k) sc[k] += ws - run;
+  own_store<CPT>(L, sc);
+  if (lane == 63) wA[wv] = ws;
+  __syncthreads();
+  const T wt = kb::lds_wave_values<BW>(wA, lane, T(0));
+  const T wex = wscan_first<BW>(wt) - wt;  // lane x < BW: offset of wavefront x
   const T A = a.A[row];
   const T rms = msafe(a.rowmax[child]);
-  const T* pr = a.Pi + (size_t)child * S;
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    const int s = threadIdx.x + k * NT;
+    const int s = tid + k * BT;
+    const int q = pos[k] > 0 ? pos[k] - 1 : 0, e = end[k] - 1;
+    const T pq = L[q] + shfl_of(wex, q / SEG), pe = L[e] + shfl_of(wex, e / SEG);
     if (s < S) {
-      udr[s] = subtree_of(t, Up, s);
-      const T pp = xexp2((a.use_col ? a.col[s] + pr[s] : pr[s]) - rms);
-      crow[s] = pp * complement_of(t, Up, s, A);
+      const T pm1 = pos[k] > 0 ? pq : T(0);
+      udr[s] = pe - pm1;
+      crow[s] = xexp2(pic[k] - rms) * (pm1 + (A - pe));
     }
   }
 }
 
 // ---- fixed-order row accumulation -------------------------------------------------------
 
+// Workgroup x takes the runs that start at sorted entries SCAT_K x .. SCAT_K x +
+// SCAT_K - 1.  Mostly a run is one row (a child row has one parent): those are
+// loaded and added together; longer runs are summed in order first.  One entry
+// per workgroup waited out a chain of four loads for 1 KB of data: 34 us per wave
+// of 2047 states against 26 us (1023-state waves of a few rows 5.2 against 5.4).
+constexpr int SCAT_K = 4;
+
 template <typename T>
 __global__ __launch_bounds__(256) void scatter_add_kernel(int S, long long n, const T* src, const int* order,
                                                           const int64_t* keys, T* dst, long long dst_stride) {
-  const long long k = blockIdx.x;
+  const long long k0 = (long long)blockIdx.x * SCAT_K;
   const int s = blockIdx.y * 256 + threadIdx.x;
   if (s >= S) return;
-  const long long key = keys[k];
-  if (key < 0 || (k > 0 && keys[k - 1] == key)) return;
-  long long e = k + 1;  // end of the run of this key (the same for every thread)
-  while (e < n && keys[e] == key) ++e;
-  // the run's rows added in order; the loads of eight rows are issued before their adds
-  T acc = 0;
-  long long j = k;
-  for (; j + 8 <= e; j += 8) {
-    T x[8];
+  long long key[SCAT_K];
+  bool one[SCAT_K], run[SCAT_K];  // the entry is a run of one row / starts a longer run
+  T x[SCAT_K], d[SCAT_K];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) x[i] = src[(size_t)order[j + i] * S + s];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) acc += x[i];
+  for (int u = 0; u < SCAT_K; ++u) {
+    const long long k = k0 + u;
+    key[u] = k < n ? keys[k] : -1;
+    const bool first = key[u] >= 0 && (k == 0 || keys[k - 1] != key[u]);
+    const bool more = first && k + 1 < n && keys[k + 1] == key[u];
+    one[u] = first && !more;
+    run[u] = more;
+    x[u] = d[u] = T(0);
+    if (one[u]) {
+      x[u] = src[(size_t)order[k] * S + s];
+      d[u] = dst[(size_t)(key[u] * dst_stride) + s];
+    }
   }
-  for (; j < e; ++j) acc += src[(size_t)order[j] * S + s];
-  dst[(size_t)(key * dst_stride) + s] += acc;
+#pragma unroll
+  for (int u = 0; u < SCAT_K; ++u)
+    if (one[u]) dst[(size_t)(key[u] * dst_stride) + s] = d[u] + x[u];
+#pragma unroll
+  for (int u = 0; u < SCAT_K; ++u) {
+    if (!run[u]) continue;
+    const long long k = k0 + u;
+    long long e = k + 2;  // end of the run of this key (the same for every thread)
+    while (e < n && keys[e] == key[u]) ++e;
+    // the run's rows added in order; the loads of eight rows are issued before their adds
+    T acc = 0;
+    long long j = k;
+    for (; j + 8 <= e; j += 8) {
+      T y[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) y[i] = src[(size_t)order[j + i] * S + s];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc += y[i];
+    }
+    for (; j < e; ++j) acc += src[(size_t)order[j] * S + s];
+    dst[(size_t)(key[u] * dst_stride) + s] += acc;
+  }
 }
 
 constexpr int SUM_CHUNK = 64;
@@ -2284,6 +2371,27 @@ static __device__ __align__(256) double scratch[KB_ESTEP_VJP_NOALLOC_MAX];
 // host side
 // =====================================================================================
 
+// The smallest workgroup whose BT * CPT positions hold a row (see estep_kernel,
+// dts_cross_kernel, pibar_vjp_kernel).
+#define KBO_SHAPE(S, ...)                                                      \
+  do {                                                                               \
+    if ((S) <= 128) { constexpr int BT = 64, CPT = 2; __VA_ARGS__; }                 \
+    else if ((S) <= 256) { constexpr int BT = 128, CPT = 2; __VA_ARGS__; }           \
+    else if ((S) <= 512) { constexpr int BT = 256, CPT = 2; __VA_ARGS__; }           \
+    else if ((S) <= 1024) { constexpr int BT = 512, CPT = 2; __VA_ARGS__; }          \
+    else if ((S) <= 2048) { constexpr int BT = 512, CPT = 4; __VA_ARGS__; }          \
+    else if ((S) <= 4096) { constexpr int BT = 1024, CPT = 4; __VA_ARGS__; }         \
+    else { constexpr int BT = 1024, CPT = 8; __VA_ARGS__; }                          \
+  } while (0)
+
+// Dispatch over the element type.
+#define KBO_TYPE(DTYPE, S, ...)                                                      \
+  do {                                                                               \
+    if (cpt_for(S) == 0) return kb::set_error(KB_ERR_ARG, "S=%d exceeds 8192", S);   \
+    if ((DTYPE) == KB_F64) { using T = double; __VA_ARGS__; }                        \
+    else { using T = float; __VA_ARGS__; }                                           \
+  } while (0)
+
 namespace {
 
 using namespace kbo_host;
@@ -2437,21 +2545,9 @@ int kb_ops_max_states(int dtype) {
 
 }  // extern "C"
 
-// The smallest shape that holds the tree (see estep_kernel).
-#define KBO_ESTEP_SHAPE(S, ...)                                                      \
-  do {                                                                               \
-    if ((S) <= 128) { constexpr int BT = 64, CPT = 2; __VA_ARGS__; }                 \
-    else if ((S) <= 256) { constexpr int BT = 128, CPT = 2; __VA_ARGS__; }           \
-    else if ((S) <= 512) { constexpr int BT = 256, CPT = 2; __VA_ARGS__; }           \
-    else if ((S) <= 1024) { constexpr int BT = 512, CPT = 2; __VA_ARGS__; }          \
-    else if ((S) <= 2048) { constexpr int BT = 512, CPT = 4; __VA_ARGS__; }          \
-    else if ((S) <= 4096) { constexpr int BT = 1024, CPT = 4; __VA_ARGS__; }         \
-    else { constexpr int BT = 1024, CPT = 8; __VA_ARGS__; }                          \
-  } while (0)
-
 template <typename T>
 static int launch_estep_rows(const kbo::OpsTree& t, const kbo::EsArgs<T>& a, hipStream_t st) {
-  KBO_ESTEP_SHAPE(t.S, {
+  KBO_SHAPE(t.S, {
     const size_t lds = (size_t)2 * (BT * CPT + 64) * sizeof(double);
     auto k = a.use_col ? kbo::estep_kernel<T, BT, CPT, true> : kbo::estep_kernel<T, BT, CPT, false>;
     if (int rc = set_lds(k, lds)) return rc;
@@ -2461,7 +2557,7 @@ static int launch_estep_rows(const kbo::OpsTree& t, const kbo::EsArgs<T>& a, hip
 }
 template <typename T>
 static int launch_estep_vjp_rows(const kbo::OpsTree& t, const kbo::EvArgs<T>& a, hipStream_t st) {
-  KBO_ESTEP_SHAPE(t.S, {
+  KBO_SHAPE(t.S, {
     const size_t lds = (size_t)2 * (BT * CPT + 64) * sizeof(double);
     auto k = kbo::estep_vjp_kernel<T, BT, CPT>;
     if (int rc = set_lds(k, lds)) return rc;
@@ -2575,9 +2671,11 @@ int launch_bwd(const kbo::OpsTree& t, const kbo::WbArgs<T>& a, int W, hipStream_
   return 0;
 }
 
-// The preorder-ownership kernel on the smallest shape that holds the row; its
-// four padded LDS rows do not hold doubles past 4096 states, where the
-// column-order kernel (four rows of S) goes on.
+// The preorder-ownership kernel on the smallest shape that holds the row (floats
+// of 513..1024 states on 1024 x 1: 19.1 us a narrow wave against 20.9 on 512 x
+// 2); its four padded LDS rows do not hold doubles past 4096 states, where the
+// column-order kernel (four rows of S) goes on.  Doubles against that kernel:
+// 1500 rows of 599 states 228 -> 79 us.
 template <typename T>
 int launch_wave_bwd(const kbo::OpsTree& t, const kbo::WbArgs<T>& a, int W, size_t lds, hipStream_t st) {
   constexpr bool F32 = std::is_same_v<T, float>;
@@ -2585,7 +2683,7 @@ int launch_wave_bwd(const kbo::OpsTree& t, const kbo::WbArgs<T>& a, int W, size_
   if (S <= 128) return launch_bwd<T, 64, 2>(t, a, W, st);
   if (S <= 256) return launch_bwd<T, 128, 2>(t, a, W, st);
   if (S <= 512) return launch_bwd<T, 256, 2>(t, a, W, st);
-  if (S <= 1024) return launch_bwd<T, 512, 2>(t, a, W, st);
+  if (S <= 1024) return launch_bwd<T, F32 ? 1024 : 512, F32 ? 1 : 2>(t, a, W, st);
   if (S <= 2048) return launch_bwd<T, 1024, 2>(t, a, W, st);
   if (S <= 4096) return launch_bwd<T, 1024, 4>(t, a, W, st);
   if constexpr (F32) return launch_bwd<T, 1024, 8>(t, a, W, st);
@@ -2744,16 +2842,18 @@ int kb_dts_cross_backward(const kb_dts_cross_io* io, void* stream) {
   const int S = io->S;
   const size_t lds = (size_t)2 * S * elem_size(io->dtype);
   if (int rc = check_lds(lds, S, io->dtype)) return rc;
-  KBO_DISPATCH(io->dtype, S, {
+  KBO_TYPE(io->dtype, S, {
     kbo::DcArgs<T> a{S, io->param_layout, io->mt_layout, io->output_ud, io->skip_inactive_ud_zero, io->N, io->ws,
                      io->side_threshold, (const T*)io->Pi, (const T*)io->Pibar, (const T*)io->v, io->active, io->sl,
                      io->sr, io->reduce_idx, io->item_idx, io->node_child1, io->node_child2, (const T*)io->wlsp, (const T*)io->log_pD,
                      (const T*)io->log_pS, (const T*)io->mt, (const T*)io->pibar_row_max, (T*)io->side_rows,
                      (T*)io->ud, (T*)io->A, io->side_active, (T*)io->grad_Pibar_l, (T*)io->grad_Pibar_r,
                      (T*)io->param_rows, (T*)io->param_sums, (T*)io->mt_rows};
-    auto k = kbo::dts_cross_kernel<T, CPT>;
-    if (int rc = set_lds(k, lds)) return rc;
-    hipLaunchKernelGGL(k, dim3((unsigned)io->N), dim3(kbo::NT), lds, st_of(stream), a);
+    KBO_SHAPE(S, {
+      auto k = kbo::dts_cross_kernel<T, BT, CPT>;
+      if (int rc = set_lds(k, lds)) return rc;
+      hipLaunchKernelGGL(k, dim3((unsigned)io->N), dim3(BT), lds, st_of(stream), a);
+    });
   });
   KBO_HIP(hipGetLastError());
   return 0;
@@ -2769,13 +2869,16 @@ int kb_pibar_vjp(const kb_tree* tr, const kb_pibar_vjp_io* io, void* stream) {
   const size_t lds = (size_t)2 * S * elem_size(io->dtype);
   if (int rc = check_lds(lds, S, io->dtype)) return rc;
   const kbo::OpsTree t = tr->dev();
-  KBO_DISPATCH(io->dtype, S, {
+  KBO_TYPE(io->dtype, S, {
     kbo::PvArgs<T> a{S, io->use_col_weights, io->N, (const T*)io->Pi, (const T*)io->col_log_probs, (const T*)io->A,
                      (const T*)io->pibar_row_max, (T*)io->ud, io->side_active, io->active, io->sl, io->sr,
                      io->reduce_idx, (T*)io->contrib};
-    auto k = kbo::pibar_vjp_kernel<T, CPT>;
-    if (int rc = set_lds(k, lds)) return rc;
-    hipLaunchKernelGGL(k, dim3((unsigned)(2 * io->N)), dim3(kbo::NT), lds, st_of(stream), t, a);
+    KBO_SHAPE(S, {
+      const size_t bytes = (size_t)BT * CPT * sizeof(T);
+      auto k = kbo::pibar_vjp_kernel<T, BT, CPT>;
+      if (int rc = set_lds(k, bytes)) return rc;
+      hipLaunchKernelGGL(k, dim3((unsigned)(2 * io->N)), dim3(BT), bytes, st_of(stream), t, a);
+    });
   });
   KBO_HIP(hipGetLastError());
   return 0;
@@ -2786,7 +2889,7 @@ int kb_rows_scatter_add(int32_t dtype, int32_t S, int64_t n, const void* src, co
   if (n <= 0 || S <= 0) return 0;
   if (!src || !order || !keys_sorted || !dst) return kb::set_error(KB_ERR_ARG, "null argument");
   if (int rc = dtype_ok(dtype)) return rc;
-  dim3 g((unsigned)n, (S + 255) / 256);
+  dim3 g((unsigned)((n + kbo::SCAT_K - 1) / kbo::SCAT_K), (S + 255) / 256);
   if (dtype == KB_F64)
     hipLaunchKernelGGL(kbo::scatter_add_kernel<double>, g, dim3(256), 0, st_of(stream), S, (long long)n,
                        (const double*)src, order, keys_sorted, (double*)dst, (long long)dst_stride);

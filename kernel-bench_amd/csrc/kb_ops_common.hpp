@@ -227,29 +227,6 @@ template <int CPT> __device__ __forceinline__ void own_load(const double* lds, d
   }
 }
 
-// float64 path sums / subtree sums over depth levels (in place).
-__device__ void level_path_sums(const OpsTree& t, double* x) {
-  for (int d = 1; d < t.n_levels; ++d) {
-    for (int i = t.lvl_ptr[d] + threadIdx.x; i < t.lvl_ptr[d + 1]; i += NT) {
-      const int n = t.lvl_node[i];
-      x[n] += x[t.par[n]];
-    }
-    __syncthreads();
-  }
-}
-__device__ void level_subtree_sums(const OpsTree& t, double* x) {
-  for (int d = t.n_levels - 2; d >= 0; --d) {
-    for (int i = t.lvl_ptr[d] + threadIdx.x; i < t.lvl_ptr[d + 1]; i += NT) {
-      const int n = t.lvl_node[i];
-      double a = 0.0;
-      if (t.c1[n] >= 0) a += x[t.c1[n]];
-      if (t.c2[n] >= 0) a += x[t.c2[n]];
-      x[n] += a;
-    }
-    __syncthreads();
-  }
-}
-
 // Ancestors-or-self path sums of per-state register values x[k] (state
 // threadIdx.x + k * NT): written as +x at the entry event and -x at the exit
 // event of each column, scanned, read back at the entry event.  Enters with
