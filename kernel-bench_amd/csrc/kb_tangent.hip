@@ -443,9 +443,10 @@ __global__ __launch_bounds__(NT) void wave_tan_kernel(OpsTree t, WtArgs<T> a) {
 //   dAS(i) = Pre(i) - PostEx(tin(i) - i),
 // so one tangent update takes two barriers (the float64 kernel above takes an
 // Euler-tour scan and two more barriers per update).
-template <int CPT>
-__global__ __launch_bounds__(NT) void wave_tan_pre_kernel(OpsTree t, WtArgs<float> a) {
-  constexpr int MAXS = NT * CPT;
+template <int BT, int CPT>
+__global__ __launch_bounds__(BT) void wave_tan_pre_kernel(OpsTree t, WtArgs<float> a) {
+  constexpr int BW = BT / 64;
+  constexpr int MAXS = BT * CPT;
   constexpr int LD = MAXS + 64;
   constexpr int ZERO = MAXS;     // padding slot: 0 in X
   constexpr int SEG = 64 * CPT;  // postorder slots per wavefront
@@ -453,7 +454,7 @@ __global__ __launch_bounds__(NT) void wave_tan_pre_kernel(OpsTree t, WtArgs<floa
   float* R = reinterpret_cast<float*>(smraw);  // the row at preorder positions: Pi, then the tangent
   float* X = R + LD;                           // the scanned values at preorder positions
   float* Q = X + LD;                           // exclusive postorder scan
-  __shared__ float wM[NW], wA[NW], wB[NW];
+  __shared__ float wM[BW], wA[BW], wB[BW];
   const int S = t.S;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const float NI = -__builtin_inff();
@@ -465,7 +466,7 @@ __global__ __launch_bounds__(NT) void wave_tan_pre_kernel(OpsTree t, WtArgs<floa
   const size_t ib = (size_t)(a.pi_ws + w) * S;
 #pragma unroll
   for (int j = 0; j < CPT; ++j) {
-    const int sc = tid + j * NT;
+    const int sc = tid + j * BT;
     if (sc < S) R[t.ppos[sc]] = a.Pi[ib + sc];
   }
   if (tid < 64) X[MAXS + tid] = 0.0f;
@@ -473,7 +474,7 @@ __global__ __launch_bounds__(NT) void wave_tan_pre_kernel(OpsTree t, WtArgs<floa
   bool okp[CPT];
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    const int i = kb::own_pos_c<NT, CPT>(k);
+    const int i = kb::own_pos_c<BT, CPT>(k);
     okp[k] = i < S;
     c1p[k] = okp[k] ? t.pc1[i] : -1;
     c2p[k] = okp[k] ? t.pc2[i] : -1;
@@ -491,7 +492,7 @@ __global__ __launch_bounds__(NT) void wave_tan_pre_kernel(OpsTree t, WtArgs<floa
     if (!okp[k]) pv[k] = NI;
     lm = fmaxf(lm, (a.use_col && okp[k] ? a.col[colk[k]] : 0.0f) + pv[k]);
   }
-  const float M = kb::block_max1<NT>(lm, wM);
+  const float M = kb::block_max1<BT>(lm, wM);
   const float Ms = M == NI ? 0.0f : M;
   // one path-sum pass over x (own positions): tot = sum x, ps = Pre - PostEx;
   // x is published in X for the postorder reads.  Two barriers.
@@ -507,12 +508,12 @@ __global__ __launch_bounds__(NT) void wave_tan_pre_kernel(OpsTree t, WtArgs<floa
     kb::lds_store_own<CPT>(X, x);
     if (lane == 63) wA[wv] = wa;
     __syncthreads();
-    const float tp = kb::lds_wave_values<NW>(wA, lane, 0.0f);
+    const float tp = kb::lds_wave_values<BW>(wA, lane, 0.0f);
     float yq[CPT];
 #pragma unroll
     for (int k = 0; k < CPT; ++k) yq[k] = X[qp[k]];
-    const float ip = kb::wave_scan_first<NW>(tp);
-    tot = kb::lane_value(ip, NW - 1);
+    const float ip = kb::wave_scan_first<BW>(tp);
+    tot = kb::lane_value(ip, BW - 1);
     const float offp = kb::lane_value(ip - tp, wv) + (wa - ta);
     float sq[CPT], tb = 0.0f;
 #pragma unroll
@@ -526,8 +527,8 @@ __global__ __launch_bounds__(NT) void wave_tan_pre_kernel(OpsTree t, WtArgs<floa
     kb::lds_store_own<CPT>(Q, sq);
     if (lane == 63) wB[wv] = wb;
     __syncthreads();
-    const float tq = kb::lds_wave_values<NW>(wB, lane, 0.0f);
-    const float eq = kb::wave_scan_first<NW>(tq) - tq;
+    const float tq = kb::lds_wave_values<BW>(wB, lane, 0.0f);
+    const float eq = kb::wave_scan_first<BW>(tq) - tq;
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       const int n = nex[k];
@@ -591,7 +592,7 @@ __global__ __launch_bounds__(NT) void wave_tan_pre_kernel(OpsTree t, WtArgs<floa
   __syncthreads();  // every read of the Pi row in R is done
 #pragma unroll
   for (int j = 0; j < CPT; ++j) {
-    const int sc = tid + j * NT;
+    const int sc = tid + j * BT;
     if (sc < S) R[t.ppos[sc]] = a.dPi_in[ib + sc];
   }
   __syncthreads();
@@ -624,7 +625,7 @@ __global__ __launch_bounds__(NT) void wave_tan_pre_kernel(OpsTree t, WtArgs<floa
       kb::lds_store_own<CPT>(X, x);
       if (lane == 63) wA[wv] = wa;
       __syncthreads();
-      const float tp = kb::lds_wave_values<NW>(wA, lane, 0.0f);
+      const float tp = kb::lds_wave_values<BW>(wA, lane, 0.0f);
       float yq[CPT];
 #pragma unroll
       for (int k = 0; k < CPT; ++k) {
@@ -632,8 +633,8 @@ __global__ __launch_bounds__(NT) void wave_tan_pre_kernel(OpsTree t, WtArgs<floa
         ch1[k] = c1p[k] >= 0 ? R[c1p[k]] : 0.0f;
         ch2[k] = c2p[k] >= 0 ? R[c2p[k]] : 0.0f;
       }
-      const float ip = kb::wave_scan_first<NW>(tp);
-      tot = kb::lane_value(ip, NW - 1);
+      const float ip = kb::wave_scan_first<BW>(tp);
+      tot = kb::lane_value(ip, BW - 1);
       const float offp = kb::lane_value(ip - tp, wv) + (wa - ta);
       float sq[CPT], tb = 0.0f;
 #pragma unroll
@@ -647,8 +648,8 @@ __global__ __launch_bounds__(NT) void wave_tan_pre_kernel(OpsTree t, WtArgs<floa
       kb::lds_store_own<CPT>(Q, sq);
       if (lane == 63) wB[wv] = wb;
       __syncthreads();
-      const float tq = kb::lds_wave_values<NW>(wB, lane, 0.0f);
-      const float eq = kb::wave_scan_first<NW>(tq) - tq;
+      const float tq = kb::lds_wave_values<BW>(wB, lane, 0.0f);
+      const float eq = kb::wave_scan_first<BW>(tq) - tq;
 #pragma unroll
       for (int k = 0; k < CPT; ++k) {
         const int n = nex[k];
@@ -677,7 +678,7 @@ __global__ __launch_bounds__(NT) void wave_tan_pre_kernel(OpsTree t, WtArgs<floa
   float* pb = a.dPibar ? a.dPibar + (size_t)grow * S : nullptr;
 #pragma unroll
   for (int j = 0; j < CPT; ++j) {
-    const int sc = tid + j * NT;
+    const int sc = tid + j * BT;
     if (sc < S) {
       const int i = t.ppos[sc];
       out[sc] = R[i];
@@ -709,22 +710,36 @@ int launch_etan(const kbo::OpsTree& t, const kbo::EtArgs<T>& a, bool f32, size_t
   return 0;
 }
 
-// float32 rows run the preorder-ownership kernel, float64 rows the float64 one
+template <int BT, int CPT>
+int launch_tan_pre(const kbo::OpsTree& t, const kbo::WtArgs<float>& a, int W, hipStream_t st) {
+  const size_t lds = (size_t)3 * (BT * CPT + 64) * sizeof(float);
+  auto k = kbo::wave_tan_pre_kernel<BT, CPT>;
+  if (int rc = set_lds(k, lds)) return rc;
+  hipLaunchKernelGGL(k, dim3(W), dim3(BT), lds, st, t, a);
+  return 0;
+}
+
+// float32 rows run the preorder-ownership kernel on the smallest workgroup that
+// holds them, float64 rows the float64 one.
 template <typename T, int CPT>
 int launch_wave_tan(const kbo::OpsTree& t, const kbo::WtArgs<T>& a, int W, size_t lds, hipStream_t st) {
   if constexpr (std::is_same_v<T, float>) {
-    const size_t lds_pre = (size_t)3 * (kbo::NT * CPT + 64) * sizeof(float);
-    auto k = kbo::wave_tan_pre_kernel<CPT>;
-    if (int rc = set_lds(k, lds_pre)) return rc;
-    hipLaunchKernelGGL(k, dim3(W), dim3(kbo::NT), lds_pre, st, t, a);
+    const int S = a.S;
+    if (S <= 128) return launch_tan_pre<64, 2>(t, a, W, st);
+    if (S <= 256) return launch_tan_pre<128, 2>(t, a, W, st);
+    if (S <= 512) return launch_tan_pre<256, 2>(t, a, W, st);
+    if (S <= 1024) return launch_tan_pre<512, 2>(t, a, W, st);
+    if (S <= 2048) return launch_tan_pre<1024, 2>(t, a, W, st);
+    if (S <= 4096) return launch_tan_pre<1024, 4>(t, a, W, st);
+    return launch_tan_pre<1024, 8>(t, a, W, st);
+  } else {
+    // the float64 kernel keeps three float64 rows of S in LDS
+    if (int rc = check_lds(lds, a.S, KB_F64)) return rc;
+    auto k = kbo::wave_tan_kernel<T, CPT>;
+    if (int rc = set_lds(k, lds)) return rc;
+    hipLaunchKernelGGL(k, dim3(W), dim3(kbo::NT), lds, st, t, a);
     return 0;
   }
-  // the float64 kernel keeps three float64 rows of S in LDS
-  if (int rc = check_lds(lds, a.S, KB_F64)) return rc;
-  auto k = kbo::wave_tan_kernel<T, CPT>;
-  if (int rc = set_lds(k, lds)) return rc;
-  hipLaunchKernelGGL(k, dim3(W), dim3(kbo::NT), lds, st, t, a);
-  return 0;
 }
 
 }  // namespace
