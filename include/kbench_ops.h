@@ -320,10 +320,10 @@ int kb_rows_scatter_add(int32_t dtype, int32_t S, int64_t n, const void* src, co
 int kb_rows_sum_into(int32_t dtype, int32_t S, int64_t n, const void* src, void* dst, double* work, void* stream);
 
 /*
- * Column sums of m <= 8 row blocks in one launch (two above 64 rows):
+ * Column sums of m <= 8 row blocks in one launch (two above 1024 rows):
  * out[j * S + s] = sum over r < n of (a[j][r * S + s] + b[j][r * S + s]),
- * b (or b[j]) null for a single addend, in row order with float64 partial
- * sums (work: m * ceil(n / 64) * S doubles, unused for n <= 64).  a and b
+ * b (or b[j]) null for a single addend, in a fixed order with float64 partial
+ * sums (work: m * ceil(n / 64) * S doubles, required for n > 64).  a and b
  * are host arrays of device pointers.  No reference kernel: it replaces the
  * glue's per-wave torch reductions of the aw tensors
  * (kbench/api/_implicit_grad.py:288-296, one .sum(0) per tensor).
@@ -335,8 +335,8 @@ int kb_rows_sum_multi(int32_t dtype, int32_t S, int64_t n, int32_t m, const void
  * Column sums of m <= 8 row blocks, each added into its own accumulator:
  * dst[j][s] += sum over r < n[j] of (a[4j][r*S+s] + ... + a[4j+k[j]-1][r*S+s])
  * with k[j] in 1..4 addends per block (each row's addends summed first, in
- * order), rows summed in order in float64 (work: m * max_j ceil(n[j] / 64) * S
- * doubles, unused when every block has at most 64 rows).  The accumulators
+ * order), rows summed in a fixed order in float64 (work: m * max_j ceil(n[j] / 64)
+ * * S doubles, required when a block has more than 64 rows).  The accumulators
  * must be distinct.  n, k, a and dst are host arrays (a: 4 entries per block,
  * device pointers).  A block of one addend gives dst exactly what
  * kb_rows_sum_into gives.  No reference kernel: it replaces the per-wave

@@ -119,3 +119,27 @@ def test_wave_adjoint_at_shape_edges_matches_oracle(leaves, kind):
     np.add.at(want, SR, ref["tree_r"])
     close(acc, want, "Pibar VJP rows")
     close(gcol, ref["col_grad"], "grad_col")
+
+
+@pytest.mark.parametrize("n", [15, 17, 1023, 1024, 1025, 2600])
+@pytest.mark.parametrize("tdt", [torch.float32, torch.float64])
+def test_column_sums_at_chunk_edges(n, tdt):
+    """Row ranges of the wavefronts and chunks of the row sums: one launch up to 1024 rows, two above."""
+    from kbench.core.kernels import _hip as H
+
+    g = torch.Generator().manual_seed(n)
+    S = 129
+    xs = [torch.randn((n, S), generator=g, dtype=torch.float64).to(device="cuda", dtype=tdt) for _ in range(3)]
+    base = torch.randn((S,), generator=g, dtype=torch.float64).to(device="cuda", dtype=tdt)
+    want = [sum(x.double() for x in grp).sum(0) for grp in ((xs[0],), (xs[1], xs[2]), xs)]
+    into, acc = base.clone(), [base.clone() for _ in want]
+    H.sum_rows_into(into, xs[0])
+    H.rows_sum_accum(list(zip(acc, ((xs[0],), (xs[1], xs[2]), tuple(xs)))))
+    multi = H.rows_sum_multi([xs[0], (xs[1], xs[2])])
+    torch.cuda.synchronize()
+    print(f"[column sums] n={n} {tdt}", flush=True)
+    # float64 sums of n values of size about 1 (n roundings of sqrt(n) 2^-53 each at the most), rounded once
+    tol = 64 * n**1.5 * 2.0**-53 + (2.0**-24 * 6 * n**0.5 if tdt == torch.float32 else 0.0)
+    assert torch.equal(into, acc[0])
+    for got, ref in ((into, base.double() + want[0]), *zip(acc, (base.double() + w for w in want)), *zip(multi, want)):
+        assert float((got.double() - ref).abs().max()) <= tol
