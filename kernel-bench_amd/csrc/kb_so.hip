@@ -305,9 +305,10 @@ __global__ __launch_bounds__(NT) void wso_kernel(OpsTree t, WsoArgs<T> a) {
 // pair of preorder / postorder scans, the two subtree sums from one pair of
 // published wavefront-local scans, the outputs written back in column order
 // through LDS.  Same mathematics as wso_kernel.
-template <int CPT>
-__global__ __launch_bounds__(NT) void wso_pre_kernel(OpsTree t, WsoArgs<float> a) {
-  constexpr int MAXS = NT * CPT;
+template <int BT, int CPT>
+__global__ __launch_bounds__(BT) void wso_pre_kernel(OpsTree t, WsoArgs<float> a) {
+  constexpr int BW = BT / 64;
+  constexpr int MAXS = BT * CPT;
   constexpr int LD = MAXS + 64;  // [MAXS] is the padding slot, kept at 0
   constexpr int ZERO = MAXS;
   constexpr int SEG = 64 * CPT;  // postorder slots per wavefront
@@ -315,7 +316,7 @@ __global__ __launch_bounds__(NT) void wso_pre_kernel(OpsTree t, WsoArgs<float> a
   extern __shared__ __align__(16) unsigned char smraw[];
   float* Lr = reinterpret_cast<float*>(smraw);  // 8 rows of LD
   auto row = [&](int j) { return Lr + (size_t)j * LD; };
-  __shared__ float wA[2 * NW], wB[2 * NW];
+  __shared__ float wA[2 * BW], wB[2 * BW];
   const int S = t.S;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const float NI = -__builtin_inff();
@@ -332,7 +333,7 @@ __global__ __launch_bounds__(NT) void wso_pre_kernel(OpsTree t, WsoArgs<float> a
   // Pi, dPi, Pibar, dPibar and v to their preorder positions (rows 0..4)
 #pragma unroll
   for (int j = 0; j < CPT; ++j) {
-    const int sc = tid + j * NT;
+    const int sc = tid + j * BT;
     if (sc < S) {
       const int p = t.ppos[sc];
       row(0)[p] = a.Pi[rb + sc];
@@ -348,7 +349,7 @@ __global__ __launch_bounds__(NT) void wso_pre_kernel(OpsTree t, WsoArgs<float> a
   bool okp[CPT];
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    const int i = kb::own_pos_c<NT, CPT>(k);
+    const int i = kb::own_pos_c<BT, CPT>(k);
     okp[k] = i < S;
     colk[k] = okp[k] ? t.pcol[i] : 0;
     c1p[k] = okp[k] ? t.pc1[i] : -1;
@@ -392,13 +393,13 @@ __global__ __launch_bounds__(NT) void wso_pre_kernel(OpsTree t, WsoArgs<float> a
   kb::lds_store_own<CPT>(row(6), dpp);
   if (lane == 63) {
     wA[wv] = wa;
-    wA[NW + wv] = wb2;
+    wA[BW + wv] = wb2;
   }
   __syncthreads();
   float anc[CPT], danc[CPT], p1[CPT], p2[CPT], dp1[CPT], dp2[CPT], rowsum, drowsum;
   {
-    const float tpa = kb::lds_wave_values<NW>(wA, lane, 0.0f);
-    const float tpb = kb::lds_wave_values<NW>(wA + NW, lane, 0.0f);
+    const float tpa = kb::lds_wave_values<BW>(wA, lane, 0.0f);
+    const float tpb = kb::lds_wave_values<BW>(wA + BW, lane, 0.0f);
     float ya[CPT], yb[CPT];
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
@@ -409,9 +410,9 @@ __global__ __launch_bounds__(NT) void wso_pre_kernel(OpsTree t, WsoArgs<float> a
       dp1[k] = c1p[k] >= 0 ? row(1)[c1p[k]] : 0.0f;
       dp2[k] = c2p[k] >= 0 ? row(1)[c2p[k]] : 0.0f;
     }
-    const float ipa = kb::wave_scan_first<NW>(tpa), ipb = kb::wave_scan_first<NW>(tpb);
-    rowsum = kb::lane_value(ipa, NW - 1);
-    drowsum = kb::lane_value(ipb, NW - 1);
+    const float ipa = kb::wave_scan_first<BW>(tpa), ipb = kb::wave_scan_first<BW>(tpb);
+    rowsum = kb::lane_value(ipa, BW - 1);
+    drowsum = kb::lane_value(ipb, BW - 1);
     const float offa = kb::lane_value(ipa - tpa, wv) + (wa - ta);
     const float offb = kb::lane_value(ipb - tpb, wv) + (wb2 - tb);
     float qa[CPT], qb[CPT], ua = 0.0f, ub = 0.0f;
@@ -432,11 +433,11 @@ __global__ __launch_bounds__(NT) void wso_pre_kernel(OpsTree t, WsoArgs<float> a
     kb::lds_store_own<CPT>(row(3), qb);
     if (lane == 63) {
       wB[wv] = xa;
-      wB[NW + wv] = xb;
+      wB[BW + wv] = xb;
     }
     __syncthreads();
-    const float tqa = kb::lds_wave_values<NW>(wB, lane, 0.0f), tqb = kb::lds_wave_values<NW>(wB + NW, lane, 0.0f);
-    const float eqa = kb::wave_scan_first<NW>(tqa) - tqa, eqb = kb::wave_scan_first<NW>(tqb) - tqb;
+    const float tqa = kb::lds_wave_values<BW>(wB, lane, 0.0f), tqb = kb::lds_wave_values<BW>(wB + BW, lane, 0.0f);
+    const float eqa = kb::wave_scan_first<BW>(tqa) - tqa, eqb = kb::wave_scan_first<BW>(tqb) - tqb;
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       const int n = nex[k];
@@ -517,12 +518,12 @@ __global__ __launch_bounds__(NT) void wso_pre_kernel(OpsTree t, WsoArgs<float> a
   // subtree sums of u and du: wavefront-local scans published in rows 5 / 6
   // (their postorder reads finished before the second barrier above)
   float scu[CPT], scd[CPT];
-  kb::local_scan_publish<NT, CPT>(scu, u, row(5), wA);
-  kb::local_scan_publish<NT, CPT>(scd, du, row(6), wA + NW);
+  kb::local_scan_publish<BT, CPT>(scu, u, row(5), wA);
+  kb::local_scan_publish<BT, CPT>(scd, du, row(6), wA + BW);
   __syncthreads();  // also publishes the child-edge terms in row 7
   float pmu[CPT], rsu[CPT], pmd[CPT], rsd[CPT], z[CPT];
-  kb::subtree_terms<NT, CPT>(scu, row(5), wA, endm1, wend, pmu, rsu);
-  kb::subtree_terms<NT, CPT>(scd, row(6), wA + NW, endm1, wend, pmd, rsd);
+  kb::subtree_terms<BT, CPT>(scu, row(5), wA, endm1, wend, pmu, rsu);
+  kb::subtree_terms<BT, CPT>(scd, row(6), wA + BW, endm1, wend, pmd, rsd);
   kb::lds_load_own<CPT>(row(7), z);
   // the output row: dself + dp' (A - sub u) + p' (dA - sub du) + the child-edge
   // term from the parent (+ rhs)
@@ -544,7 +545,7 @@ __global__ __launch_bounds__(NT) void wso_pre_kernel(OpsTree t, WsoArgs<float> a
   float* const outs[7] = {a.out, a.aw0, a.aw1, a.aw2, a.aw3, a.aw4, a.aw345};
 #pragma unroll
   for (int j = 0; j < CPT; ++j) {
-    const int sc = tid + j * NT;
+    const int sc = tid + j * BT;
     if (sc < S) {
       const int p = t.ppos[sc];
       float ov = row(0)[p];
@@ -720,9 +721,10 @@ __global__ __launch_bounds__(NT) void dso_tree_kernel(OpsTree t, DsoArgs<T> a) {
 // from wavefront-local scans published behind one barrier, and the outputs go
 // back to column order through LDS.  Same terms as dso_tree_kernel, in
 // float32 with the hardware exp2.
-template <int CPT>
-__global__ __launch_bounds__(NT) void dso_tree_pre_kernel(OpsTree t, DsoArgs<float> a) {
-  constexpr int MAXS = NT * CPT;
+template <int BT, int CPT>
+__global__ __launch_bounds__(BT) void dso_tree_pre_kernel(OpsTree t, DsoArgs<float> a) {
+  constexpr int BW = BT / 64;
+  constexpr int MAXS = BT * CPT;
   constexpr int LD = MAXS + 64;  // [MAXS] is the padding slot, kept at 0
   constexpr int ZERO = MAXS;
   constexpr int SEG = 64 * CPT;  // positions per wavefront
@@ -730,7 +732,7 @@ __global__ __launch_bounds__(NT) void dso_tree_pre_kernel(OpsTree t, DsoArgs<flo
   extern __shared__ __align__(16) unsigned char smraw[];
   float* Lr = reinterpret_cast<float*>(smraw);  // rows: ud, dud (then their scans), Pi (then the output), dPi
   auto row = [&](int j) { return Lr + (size_t)j * LD; };
-  __shared__ float wA[NW], wB[NW];
+  __shared__ float wA[BW], wB[BW];
   const int S = t.S;
   const int tid = threadIdx.x;
   const float NI = -__builtin_inff();
@@ -741,7 +743,7 @@ __global__ __launch_bounds__(NT) void dso_tree_pre_kernel(OpsTree t, DsoArgs<flo
   const float rms = rm == NI ? 0.0f : rm;
 #pragma unroll
   for (int j = 0; j < CPT; ++j) {
-    const int sc = tid + j * NT;
+    const int sc = tid + j * BT;
     if (sc < S) {
       const int p = t.ppos[sc];
       row(0)[p] = a.ud[rb + sc];
@@ -756,7 +758,7 @@ __global__ __launch_bounds__(NT) void dso_tree_pre_kernel(OpsTree t, DsoArgs<flo
   bool okp[CPT];
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
-    const int q = kb::own_pos_c<NT, CPT>(k);
+    const int q = kb::own_pos_c<BT, CPT>(k);
     okp[k] = q < S;
     colk[k] = okp[k] ? t.pcol[q] : 0;
     endm1[k] = okp[k] ? t.pend[colk[k]] - 1 : ZERO;
@@ -772,12 +774,12 @@ __global__ __launch_bounds__(NT) void dso_tree_pre_kernel(OpsTree t, DsoArgs<flo
   for (int k = 0; k < CPT; ++k)
     if (!okp[k]) x[k] = dx[k] = 0.0f;  // positions past S were not written: out of the scans
   float sx[CPT], sdx[CPT];
-  kb::local_scan_publish<NT, CPT>(sx, x, row(0), wA);
-  kb::local_scan_publish<NT, CPT>(sdx, dx, row(1), wB);
+  kb::local_scan_publish<BT, CPT>(sx, x, row(0), wA);
+  kb::local_scan_publish<BT, CPT>(sdx, dx, row(1), wB);
   __syncthreads();
   float pm1[CPT], rest[CPT], dpm1[CPT], drest[CPT];
-  kb::subtree_terms<NT, CPT>(sx, row(0), wA, endm1, wend, pm1, rest);
-  kb::subtree_terms<NT, CPT>(sdx, row(1), wB, endm1, wend, dpm1, drest);
+  kb::subtree_terms<BT, CPT>(sx, row(0), wA, endm1, wend, pm1, rest);
+  kb::subtree_terms<BT, CPT>(sdx, row(1), wB, endm1, wend, dpm1, drest);
   float c[CPT];
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
@@ -791,7 +793,7 @@ __global__ __launch_bounds__(NT) void dso_tree_pre_kernel(OpsTree t, DsoArgs<flo
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < CPT; ++j) {
-    const int sc = tid + j * NT;
+    const int sc = tid + j * BT;
     if (sc < S) {
       const float v = row(2)[t.ppos[sc]];
       a.side[rb + sc] += v;
@@ -806,17 +808,27 @@ using namespace kbo_host;
 
 namespace {
 
-// float32 rows of up to 4096 states run the preorder-ownership kernel, the
-// others the generic one (float64 arithmetic, float32 for float32 rows too
+template <int BT, int CPT>
+int launch_wso_pre(const kbo::OpsTree& t, const kbo::WsoArgs<float>& a, int W, hipStream_t st) {
+  const size_t lds = (size_t)8 * (BT * CPT + 64) * sizeof(float);
+  auto k = kbo::wso_pre_kernel<BT, CPT>;
+  if (int rc = set_lds(k, lds)) return rc;
+  hipLaunchKernelGGL(k, dim3(W), dim3(BT), lds, st, t, a);
+  return 0;
+}
+
+// float32 rows of up to 4096 states run the preorder-ownership kernel on the
+// smallest workgroup that holds them, the others the generic one (float64 arithmetic, float32 for float32 rows too
 // long for three float64 LDS rows)
 template <typename T, int CPT>
 int launch_wso(const kbo::OpsTree& t, const kbo::WsoArgs<T>& a, int W, bool f32, size_t lds, hipStream_t st) {
   if constexpr (std::is_same_v<T, float> && CPT <= 4) {  // (eight LDS rows: up to 4096 positions)
-    const size_t lds_pre = (size_t)8 * (kbo::NT * CPT + 64) * sizeof(float);
-    auto k = kbo::wso_pre_kernel<CPT>;
-    if (int rc = set_lds(k, lds_pre)) return rc;
-    hipLaunchKernelGGL(k, dim3(W), dim3(kbo::NT), lds_pre, st, t, a);
-    return 0;
+    if (a.S <= 128) return launch_wso_pre<64, 2>(t, a, W, st);
+    if (a.S <= 256) return launch_wso_pre<128, 2>(t, a, W, st);
+    if (a.S <= 512) return launch_wso_pre<256, 2>(t, a, W, st);
+    if (a.S <= 1024) return launch_wso_pre<512, 2>(t, a, W, st);
+    if (a.S <= 2048) return launch_wso_pre<1024, 2>(t, a, W, st);
+    return launch_wso_pre<1024, 4>(t, a, W, st);
   }
   if constexpr (std::is_same_v<T, float> && CPT == 8) {
     if (f32) {  // rows too long for three float64 LDS rows
@@ -850,21 +862,34 @@ int launch_eso(const kbo::OpsTree& t, const kbo::EsoArgs<T>& a, bool f32, size_t
   return 0;
 }
 
-// float32 rows: the preorder-ownership tree kernel; the others the float64 one
+template <int BT, int CPT>
+int launch_dso_tree_pre(const kbo::OpsTree& t, const kbo::DsoArgs<float>& a, hipStream_t st) {
+  const size_t lds = (size_t)4 * (BT * CPT + 64) * sizeof(float);
+  auto k = kbo::dso_tree_pre_kernel<BT, CPT>;
+  if (int rc = set_lds(k, lds)) return rc;
+  hipLaunchKernelGGL(k, dim3((unsigned)(2 * a.N)), dim3(BT), lds, st, t, a);
+  return 0;
+}
+
+// float32 rows: the preorder-ownership tree kernel on the smallest workgroup
+// that holds them; the others the float64 one
 template <typename T, int CPT>
 int launch_dso_tree(const kbo::OpsTree& t, const kbo::DsoArgs<T>& a, size_t lds, hipStream_t st) {
-  const dim3 grid((unsigned)(2 * a.N));
   if constexpr (std::is_same_v<T, float>) {
-    const size_t lds_pre = (size_t)4 * (kbo::NT * CPT + 64) * sizeof(float);
-    auto k = kbo::dso_tree_pre_kernel<CPT>;
-    if (int rc = set_lds(k, lds_pre)) return rc;
-    hipLaunchKernelGGL(k, grid, dim3(kbo::NT), lds_pre, st, t, a);
+    if (a.S <= 128) return launch_dso_tree_pre<64, 2>(t, a, st);
+    if (a.S <= 256) return launch_dso_tree_pre<128, 2>(t, a, st);
+    if (a.S <= 512) return launch_dso_tree_pre<256, 2>(t, a, st);
+    if (a.S <= 1024) return launch_dso_tree_pre<512, 2>(t, a, st);
+    if (a.S <= 2048) return launch_dso_tree_pre<1024, 2>(t, a, st);
+    if (a.S <= 4096) return launch_dso_tree_pre<1024, 4>(t, a, st);
+    return launch_dso_tree_pre<1024, 8>(t, a, st);
+  } else {
+    const dim3 grid((unsigned)(2 * a.N));
+    auto k = kbo::dso_tree_kernel<T, CPT>;
+    if (int rc = set_lds(k, lds)) return rc;
+    hipLaunchKernelGGL(k, grid, dim3(kbo::NT), lds, st, t, a);
     return 0;
   }
-  auto k = kbo::dso_tree_kernel<T, CPT>;
-  if (int rc = set_lds(k, lds)) return rc;
-  hipLaunchKernelGGL(k, grid, dim3(kbo::NT), lds, st, t, a);
-  return 0;
 }
 
 }  // namespace
