@@ -859,8 +859,8 @@ static int forward_setup(kb_plan* p, const kb_forward_io* io, hipStream_t st, kb
     // states (config 3): the narrow shape wins on levels of less than one row
     // per CU and on the leaf level (no split term; the last round of 512 x 4
     // rows would run one row per CU), the 512 x 4 shape on the others (levels
-    // of 570..1428 rows: 4-6 us each).  Shorter rows keep the earlier rule,
-    // the narrow shape below six rows per CU.
+    // of 570..1428 rows: 4-6 us each).  Rows of 513..1024 states take the
+    // narrow shape (512 x 2 against 256 x 4) below six rows per CU.
     int dev = 0, n_cu = 0;
     KB_HIP(hipGetDevice(&dev));
     KB_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
@@ -941,12 +941,11 @@ static int ensure_backward_work(kb_plan* p, int use_col) {
   int dev = 0, n_cu = 0;
   KB_HIP(hipGetDevice(&dev));
   KB_HIP(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
-  // launch shape: 1024 x 2 (more, narrower threads: four wavefronts per SIMD
-  // instead of two) on every level of rows of 1025..2048 states, where it
-  // measured faster on every level (config 3: 1.77 vs 1.96 ms); on shorter
-  // rows 512 x 4 on levels with at least two rows per workgroup slot and
-  // 1024 x 2 on the smaller ones; KB_BWD_VARIANT=0 / 2 forces one shape
-  // everywhere
+  // launch shape: two positions per thread on the smallest workgroup that holds
+  // the row (more, narrower threads: for 1025..2048 states 1024 x 2 measured
+  // faster than 512 x 4 on every level, config 3: 1.77 vs 1.96 ms);
+  // KB_BWD_VARIANT=0 takes four positions per thread past 512 states, =2
+  // 1024 x 2 everywhere (768 x 2 for 1025..1536 states)
   const char* vv = getenv("KB_BWD_VARIANT");
   const int variant = (vv && vv[0] == '2') ? 2 : (vv && vv[0] == '0') ? 0 : 1;
   // rows of 2049..8192 states: the low-register kernel (KB_BWD_LARGE=0: the

@@ -60,8 +60,7 @@ __global__ __launch_bounds__(NT) void bwd_row_kernel(BwdParams P, int first, int
   const int tid = threadIdx.x;
   constexpr int ZERO = MAXS;
 
-  // The 1024 x 2 shape (rows of 1025..2048 states on every level, shorter
-  // rows on levels with about one row per workgroup) fetches rows when needed
+  // The 1024 x 2 shape (rows of 1537..2048 states) fetches rows when needed
   // instead of one row ahead (128 VGPRs at 16 waves).
   constexpr bool AHEAD = NT < 1024;
   // the first split's child rows are prefetched into registers during the
@@ -1157,6 +1156,12 @@ void launch_bwd_wave(const BwdParams& P, int first, int W, int nb, int poff, hip
   if (launch_bwd_large(P, first, W, nb, poff, st)) return;
   const int S = P.S;
   if (P.variant == 2) {
+    // up to 1536 states: 768 threads leave registers for fetching a row ahead,
+    // and no quarter of the wavefronts idle (1399 states, 22 levels: 833 -> 818
+    // us; its levels of a few hundred rows 109 -> 101 us)
+    if (S > 1024) {
+      KB_BWD_CASE(768, 2)
+    }
     KB_BWD_CASE(1024, 2)
   }
   KB_BWD_CASE(64, 2)
@@ -1184,6 +1189,9 @@ void launch_bwd_wave(const BwdParams& P, int first, int W, int nb, int poff, hip
 int bwd_blocks_per_cu(int S, int use_col, int variant, int large) {
   if (kb_use_large(S, large)) return bwd_large_blocks_per_cu(S, use_col);
   if (variant == 2) {
+    if (S > 1024) {
+      KB_BWD_OCC(768, 2)
+    }
     KB_BWD_OCC(1024, 2)
   }
   KB_BWD_OCC(64, 2)

@@ -254,7 +254,7 @@ __global__ __launch_bounds__(NT, (NT == 1024 && CPT == 2) ? 8 : 1) void fwd_row_
 // Minimum waves per SIMD (the second launch-bounds argument): 6 keeps three
 // 512 x 4 workgroups resident per CU (at most 80 VGPRs; the weighted variant
 // would spill).
-#define FWD_MIN_WAVES(NT, CPT, W) (((NT) == 512 && (CPT) == 4 && !(W)) ? 6 : 1)
+#define FWD_MIN_WAVES(NT, CPT, W) ((((NT) == 512 || (NT) == 384) && (CPT) == 4 && !(W)) ? 6 : 1)
 
 // the LDS word at a byte offset, and the value of lane (byte / 4)
 __device__ __forceinline__ float lds_at(const float* p, unsigned byte) {
@@ -693,7 +693,14 @@ void launch_fwd_wave(const FwdParams& P, int first, int W, hipStream_t st) {
   // 1024 x 2: on every level by the knob; by default on rows of 1025..2048
   // states where few rows share a CU (narrow_below, forward_setup).  Shorter
   // rows never take it: half or more of its wavefronts would carry padding.
+  // Rows of 1025..1536 states leave a quarter or more of a 2048-position
+  // workgroup idle: 768 x 2 and 384 x 4 in place of 1024 x 2 and 512 x 4
+  // (1399 states, 22 levels: 590 -> 545 us).
+  const bool three = P.wide == 0 && S > 1024;
   if (P.wide == 2 || (P.wide == 0 && S > 1024 && W < P.narrow_below)) {
+    if (three) {
+      KB_FWD_CASE(768, 2, fwd_row_kernel)
+    }
     KB_FWD_CASE(1024, 2, fwd_row_kernel)
   }
   KB_FWD_CASE(64, 2, fwd_row_kernel)
@@ -703,6 +710,9 @@ void launch_fwd_wave(const FwdParams& P, int first, int W, hipStream_t st) {
     KB_FWD_CASE(512, 2, fwd_row_kernel)
   }
   KB_FWD_CASE(256, 4, fwd_row_kernel)
+  if (three) {
+    KB_FWD_CASE(384, 4, fwd_row_kernel)
+  }
   KB_FWD_CASE(512, 4, fwd_row_kernel)
   KB_FWD_CASE(1024, 4, fwd_row_kernel)
   if (P.large) {

@@ -46,11 +46,10 @@ __device__ __forceinline__ float wave_prev_lane(float x) {
 
 // Per-wavefront values published in LDS (w[0..NW-1]), read by lanes 0..NW-1
 // (zero elsewhere) without a branch, so the scheduler can issue the read
-// together with the gathers around it.  NW is a power of two.
+// together with the gathers around it.
 template <int NW, typename T>
 __device__ __forceinline__ T lds_wave_values(const T* w, int lane, T zero) {
-  static_assert((NW & (NW - 1)) == 0, "power of two");
-  const T x = w[lane & (NW - 1)];
+  const T x = w[(NW & (NW - 1)) == 0 ? lane & (NW - 1) : min(lane, NW - 1)];
   return lane < NW ? x : zero;
 }
 

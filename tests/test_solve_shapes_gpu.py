@@ -1,8 +1,8 @@
 """The whole-pass driver at the edges of its launch shapes, against the float64 oracle.
 
 Row kernels, E step and backward epilogue take the smallest workgroup that holds the tree
-(128, 256, 512, 1024, 2048, 4096 or 8192 positions): S = 2 L - 1 just below and just above
-each of the first six, and the largest, with few families so that the oracle stays quick.
+(128, 256, 512, 1024, 1536, 2048, 4096 or 8192 positions): S = 2 L - 1 just below and just above
+each of them, with few families so that the oracle stays quick.
 """
 
 import numpy as np
@@ -14,7 +14,7 @@ import kbtest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("leaves", [2, 33, 64, 65, 128, 129, 256, 257, 512, 513, 2049, 4096])
+@pytest.mark.parametrize("leaves", [2, 33, 64, 65, 128, 129, 256, 257, 512, 513, 768, 769, 1024, 2049, 4096])
 def test_solve_at_shape_edges_matches_oracle(leaves):
     import kbench_oracle as O
     from kbench import synth
