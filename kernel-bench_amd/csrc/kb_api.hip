@@ -129,7 +129,7 @@ struct kb_plan {
   float* b_rhsc = nullptr;
   unsigned char* b_m_mask = nullptr;
   unsigned char* b_cls_active = nullptr;
-  float* b_contrib = nullptr; double* b_partial = nullptr; double* b_acc = nullptr;
+  float* b_contrib = nullptr; double* b_acc = nullptr;
   float* b_om_const = nullptr;  // owner-major constants of the large backward kernel
   int* b_status = nullptr;
   int* h_status = nullptr;  // pinned host copy of b_status (kb_backward_stats)
@@ -980,16 +980,12 @@ static int ensure_backward_work(kb_plan* p, int use_col) {
   p->b_n_partials = nb_max;
   if (p->b_contrib) {
     (void)hipFree(p->b_contrib);
-    (void)hipFree(p->b_partial);
     for (auto& ptr : p->owned)
-      if (ptr == (void*)p->b_contrib || ptr == (void*)p->b_partial) ptr = nullptr;
+      if (ptr == (void*)p->b_contrib) ptr = nullptr;
     p->b_contrib = nullptr;
-    p->b_partial = nullptr;
     int rc = 0;
     rc |= alloc(&p->b_contrib, (size_t)2 * std::max(1, p->b_n_partials) * p->b_slot);
-    rc |= alloc(&p->b_partial, (size_t)kb::reduce_chunks(2 * std::max(1, p->b_n_partials)) * 8 * S);
     p->owned.push_back(p->b_contrib);
-    p->owned.push_back(p->b_partial);
     return rc ? KB_ERR_HIP : 0;
   }
   const int64_t NS = p->n_splits;
@@ -1005,7 +1001,6 @@ static int ensure_backward_work(kb_plan* p, int use_col) {
   rc |= alloc(&p->b_cls_active, (size_t)std::max(1, p->n_cls0));
   rc |= alloc(&p->b_ck_any, (size_t)std::max(1, p->n_chunks0));
   rc |= alloc(&p->b_contrib, (size_t)2 * std::max(1, p->b_n_partials) * p->b_slot);
-  rc |= alloc(&p->b_partial, (size_t)kb::reduce_chunks(2 * std::max(1, p->b_n_partials)) * 8 * S);
   rc |= alloc(&p->b_acc, (size_t)8 * S);
   rc |= alloc(&p->b_status, 2);
   rc |= alloc(&p->b_DL, S);
@@ -1020,7 +1015,7 @@ static int ensure_backward_work(kb_plan* p, int use_col) {
   for (void* ptr : {(void*)p->b_Ebar, (void*)p->b_E, (void*)p->b_mt, (void*)p->b_col,
                     (void*)p->b_staging, (void*)p->b_split_on, (void*)p->b_mask, (void*)p->b_contrib,
                     (void*)p->b_rhs0, (void*)p->b_rhsc, (void*)p->b_cls_active, (void*)p->b_ck_any, (void*)p->b_m_mask,
-                    (void*)p->b_partial, (void*)p->b_acc, (void*)p->b_status, (void*)p->b_DL,
+                    (void*)p->b_acc, (void*)p->b_status, (void*)p->b_DL,
                     (void*)p->b_SL1, (void*)p->b_SL2, (void*)p->b_pS, (void*)p->b_pD})
     p->owned.push_back(ptr);
   return rc ? KB_ERR_HIP : 0;
@@ -1155,8 +1150,7 @@ static int backward_finish(kb_plan* p, const kb_backward_io* io, const kb::BwdPa
   if (p->n_levels > 0)
     kb::launch_bwd_buckets_large(B, p->level_ptr[1], p->C - p->level_ptr[1], p->n_cls0, p->b_nb_max, st);
   KB_HIP(hipGetLastError());
-  kb::launch_bwd_reduce(p->b_contrib, n_partials, S, p->b_slot, kb::kb_slot_ld(S, p->b_large), p->b_partial,
-                        p->d_pre, p->b_acc, st);
+  kb::launch_bwd_reduce(p->b_contrib, n_partials, S, p->b_slot, kb::kb_slot_ld(S, p->b_large), p->d_pcol, p->b_acc, st);
   KB_HIP(hipGetLastError());
   if (io->acc_out)
     KB_HIP(hipMemcpyAsync(io->acc_out, p->b_acc, (size_t)8 * S * sizeof(double), hipMemcpyDeviceToDevice, st));

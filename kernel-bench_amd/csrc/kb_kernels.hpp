@@ -51,7 +51,8 @@ struct FwdParams {
   PreDev pre;
   int S;
   int wide;                   // 1: 256 x 8, 2: 1024 x 2 on every level, 3: no narrow shape
-  int narrow_below;           // wide == 0: 1024 x 2 on levels with fewer rows than this (and the leaf level)
+  int narrow_below;           // wide == 0: two positions per thread on levels with fewer rows than this (past
+                              // 1024 states also on the leaf level)
   int n_sweeps;               // pi_iters - 1
   int use_col;
   // per-position constants: one [S] row in preorder, shared by every row
@@ -235,11 +236,10 @@ void launch_bwd_buckets_large(const BwdParams& P, int first, int n_rows, int n_c
 // Level-0 adjoint rows, masks and class sums.
 void launch_bwd_level0_prep(const BwdParams& P, int n_members, int n_cls, hipStream_t st);
 // Sums the bucket rows of C workgroup slots (slot_stride floats apart, bucket
-// rows ld floats apart, preorder positions) in slot order into out [8, S] in
-// column order (column s at preorder position pre[s]).
-void launch_bwd_reduce(const float* contrib, int C, int S, size_t slot_stride, int ld, double* partial, const int* pre,
-                       double* out, hipStream_t st);
-int reduce_chunks(int C);
+// rows ld floats apart, preorder positions) in a fixed order into out [8, S] in
+// column order (preorder position i is column pcol[i]).
+void launch_bwd_reduce(const float* contrib, int C, int S, size_t slot_stride, int ld, const int* pcol, double* out,
+                       hipStream_t st);
 void launch_epilogue(const EpiParams& P, hipStream_t st);
 
 }  // namespace kb

@@ -3,14 +3,16 @@
 // reference function each replaces: include/kbench_ops.h).
 //
 // Design (MI355X):
-//  * one 1024-thread workgroup per row (item row, clade row, split or split
-//    side); thread t owns states t + k*1024 (k < CPT), so global row accesses
-//    are coalesced;
-//  * the species tree is described once by preorder positions and an Euler
-//    tour (kb_tree); ancestors-or-self path sums are one prefix scan over the
-//    Euler tour (+x on entry, -x on exit) and subtree sums one prefix scan
-//    over preorder positions, both in LDS, independent of the tree depth;
-//  * the E-step kernels (O(S) work) run in float64 and sum over tree levels;
+//  * one workgroup per row (item row, clade row, split or split side), the
+//    smallest whose positions hold the row (64 to 1024 threads of 2 to 8);
+//    global row accesses are coalesced (column t + k * threads), and the kernels
+//    that sum over the tree move the row to preorder positions in LDS, thread t
+//    owning positions t*CPT + k;
+//  * the species tree is described once by preorder positions (kb_tree);
+//    ancestors-or-self path sums are a preorder scan less a postorder scan and
+//    subtree sums differences of one preorder scan, in registers with one
+//    exchange per scan, independent of the tree depth;
+//  * the E-step kernels (O(S) work) run in float64;
 //  * no atomics: cross-row accumulations are written as rows and summed in a
 //    fixed order by kb_rows_scatter_add / kb_rows_sum_into.
 #include <hip/hip_runtime.h>
