@@ -123,8 +123,10 @@ int kb_estep_vjp_noalloc(const kb_tree* tree, const kb_estep_vjp_io* io, void* s
  * pi_ws + w (pi_ws = input_ws, or ws); output row Pi_out row ws + w.  With
  * dts (nullable) the split term of row w joins the LSE.  store_final_pibar
  * also writes Pibar row ws + w and pibar_row_max[ws + w] from the new row;
- * pi_residual (nullable, float32 [C]) gets max |Pi_new - Pi_in| over finite
- * entries.  In-place use (Pi_in == Pi_out, Pi_out == Pibar) is allowed.
+ * pi_residual (nullable, float32 [C]) gets max |Pi_new - Pi_in| over the
+ * entries that are above -inf in both rows, NaN if one of them is NaN.  A NaN
+ * in Pi_in, dts or a leaf value makes NaN of every entry whose terms read it
+ * (the transfer sums of its row are left out).  In-place use (Pi_in == Pi_out, Pi_out == Pibar) is allowed.
  * n_sweeps > 1 runs that many sweeps in one launch with the row kept on chip
  * (bitwise equal to n_sweeps one-sweep calls chained through Pi_out; only the
  * last sweep is written, and pi_residual is the last sweep's); 0 or 1 is one.

@@ -694,14 +694,15 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
     const int lpos = has_leaf ? t.ppos[lstate] : -1;
     const T lval = has_leaf ? a.leaf_logp[(size_t)item * S + lstate] : NI;
     T* out = a.Pi_out + (size_t)grow * S;
-    // largest and (negated) smallest finite input; one that is NaN or +inf
-    // makes the range infinite
-    T hi = lval, lo = lval == NI ? NI : -lval;
+    // Largest and (negated) smallest finite input.  tmax may drop a NaN but never
+    // a +inf: a NaN is kept as +inf in lo, a +inf in hi.
+    T hi = NI, lo = NI;
     auto span = [&](T x) {
       hi = tmax(hi, x);
       lo = tmax(lo, x == NI ? NI : x == x ? -x : -NI);
     };
     auto publish_span = [&]() {
+      span(lval);
       hi = wmax63(hi);
       lo = wmax63(lo);
       if (lane == 63) {
@@ -730,8 +731,9 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
     for (int k = 0; k < CPT; ++k)
       if (own(k) >= S) pr[k] = dd[k] = NI;
     for (int sweep = 0;; ++sweep) {
-      // (hi and lo of a row without finite entries are -inf)
-      if (!cbad && (hi == NI || hi + lo <= R)) {
+      // (-inf of a row of -inf; +inf or NaN, which fail the test, of a row with a
+      // NaN or +inf)
+      if (!cbad && hi + lo <= R) {
         // an integer reference: Pi - Ms and the exponent of the result are exact,
         // and the result is rounded once
         const T Ms = xceil(msafe(hi));
@@ -812,18 +814,20 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
       }
       if (a.resid && sweep + 1 >= a.n_sweeps) {
         T ldiff = T(0);
+        bool nan = false;
 #pragma unroll
         for (int k = 0; k < CPT; ++k)
           if (res[k] != NI && pr[k] != NI) {
             const T df = res[k] - pr[k];
-            ldiff = tmax(ldiff, df < T(0) ? -df : df);
+            nan = nan || df != df;
+            ldiff = df == df ? tmax(ldiff, df < T(0) ? -df : df) : ldiff;
           }
         ldiff = wg_max(ldiff);
+        if (__syncthreads_or(nan)) ldiff = __builtin_nanf("");
         if (tid == 0) a.resid[grow] = (float)ldiff;
       }
       if (!CHAINS || sweep + 1 >= a.n_sweeps) break;
-      hi = lval;
-      lo = lval == NI ? NI : -lval;
+      hi = lo = NI;
 #pragma unroll
       for (int k = 0; k < CPT; ++k) {
         pr[k] = res[k];

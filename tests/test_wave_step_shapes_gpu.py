@@ -123,3 +123,41 @@ def test_float64_chain_is_bitwise_its_single_sweeps(leaves, monkeypatch):
     chain = _device_sweep(case, torch.float64, True, sweeps=3)
     for a, b in zip(one[:3], chain[:3]):
         assert np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("leaves,kind", [(n, k) for n in (1, 32, 64, 300, 512, 700, 1024, 1501)
+                                         for k in ("float32", "float64")])
+def test_nan_rows_stay_nan(leaves, kind):
+    """A NaN entry reaches every entry that reads it, whatever else the row holds (the pattern of the oracle)."""
+    dt, tdt = (np.float32, torch.float32) if kind == "float32" else (np.float64, torch.float64)
+    for weighted, leaf, nan_dts in ((False, False, False), (False, False, True), (True, False, True),
+                                    (False, True, False)):
+        if leaves == 1 and weighted:
+            continue
+        tree, h, S, Pi, dts, c, col, items, leaf_state, consts = _case(leaves, dt, weighted, False, leaf)
+        Pi[0] = np.nan
+        Pi[1] = -np.inf
+        Pi[1, S // 3] = np.nan
+        Pi[2] = -20.0
+        Pi[2, S - 1] = np.nan
+        dts[1] = dts[3] = -np.inf
+        if nan_dts:
+            dts[0] = np.nan
+            dts[3, S // 2] = np.nan
+        if leaf:  # a NaN leaf value, a finite one in a NaN row, and one beside a NaN
+            consts.leaf_logp[items[5], leaf_state[5]] = c["leaf"][items[5], leaf_state[5]] = np.nan
+        case = (tree, h, S, Pi, dts, c, col, items, leaf_state, consts)
+        print(f"[nan] S={S} {kind} weighted={weighted} leaf={leaf} nan_dts={nan_dts}", flush=True)
+        out, pibar, _, resid = _device_sweep(case, tdt, weighted)
+        with np.errstate(all="ignore"):
+            ref = O.wave_sweep(Pi, items, consts, O.Tree.from_helpers(h), leaf_state=leaf_state,
+                               dts_r=None if leaf else dts)
+        assert np.isnan(ref[0]).all() and np.isnan(ref[1]).any() and not np.isnan(ref[4]).any()
+        assert np.array_equal(np.isnan(out), np.isnan(ref)), "NaN"
+        assert np.array_equal(np.isneginf(out), np.isneginf(ref)), "-inf"
+        nan_row = np.isnan(ref).any(axis=1)
+        assert np.isneginf(pibar[nan_row]).all(), "Pibar of a NaN row"
+        # a NaN difference (of entries that are both above -inf) makes the residual NaN
+        f = ~np.isneginf(ref) & ~np.isneginf(Pi)
+        want = np.isnan(np.where(f, ref - np.where(f, Pi, 0.0), 0.0)).any(axis=1)
+        assert np.array_equal(np.isnan(resid.cpu().numpy()), want), "residual"
