@@ -478,9 +478,12 @@ struct WsArgs {
 // A sweep is evaluated in linear space relative to the row's largest entry,
 // 2^-M y' = a x + emc (rowsum - ps) + k1 x[c1] + k2 x[c2] + (leaf + dts) 2^-M,
 // so an entry takes one exponential per input and one logarithm instead of
-// seven and two.  Rows (or constants) whose finite values span more than R
-// binary orders, and non-finite ones, are evaluated term by term in log space,
-// where nothing underflows: both forms in one kernel, chosen per row.
+// seven and two.  The smallest product that a sum may consist of is the row's
+// smallest entry times the smallest constant (for the transfer term, times the
+// smallest weight): a row is swept in linear space where that lies at most RANGE
+// binary orders below its largest entry, a few above the smallest normal number.
+// Any other row, and one with a NaN or +inf, is evaluated term by term in log
+// space, where nothing underflows: both forms in one kernel, chosen per row.
 //
 // A workgroup walks its rows with the position tables and the linear constants
 // in registers (formed again when the item changes) and the next row's loads
@@ -514,7 +517,8 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
   constexpr int MAXS = BT * CPT, BW = BT / 64, ZERO = MAXS, SEG = 64 * CPT, LD = MAXS + 64;
   constexpr int NONE = 0xffff;
   constexpr bool CHAINS = !std::is_same_v<T, float>;  // (float chains: wave_step_lin_kernel)
-  constexpr T R = std::is_same_v<T, float> ? T(60) : T(400);
+  constexpr T RANGE = std::is_same_v<T, float> ? T(120) : T(1000);
+  constexpr T HIGH = std::is_same_v<T, float> ? T(60) : T(400);  // the largest constant (log2)
   extern __shared__ __align__(16) unsigned char smraw[];
   T* X = reinterpret_cast<T*>(smraw);  // the row's values at preorder positions; [ZERO] stays 0
   T* Q = X + LD;                       // the split term, then the postorder scan
@@ -547,25 +551,37 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
     X[MAXS + tid] = T(0);
     Q[MAXS + tid] = T(0);
   }
+  // the largest value over the workgroup (two barriers)
+  auto wg_max = [&](T x) {
+    x = wmax63(x);
+    __syncthreads();
+    if (lane == 63) wA[wv] = x;
+    __syncthreads();
+    return wmax_first<BW>(wA, lane);
+  };
+  // Binary orders by which a factor 2^lg may lower what it multiplies, at least
+  // 0; +inf if it is NaN or larger than HIGH.
+  auto depth = [&](T lg) { return lg == NI ? T(0) : lg <= HIGH ? tmax(-lg, T(0)) : -NI; };
   T cw[WEIGHTED ? CPT : 1], cwq[WEIGHTED ? CPT : 1];
-  bool out_of_range = false;
-  auto ranged = [&](T x) { out_of_range = out_of_range || !((x >= -R && x <= R) || x == NI); };
+  T wdepth = T(0), whigh = T(0);  // of the weights: the largest depth, the largest log2 above 0
   if constexpr (WEIGHTED) {
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       cw[k] = cwq[k] = T(0);
       if (own(k) < S) {
         const T c = a.col[t.pcol[own(k)]];
-        ranged(c);
+        wdepth = tmax(wdepth, depth(c));
+        whigh = tmax(whigh, c);
         cw[k] = xexp2(c);
         cwq[k] = xexp2(a.col[t.pcol[cq[k] >> 16]]);
       }
     }
+    wdepth = wg_max(wdepth);
+    whigh = wg_max(tmax(whigh, T(0)));
   }
-  const bool col_out = out_of_range;
   T kr[4][KC ? 1 : CPT];
-  auto load_consts = [&](size_t cb) {  // -> a constant is out of range
-    out_of_range = col_out;
+  auto load_consts = [&](size_t cb) {  // -> the largest depth of the products of constants
+    T deep = wdepth;
     T ca[CPT], ce[CPT], ck1[CPT], ck2[CPT];
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
@@ -575,18 +591,18 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
         const T dl = a.DL[ci], eb = a.Ebar[ci], em = a.E[ci] + a.mt[ci];
         ca[k] = xexp2(dl) + xexp2(eb);
         ce[k] = xexp2(em);
-        ranged(dl);
-        ranged(eb);
-        ranged(em);
+        // (of the sum dl and eb the larger one counts; dl > eb fails for a NaN)
+        deep = tmax(deep, dl != dl ? -NI : depth(dl > eb ? dl : eb));
+        deep = tmax(deep, em + whigh <= HIGH ? depth(em) + (em == NI ? T(0) : wdepth) : -NI);
         if (t.pc1[own(k)] >= 0) {
           const T s1 = a.SL1[ci];
           ck1[k] = xexp2(s1);
-          ranged(s1);
+          deep = tmax(deep, depth(s1));
         }
         if ((cq[k] & 0xffff) != ZERO) {
           const T s2 = a.SL2[ci];
           ck2[k] = xexp2(s2);
-          ranged(s2);
+          deep = tmax(deep, depth(s2));
         }
       }
     }
@@ -604,7 +620,7 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
         kr[3][k] = ck2[k];
       }
     }
-    return __syncthreads_or(out_of_range) != 0;
+    return wg_max(deep);
   };
   auto konst = [&](int j, T (&v)[CPT]) {
     if constexpr (KC) {
@@ -660,16 +676,8 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
       ps[k] = (sp[k] + offp) - (Q[n] + (BW > 1 ? shfl_of(eq, n / SEG) : T(0)));
     }
   };
-  // the largest value over the workgroup (two barriers)
-  auto wg_max = [&](T x) {
-    x = wmax63(x);
-    __syncthreads();
-    if (lane == 63) wA[wv] = x;
-    __syncthreads();
-    return wmax_first<BW>(wA, lane);
-  };
   long long citem = -1;
-  bool cbad = false;
+  T deep = T(0);
   for (int w = blockIdx.x; w < a.W; w += gridDim.x) {
     // (opaque in every row: the LDS addresses formed from the packed tables
     // would otherwise be kept in registers through the loop)
@@ -678,7 +686,7 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
     const long long grow = a.ws + w;
     const long long item = a.item[grow];
     const size_t cb = (size_t)(item * a.cstride);
-    if (citem < 0 || (a.cstride != 0 && item != citem)) cbad = load_consts(cb);
+    if (citem < 0 || (a.cstride != 0 && item != citem)) deep = load_consts(cb);
     citem = item;
     const T* in = a.Pi_in + (size_t)(a.pi_ws + w) * S;
     const T* dt = a.dts ? a.dts + (size_t)w * S : nullptr;
@@ -731,9 +739,9 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
     for (int k = 0; k < CPT; ++k)
       if (own(k) >= S) pr[k] = dd[k] = NI;
     for (int sweep = 0;; ++sweep) {
-      // (-inf of a row of -inf; +inf or NaN, which fail the test, of a row with a
-      // NaN or +inf)
-      if (!cbad && hi + lo <= R) {
+      // (-inf for a row of -inf; +inf or NaN, which fail the test, for a row or
+      // constants with a NaN or +inf)
+      if (hi + lo + deep <= RANGE) {
         // an integer reference: Pi - Ms and the exponent of the result are exact,
         // and the result is rounded once
         const T Ms = xceil(msafe(hi));

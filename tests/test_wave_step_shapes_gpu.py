@@ -1,9 +1,9 @@
 """``compute_wave_step`` at the edges of its launch shapes and of its two row forms, against the oracle.
 
-A row (with its constants) whose finite values span at most 60 binary orders (float32; 400 in
-float64) is swept in linear space, any other term by term in log space.  Rows of both kinds,
-rows with -inf entries, a single finite entry or none, and two items whose constants alternate
-over the rows share one launch.
+A row whose span times its smallest constant (and weight) covers at most 120 binary orders
+(float32; 1000 in float64) is swept in linear space, any other term by term in log space.  Rows of
+both kinds, rows with -inf entries, a single finite entry or none, and two items whose constants
+alternate over the rows share one launch.
 """
 
 import numpy as np
@@ -161,3 +161,68 @@ def test_nan_rows_stay_nan(leaves, kind):
         f = ~np.isneginf(ref) & ~np.isneginf(Pi)
         want = np.isnan(np.where(f, ref - np.where(f, Pi, 0.0), 0.0)).any(axis=1)
         assert np.array_equal(np.isnan(resid.cpu().numpy()), want), "residual"
+
+
+@pytest.mark.parametrize("leaves,kind", [(n, k) for n in (2, 64, 65, 300, 600, 1024, 1501)
+                                         for k in ("float32", "float64")])
+def test_products_below_the_linear_range(leaves, kind):
+    """Entries that only a product below the smallest normal number decides: compared in log2, where a
+    flush to 0 shows as -inf.  Rows 0 and 1: one column of small weight and small Pi feeds the transfer
+    term of all others, and the split term sets the row's largest entry (three factors, each of which
+    alone would fit; two without weights).  Row 2: Pi over twice the format's range of exponents and no
+    transfer.  Rows 3 and 4: small DL, Ebar, SL1 and SL2 times a small Pi.  Row 5: the products of row 0
+    where the linear range just holds them."""
+    dt, tdt = (np.float32, torch.float32) if kind == "float32" else (np.float64, torch.float64)
+    f32 = dt == np.float32
+    rng = np.random.default_rng(leaves)
+    from kbench import synth
+
+    tree = synth.yule_tree(leaves, rng)
+    h = synth.state_helpers_from_tree(tree)
+    S, root = tree.S, tree.root
+    rnd = lambda a: np.asarray(a).astype(dt).astype(np.float64)
+    col_low, em_low, pi_low = (-50.0, -50.0, -55.0) if f32 else (-390.0, -390.0, -390.0)
+    for weighted in (False, True):
+        c = {k: rng.uniform(-4.0, -0.5, (2, S)) for k in ("DL", "Ebar", "E", "SL1", "SL2", "leaf", "mt")}
+        c["E"][:] = em_low
+        Pi, dts = np.full((W, S), -np.inf), np.full((W, S), -np.inf)
+        col = np.full(S, -np.log2(S))
+        feed = 0  # a leaf: no column but itself has it among its ancestors
+        if weighted:
+            col[:] = -3.0
+            col[feed] = col_low
+        else:
+            c["E"][:] = 2.0 * em_low
+        c["mt"][:] = 0.0
+        Pi[0, feed], dts[0, root] = -5.0 + pi_low, -5.0
+        Pi[1, feed], dts[1, root] = -300.0 + pi_low, -300.0
+        Pi[5, feed], dts[5, root] = -5.0, -5.0 - (3.0 if f32 else 200.0)
+        # rows 2 to 4 are of items without transfers
+        c["E"][0] = -np.inf
+        items = np.array([1, 1, 0, 0, 0, 1])
+        reach = 250.0 if f32 else 2100.0
+        Pi[2] = -10.0 - np.linspace(0.0, reach, S)[rng.permutation(S)]
+        Pi[3:5] = -20.0
+        low = rng.permutation(S)[: max(1, S // 3)]
+        Pi[3:5, low] = -20.0 - (70.0 if f32 else 600.0)
+        for k, name in enumerate(("DL", "Ebar")):
+            c[name][0, low] = -80.0 - k if f32 else -700.0 - k
+        inner = np.nonzero(np.asarray(h["node_child1"]) < S)[0][: max(1, leaves // 3)]
+        for name in ("SL1", "SL2"):
+            c[name][0, inner] = -85.0 if f32 else -710.0
+        c, Pi, dts, col = {k: rnd(v) for k, v in c.items()}, rnd(Pi), rnd(dts), rnd(col)
+        consts = O.WaveConsts(mt=c["mt"], DL=c["DL"], Ebar=c["Ebar"], E=c["E"], SL1=c["SL1"], SL2=c["SL2"],
+                              leaf_logp=c["leaf"], col=col, use_col_weights=weighted)
+        case = (tree, h, S, Pi, dts, c, col, items, None, consts)
+        print(f"[small] S={S} {kind} weighted={weighted}", flush=True)
+        out, _, _, _ = _device_sweep(case, tdt, weighted)
+        with np.errstate(all="ignore"):
+            ref = O.wave_sweep(Pi, items, consts, O.Tree.from_helpers(h), dts_r=dts)
+        if S > 3:
+            assert np.isfinite(ref[:2]).sum() >= S  # (the test holds what it says it does)
+        eps = np.finfo(dt).eps
+        assert np.array_equal(np.isneginf(out), np.isneginf(ref)), (weighted, "entries of probability 0")
+        f = np.isfinite(ref)
+        # a log2 value carries a few roundings of its own size and of its inputs'
+        tol = 4.0 * eps * (np.abs(ref[f]) + np.abs(Pi[np.isfinite(Pi)]).max()) + 16.0 * eps
+        assert (np.abs(out[f] - ref[f]) <= tol).all(), (weighted, np.abs(out[f] - ref[f]).max())
