@@ -536,13 +536,15 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
   // row).  Child1 of i is i + 1.
   unsigned cq[CPT], np[CPT];
   auto load_tables = [&]() {
+    int c2[CPT], q[CPT], nex[CPT];
+    kb::gld_own<CPT>(t.pc2, S, c2, -1);
+    kb::gld_own<CPT>(t.ppost, S, q, ZERO);
+    kb::gld_own<CPT>(t.pnex, S, nex, 0);
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
-      const int i = kb::own_pos_c<BT, CPT>(k);
-      const int c2 = i < S ? t.pc2[i] : -1, q = i < S ? t.ppost[i] : ZERO;
-      cq[k] = (unsigned)(c2 >= 0 ? c2 : ZERO) | ((unsigned)q << 16);
+      cq[k] = (unsigned)(c2[k] >= 0 ? c2[k] : ZERO) | ((unsigned)q[k] << 16);
       const int sc = tid + k * BT;
-      np[k] = (unsigned)(i < S ? t.pnex[i] : 0) | ((unsigned)(sc < S ? t.ppos[sc] : NONE) << 16);
+      np[k] = (unsigned)nex[k] | ((unsigned)(sc < S ? t.ppos[sc] : NONE) << 16);
     }
   };
   load_tables();
@@ -766,59 +768,61 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
           res[k] = z > T(0) ? flog2(mantissa(z)) + (Ms + (T)exponent(z)) : NI;
         }
       } else {
-        // term by term in log space: values 2^(col + Pi - M) in Q, Pi in X, the
-        // path sums by following the parents; the results go straight to the
-        // output row and are read back
-        T lm = NI;
+        // Term by term in log space: the others' sums from the same scans over
+        // 2^(col + Pi - M).  Then they go to Q and Pi to X in column order, so that
+        // the entries are evaluated with coalesced reads of the constants, each
+        // result in the place of its sum in Q.  Rows of this kind only, against
+        // sums by following the parents entry by entry and reads at preorder
+        // positions: 2140 rows of 2047 floats over 200 orders 226 -> 53 us, 650 of
+        // 8191 543 -> 166 us, 600 of 2047 on a tree of depth 1023 981 -> 25 us.
+        {
+          T lm = NI, x[CPT], x2[CPT], ps[CPT], tot, x1last;
 #pragma unroll
-        for (int k = 0; k < CPT; ++k)
-          if (own(k) < S) lm = tmax(lm, a.use_col ? a.col[t.pcol[own(k)]] + pr[k] : pr[k]);
-        const T M = wg_max(lm);
-        const T Mw = msafe(M);
-        T ls = T(0);
-#pragma unroll
-        for (int k = 0; k < CPT; ++k)
-          if (own(k) < S) {
-            const T xw = xexp2((a.use_col ? a.col[t.pcol[own(k)]] + pr[k] : pr[k]) - Mw);
-            X[own(k)] = pr[k];
-            Q[own(k)] = xw;
-            ls += xw;
+          for (int k = 0; k < CPT; ++k) {
+            x[k] = WEIGHTED && own(k) < S ? a.col[t.pcol[own(k)]] + pr[k] : pr[k];
+            lm = tmax(lm, x[k]);
           }
-        const T wa = lane_of(wscan(ls), 63);
-        if (lane == 63) wP[wv] = wa;
-        __syncthreads();
-        T tot = wP[0];
-#pragma unroll 1
-        for (int i = 1; i < BW; ++i) tot += wP[i];
-#pragma unroll 1
-        for (int i = tid * CPT; i < min(S, tid * CPT + CPT); ++i) {
-          const int sc = t.pcol[i];
-          const size_t ci = cb + sc;
-          T ps = T(0);
-          for (int n = sc; n >= 0; n = t.par[n]) ps += Q[t.ppos[n]];
-          const T denom = tot - ps, p = X[i];
-          const int c1 = t.pc1[i], c2 = t.pc2[i];
-          const T pibar = denom > T(0) ? xlog2(denom) + M + a.mt[ci] : NI;
-          const T t0 = a.DL[ci] + p;
-          const T t1 = p + a.Ebar[ci];
-          const T t2 = pibar + a.E[ci];
-          const T t3 = a.SL1[ci] + (c1 >= 0 ? X[c1] : NI);
-          const T t4 = a.SL2[ci] + (c2 >= 0 ? X[c2] : NI);
-          const T t5 = i == lpos ? lval : NI;
-          const T d = a.dts ? a.dts[(size_t)w * S + sc] : NI;
-          const T m = tmax(tmax(tmax(tmax(t0, t1), tmax(t2, t3)), tmax(t4, t5)), d);
-          const T ms = msafe(m);
-          const T sum = xexp2(t0 - ms) + xexp2(t1 - ms) + xexp2(t2 - ms) + xexp2(t3 - ms) + xexp2(t4 - ms) +
-                        xexp2(t5 - ms) + xexp2(d - ms);
-          out[sc] = xlog2(sum) + m;
-        }
+          const T M = wg_max(lm);
+          const T Mw = msafe(M);
 #pragma unroll
-        for (int k = 0; k < CPT; ++k) res[k] = own(k) < S ? out[t.pcol[own(k)]] : NI;
-        __syncthreads();  // X and Q are written again below
-        // tables and constants are read again, so that this branch, which few
-        // rows take, does not hold the others' registers
-        load_tables();
-        citem = -1;
+          for (int k = 0; k < CPT; ++k) x[k] = own(k) < S ? xexp2(x[k] - Mw) : T(0);
+          path_sums(std::false_type{}, std::false_type{}, x, ps, tot, x2, x1last);
+          __syncthreads();  // X and Q were read
+#pragma unroll
+          for (int k = 0; k < CPT; ++k) {
+            ps[k] = tot - ps[k];
+            if (own(k) < S) X[t.pcol[own(k)]] = pr[k];
+          }
+          own_store<CPT>(Q, ps);
+          __syncthreads();
+#pragma unroll 1
+          for (int sc = tid; sc < S; sc += BT) {
+            const size_t ci = cb + sc;
+            const int i = t.ppos[sc], c1 = t.c1[sc], c2 = t.c2[sc];
+            const T denom = Q[i], p = X[sc];
+            const T d = a.dts ? a.dts[(size_t)w * S + sc] : NI;
+            const T pibar = denom > T(0) ? xlog2(denom) + M + a.mt[ci] : NI;
+            const T t0 = a.DL[ci] + p;
+            const T t1 = p + a.Ebar[ci];
+            const T t2 = pibar + a.E[ci];
+            const T t3 = a.SL1[ci] + (c1 >= 0 ? X[c1] : NI);
+            const T t4 = a.SL2[ci] + (c2 >= 0 ? X[c2] : NI);
+            const T t5 = i == lpos ? lval : NI;
+            const T m = tmax(tmax(tmax(tmax(t0, t1), tmax(t2, t3)), tmax(t4, t5)), d);
+            const T ms = msafe(m);
+            T sum = xexp2(t0 - ms) + xexp2(t1 - ms) + xexp2(t2 - ms) + xexp2(t3 - ms) + xexp2(t4 - ms) + xexp2(t5 - ms);
+            if (a.dts) sum += xexp2(d - ms);
+            Q[i] = xlog2(sum) + m;
+          }
+          __syncthreads();
+          own_load<CPT>(Q, res);
+#pragma unroll
+          for (int k = 0; k < CPT; ++k)
+            if (own(k) >= S) res[k] = NI;
+        }
+        // (where registers are short the tables are read again, so that this branch
+        // does not hold them)
+        if constexpr (step_min_waves<T>(CPT) > 1 || CPT == 8) load_tables();
       }
       if (a.resid && sweep + 1 >= a.n_sweeps) {
         T ldiff = T(0);

@@ -226,3 +226,56 @@ def test_products_below_the_linear_range(leaves, kind):
         # a log2 value carries a few roundings of its own size and of its inputs'
         tol = 4.0 * eps * (np.abs(ref[f]) + np.abs(Pi[np.isfinite(Pi)]).max()) + 16.0 * eps
         assert (np.abs(out[f] - ref[f]) <= tol).all(), (weighted, np.abs(out[f] - ref[f]).max())
+
+
+def test_wide_rows_of_a_deep_tree():
+    """Rows swept in log space on a tree of depth 1023: the oracle's values, at a few times the cost of rows
+    swept in linear space (walking to the root from every entry took 50 times as long)."""
+    from kbench import synth
+    from kbench.core.kernels import wave_step
+
+    L, rows = 1024, 600
+    S = 2 * L - 1
+    parent, c1, c2 = np.full(S, -1, np.int64), np.full(S, S, np.int64), np.full(S, S, np.int64)
+    for j in range(L - 1):  # internal node L + j: leaf j + 1 and the internal node below (the lowest: two leaves)
+        c1[L + j], c2[L + j] = (0, 1) if j == 0 else (j + 1, L + j - 1)
+        parent[c1[L + j]] = parent[c2[L + j]] = L + j
+    tree = synth._finish_tree(synth.SpeciesTree(L, parent, c1, c2, np.zeros(S)))
+    h = synth.state_helpers_from_tree(tree)
+    assert h["max_ancestor_depth"] == L
+    rng = np.random.default_rng(5)
+    f32 = lambda a: np.asarray(a, np.float32).astype(np.float64)
+    c = {k: f32(rng.uniform(-4.0, -0.5, (1, S))) for k in ("DL", "Ebar", "E", "SL1", "SL2", "leaf", "mt")}
+    col = f32(np.full(S, -np.log2(S)))
+    consts = O.WaveConsts(mt=c["mt"], DL=c["DL"], Ebar=c["Ebar"], E=c["E"], SL1=c["SL1"], SL2=c["SL2"],
+                          leaf_logp=c["leaf"], col=col, use_col_weights=False)
+    t = lambda a: torch.as_tensor(np.ascontiguousarray(a), dtype=torch.float32, device="cuda")
+    ints = lambda a: torch.as_tensor(np.asarray(a), dtype=torch.int64, device="cuda")
+    dev = [t(c[k]) for k in ("mt", "DL", "Ebar", "E", "SL1", "SL2")]
+    topo = [ints(h[k]) for k in ("node_child1", "node_child2", "node_parent")]
+    rest = dict(leaf_state_idx=ints(np.zeros(rows)), leaf_logp=t(c["leaf"]), item_idx=ints(np.zeros(rows)),
+                pibar_row_max=t(np.zeros(rows)), store_final_pibar=False, has_leaf_term=False, use_col_weights=False)
+    took = {}
+    for span in (30.0, 200.0):
+        Pi = f32(-10.0 - rng.uniform(0.0, span, (rows, S)))
+        src, out, colt = t(Pi), t(np.zeros((rows, S))), t(col)
+        sweep = lambda: wave_step.compute_wave_step(src, out, out, 0, rows, S, *dev, colt, *topo, L, None, **rest)
+        sweep()
+        times = []
+        for _ in range(7):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            sweep()
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        took[span] = float(np.median(times))
+        with np.errstate(all="ignore"):
+            ref = O.wave_sweep(Pi, np.zeros(rows, np.int64), consts, O.Tree.from_helpers(h))
+        eps = np.finfo(np.float32).eps
+        unit = np.exp2((c["E"] + c["mt"])[0]) * np.exp2(Pi).sum(axis=1, keepdims=True)  # the transfer term's noise
+        y, y_ref = np.exp2(out.cpu().numpy().astype(np.float64)), np.exp2(ref)
+        size = 4.0 * eps * np.abs(Pi).max() + 16.0 * eps
+        assert (np.abs(y - y_ref) <= size * y_ref + eps * (8.0 + 2.0 * np.sqrt(S)) * unit).all(), span
+    print(f"[deep tree] {took}", flush=True)
+    assert took[200.0] <= 8.0 * took[30.0]
