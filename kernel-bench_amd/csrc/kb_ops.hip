@@ -159,8 +159,10 @@ __device__ void estep_row_log(const OpsTree& t, const EsArgs<T>& a, size_t base,
 //   e' = 2^pS e[c1] e[c2] + 2^pD e^2 + e 2^mt (rowsum - ps) + 2^pL,
 // path sums from an inclusive preorder and an exclusive postorder register
 // scan, two barriers per step, and no exponential or logarithm inside the
-// iteration.  Rows with a parameter or start outside [-400, 400] (log2), which
-// products of float64 might not hold, are evaluated in log space.
+// iteration.  Rows with a parameter or start outside [-400, 200] (log2) are
+// evaluated in log space: a step multiplies up to four of these values, and what
+// falls below the smallest double vanishes next to 2^pL.  A row whose iterates
+// outgrow float64 (which then stay infinite or NaN) starts again there.
 // Bound by one row's latency (two barriers and two scans a step).  100 rows of
 // 1023 states: 16 iterations and one step 290 -> 39 us (against a 1024-thread
 // workgroup summing by tree levels, with eight transcendentals an entry and
@@ -178,9 +180,9 @@ __global__ __launch_bounds__(BT) void estep_kernel(OpsTree t, EsArgs<T> a) {
   const size_t base = (size_t)blockIdx.x * S;
   const double NI = -__builtin_inf();
   int colk[CPT], c2p[CPT], nex[CPT], qp[CPT];
-  bool h1[CPT], ranged = true;
+  bool h1[CPT], linear = true;
   double e[CPT], kS[CPT], kD[CPT], kL[CPT], kM[CPT], w[WEIGHTED ? CPT : 1], wq[WEIGHTED ? CPT : 1];
-  auto in_range = [&](double x) { ranged = ranged && x >= -400.0 && x <= 400.0; };
+  auto in_range = [&](double x) { linear = linear && x >= -400.0 && x <= 200.0; };
 #pragma unroll
   for (int k = 0; k < CPT; ++k) {
     const int i = tid * CPT + k;
@@ -218,15 +220,12 @@ __global__ __launch_bounds__(BT) void estep_kernel(OpsTree t, EsArgs<T> a) {
     }
   }
   if (tid < 64) X[MAXS + tid] = Q[MAXS + tid] = 0.0;
-  if (!__syncthreads_and(ranged)) {
-    estep_row_log<T, BT, CPT>(t, a, base, X, Q, red);
-    return;
-  }
+  linear = __syncthreads_and(linear);
   const double hi = exp2(a.tol), lo = exp2(-a.tol);
   bool ok = true;  // the last update moved the own positions by less than tol
   double e1[CPT], e2[CPT], ps[CPT], tot = 0.0;
   int it = 0;
-  for (;;) {
+  if (linear) for (;;) {
     double sp[CPT], ta = 0.0;
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
@@ -310,6 +309,16 @@ __global__ __launch_bounds__(BT) void estep_kernel(OpsTree t, EsArgs<T> a) {
         e[k] = en;
       }
     ++it;
+  }
+  if (linear) {
+    bool finite = tot < __builtin_inf();
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) finite = finite && e[k] < __builtin_inf();
+    linear = __syncthreads_and(finite);
+  }
+  if (!linear) {
+    estep_row_log<T, BT, CPT>(t, a, base, X, Q, red);
+    return;
   }
 #pragma unroll
   for (int k = 0; k < CPT; ++k)

@@ -1,6 +1,6 @@
 """The per-call E step, its fixed point and its VJP at the edges of their launch shapes, against the oracle.
 
-Item rows whose parameters all lie in [-400, 400] (log2) run in linear float64, any other row in
+Item rows whose parameters all lie in [-400, 200] (log2) run in linear float64, any other row in
 log space: one row of each launch has a probability of 0 and one a rate of 2^-600.
 """
 
@@ -71,3 +71,45 @@ def test_e_step_rows_match_oracle(leaves, weighted):
     grads = torch.autograd.grad(out, leaves_, grad_outputs=[t(c) for c in cot])
     for name, a, b in zip(("E", "pS", "pD", "pL", "mt", "col"), grads, ref_g):
         assert np.abs(a.cpu().numpy() - b).max() <= 1e-10 * max(1.0, np.abs(b).max()), name
+
+
+@pytest.mark.parametrize("leaves", [2, 64, 300, 1024, 2049])
+def test_large_values_stay_finite(leaves):
+    """Steps whose products pass 2^1024 (unnormalised rates), and a fixed point that grows past it: log space."""
+    from kbench import synth
+    from kbench.core.kernels.e_step import e_fixed_point_triton, e_step_triton_autograd
+
+    rng = np.random.default_rng(leaves)
+    h = synth.state_helpers_from_tree(synth.yule_tree(leaves, rng))
+    S, G = 2 * leaves - 1, 3
+    otree = O.Tree.from_helpers(h)
+    t = lambda a: torch.as_tensor(np.ascontiguousarray(a), dtype=torch.float64, device="cuda")
+    topo = [torch.as_tensor(np.asarray(h[k])).cuda() for k in ("node_parent", "node_child1", "node_child2")]
+    topo.append(int(h["max_ancestor_depth"]))
+    print(f"[large e] S={S}", flush=True)
+    for weighted in (False, True):
+        col = rng.uniform(190.0, 199.0, S) if weighted else np.full(S, -np.log2(S))
+        E, pS, pD, pL, mt = (rng.uniform(-3.0, -1.0, (G, S)) for _ in range(5))
+        E[1], pS[1], pD[1], mt[1] = (rng.uniform(340.0, 399.0, S) for _ in range(4))
+        E[2] = 199.0
+        mt[2] = pD[2] = 190.0
+        out = e_step_triton_autograd(*(t(x) for x in (E, pS, pD, pL, mt, col)), *topo, use_col_weights=weighted)
+        with np.errstate(all="ignore"):
+            ref = O.e_step(E, pS, pD, pL, mt, col, otree, weighted)
+        for a, b in zip(out, ref):
+            a = a.cpu().numpy()
+            assert np.array_equal(np.isfinite(a), np.isfinite(b))
+            f = np.isfinite(b)
+            assert np.abs(a[f] - b[f]).max(initial=0.0) <= 1e-10 * max(1.0, np.abs(b[f]).max(initial=0.0))
+        # no transfers to speak of and every other rate 1: the exponents double with every step
+        one = np.zeros((G, S))
+        got = e_fixed_point_triton(t(one + 150.0), *(t(one + x) for x in (0.0, 0.0, 0.0, -390.0)), t(col), *topo,
+                                   max_iter=3, tol=1e-8, use_col_weights=weighted)
+        with np.errstate(all="ignore"):
+            want = O.e_fixed_point(one + 150.0, one, one, one, one - 390.0, col, otree, weighted, 3, 1e-8)
+        assert np.isfinite(want[0]).all() and want[0].max() > 1100.0
+        for a, b in zip(got, want):
+            a = a.cpu().numpy()
+            assert np.array_equal(np.isfinite(a), np.isfinite(b))
+            f = np.isfinite(b)
+            assert np.abs(a[f] - b[f]).max(initial=0.0) <= 1e-9 * np.abs(b[f]).max(initial=1.0)
