@@ -61,7 +61,7 @@ int kb_ops_max_states(int dtype);
  *         iterate from E until max_s |E_new - E| < tol (each item row stops on
  *         its own) or max_iter steps; E_out is the last iterate and
  *         E_s1/E_s2/Ebar are evaluated at it.  n_iter [G] (nullable, int32).
- * Arithmetic is float64 whatever `dtype`.
+ * Arithmetic is float64 whatever `dtype`.  E_out may be E.
  */
 typedef struct kb_estep_io {
   int32_t dtype, G, mode, use_col_weights, max_iter;

@@ -120,7 +120,7 @@ __device__ void estep_row_log(const OpsTree& t, const EsArgs<T>& a, size_t base,
       a.Es1[base + s] = (T)child(t.c1[s]);
       a.Es2[base + s] = (T)child(t.c2[s]);
       a.Ebar[base + s] = (T)ebar_of(s);
-      const T d = en - a.E[base + s];
+      const T d = en - (T)Ev[s];  // (E may have been E_out)
       ld = fmax(ld, (double)(d < T(0) ? -d : d));
     }
     const double md = wg_max_of<BT>(ld, red);
@@ -276,19 +276,30 @@ __global__ __launch_bounds__(BT) void estep_kernel(OpsTree t, EsArgs<T> a) {
     if (stop) break;
     if (a.mode == 0) {
       double ld = 0.0;
+      T E0[CPT], E1[CPT], E2[CPT];  // all of E is read before any of E_out, which may be E, is written
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) {
+        E0[k] = E1[k] = E2[k] = (T)NI;
+        if (colk[k] >= 0) {
+          const int c1 = t.c1[colk[k]], c2 = t.c2[colk[k]];
+          E0[k] = a.E[base + colk[k]];
+          if (c1 >= 0) E1[k] = a.E[base + c1];
+          if (c2 >= 0) E2[k] = a.E[base + c2];
+        }
+      }
+      __syncthreads();
 #pragma unroll
       for (int k = 0; k < CPT; ++k)
         if (colk[k] >= 0) {
           const size_t o = base + colk[k];
           const double na = tot - ps[k];
           const double en = kS[k] * e1[k] * e2[k] + kD[k] * e[k] * e[k] + (na > 0.0 ? e[k] * kM[k] * na : 0.0) + kL[k];
-          const T En = (T)log2(en), Eo = a.E[o];
+          const T En = (T)log2(en);
           a.E_out[o] = En;
           a.Ebar[o] = (T)(na > 0.0 ? log2(na) + (double)a.mt[o] : NI);
-          const int c1 = t.c1[colk[k]], c2 = t.c2[colk[k]];
-          a.Es1[o] = c1 >= 0 ? a.E[base + c1] : (T)NI;
-          a.Es2[o] = c2 >= 0 ? a.E[base + c2] : (T)NI;
-          const T d = En - Eo;
+          a.Es1[o] = E1[k];
+          a.Es2[o] = E2[k];
+          const T d = En - E0[k];
           ld = fmax(ld, (double)(d < T(0) ? -d : d));
         }
       if (a.max_diff) {

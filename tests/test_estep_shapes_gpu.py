@@ -113,3 +113,37 @@ def test_large_values_stay_finite(leaves):
             assert np.array_equal(np.isfinite(a), np.isfinite(b))
             f = np.isfinite(b)
             assert np.abs(a[f] - b[f]).max(initial=0.0) <= 1e-9 * np.abs(b[f]).max(initial=1.0)
+
+
+@pytest.mark.parametrize("leaves", [2, 65, 300, 1024, 2049])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_e_out_may_be_e(leaves, mode):
+    """The entry point called in place gives the bits of a call with a row block of its own, in both forms."""
+    from kbench import synth
+    from kbench.core.kernels import _hip as H
+
+    rng = np.random.default_rng(leaves)
+    h = synth.state_helpers_from_tree(synth.yule_tree(leaves, rng))
+    S, G = 2 * leaves - 1, 3
+    print(f"[in place] S={S} mode={mode}", flush=True)
+    tree = H.tree_from_parent(*(torch.as_tensor(np.asarray(h[k])).cuda()
+                                for k in ("node_parent", "node_child1", "node_child2")))
+    t = lambda a: torch.as_tensor(np.ascontiguousarray(a), dtype=torch.float32, device="cuda")
+    par = [rng.uniform(-5.0, -2.0, (G, S)) for _ in range(3)] + [rng.uniform(-16.0, -12.0, (G, S))]
+    par[1][1] = -np.inf  # a row in log space
+    par, col = [t(x) for x in par], t(np.full(S, -np.log2(S)))
+    E = t(rng.uniform(-3.0, -1.0, (G, S)))
+    res = []
+    for in_place in (False, True):
+        src = E.clone()
+        outs = [src if in_place else torch.empty_like(E)] + [torch.empty_like(E) for _ in range(3)]
+        diff = torch.full((G,), -7.0, device="cuda")
+        io = H.KbEStepIO(dtype=H.KB_F32, G=G, mode=mode, use_col_weights=0, max_iter=20, tol=1e-6, E=H.ptr(src),
+                         log_pS=H.ptr(par[0]), log_pD=H.ptr(par[1]), log_pL=H.ptr(par[2]), max_coupling=H.ptr(par[3]),
+                         col_log_probs=H.ptr(col), E_out=H.ptr(outs[0]), E_s1=H.ptr(outs[1]), E_s2=H.ptr(outs[2]),
+                         Ebar=H.ptr(outs[3]), max_diff=H.ptr(diff), n_iter=None)
+        H.check(H.lib().kb_estep(tree.handle, io, H.stream(E.device)))
+        torch.cuda.synchronize()
+        res.append([x.cpu() for x in outs] + [diff.cpu()])
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
