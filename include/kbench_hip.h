@@ -48,8 +48,8 @@ typedef struct kb_layout {
   const int64_t* node_parent;        /* [S], -1 at the root */
   const int64_t* node_child1;        /* [S], >= S: none */
   const int64_t* node_child2;        /* [S] */
-  const int64_t* node_subtree_start; /* [S] preorder index */
-  const int64_t* node_subtree_end;   /* [S] preorder index + subtree size */
+  const int64_t* node_subtree_start; /* [S] preorder index (not read: the plan makes its own preorder) */
+  const int64_t* node_subtree_end;   /* [S] preorder index + subtree size (not read) */
   const float* unnorm_row_max;       /* [S] */
   const int64_t* leaf_state_index;   /* [C], -1 for non-leaf rows */
   const int64_t* rate_item_idx;      /* [C] */

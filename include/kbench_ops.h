@@ -38,8 +38,8 @@ extern "C" {
 #define KB_F64 1
 
 /*
- * Species-tree tables for the per-wrapper kernels (preorder, Euler tour, depth
- * levels), built from the reference's state_helpers arrays (host pointers):
+ * Species-tree tables for the per-wrapper kernels (preorder, Euler tour), built
+ * from the reference's state_helpers arrays (host pointers):
  * node_parent [S] (-1 at the root), node_child1/2 [S] (a value outside [0, S)
  * means "no child").  Replaces the per-launch ancestor chase bounded by
  * max_ancestor_depth and the compact_level_* tables (pristine

@@ -66,7 +66,7 @@ int alloc(T** dst, size_t n) {
 
 struct kb_plan {
   int S = 0, C = 0, n_fam = 0, n_waves = 0;
-  int n_jump = 0, n_blevels = 0;
+  int n_jump = 0, n_blevels = 0;  // of the tree (kb_plan_info): pointer-jump rounds, bottom-up levels
   std::vector<int> wave_start, wave_size, wave_split;
   // dependency levels: rows grouped by clade-DAG depth (0 = no splits); a row
   // only reads its own children, so level order is a valid schedule
@@ -101,12 +101,8 @@ struct kb_plan {
   int* d_cls_rows = nullptr;
   int* d_row_kind = nullptr;  // 1: row of a leaf wave (leaf initialisation), 0: split row
   // device tables
-  int* d_parent = nullptr; int* d_c1 = nullptr; int* d_c2 = nullptr; int* d_jump = nullptr;
-  int* d_blevel_ptr = nullptr; int* d_blevel_node = nullptr;
-  int* d_sub_start = nullptr; int* d_sub_end = nullptr;
-  int* d_item = nullptr; int* d_leaf = nullptr; int* d_roots = nullptr;
+  int* d_leaf = nullptr; int* d_roots = nullptr;
   int* d_split_ptr = nullptr; int* d_split_l = nullptr; int* d_split_r = nullptr; float* d_split_lsp = nullptr;
-  int* d_split_parent = nullptr;
   int* d_child_ptr = nullptr; int* d_child_in = nullptr;
   int* d_bslot = nullptr;  // [KB_BREC * C] the backward's record of every schedule slot
   float* d_unnorm = nullptr;
@@ -120,8 +116,7 @@ struct kb_plan {
   int* d_pflag = nullptr; int* d_endpos = nullptr; int* d_tin = nullptr; int* d_euler = nullptr;
   int* d_post = nullptr;
   int* d_om_tab = nullptr;  // owner-major position tables of the large backward kernel (2048 < S <= 8192)
-  double* E64 = nullptr; int* n_e_iter = nullptr; double* loss_terms = nullptr; double* loss64 = nullptr;
-  int* d_root_index = nullptr;
+  int* n_e_iter = nullptr; double* loss_terms = nullptr; double* loss64 = nullptr;
   int64_t n_splits = 0;
   // backward work (allocated on first use)
   float* b_staging = nullptr; unsigned char* b_split_on = nullptr; unsigned char* b_mask = nullptr;
@@ -137,7 +132,6 @@ struct kb_plan {
   float* b_Ebar = nullptr; float* b_E = nullptr; float* b_mt = nullptr; float* b_col = nullptr;
   int b_nb_max = 0, b_n_partials = 0, b_variant = 0, b_large = 1;
   size_t b_slot = 0;  // floats per workgroup slot of b_contrib
-  std::vector<int> b_poff;
   // kb_solve: rows of the families whose root lies at a level <= overlap_cut
   // come first in their level's backward schedule (n_early of them); those of
   // levels overlap_low .. overlap_cut are solved on a second stream while the
@@ -167,22 +161,6 @@ struct kb_plan {
     t.tin = d_tin;
     t.euler = d_euler;
     t.post = d_post;
-    return t;
-  }
-
-  kb::TreeDev tree() const {
-    kb::TreeDev t;
-    t.S = S;
-    t.n_jump = n_jump;
-    t.n_blevels = n_blevels;
-    t.parent = d_parent;
-    t.c1 = d_c1;
-    t.c2 = d_c2;
-    t.jump = d_jump;
-    t.blevel_ptr = d_blevel_ptr;
-    t.blevel_node = d_blevel_node;
-    t.sub_start = d_sub_start;
-    t.sub_end = d_sub_end;
     return t;
   }
 };
@@ -219,15 +197,13 @@ int kb_plan_create(const kb_layout* L, kb_plan** out) {
   p->n_waves = L->n_waves;
 
   // ---- species tree
-  std::vector<int> parent(S), c1(S), c2(S), depth(S, -1), ss(S), se(S);
+  std::vector<int> parent(S), c1(S), c2(S), depth(S, -1);
   for (int s = 0; s < S; ++s) {
     int64_t pa = L->node_parent[s];
     parent[s] = (pa >= 0 && pa < S) ? (int)pa : -1;
     int64_t a = L->node_child1[s], b = L->node_child2[s];
     c1[s] = (a >= 0 && a < S) ? (int)a : -1;
     c2[s] = (b >= 0 && b < S) ? (int)b : -1;
-    ss[s] = (int)L->node_subtree_start[s];
-    se[s] = (int)L->node_subtree_end[s];
   }
   // depth by walking to the root (bounded: a cycle is a layout error)
   int max_chain = 1;
@@ -245,25 +221,11 @@ int kb_plan_create(const kb_layout* L, kb_plan** out) {
   }
   int n_jump = 0;
   while ((1 << n_jump) < max_chain) ++n_jump;
-  std::vector<int> jump((size_t)std::max(n_jump, 1) * S, -1);
-  for (int s = 0; s < S; ++s) jump[s] = parent[s];
-  for (int t = 1; t < n_jump; ++t)
-    for (int s = 0; s < S; ++s) {
-      int a = jump[(size_t)(t - 1) * S + s];
-      jump[(size_t)t * S + s] = a >= 0 ? jump[(size_t)(t - 1) * S + a] : -1;
-    }
   int maxd = 0;
   for (int s = 0; s < S; ++s) maxd = std::max(maxd, depth[s]);
-  std::vector<int> bptr(1, 0), bnode;
-  for (int d = maxd; d >= 0; --d) {
-    bool any = false;
-    for (int s = 0; s < S; ++s)
-      if (depth[s] == d && (c1[s] >= 0 || c2[s] >= 0)) {
-        bnode.push_back(s);
-        any = true;
-      }
-    if (any) bptr.push_back((int)bnode.size());
-  }
+  std::vector<char> has_internal(maxd + 1, 0);  // depth levels with an internal node
+  for (int s = 0; s < S; ++s)
+    if (c1[s] >= 0 || c2[s] >= 0) has_internal[depth[s]] = 1;
   // preorder (child1 first) and its Euler tour
   std::vector<int> pre(S, -1), pcol(S), c1pos(S), c2pos(S), ppos(S), pflag(S, 0), endpos(S), tin(S), euler;
   {
@@ -325,7 +287,7 @@ int kb_plan_create(const kb_layout* L, kb_plan** out) {
     }
   }
   p->n_jump = n_jump;
-  p->n_blevels = (int)bptr.size() - 1;
+  p->n_blevels = (int)std::count(has_internal.begin(), has_internal.end(), 1);
 
   // ---- rows, splits, waves (int64 values range-checked before narrowing)
   std::vector<int> item(C), leaf(C), roots(L->n_fam);
@@ -395,7 +357,7 @@ int kb_plan_create(const kb_layout* L, kb_plan** out) {
   }
   for (int r = 0; r < C; ++r) cnt[r + 1] += cnt[r];
   std::vector<int> sptr(cnt), fill(cnt.begin(), cnt.end() - 1);
-  std::vector<int> sl(NS), sr(NS), spar(NS);
+  std::vector<int> sl(NS), sr(NS);
   std::vector<float> slsp(NS);
   for (int64_t i = 0; i < NS; ++i) {  // stable: keeps the layout's split order per parent
     int pr = (int)L->split_parent[i];
@@ -403,7 +365,6 @@ int kb_plan_create(const kb_layout* L, kb_plan** out) {
     sl[pos] = (int)L->split_left[i];
     sr[pos] = (int)L->split_right[i];
     slsp[pos] = (float)L->split_log_prob[i];
-    spar[pos] = pr;
   }
   // child -> incoming (split, side) CSR in increasing split order: fixed gather order
   std::vector<int> ccnt(C + 1, 0);
@@ -522,26 +483,15 @@ int kb_plan_create(const kb_layout* L, kb_plan** out) {
   p->n_chunks0 = (int)ck_ptr.size() - 1;
 
   int rc = 0;
-  rc |= upload(&p->d_parent, parent);
-  rc |= upload(&p->d_c1, c1);
-  rc |= upload(&p->d_c2, c2);
-  rc |= upload(&p->d_jump, jump);
-  rc |= upload(&p->d_blevel_ptr, bptr);
-  rc |= upload(&p->d_blevel_node, bnode);
-  rc |= upload(&p->d_sub_start, ss);
-  rc |= upload(&p->d_sub_end, se);
-  rc |= upload(&p->d_item, item);
   rc |= upload(&p->d_leaf, leaf);
   rc |= upload(&p->d_roots, roots);
   rc |= upload(&p->d_split_ptr, sptr);
   rc |= upload(&p->d_split_l, sl);
   rc |= upload(&p->d_split_r, sr);
   rc |= upload(&p->d_split_lsp, slsp);
-  rc |= upload(&p->d_split_parent, spar);
   rc |= upload(&p->d_child_ptr, ccnt);
   rc |= upload(&p->d_child_in, cin);
   rc |= upload(&p->d_unnorm, unnorm);
-  rc |= upload(&p->d_root_index, root_index);
   {
     // kb_solve's overlap (KB_OVERLAP_CUT = c): every row of a family whose
     // root lies at level <= c moves to the front of its level's backward
@@ -745,19 +695,14 @@ int kb_plan_create(const kb_layout* L, kb_plan** out) {
   rc |= alloc(&p->lin_emc, S);
   rc |= alloc(&p->lin_k1, S);
   rc |= alloc(&p->lin_k2, S);
-  rc |= alloc(&p->E64, S);
   rc |= alloc(&p->n_e_iter, 1);
   rc |= alloc(&p->loss_terms, std::max(1, L->n_fam));
   rc |= alloc(&p->loss64, 1);
-  for (void* ptr : {(void*)p->d_parent, (void*)p->d_c1, (void*)p->d_c2, (void*)p->d_jump, (void*)p->d_blevel_ptr,
-                    (void*)p->d_blevel_node, (void*)p->d_sub_start,
-                    (void*)p->d_sub_end, (void*)p->d_item, (void*)p->d_leaf, (void*)p->d_roots, (void*)p->d_split_ptr,
-                    (void*)p->d_split_l, (void*)p->d_split_r, (void*)p->d_split_lsp, (void*)p->d_split_parent,
-                    (void*)p->d_child_ptr, (void*)p->d_child_in, (void*)p->d_bslot, (void*)p->d_unnorm, (void*)p->c_DL, (void*)p->c_SL1,
+  for (void* ptr : {(void*)p->d_leaf, (void*)p->d_roots, (void*)p->d_split_ptr,
+                    (void*)p->d_split_l, (void*)p->d_split_r, (void*)p->d_split_lsp, (void*)p->d_child_ptr, (void*)p->d_child_in, (void*)p->d_bslot, (void*)p->d_unnorm, (void*)p->c_DL, (void*)p->c_SL1,
                     (void*)p->c_SL2, (void*)p->c_pS, (void*)p->c_pD, (void*)p->c_colw, (void*)p->lin_a,
-                    (void*)p->lin_emc, (void*)p->lin_k1, (void*)p->lin_k2, (void*)p->E64, (void*)p->n_e_iter,
-                    (void*)p->loss_terms, (void*)p->loss64, (void*)p->d_root_index,
-                    (void*)p->d_sched_rows, (void*)p->d_row_kind, (void*)p->d_pre, (void*)p->d_pcol,
+                    (void*)p->lin_emc, (void*)p->lin_k1, (void*)p->lin_k2, (void*)p->n_e_iter,
+                    (void*)p->loss_terms, (void*)p->loss64, (void*)p->d_sched_rows, (void*)p->d_row_kind, (void*)p->d_pre, (void*)p->d_pcol,
                     (void*)p->d_fsched, (void*)p->d_fsplit_l, (void*)p->d_fsplit_r, (void*)p->d_dup_ptr,
                     (void*)p->d_dup_rows, (void*)p->d_cls_ptr, (void*)p->d_cls_rows, (void*)p->d_ck_ptr, (void*)p->d_cls_ck_ptr, (void*)p->d_rep_of, (void*)p->d_m_side_ptr, (void*)p->d_m_side, (void*)p->d_m_root,
                     (void*)p->d_dts,
@@ -799,7 +744,6 @@ static int forward_setup(kb_plan* p, const kb_forward_io* io, hipStream_t st, kb
   const int S = p->S;
 
   kb::EStepParams E{};
-  E.tr = p->tree();
   E.pd = p->predev();
   E.S = S;
   E.theta = io->theta;
@@ -819,7 +763,6 @@ static int forward_setup(kb_plan* p, const kb_forward_io* io, hipStream_t st, kb
   E.log_pL = io->log_pL;
   E.mt = io->max_coupling;
   E.col_log_probs = io->col_log_probs;
-  E.E64 = p->E64;
   E.n_iter_out = p->n_e_iter;
   E.c_DL = p->c_DL;
   E.c_SL1 = p->c_SL1;
@@ -831,7 +774,6 @@ static int forward_setup(kb_plan* p, const kb_forward_io* io, hipStream_t st, kb
   E.c_E = p->c_E;
   E.c_mt = p->c_mt;
   E.c_col = p->c_col;
-  E.pre = p->d_pre;
   E.lin_a = p->lin_a;
   E.lin_emc = p->lin_emc;
   E.lin_k1 = p->lin_k1;
@@ -840,7 +782,6 @@ static int forward_setup(kb_plan* p, const kb_forward_io* io, hipStream_t st, kb
   KB_HIP(hipGetLastError());
 
   F = kb::FwdParams{};
-  F.tr = p->tree();
   F.S = S;
   F.n_sweeps = io->pi_iters - 1;
   F.use_col = io->use_col_weights;
@@ -1070,7 +1011,6 @@ static int backward_setup(kb_plan* p, const kb_backward_io* io, hipStream_t st, 
   kb::launch_bwd_consts(K, st);
 
   B = kb::BwdParams{};
-  B.tr = p->tree();
   B.S = S;
   B.n_terms = io->neumann_terms;
   B.rtol = (float)io->neumann_rtol;
@@ -1092,7 +1032,6 @@ static int backward_setup(kb_plan* p, const kb_backward_io* io, hipStream_t st, 
   B.pibar = io->pibar;
   B.rowmax = io->pibar_row_max;
   B.leaf_state = p->d_leaf;
-  B.root_index = p->d_root_index;
   B.split_ptr = p->d_split_ptr;
   B.split_l = p->d_split_l;
   B.split_r = p->d_split_r;
@@ -1156,7 +1095,6 @@ static int backward_finish(kb_plan* p, const kb_backward_io* io, const kb::BwdPa
     KB_HIP(hipMemcpyAsync(io->acc_out, p->b_acc, (size_t)8 * S * sizeof(double), hipMemcpyDeviceToDevice, st));
 
   kb::EpiParams X{};
-  X.tr = p->tree();
   X.pd = p->predev();
   X.S = S;
   X.E = io->E;
@@ -1263,7 +1201,6 @@ int kb_e_adjoint(kb_plan* p, const kb_e_adjoint_io* io, void* stream) {
   if (!(io->bicgstab_tol > 0.0)) return set_error(KB_ERR_ARG, "tol must be positive");
   if (!(io->bicgstab_breakdown_tol > 0.0)) return set_error(KB_ERR_ARG, "breakdown_tol must be positive");
   kb::EpiParams X{};
-  X.tr = p->tree();
   X.pd = p->predev();
   X.S = p->S;
   X.E = io->E;

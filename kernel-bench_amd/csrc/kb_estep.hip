@@ -273,7 +273,6 @@ __global__ __launch_bounds__(NT) void estep_pre_kernel(EStepParams P) {
     P.E_s1[s] = (float)Es1;
     P.E_s2[s] = (float)Es2;
     P.Ebar[s] = (float)Ebar;
-    if (P.E64) P.E64[s] = E;
     P.mt[s] = (float)mt[k];
     P.col_log_probs[s] = (float)cl[k];
     if (P.statewise) {

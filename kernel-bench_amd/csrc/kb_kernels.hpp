@@ -15,10 +15,8 @@ int set_error(int code, const char* fmt, ...);
 // parameters + E-step (kb_estep.hip)
 // ----------------------------------------------------------------------------
 struct EStepParams {
-  TreeDev tr;
-  PreDev pd;                  // preorder tables
+  PreDev pd;                  // preorder tables (also the layout of the c_* / lin_* constants)
   int S;
-  const int* pre;             // [S] column -> preorder position (layout of the c_* / lin_* constants)
   const float* theta;         // [S,3] (statewise) or [3]
   int statewise;
   const float* col_weights;   // [S]
@@ -31,7 +29,6 @@ struct EStepParams {
   float* E; float* E_s1; float* E_s2; float* Ebar;
   float* log_pS; float* log_pD; float* log_pL;   // [S] statewise, [1] global
   float* mt; float* col_log_probs;               // [S]
-  double* E64;                                    // optional float64 E
   int* n_iter_out;
   // constants of the row kernels (float32, [S], preorder positions)
   float* c_DL; float* c_SL1; float* c_SL2; float* c_pS; float* c_pD; float* c_colw;
@@ -47,7 +44,6 @@ void launch_loss(const float* pi, const int* root_rows, const float* E, int S, i
 // forward wave kernels (kb_fwd.hip)
 // ----------------------------------------------------------------------------
 struct FwdParams {
-  TreeDev tr;
   PreDev pre;
   int S;
   int wide;                   // 1: 256 x 8, 2: 1024 x 2 on every level, 3: no narrow shape
@@ -121,7 +117,6 @@ enum BrecField {
 };
 
 struct BwdParams {
-  TreeDev tr;
   PreDev pre;
   int S;
   int n_terms;                // neumann_terms
@@ -135,7 +130,7 @@ struct BwdParams {
   const float* mt; const float* col;
   const float* pD; const float* pS;  // [S] split-term rates (pS is also the leaf term's log pS)
   const float* pi; const float* pibar; const float* rowmax;
-  const int* leaf_state; const int* root_index;
+  const int* leaf_state;
   const int* split_ptr; const int* split_l; const int* split_r; const float* split_lsp;
   const int* child_ptr; const int* child_in;
   const int* bslot;           // [KB_BREC * C] record of every schedule slot (BrecField)
@@ -195,7 +190,6 @@ __host__ __device__ inline int kb_slot_ld(int S, int large) {
 }
 
 struct EpiParams {
-  TreeDev tr;
   PreDev pd;                  // preorder tables
   int S;
   const float* E; const float* log_pS; const float* log_pD; const float* log_pL; const float* mt;

@@ -2514,8 +2514,8 @@ int kb_tree_create(int32_t S, const int64_t* parent, const int64_t* child1, cons
     if (par[s] >= 0 && c1[par[s]] != s && c2[par[s]] != s)
       return kb::set_error(KB_ERR_ARG, "node %d is not a child of its parent %d", s, par[s]);
   }
-  // preorder DFS (child1 first), Euler tour, depths
-  std::vector<int> pcol, ppos(S, -1), pend(S, 0), tin(S, 0), ev, depth(S, 0);
+  // preorder DFS (child1 first), Euler tour
+  std::vector<int> pcol, ppos(S, -1), pend(S, 0), tin(S, 0), ev;
   pcol.reserve(S);
   ev.reserve(2 * S);
   std::vector<std::pair<int, int>> stack;  // (node, state) 0: enter, 1: exit
@@ -2530,14 +2530,8 @@ int kb_tree_create(int32_t S, const int64_t* parent, const int64_t* child1, cons
       tin[n] = (int)ev.size();
       ev.push_back(n << 1);
       stack.push_back({n, 1});
-      if (c2[n] >= 0) {
-        depth[c2[n]] = depth[n] + 1;
-        stack.push_back({c2[n], 0});
-      }
-      if (c1[n] >= 0) {
-        depth[c1[n]] = depth[n] + 1;
-        stack.push_back({c1[n], 0});
-      }
+      if (c2[n] >= 0) stack.push_back({c2[n], 0});
+      if (c1[n] >= 0) stack.push_back({c1[n], 0});
     } else {
       pend[n] = (int)pcol.size();
       ev.push_back((n << 1) | 1);
@@ -2545,15 +2539,6 @@ int kb_tree_create(int32_t S, const int64_t* parent, const int64_t* child1, cons
   }
   if ((int)pcol.size() != S)
     return kb::set_error(KB_ERR_ARG, "species tree is not connected (%zu of %d nodes reachable)", pcol.size(), S);
-  int max_d = 0;
-  for (int s = 0; s < S; ++s) max_d = std::max(max_d, depth[s]);
-  std::vector<int> lvl_ptr(max_d + 2, 0), lvl_node(S);
-  for (int s = 0; s < S; ++s) ++lvl_ptr[depth[s] + 1];
-  for (int d = 0; d <= max_d; ++d) lvl_ptr[d + 1] += lvl_ptr[d];
-  {
-    std::vector<int> fill(lvl_ptr.begin(), lvl_ptr.end() - 1);
-    for (int s = 0; s < S; ++s) lvl_node[fill[depth[s]]++] = s;
-  }
   // preorder-position tables of the contiguous-ownership sweeps
   std::vector<int> pc1(S), pc2(S), pnex(S), ppost;
   ppost.reserve(S);
@@ -2567,7 +2552,6 @@ int kb_tree_create(int32_t S, const int64_t* parent, const int64_t* child1, cons
     if (e & 1) ppost.push_back(ppos[e >> 1]);
   kb_tree* t = new kb_tree();
   t->S = S;
-  t->n_levels = max_d + 1;
   int rc = 0;
   rc |= put(&t->par, par);
   rc |= put(&t->c1, c1);
@@ -2577,8 +2561,6 @@ int kb_tree_create(int32_t S, const int64_t* parent, const int64_t* child1, cons
   rc |= put(&t->pcol, pcol);
   rc |= put(&t->ppos, ppos);
   rc |= put(&t->pend, pend);
-  rc |= put(&t->lvl_ptr, lvl_ptr);
-  rc |= put(&t->lvl_node, lvl_node);
   rc |= put(&t->pc1, pc1);
   rc |= put(&t->pc2, pc2);
   rc |= put(&t->pnex, pnex);
@@ -2593,7 +2575,7 @@ int kb_tree_create(int32_t S, const int64_t* parent, const int64_t* child1, cons
 
 void kb_tree_destroy(kb_tree* t) {
   if (!t) return;
-  for (int* p : {t->par, t->c1, t->c2, t->ev, t->tin, t->pcol, t->ppos, t->pend, t->lvl_ptr, t->lvl_node, t->pc1,
+  for (int* p : {t->par, t->c1, t->c2, t->ev, t->tin, t->pcol, t->ppos, t->pend, t->pc1,
                  t->pc2, t->pnex, t->ppost})
     if (p) (void)hipFree(p);
   delete t;

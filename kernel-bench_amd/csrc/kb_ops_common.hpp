@@ -19,7 +19,7 @@ constexpr int NT = 1024;
 constexpr int NW = NT / 64;
 
 struct OpsTree {
-  int S, n_levels;
+  int S;
   const int* par;       // [S] parent column, -1 at the root
   const int* c1;        // [S] child columns, -1 if none
   const int* c2;
@@ -28,8 +28,6 @@ struct OpsTree {
   const int* pcol;      // [S] preorder position -> column
   const int* ppos;      // [S] column -> preorder position
   const int* pend;      // [S] column -> exclusive end of its subtree (preorder)
-  const int* lvl_ptr;   // [n_levels + 1] depth levels, root level first
-  const int* lvl_node;  // [S]
   const int* pc1;       // [S] preorder position -> position of child1, -1 if none
   const int* pc2;       // [S] preorder position -> position of child2, -1 if none
   const int* pnex;      // [S] preorder position i -> tin(column) - i, the postorder slots before entering i
@@ -143,18 +141,13 @@ __device__ void path_sums(const OpsTree& t, const T* x, T* ev2, T* ps, T* red) {
 }
 
 // Preorder prefix scan of u (column order, LDS) into pre[] (LDS, S); then
-// the sum of u over the subtree of s is pre[pend[s]-1] - pre[ppos[s]-1] and
-// over its complement pre[ppos[s]-1] + (total - pre[pend[s]-1]).
+// the sum of u over the complement of the subtree of s is
+// pre[ppos[s]-1] + (total - pre[pend[s]-1]).
 template <typename T>
 __device__ void subtree_scan(const OpsTree& t, const T* u, T* pre, T* red) {
   for (int s = threadIdx.x; s < t.S; s += NT) pre[t.ppos[s]] = u[s];
   __syncthreads();
   block_scan(pre, t.S, red);
-}
-template <typename T>
-__device__ __forceinline__ T subtree_of(const OpsTree& t, const T* pre, int s) {
-  const int p = t.ppos[s], e = t.pend[s];
-  return pre[e - 1] - (p > 0 ? pre[p - 1] : T(0));
 }
 template <typename T>
 __device__ __forceinline__ T complement_of(const OpsTree& t, const T* pre, int s, T total) {
@@ -287,13 +280,12 @@ __device__ void reg_subtree_sums(const OpsTree& t, const V (&x)[CPT], V (&sub)[C
 // =====================================================================================
 
 struct kb_tree {
-  int S = 0, n_levels = 0;
+  int S = 0;
   int *par = nullptr, *c1 = nullptr, *c2 = nullptr, *ev = nullptr, *tin = nullptr;
-  int *pcol = nullptr, *ppos = nullptr, *pend = nullptr, *lvl_ptr = nullptr, *lvl_node = nullptr;
+  int *pcol = nullptr, *ppos = nullptr, *pend = nullptr;
   int *pc1 = nullptr, *pc2 = nullptr, *pnex = nullptr, *ppost = nullptr;
   kbo::OpsTree dev() const {
-    return kbo::OpsTree{S, n_levels, par, c1, c2, ev, tin, pcol, ppos, pend, lvl_ptr, lvl_node,
-                        pc1, pc2, pnex, ppost};
+    return kbo::OpsTree{S, par, c1, c2, ev, tin, pcol, ppos, pend, pc1, pc2, pnex, ppost};
   }
 };
 

@@ -191,73 +191,6 @@ __device__ __forceinline__ float block_max1(float x, float* wtot) {
   return t;
 }
 
-// In-place inclusive scan over positions of v[k] (slot k of this lane).
-// Returns the block total.
-template <int NT, int N>
-__device__ __forceinline__ float block_scan_incl(float (&v)[N], float* wtot) {
-  constexpr int NW = NT / 64;
-  float carry = 0.0f;
-#pragma unroll
-  for (int k = 0; k < N; ++k) {
-    const float s = wave_scan_incl(v[k]);
-    v[k] = s + carry;
-    carry += lane_value(s, 63);
-  }
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) wtot[w] = carry;
-  __syncthreads();
-  float off = 0.0f, total = 0.0f;
-#pragma unroll
-  for (int i = 0; i < NW; ++i) {
-    const float t = wtot[i];
-    if (i < w) off += t;
-    total += t;
-  }
-#pragma unroll
-  for (int k = 0; k < N; ++k) v[k] += off;
-  return total;
-}
-
-// Two scans sharing one barrier (wtot holds 2*NW floats).
-template <int NT, int N>
-__device__ __forceinline__ void block_scan_incl2(float (&a)[N], float (&b)[N], float* wtot, float& ta, float& tb) {
-  constexpr int NW = NT / 64;
-  float ca = 0.0f, cb = 0.0f;
-#pragma unroll
-  for (int k = 0; k < N; ++k) {
-    const float sa = wave_scan_incl(a[k]);
-    const float sb = wave_scan_incl(b[k]);
-    a[k] = sa + ca;
-    b[k] = sb + cb;
-    ca += lane_value(sa, 63);
-    cb += lane_value(sb, 63);
-  }
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    wtot[w] = ca;
-    wtot[NW + w] = cb;
-  }
-  __syncthreads();
-  float oa = 0.0f, ob = 0.0f;
-  ta = 0.0f;
-  tb = 0.0f;
-#pragma unroll
-  for (int i = 0; i < NW; ++i) {
-    const float x = wtot[i], y = wtot[NW + i];
-    if (i < w) {
-      oa += x;
-      ob += y;
-    }
-    ta += x;
-    tb += y;
-  }
-#pragma unroll
-  for (int k = 0; k < N; ++k) {
-    a[k] += oa;
-    b[k] += ob;
-  }
-}
-
 // ---- preorder tables ---------------------------------------------------------
 
 struct PreDev {
@@ -278,12 +211,6 @@ struct PreDev {
 template <int NT, int CPT>
 __device__ __forceinline__ int own_pos(int k) {
   return (threadIdx.x >> 6) * (64 * CPT) + k * 64 + (threadIdx.x & 63);
-}
-
-// Euler event of slot j (< 2*CPT) of this thread.
-template <int NT, int CPT>
-__device__ __forceinline__ int own_event(int j) {
-  return (threadIdx.x >> 6) * (128 * CPT) + j * 64 + (threadIdx.x & 63);
 }
 
 // Per-thread copy of the preorder tables of its own positions and events.
@@ -432,30 +359,6 @@ __device__ __forceinline__ void lds_load_own(const float* lds, float (&v)[CPT]) 
   }
 }
 
-// In-place inclusive scan over positions of contiguously owned v[]; returns the
-// block total.  One barrier; callers alternate `wtot` arrays.
-template <int NT, int CPT>
-__device__ __forceinline__ float block_scan_incl_c(float (&v)[CPT], float* wtot) {
-  constexpr int NW = NT / 64;
-#pragma unroll
-  for (int k = 1; k < CPT; ++k) v[k] += v[k - 1];
-  const float tsum = v[CPT - 1];
-  const float ws = wave_scan_incl(tsum);
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 63) wtot[w] = ws;
-  __syncthreads();
-  float off = ws - tsum, total = 0.0f;
-#pragma unroll
-  for (int i = 0; i < NW; ++i) {
-    const float t = wtot[i];
-    if (i < w) off += t;
-    total += t;
-  }
-#pragma unroll
-  for (int k = 0; k < CPT; ++k) v[k] += off;
-  return total;
-}
-
 // Subtree sums with one barrier.  Before it, local_scan_publish stores the
 // wavefront-local inclusive scan of u (own positions) at L and the wavefront
 // total at wt[wavefront]; after it, subtree_terms gives for every own
@@ -496,44 +399,6 @@ __device__ __forceinline__ void subtree_terms(const float (&sc)[CPT], const floa
   for (int k = 0; k < CPT; ++k) {
     pm1[k] = k == 0 ? p0 : sc[k - 1] + woff;
     rest[k] = A - (le[k] + __shfl(wexcl, wend[k], 64));
-  }
-}
-
-// Two contiguous-ownership scans sharing one barrier (wtot holds 2*NW floats).
-template <int NT, int CPT>
-__device__ __forceinline__ void block_scan_incl2_c(float (&a)[CPT], float (&b)[CPT], float* wtot, float& ta,
-                                                   float& tb) {
-  constexpr int NW = NT / 64;
-#pragma unroll
-  for (int k = 1; k < CPT; ++k) {
-    a[k] += a[k - 1];
-    b[k] += b[k - 1];
-  }
-  const float sa = a[CPT - 1], sb = b[CPT - 1];
-  const float wa = wave_scan_incl(sa), wb = wave_scan_incl(sb);
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 63) {
-    wtot[w] = wa;
-    wtot[NW + w] = wb;
-  }
-  __syncthreads();
-  float oa = wa - sa, ob = wb - sb;
-  ta = 0.0f;
-  tb = 0.0f;
-#pragma unroll
-  for (int i = 0; i < NW; ++i) {
-    const float x = wtot[i], y = wtot[NW + i];
-    if (i < w) {
-      oa += x;
-      ob += y;
-    }
-    ta += x;
-    tb += y;
-  }
-#pragma unroll
-  for (int k = 0; k < CPT; ++k) {
-    a[k] += oa;
-    b[k] += ob;
   }
 }
 
@@ -579,21 +444,6 @@ struct OwnTablesC {
     }
   }
 };
-
-// Coalesced load of a global row (column order) into LDS at preorder
-// positions, then into v[] (own positions).  One barrier; the caller separates
-// reuse of `lds` with a barrier.  Positions >= S read `fill`.
-template <int NT, int CPT>
-__device__ __forceinline__ void load_row_pre(const PreDev& T, const float* grow, float* lds, float (&v)[CPT],
-                                             float fill) {
-  for (int s = threadIdx.x; s < T.S; s += NT) lds[T.pre[s]] = grow[s];
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < CPT; ++k) {
-    const int i = own_pos<NT, CPT>(k);
-    v[k] = i < T.S ? lds[i] : fill;
-  }
-}
 
 // Own positions -> LDS -> coalesced global row in column order.  One barrier.
 template <int NT, int CPT>
