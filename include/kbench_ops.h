@@ -316,8 +316,9 @@ int kb_rows_scatter_add(int32_t dtype, int32_t S, int64_t n, const void* src, co
 
 /*
  * dst[s] += sum over r < n of src[r * S + s] (fixed order, float64 partial
- * sums; work: ceil(n / 64) * S doubles).  Replaces atomic column reductions
- * into grad_col_log_probs (pristine wave_backward.py:700-733, 2320-2327).
+ * sums; work: ceil(n / 1024) * S doubles, used past 1024 rows, never null).
+ * Replaces atomic column reductions into grad_col_log_probs (pristine
+ * wave_backward.py:700-733, 2320-2327).
  */
 int kb_rows_sum_into(int32_t dtype, int32_t S, int64_t n, const void* src, void* dst, double* work, void* stream);
 
@@ -325,9 +326,9 @@ int kb_rows_sum_into(int32_t dtype, int32_t S, int64_t n, const void* src, void*
  * Column sums of m <= 8 row blocks in one launch (two above 1024 rows):
  * out[j * S + s] = sum over r < n of (a[j][r * S + s] + b[j][r * S + s]),
  * b (or b[j]) null for a single addend, in a fixed order with float64 partial
- * sums (work: m * ceil(n / 64) * S doubles, required for n > 64).  a and b
- * are host arrays of device pointers.  No reference kernel: it replaces the
- * glue's per-wave torch reductions of the aw tensors
+ * sums (work: m * ceil(n / 1024) * S doubles, used for n > 1024, not null for
+ * n > 64).  a and b are host arrays of device pointers.  No reference kernel:
+ * it replaces the glue's per-wave torch reductions of the aw tensors
  * (kbench/api/_implicit_grad.py:288-296, one .sum(0) per tensor).
  */
 int kb_rows_sum_multi(int32_t dtype, int32_t S, int64_t n, int32_t m, const void* const* a, const void* const* b,
@@ -337,8 +338,9 @@ int kb_rows_sum_multi(int32_t dtype, int32_t S, int64_t n, int32_t m, const void
  * Column sums of m <= 8 row blocks, each added into its own accumulator:
  * dst[j][s] += sum over r < n[j] of (a[4j][r*S+s] + ... + a[4j+k[j]-1][r*S+s])
  * with k[j] in 1..4 addends per block (each row's addends summed first, in
- * order), rows summed in a fixed order in float64 (work: m * max_j ceil(n[j] / 64)
- * * S doubles, required when a block has more than 64 rows).  The accumulators
+ * order), rows summed in a fixed order in float64 (work: m * max_j ceil(n[j] /
+ * 1024) * S doubles, used when a block has more than 1024 rows, not null when one
+ * has more than 64).  The accumulators
  * must be distinct.  n, k, a and dst are host arrays (a: 4 entries per block,
  * device pointers).  A block of one addend gives dst exactly what
  * kb_rows_sum_into gives.  No reference kernel: it replaces the per-wave

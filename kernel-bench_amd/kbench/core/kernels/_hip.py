@@ -244,8 +244,18 @@ def scatter_add_rows(dst: torch.Tensor, src: torch.Tensor, keys, *, row_stride=N
     wrote(dst)
 
 
+_SUM_CHUNK = 1024  # rows that one launch of the column sums takes
+
+
+def _sum_work(blocks, n, S, device):
+    """The float64 partial sums of column sums over ``n`` rows: one row per block and chunk past one chunk (the
+    entry points ask for a pointer below that too, and do not use it)."""
+    chunks = (n + _SUM_CHUNK - 1) // _SUM_CHUNK
+    return torch.empty((blocks * chunks * S if chunks > 1 else 1,), device=device, dtype=torch.float64)
+
+
 def rows_sum_multi(blocks) -> torch.Tensor:
-    """[m, S] column sums of up to 8 [n, S] row blocks, in row order with float64 partial sums.
+    """[m, S] column sums of up to 8 [n, S] row blocks, in a fixed order with float64 partial sums.
 
     Each entry of ``blocks`` is a tensor or a pair of tensors (summed elementwise in the
     reduction); all share n, S, dtype and device.
@@ -262,8 +272,7 @@ def rows_sum_multi(blocks) -> torch.Tensor:
         for t in (x,) if y is None else (x, y):
             _check_rows(t, n, S, first, "rows_sum_multi")
     out = torch.empty((m, S), device=first.device, dtype=first.dtype)
-    chunks = (n + 63) // 64
-    work = torch.empty((m * chunks * S if chunks > 1 else 1,), device=first.device, dtype=torch.float64)
+    work = _sum_work(m, n, S, first.device)
     a = (ct.c_void_p * m)(*[ptr(x) for x, _ in pairs])
     b = (ct.c_void_p * m)(*[ptr(y) if y is not None else None for _, y in pairs])
     check(lib().kb_rows_sum_multi(dtype_code(first.dtype), S, n, m, a, b, ptr(out), ptr(work), stream(first.device)))
@@ -271,11 +280,11 @@ def rows_sum_multi(blocks) -> torch.Tensor:
 
 
 def rows_sum_accum(blocks) -> None:
-    """dst += column sums of row blocks, all in one launch (two above 64 rows).
+    """dst += column sums of row blocks, all in one launch (two above 1024 rows).
 
     ``blocks``: up to 8 pairs (dst, addends): dst a contiguous [S] tensor (distinct
     per block), addends a [n, S] tensor or a tuple of up to 4 of them whose sum is
-    the block's rows; rows summed in order in float64, as ``sum_rows_into`` does.
+    the block's rows; rows summed in a fixed order in float64, as ``sum_rows_into`` does.
     """
     import ctypes as ct
 
@@ -297,8 +306,7 @@ def rows_sum_accum(blocks) -> None:
                 or d.numel() != S):
             raise ValueError("rows_sum_accum: every accumulator must be a contiguous tensor of S elements with the "
                              "addends' dtype and device")
-    chunks = max((x + 63) // 64 for x in n)
-    work = torch.empty((m * chunks * S if chunks > 1 else 1,), device=first.device, dtype=torch.float64)
+    work = _sum_work(m, max(n), S, first.device)
     addends = []
     for _, a in blocks:
         addends += [ptr(x) for x in a] + [None] * (4 - len(a))
@@ -319,11 +327,11 @@ def _check_rows(t, n, S, first, what):
 
 
 def sum_rows_into(dst: torch.Tensor, src: torch.Tensor) -> None:
-    """dst += src.sum(0), in row order with float64 partial sums."""
+    """dst += src.sum(0), in a fixed order with float64 partial sums."""
     n = int(src.shape[0])
     if n == 0:
         return
     S = int(src.shape[1])
-    work = torch.empty(((n + 63) // 64) * S, device=src.device, dtype=torch.float64)
+    work = _sum_work(1, n, S, src.device)
     check(lib().kb_rows_sum_into(dtype_code(src.dtype), S, n, ptr(src), ptr(dst), ptr(work), stream(src.device)))
     wrote(dst)
