@@ -162,7 +162,12 @@ struct BwdParams {
   const int* ck_ptr;          // [chunks + 1] member (cls_rows) ranges
   const int* cls_ck_ptr;      // [classes + 1] chunk ranges
   unsigned char* ck_any;      // [chunks] any member of the chunk active
+  // Up to 512 bytes the compiler loads the block ahead of its uses and spills
+  // more scalar registers: bwd_row_kernel<64, 2> 13.6 -> 14.6 us a launch, <256,
+  // 2> 17.4 -> 18.2 us.
+  int beyond_512[6];
 };
+static_assert(sizeof(BwdParams) > 512, "see beyond_512");
 
 constexpr int KB_CHUNK0 = 8;
 // Workgroup slot of bwd_row_large_kernel: KB_LARGE_SLOT_ROWS rows of
