@@ -4,14 +4,16 @@
 //
 // Design (MI355X):
 //  * one workgroup per row (item row, clade row, split or split side), the
-//    smallest whose positions hold the row (64 to 1024 threads of 2 to 8);
+//    smallest of a list of shapes (64 to 1024 threads of 1 to 8 positions, powers
+//    of two) that holds the row;
 //    global row accesses are coalesced (column t + k * threads), and the kernels
 //    that sum over the tree move the row to preorder positions in LDS, thread t
 //    owning positions t*CPT + k;
 //  * the species tree is described once by preorder positions (kb_tree);
 //    ancestors-or-self path sums are a preorder scan less a postorder scan and
 //    subtree sums differences of one preorder scan, in registers with one
-//    exchange per scan, independent of the tree depth;
+//    exchange per scan, independent of the tree depth (but for estep_row_log,
+//    which follows the parents);
 //  * the E-step kernels (O(S) work) run in float64;
 //  * no atomics: cross-row accumulations are written as rows and summed in a
 //    fixed order by kb_rows_scatter_add / kb_rows_sum_into.
@@ -276,18 +278,14 @@ __global__ __launch_bounds__(BT) void estep_kernel(OpsTree t, EsArgs<T> a) {
     if (stop) break;
     if (a.mode == 0) {
       double ld = 0.0;
-      T E0[CPT], E1[CPT], E2[CPT];  // all of E is read before any of E_out, which may be E, is written
+      // E itself for the children (X's readers have passed a barrier); all of it is
+      // read before any of E_out, which may be E, is written
+      double E0[CPT];
 #pragma unroll
-      for (int k = 0; k < CPT; ++k) {
-        E0[k] = E1[k] = E2[k] = (T)NI;
-        if (colk[k] >= 0) {
-          const int c1 = t.c1[colk[k]], c2 = t.c2[colk[k]];
-          E0[k] = a.E[base + colk[k]];
-          if (c1 >= 0) E1[k] = a.E[base + c1];
-          if (c2 >= 0) E2[k] = a.E[base + c2];
-        }
-      }
+      for (int k = 0; k < CPT; ++k) E0[k] = colk[k] >= 0 ? (double)a.E[base + colk[k]] : NI;
+      own_store<CPT>(X, E0);
       __syncthreads();
+      const double E1last = X[tid * CPT + CPT];
 #pragma unroll
       for (int k = 0; k < CPT; ++k)
         if (colk[k] >= 0) {
@@ -297,9 +295,9 @@ __global__ __launch_bounds__(BT) void estep_kernel(OpsTree t, EsArgs<T> a) {
           const T En = (T)log2(en);
           a.E_out[o] = En;
           a.Ebar[o] = (T)(na > 0.0 ? log2(na) + (double)a.mt[o] : NI);
-          a.Es1[o] = E1[k];
-          a.Es2[o] = E2[k];
-          const T d = En - E0[k];
+          a.Es1[o] = (T)(h1[k] ? (k + 1 < CPT ? E0[k + 1 < CPT ? k + 1 : k] : E1last) : NI);
+          a.Es2[o] = (T)(c2p[k] != ZERO ? X[c2p[k]] : NI);
+          const T d = En - (T)E0[k];
           ld = fmax(ld, (double)(d < T(0) ? -d : d));
         }
       if (a.max_diff) {
@@ -321,13 +319,8 @@ __global__ __launch_bounds__(BT) void estep_kernel(OpsTree t, EsArgs<T> a) {
       }
     ++it;
   }
-  if (linear) {
-    bool finite = tot < __builtin_inf();
-#pragma unroll
-    for (int k = 0; k < CPT; ++k) finite = finite && e[k] < __builtin_inf();
-    linear = __syncthreads_and(finite);
-  }
-  if (!linear) {
+  // (the total of every thread; no weight is 0, so one infinite or NaN e makes it so)
+  if (!(linear && tot < __builtin_inf())) {
     estep_row_log<T, BT, CPT>(t, a, base, X, Q, red);
     return;
   }
@@ -489,25 +482,6 @@ struct WsArgs {
   const T* leaf_logp;
 };
 
-// One sweep of rows [ws, ws + W) (float64: n_sweeps of them), one workgroup
-// per row in flight.  Threads own preorder positions: the path sums are an
-// inclusive preorder scan minus an exclusive postorder scan, both in registers
-// (two barriers), and the row passes through LDS once each way between column
-// and preorder order.
-//
-// A sweep is evaluated in linear space relative to the row's largest entry,
-// 2^-M y' = a x + emc (rowsum - ps) + k1 x[c1] + k2 x[c2] + (leaf + dts) 2^-M,
-// so an entry takes one exponential per input and one logarithm instead of
-// seven and two.  The smallest product that a sum may consist of is the row's
-// smallest entry times the smallest constant (for the transfer term, times the
-// smallest weight): a row is swept in linear space where that lies at most RANGE
-// binary orders below its largest entry, a few above the smallest normal number.
-// Any other row, and one with a NaN or +inf, is evaluated term by term in log
-// space, where nothing underflows: both forms in one kernel, chosen per row.
-//
-// A workgroup walks its rows with the position tables and the linear constants
-// in registers (formed again when the item changes) and the next row's loads
-// in flight.  Measured: see launch_wave_step.
 // hardware exponential and logarithm for float (arguments that keep clear of
 // denormals, or whose denormal results vanish next to the sums they enter)
 __device__ __forceinline__ float fexp2(float x) { return kb::exp2_hw(x); }
@@ -532,6 +506,26 @@ constexpr int step_min_waves(int cpt) { return std::is_same_v<T, float> && cpt =
 template <typename T>
 __host__ __device__ constexpr bool step_consts_in_lds(int maxs) { return 4 * maxs * (int)sizeof(T) <= 64 * 1024; }
 
+// One sweep of rows [ws, ws + W) (float64: n_sweeps of them), one workgroup
+// per row in flight.  Threads own preorder positions: the path sums are an
+// inclusive preorder scan minus an exclusive postorder scan, both in registers
+// (two barriers), and the row passes through LDS once each way between column
+// and preorder order.
+//
+// A sweep is evaluated in linear space relative to the row's largest entry,
+// 2^-M y' = a x + emc (rowsum - ps) + k1 x[c1] + k2 x[c2] + (leaf + dts) 2^-M,
+// so an entry takes one exponential per input and one logarithm instead of
+// seven and two.  The smallest product that a sum may consist of is the row's
+// smallest entry times the smallest constant (for the transfer term, times the
+// smallest weight): a row is swept in linear space where that lies at most RANGE
+// binary orders below its largest entry, a few above the smallest normal number.
+// Any other row, and one with a NaN or +inf, is evaluated term by term in log
+// space, where nothing underflows: both forms in one kernel, chosen per row.
+//
+// A workgroup walks its rows with the position tables in registers and the linear
+// constants in LDS (step_consts_in_lds; else in registers), formed again when the
+// item changes.  A row is loaded when it begins: its latency is hidden by the
+// other rows of the CU.  Measured: see launch_wave_step.
 template <typename T, int BT, int CPT, bool WEIGHTED>
 __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(OpsTree t, WsArgs<T> a) {
   constexpr int MAXS = BT * CPT, BW = BT / 64, ZERO = MAXS, SEG = 64 * CPT, LD = MAXS + 64;
@@ -2687,15 +2681,16 @@ int launch_wave_step(const kbo::OpsTree& t, const kbo::WsArgs<T>& a, int W, hipS
   }
   // The smallest shape that holds the row.  Times of the 15 sweeps and the split
   // term of a wave through the wrappers, against one 1024-thread workgroup per
-  // row with an Euler-tour scan and log-space sums: 2047 states, 2140 rows 1044 ->
-  // 514 us (512 x 4; 1024 x 2 579 us); 1023 states, 1908 rows 658 -> 279 us (512
-  // x 2; 256 x 4 314 us); 127 states, 2104 rows 567 -> 246 us (the calls' host
-  // time); 4095 states, 721 rows 644 -> 517 us; 7999 states, 652 rows 2338 ->
-  // 1711 us.  float64: 2047 states 3440 -> 1170 us (512 x 4; 1024 x 2 spills,
-  // 1470 us), 1023 states 1342 -> 590 us (256 x 4; 512 x 2 700 us), 511 states
-  // 1024 -> 335 us.  A sweep of 2140 x 2047 floats moves 53 MB (10 us at 5.3
-  // TB/s) in about 32 us: barriers and the LDS round trips of a row, with two to
-  // three rows per CU.
+  // row with an Euler-tour scan and log-space sums: 127 states, 5015 rows 1240 ->
+  // 243 us; 1023 states, 2386 rows 817 -> 325 us; 2047 states, 2140 rows 1047 ->
+  // 479 us (weighted 1057 -> 541 us); 4095 states, 721 rows 650 -> 495 us; 7999
+  // states, 515 rows 2300 -> 1480 us.  float64: 511 states, 2550 rows 1289 -> 418
+  // us, 1023 states 1667 -> 704 us, 2047 states 3434 -> 1236 us.  (Other shapes
+  // for one size: 2047 floats on 1024 x 2 an eighth slower than on 512 x 4, 1023
+  // on 256 x 4 an eighth slower than on 512 x 2; doubles of 2047 on 1024 x 2 spill,
+  // a quarter slower, of 1023 on 512 x 2 a fifth.)  A sweep of 2140 x 2047 floats
+  // moves 53 MB (10 us at 5.3 TB/s) in about 30 us: barriers and the LDS round
+  // trips of a row, with two to three rows per CU.
   const int S = t.S;
   constexpr bool F32 = std::is_same_v<T, float>;
   if (S <= 128) return launch_step<T, 64, 2>(t, a, W, st);
