@@ -128,8 +128,9 @@ int kb_estep_vjp_noalloc(const kb_tree* tree, const kb_estep_vjp_io* io, void* s
  * in Pi_in, dts or a leaf value makes NaN of every entry whose terms read it
  * (the transfer sums of its row are left out).  In-place use (Pi_in == Pi_out, Pi_out == Pibar) is allowed.
  * n_sweeps > 1 runs that many sweeps in one launch with the row kept on chip
- * (bitwise equal to n_sweeps one-sweep calls chained through Pi_out; only the
- * last sweep is written, and pi_residual is the last sweep's); 0 or 1 is one.
+ * (equal to n_sweeps one-sweep calls chained through Pi_out: bitwise for float64
+ * rows, to float32 rounding for float32 rows; only the last sweep is written, and
+ * pi_residual is the last sweep's); 0 or 1 is one.
  */
 typedef struct kb_wave_step_io {
   int32_t dtype, S, W, use_col_weights, use_leaf_index, store_final_pibar, n_sweeps;

@@ -931,7 +931,8 @@ static int ensure_backward_work(kb_plan* p, int use_col) {
   }
   const int64_t NS = p->n_splits;
   int rc = 0;
-  // (the large-row kernels keep the family roots' v behind the child sides)
+  // (the large-row kernels keep the family roots' v behind the child sides; up to
+  // 2048 states they run only with KB_BWD_LARGE=2, which may change between calls)
   const int64_t n_stage = 2 * NS + (S > 1024 && S <= 8192 ? p->n_fam : 0);
   rc |= alloc(&p->b_staging, (size_t)std::max<int64_t>(1, n_stage) * kb::kb_stage_ld(S) + kb::KB_STAGE_TAIL);
   rc |= alloc(&p->b_split_on, (size_t)std::max<int64_t>(1, NS));

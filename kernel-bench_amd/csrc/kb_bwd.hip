@@ -1158,7 +1158,8 @@ void launch_bwd_wave(const BwdParams& P, int first, int W, int nb, int poff, hip
   if (P.variant == 2) {
     // up to 1536 states: 768 threads leave registers for fetching a row ahead,
     // and no quarter of the wavefronts idle (1399 states, 22 levels: 833 -> 818
-    // us; its levels of a few hundred rows 109 -> 101 us)
+    // us; its levels of a few hundred rows 109 -> 101 us).  The like of it for
+    // 513..768, 2049..3072 and 4097..6144 states is not built.
     if (S > 1024) {
       KB_BWD_CASE(768, 2)
     }

@@ -1,4 +1,5 @@
-// Backward row kernel for species trees of 2049 to 8192 nodes.
+// Backward row kernel for species trees of 2049 to 8192 nodes (of 1025 to 8192
+// with KB_BWD_LARGE=2).
 //
 // Same per-row mathematics as bwd_row_kernel (kb_bwd.hip; reference
 // kbench/api/_implicit_grad.py:97-370 driving pristine wave_backward.py):

@@ -695,7 +695,8 @@ void launch_fwd_wave(const FwdParams& P, int first, int W, hipStream_t st) {
   // rows never take it: half or more of its wavefronts would carry padding.
   // Rows of 1025..1536 states leave a quarter or more of a 2048-position
   // workgroup idle: 768 x 2 and 384 x 4 in place of 1024 x 2 and 512 x 4
-  // (1399 states, 22 levels: 590 -> 545 us).
+  // (1399 states, 22 levels: 590 -> 545 us).  The like of them for 513..768,
+  // 2049..3072 and 4097..6144 states is not built.
   const bool three = P.wide == 0 && S > 1024;
   if (P.wide == 2 || (P.wide == 0 && S > 1024 && W < P.narrow_below)) {
     if (three) {
