@@ -1253,8 +1253,8 @@ void launch_bwd_consts(const BwdConstArgs& A, hipStream_t st) {
 // equal range of the slots each (eight loads ahead of their float64 adds), and
 // the wavefronts' sums are added in order and written in column order.  One
 // launch instead of a pass of partial sums and one over those: 8191 states, 416
-// slots 49 -> 25 us, 127 states 8.6 -> 3.8 us and a launch (whole solves 15 to 20
-// us less).
+// slots 49 -> 25 us, 127 states 8.6 -> 3.8 us and a launch (whole solves of 127 and
+// 511 states 17 to 20 us less, of 2047 within the spread).
 constexpr int RED_G = 16;
 
 __global__ __launch_bounds__(64 * RED_G) void bwd_reduce_kernel(const float* contrib, int C, int S, size_t slot_stride,

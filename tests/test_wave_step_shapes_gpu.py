@@ -3,7 +3,8 @@
 A row whose span times its smallest constant (and weight) covers at most 120 binary orders
 (float32; 1000 in float64) is swept in linear space, any other term by term in log space.  Rows of
 both kinds, rows with -inf entries, a single finite entry or none, and two items whose constants
-alternate over the rows share one launch.
+alternate over the rows share one launch.  That the switch lies where it must is the claim of
+test_products_below_the_linear_range: in the other rows a transfer term hides what underflows.
 """
 
 import numpy as np
