@@ -531,6 +531,9 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
   constexpr int MAXS = BT * CPT, BW = BT / 64, ZERO = MAXS, SEG = 64 * CPT, LD = MAXS + 64;
   constexpr int NONE = 0xffff;
   constexpr bool CHAINS = !std::is_same_v<T, float>;  // (float chains: wave_step_lin_kernel)
+  // the constants are formed only for a row whose span leaves room for them (inside
+  // the loop of a chain that would cost registers: doubles 84 -> 116 us a sweep)
+  constexpr bool LAZY = !CHAINS;
   constexpr T RANGE = std::is_same_v<T, float> ? T(120) : T(1000);
   constexpr T HIGH = std::is_same_v<T, float> ? T(60) : T(400);  // the largest constant (log2)
   extern __shared__ __align__(16) unsigned char smraw[];
@@ -596,47 +599,72 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
     whigh = wg_max(tmax(whigh, T(0)));
   }
   T kr[4][KC ? 1 : CPT];
-  auto load_consts = [&](size_t cb) {  // -> the largest depth of the products of constants
+  // The constants at cb, read in column order (coalesced) and moved to the own
+  // positions through LDS (X and Q free); returns the largest depth of their
+  // products.  Against reads at preorder positions: one item 35 -> 31 us a sweep
+  // (2140 rows of 2047 floats), another item with every row 62 -> 41 us (650 of
+  // 8191 191 -> 134 us).
+  if constexpr (KC) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      for (int i = S + tid; i < MAXS; i += BT) Kc[j * MAXS + i] = T(0);
+  }
+  auto load_consts = [&](size_t cb) {
     T deep = wdepth;
     T ca[CPT], ce[CPT], ck1[CPT], ck2[CPT];
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
+      const int sc = tid + k * BT;
       ca[k] = ce[k] = ck1[k] = ck2[k] = T(0);
-      if (own(k) < S) {
-        const size_t ci = cb + t.pcol[own(k)];
-        const T dl = a.DL[ci], eb = a.Ebar[ci], em = a.E[ci] + a.mt[ci];
+      if (sc < S) {
+        const size_t ci = cb + sc;
+        const T dl = a.DL[ci], eb = a.Ebar[ci], em = a.E[ci] + a.mt[ci], s1 = a.SL1[ci], s2 = a.SL2[ci];
         ca[k] = xexp2(dl) + xexp2(eb);
         ce[k] = xexp2(em);
         // (of the sum dl and eb the larger one counts; dl > eb fails for a NaN)
         deep = tmax(deep, dl != dl ? -NI : depth(dl > eb ? dl : eb));
         deep = tmax(deep, em + whigh <= HIGH ? depth(em) + (em == NI ? T(0) : wdepth) : -NI);
-        if (t.pc1[own(k)] >= 0) {
-          const T s1 = a.SL1[ci];
+        if (t.c1[sc] >= 0) {
           ck1[k] = xexp2(s1);
           deep = tmax(deep, depth(s1));
         }
-        if ((cq[k] & 0xffff) != ZERO) {
-          const T s2 = a.SL2[ci];
+        if (t.c2[sc] >= 0) {
           ck2[k] = xexp2(s2);
           deep = tmax(deep, depth(s2));
         }
       }
     }
-    if constexpr (KC) {
-      own_store<CPT>(Kc, ca);
-      own_store<CPT>(Kc + MAXS, ce);
-      own_store<CPT>(Kc + 2 * MAXS, ck1);
-      own_store<CPT>(Kc + 3 * MAXS, ck2);
-    } else {
+    auto put = [&](T* dst, const T (&v)[CPT]) {
 #pragma unroll
-      for (int k = 0; k < CPT; ++k) {
-        kr[0][k] = ca[k];
-        kr[1][k] = ce[k];
-        kr[2][k] = ck1[k];
-        kr[3][k] = ck2[k];
-      }
+      for (int k = 0; k < CPT; ++k)
+        if (tid + k * BT < S) dst[np[k] >> 16] = v[k];
+    };
+    if constexpr (KC) {
+      put(Kc, ca);
+      put(Kc + MAXS, ce);
+      put(Kc + 2 * MAXS, ck1);
+      put(Kc + 3 * MAXS, ck2);
+    } else {
+      auto get = [&](const T* src, T (&v)[CPT]) {
+        own_load<CPT>(src, v);
+#pragma unroll
+        for (int k = 0; k < CPT; ++k)
+          if (own(k) >= S) v[k] = T(0);
+      };
+      __syncthreads();  // the row was read from X and Q
+      put(X, ca);
+      put(Q, ce);
+      __syncthreads();
+      get(X, kr[0]);
+      get(Q, kr[1]);
+      __syncthreads();
+      put(X, ck1);
+      put(Q, ck2);
+      __syncthreads();
+      get(X, kr[2]);
+      get(Q, kr[3]);
     }
-    return wg_max(deep);
+    return wg_max(deep);  // (its barriers: Kc is written, X and Q are free)
   };
   auto konst = [&](int j, T (&v)[CPT]) {
     if constexpr (KC) {
@@ -702,8 +730,6 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
     const long long grow = a.ws + w;
     const long long item = a.item[grow];
     const size_t cb = (size_t)(item * a.cstride);
-    if (citem < 0 || (a.cstride != 0 && item != citem)) deep = load_consts(cb);
-    citem = item;
     const T* in = a.Pi_in + (size_t)(a.pi_ws + w) * S;
     const T* dt = a.dts ? a.dts + (size_t)w * S : nullptr;
     T vin[CPT], vdt[CPT];  // columns tid + j*BT
@@ -712,6 +738,10 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
       const int sc = tid + j * BT;
       vin[j] = sc < S ? kb::ldg(in, sc) : NI;
       vdt[j] = dt && sc < S ? kb::ldg(dt, sc) : NI;
+    }
+    if constexpr (!LAZY) {
+      if (citem < 0 || (a.cstride != 0 && item != citem)) deep = load_consts(cb);
+      citem = item;
     }
     const long long lstate = a.use_leaf ? a.leaf_state[grow] : -1;
     const bool has_leaf = lstate >= 0 && lstate < S;
@@ -755,9 +785,15 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
     for (int k = 0; k < CPT; ++k)
       if (own(k) >= S) pr[k] = dd[k] = NI;
     for (int sweep = 0;; ++sweep) {
+      if constexpr (LAZY) {
+        if (hi + lo <= RANGE && (citem < 0 || (a.cstride != 0 && item != citem))) {
+          deep = load_consts(cb);
+          citem = item;
+        }
+      }
       // (-inf for a row of -inf; +inf or NaN, which fail the test, for a row or
       // constants with a NaN or +inf)
-      if (hi + lo + deep <= RANGE) {
+      if (hi + lo <= RANGE && hi + lo + deep <= RANGE) {
         // an integer reference: Pi - Ms and the exponent of the result are exact,
         // and the result is rounded once
         const T Ms = xceil(msafe(hi));
@@ -787,8 +823,8 @@ __global__ __launch_bounds__(BT, step_min_waves<T>(CPT)) void wave_step_kernel(O
         // the entries are evaluated with coalesced reads of the constants, each
         // result in the place of its sum in Q.  Rows of this kind only, against
         // sums by following the parents entry by entry and reads at preorder
-        // positions: 2140 rows of 2047 floats over 200 orders 226 -> 53 us, 650 of
-        // 8191 543 -> 166 us, 600 of 2047 on a tree of depth 1023 981 -> 25 us.
+        // positions: 2140 rows of 2047 floats over 200 orders 226 -> 46 us, 650 of
+        // 8191 543 -> 115 us, 600 of 2047 on a tree of depth 1023 981 -> 20 us.
         {
           T lm = NI, x[CPT], x2[CPT], ps[CPT], tot, x1last;
 #pragma unroll
@@ -2682,14 +2718,14 @@ int launch_wave_step(const kbo::OpsTree& t, const kbo::WsArgs<T>& a, int W, hipS
   // The smallest shape that holds the row.  Times of the 15 sweeps and the split
   // term of a wave through the wrappers, against one 1024-thread workgroup per
   // row with an Euler-tour scan and log-space sums: 127 states, 5015 rows 1240 ->
-  // 243 us; 1023 states, 2386 rows 817 -> 325 us; 2047 states, 2140 rows 1047 ->
-  // 479 us (weighted 1057 -> 541 us); 4095 states, 721 rows 650 -> 495 us; 7999
-  // states, 515 rows 2300 -> 1480 us.  float64: 511 states, 2550 rows 1289 -> 418
-  // us, 1023 states 1667 -> 704 us, 2047 states 3434 -> 1236 us.  (Other shapes
+  // 243 us; 1023 states, 2386 rows 817 -> 285 us; 2047 states, 2140 rows 1047 ->
+  // 441 us (weighted 1057 -> 492 us); 4095 states, 721 rows 650 -> 364 us; 7999
+  // states, 515 rows 2300 -> 1360 us.  float64: 511 states, 2550 rows 1289 -> 403
+  // us, 1023 states 1667 -> 687 us, 2047 states 3434 -> 1220 us.  (Other shapes
   // for one size: 2047 floats on 1024 x 2 an eighth slower than on 512 x 4, 1023
   // on 256 x 4 an eighth slower than on 512 x 2; doubles of 2047 on 1024 x 2 spill,
   // a quarter slower, of 1023 on 512 x 2 a fifth.)  A sweep of 2140 x 2047 floats
-  // moves 53 MB (10 us at 5.3 TB/s) in about 30 us: barriers and the LDS round
+  // moves 53 MB (10 us at 5.3 TB/s) in about 28 us: barriers and the LDS round
   // trips of a row, with two to three rows per CU.
   const int S = t.S;
   constexpr bool F32 = std::is_same_v<T, float>;

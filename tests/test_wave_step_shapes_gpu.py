@@ -280,3 +280,64 @@ def test_wide_rows_of_a_deep_tree():
         assert (np.abs(y - y_ref) <= size * y_ref + eps * (8.0 + 2.0 * np.sqrt(S)) * unit).all(), span
     print(f"[deep tree] {took}", flush=True)
     assert took[200.0] <= 8.0 * took[30.0]
+
+
+@pytest.mark.parametrize("leaves,kind,rows", [
+    (64, "float32", 14000), (300, "float32", 4000), (512, "float32", 2600), (1024, "float32", 2000),
+    (1501, "float32", 1100), (2049, "float32", 700), (64, "float64", 14000), (300, "float64", 4000),
+    (512, "float64", 2600), (1024, "float64", 1500), (1501, "float64", 800)])
+def test_rows_do_not_depend_on_their_predecessors(leaves, kind, rows):
+    """More rows than workgroups: each walks rows of several items, with and without room for the linear
+    form, and of none but -inf.  The same rows in another order give the same bits; a sample is the oracle's."""
+    from kbench import synth
+    from kbench.core.kernels import wave_step
+
+    dt, tdt = (np.float32, torch.float32) if kind == "float32" else (np.float64, torch.float64)
+    rng = np.random.default_rng(leaves)
+    tree = synth.yule_tree(leaves, rng)
+    h = synth.state_helpers_from_tree(tree)
+    S, G = tree.S, 5
+    print(f"[predecessors] S={S} {kind} rows={rows}", flush=True)
+    rnd = lambda a: np.asarray(a).astype(dt).astype(np.float64)
+    c = {k: rnd(rng.uniform(-6.0, -0.5, (G, S))) for k in ("DL", "Ebar", "E", "SL1", "SL2", "leaf", "mt")}
+    c["DL"][4] = rnd(c["DL"][4] - (150.0 if dt == np.float32 else 1100.0))  # no row of this item is linear
+    c["Ebar"][4] = -np.inf
+    col = rnd(np.log2(rng.dirichlet(np.full(S, 50.0))))
+    g = torch.Generator(device="cuda").manual_seed(leaves)
+    Pi = -10.0 - 30.0 * torch.rand((rows, S), generator=g, device="cuda", dtype=tdt)
+    kinds = torch.randint(0, 6, (rows,), generator=g, device="cuda")
+    Pi[kinds == 4] *= 6.0 if dt == np.float32 else 50.0
+    Pi[kinds == 5] = -float("inf")
+    dts = Pi - 3.0
+    items = torch.randint(0, G, (rows,), generator=g, device="cuda")
+    t = lambda a: torch.as_tensor(np.ascontiguousarray(a), dtype=tdt, device="cuda")
+    ints = lambda a: torch.as_tensor(np.asarray(a), dtype=torch.int64, device="cuda")
+    dev, colt, leaf = [t(c[k]) for k in ("mt", "DL", "Ebar", "E", "SL1", "SL2")], t(col), t(c["leaf"])
+    topo, zero = [ints(h[k]) for k in ("node_child1", "node_child2", "node_parent")], ints(np.zeros(rows))
+
+    def sweep(order):
+        out, pibar = torch.empty_like(Pi), torch.empty_like(Pi)
+        rmax = torch.empty((rows,), dtype=tdt, device="cuda")
+        wave_step.compute_wave_step(
+            Pi[order].contiguous(), out, pibar, 0, rows, S, *dev, colt, *topo, int(h["max_ancestor_depth"]),
+            dts[order].contiguous(), leaf_state_idx=zero, leaf_logp=leaf, item_idx=items[order].contiguous(),
+            pibar_row_max=rmax, store_final_pibar=True, has_leaf_term=False, use_col_weights=True)
+        back = torch.argsort(order)
+        return out[back], pibar[back], rmax[back]
+
+    a = sweep(torch.arange(rows, device="cuda"))
+    b = sweep(torch.randperm(rows, generator=g, device="cuda"))
+    for x, y in zip(a, b):
+        assert torch.equal(x, y)
+    pick = rng.choice(rows, 40, replace=False)
+    take = lambda x: x[torch.as_tensor(pick, device="cuda")].double().cpu().numpy()
+    consts = O.WaveConsts(mt=c["mt"], DL=c["DL"], Ebar=c["Ebar"], E=c["E"], SL1=c["SL1"], SL2=c["SL2"],
+                          leaf_logp=c["leaf"], col=col, use_col_weights=True)
+    P, it = take(Pi), items.cpu().numpy()[pick]
+    with np.errstate(all="ignore"):
+        ref = O.wave_sweep(P, it, consts, O.Tree.from_helpers(h), dts_r=take(dts))
+        unit = np.exp2((c["E"] + c["mt"])[it]) * np.exp2(P + col).sum(axis=1, keepdims=True)  # the transfer's noise
+    eps = np.finfo(dt).eps
+    y, y_ref = np.exp2(take(a[0])), np.exp2(ref)
+    size = 4.0 * eps * np.abs(P[np.isfinite(P)]).max() + 16.0 * eps
+    assert (np.abs(y - y_ref) <= size * y_ref + eps * (8.0 + 2.0 * np.sqrt(S)) * unit).all()
